@@ -225,11 +225,17 @@ def _context(bf16):
     return _contexts[bf16].handle
 
 
+def _block(shape, bf16=False):
+    """A tensor that lies inside a larger allocation, as a block of the framework's own pool does."""
+    dtype, head = (torch.bfloat16 if bf16 else torch.float32), 4096
+    raw = torch.empty(head + math.prod(shape) * (2 if bf16 else 4), dtype=torch.uint8, device="cuda")
+    return raw[head:].view(dtype).view(shape)
+
+
 def _normal(shape, seed, which, scale=1.0, bf16=False):
     g = torch.Generator(device="cuda")
     g.manual_seed(seed * 16 + which)
-    t = torch.randn(shape, generator=g, device="cuda").mul_(scale)
-    return t.bfloat16() if bf16 else t
+    return _block(shape, bf16).copy_(torch.randn(shape, generator=g, device="cuda").mul_(scale))
 
 
 def _rectified(shape, seed, which, bf16):
@@ -240,10 +246,6 @@ def _rectified(shape, seed, which, bf16):
 def _gated(shape, seed, which, bf16, scale=1.0):
     """A gradient as it leaves a rectifier's backward: half of its elements zero."""
     return _normal(shape, seed, which, scale, bf16).mul_(_normal(shape, seed, which + 1) > 0)
-
-
-def _empty(shape, bf16=False):
-    return torch.empty(shape, dtype=torch.bfloat16 if bf16 else torch.float32, device="cuda")
 
 
 def _conv_sizes(case):
@@ -263,10 +265,10 @@ def _prepare_conv(case, seed):
     s["workspace"] = torch.empty(need, dtype=torch.uint8, device="cuda") if need else None
     s["ws"] = (s["workspace"].data_ptr() if need else None, need)
     if case["pass"] == "fwd":
-        s["b"], s["y"] = _normal(ys[1], seed, 2), _empty(ys, bf16)
+        s["b"], s["y"] = _normal((ys[1],), seed, 2), _block(ys, bf16)
     else:
         s["dy"] = _gated(ys, seed, 2, bf16)
-        s["dx"], s["dw"], s["db"] = _empty(xs, bf16), _empty(ws), _empty(ys[1])
+        s["dx"], s["dw"], s["db"] = _block(xs, bf16), _block(ws), _block((ys[1],))
     return s
 
 
@@ -299,8 +301,8 @@ def _prepare_block(case, seed):
     s = {"kind": "block", "lrn": case["lrn"], "ctx": _context(bf16), "dims": xs, "count": math.prod(xs),
          "g": be.shape(*xs, 0, case["window"], case["window"], 0, 0, 2, 2), "x": _normal(xs, seed, 0, 1.5, bf16), "dy": _normal(ys, seed, 1, 1.0, bf16)}
     for name in ("a", "da", "dx") + (("u", "du") if case["lrn"] else ()):
-        s[name] = _empty(xs, bf16)
-    s["y"] = _empty(ys, bf16)
+        s[name] = _block(xs, bf16)
+    s["y"] = _block(ys, bf16)
     return s
 
 
@@ -332,7 +334,7 @@ def _work_block(case):
 def _prepare_fc(case, seed):
     n, ci, co, bf16 = case["n"], case["c_in"], case["c_out"], case["bf16"]
     return {"kind": "fc", "ctx": _context(bf16), "dims": (n, ci, co), "x": _rectified((n, ci), seed, 0, bf16), "w": _normal((co, ci), seed, 1, math.sqrt(2.0 / ci)),
-            "b": _normal((co,), seed, 2), "dy": _gated((n, co), seed, 3, bf16, 1.0 / n), "y": _empty((n, co), bf16), "dx": _empty((n, ci), bf16)}
+            "b": _normal((co,), seed, 2), "dy": _gated((n, co), seed, 3, bf16, 1.0 / n), "y": _block((n, co), bf16), "dx": _block((n, ci), bf16)}
 
 
 def _run_fc(s):
