@@ -392,3 +392,35 @@ def test_conv_bf16_tensors_at_odd_element_offsets(ctx):
         assert_close_bf16(got_y, oracle.conv_fwd(og, x, wr, b), "fwd")
         assert_close_bf16(got_gx, oracle.conv_bwd_data(og, dy, wr), "bwd data")
         assert_close(gw.download(w.shape), oracle.conv_bwd_filter_sgd(og, x, dy, np.zeros_like(w), 1.0), 1e-4, "bwd filter")
+
+
+def test_pixel_pair_loads_stay_inside_the_tensors(ctx):
+    """A pair of neighbouring pixels is one 32-bit load. Beside the first image row of a tensor such a pair lies before the
+    tensor's first element, which need not be mapped: tensors of their own (device allocations of 11 MB, each at the start
+    of a mapping) must give the bits that the same tensors give inside the context's pool. 5x5 window, padding 2, even
+    rows: forward, backward data and backward filter all fetch pairs here."""
+    torch = pytest.importorskip("torch")
+    n, c, hw, k, r = 150, 64, 24, 64, 5
+    g = be.shape(n, c, hw, hw, k, r, r, 2, 2, 1, 1)
+    rng = np.random.default_rng(17)
+    x, dy = rnd(rng, (n, c, hw, hw)), rnd(rng, (n, k, hw, hw))
+    w = (rng.standard_normal((k, c, r, r)) * 0.05).astype(np.float32)
+    announce("pixel pairs, tensors of their own")
+    with Dev(ctx) as d:
+        dx_, ddy, dw_ = d.act(x), d.act(dy), d.f32(w)
+        y, dx, dw = d.empty_act(dy.shape), d.empty_act(x.shape), d.raw(w.nbytes)
+        check(lib.vdnn_conv_fwd(ctx.handle, None, g, 0, dx_.ptr, dw_.ptr, None, y.ptr, None, 0))
+        check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, ddy.ptr, dw_.ptr, dx.ptr, None, 0))
+        check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, dx_.ptr, ddy.ptr, dw.ptr, None, 0))
+        want = [y.download(dy.shape, np.uint16), dx.download(x.shape, np.uint16), dw.download(w.shape)]
+    up = lambda a: torch.from_numpy(to_bf16_bits(a).view(np.int16)).cuda()
+    tx, tdy, tw = up(x), up(dy), torch.from_numpy(w).cuda()
+    ty, tdx, tdw = torch.empty_like(tdy), torch.empty_like(tx), torch.empty_like(tw)
+    torch.cuda.synchronize()
+    check(lib.vdnn_conv_fwd(ctx.handle, None, g, 0, tx.data_ptr(), tw.data_ptr(), None, ty.data_ptr(), None, 0))
+    check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, tdy.data_ptr(), tw.data_ptr(), tdx.data_ptr(), None, 0))
+    check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, tx.data_ptr(), tdy.data_ptr(), tdw.data_ptr(), None, 0))
+    ctx.synchronize()
+    got = [ty.cpu().numpy().view(np.uint16), tdx.cpu().numpy().view(np.uint16), tdw.cpu().numpy()]
+    for a, b in zip(got, want):
+        assert np.array_equal(a, b)

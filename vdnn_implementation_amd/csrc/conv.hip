@@ -1273,7 +1273,7 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
                 }
 #define VDNN_WGRAD_TAP_H(NTAP)                                                                                              \
                 do {                                                                                                        \
-                    if (g.sw == 1) {                                                                                        \
+                    if (g.sw == 1 && g.W >= 2) {                                                                                      \
                         LoadIm2colRedTapH<NTAP, true> bl{x, g.N, g.C, g.H, g.W, g.R, g.S, g.P, g.Q, g.ph, g.pw, g.sh, g.sw, N, dh.kchunk, dh.K, dC, dS}; \
                         rch = narrow ? launch_igemm<64, 256, LoadDyRedIncH, LoadIm2colRedTapH<NTAP, true>, StoreFilterTap, true>(ctx, st, kBwdFilterHalfNames.t64, al, bl, ept, dh) \
                                      : launch_igemm<128, 128, LoadDyRedIncH, LoadIm2colRedTapH<NTAP, true>, StoreFilterTap, true>(ctx, st, kBwdFilterHalfNames.t128, al, bl, ept, dh); \

@@ -408,8 +408,7 @@ struct LoadIm2colRedTapH {
     template <int T>
     __device__ __forceinline__ void load(State<T>& st, int, int, int, Regs<T>& r) const {
         int base0[NTAP], base1[NTAP];
-        unsigned keep[NTAP]; // PAIR32: which halves of the loaded word lie inside the image
-        int down[NTAP];      // PAIR32: 16 when the word was fetched one element lower
+        unsigned take[NTAP]; // PAIR32: v_perm_b32 selector of the two elements from the loaded word (0x0c: a zero byte)
 #pragma unroll
         for (int g = 0; g < NTAP; g++) {
             const int ih = g == 0 ? st.ih : st.ih + st.dih[g], iw = g == 0 ? st.iw : st.iw + st.diw[g];
@@ -417,17 +416,17 @@ struct LoadIm2colRedTapH {
             const bool row_ok = (unsigned)ih < (unsigned)H;
             const bool ok0 = (unsigned)iw < (unsigned)W, ok1 = (unsigned)(iw + sw) < (unsigned)W;
             if (PAIR32) {
-                // A pair whose second pixel reads past the right edge is fetched one element lower and shifted
-                // down afterwards: its first element may be the last one of the descriptor's range, and a
-                // 32-bit load that crosses the end of the range returns zero.
-                base0[g] = (ok1 ? o : o - 2) | (row_ok ? 0 : SENT);
+                // Only elements of the tensor are read (see LoadIm2colPixTapH2): a pair whose second pixel reads past the
+                // right edge is fetched one element lower (its first element may be the last one of the descriptor's
+                // range, and a 32-bit load that crosses the end of the range returns zero), a pair whose first pixel
+                // reads left of the image one element higher, a pair with neither inside not at all.
+                base0[g] = (ok0 ? (ok1 ? o : o - 2) : o + 2) | ((row_ok & (ok0 | ok1)) ? 0 : SENT);
                 base1[g] = 0;
-                down[g] = ok1 ? 0 : 16;
-                keep[g] = (ok0 ? 0x0000FFFFu : 0u) | (ok1 ? 0xFFFF0000u : 0u);
+                take[g] = ok0 ? (ok1 ? 0x03020100u : 0x0c0c0302u) : 0x01000c0cu;
             } else {
                 base0[g] = o | ((row_ok & ok0) ? 0 : SENT);
                 base1[g] = (o + sw * 2) | ((row_ok & ok1) ? 0 : SENT);
-                keep[g] = 0; down[g] = 0;
+                take[g] = 0;
             }
         }
         constexpr int PERG = T / 16 / NTAP;
@@ -437,7 +436,7 @@ struct LoadIm2colRedTapH {
             if (PAIR32) {
                 // the pair is two neighbouring elements of an input row: one load (two-byte alignment suffices)
                 const unsigned word = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(st.rsrc, base0[i / PERG], (i % PERG) * plane16, 0);
-                r.s[i] = __builtin_amdgcn_alignbit(0u, word, (unsigned)down[i / PERG]) & keep[i / PERG];
+                r.s[i] = __builtin_amdgcn_perm(0u, word, take[i / PERG]);
             } else {
                 const unsigned lo = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(st.rsrc, base0[i / PERG], (i % PERG) * plane16, 0);
                 const unsigned hi = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(st.rsrc, base1[i / PERG], (i % PERG) * plane16, 0);
@@ -643,9 +642,11 @@ namespace vdnn {
 // neighbouring elements of an input row through any tap: one 32-bit load (two-byte alignment suffices for
 // buffer loads, and with consecutive lanes on consecutive pairs a wavefront's load still covers one run of
 // a plane). Item = (pixel pair, eight consecutive channels): eight loads, a 2x8 transpose of 16-bit values
-// (v_perm_b32), two 128-bit LDS stores. A pixel left or right of the image is read from the neighbouring row
-// and masked; a pair whose second pixel is past the right edge is fetched one element lower (the last element
-// of the descriptor's range must not be the first half of a word) and unpacked from the upper halves.
+// (v_perm_b32), two 128-bit LDS stores. Only elements of the tensor are read: a pair whose second pixel is past the
+// right edge is fetched one element lower and its first pixel unpacked from the upper halves, a pair whose first pixel
+// is left of the image one element higher and its second pixel unpacked from the lower halves, a pair with neither
+// inside is not fetched. (The elements beside an image row belong to its neighbours, but what lies before the first row
+// of the tensor belongs to somebody else, or to nobody: reading and masking it faulted where the tensor began a mapping.)
 // Needs an even output row length, unit column stride in forward, at most 16 taps per filter row.
 template <int MODE>
 struct LoadIm2colPixTapH2 {
@@ -699,9 +700,10 @@ struct LoadIm2colPixTapH2 {
 #pragma unroll
         for (int i = 0; i < T / 128; i++) {
             const unsigned m0 = (unsigned)bit_to_all_ones(st.colbad[i], 2 * ts), m1 = (unsigned)bit_to_all_ones(st.colbad[i], 2 * ts + 1);
-            // second pixel outside: fetch one element lower, the first pixel is then the upper half of each word
-            const int voff = (st.vbase[i] + (int)(m1 & 0xFFFFFFFEu)) | bit_to_all_ones(st.invrow[i], tr); // m1 is 0 or -1: adds -2
-            const unsigned sel0 = m1 ? 0x07060302u : 0x05040100u;
+            // m0, m1: all ones where the first (second) pixel lies outside: one element higher (+2), one lower (-2)
+            const int move = (int)((m0 & 2u) + (m1 & 0xFFFFFFFEu));
+            const int voff = (st.vbase[i] + move) | (int)(m0 & m1) | bit_to_all_ones(st.invrow[i], tr);
+            const unsigned sel0 = m1 ? 0x07060302u : 0x05040100u, sel1 = m0 ? 0x05040100u : 0x07060302u;
             const int ch = cb * KH + 8 * (g0 + (NT / PAIRS) * i);
             const int soff = (ch * plane + tapoff) * 2, step = plane * 2;
             unsigned c[8];
@@ -709,8 +711,8 @@ struct LoadIm2colPixTapH2 {
             for (int e = 0; e < 8; e++) c[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(st.rsrc, voff, soff + e * step, 0);
             r.v[i][0].x = __builtin_amdgcn_perm(c[1], c[0], sel0) & ~m0; r.v[i][0].y = __builtin_amdgcn_perm(c[3], c[2], sel0) & ~m0;
             r.v[i][0].z = __builtin_amdgcn_perm(c[5], c[4], sel0) & ~m0; r.v[i][0].w = __builtin_amdgcn_perm(c[7], c[6], sel0) & ~m0;
-            r.v[i][1].x = __builtin_amdgcn_perm(c[1], c[0], 0x07060302u) & ~m1; r.v[i][1].y = __builtin_amdgcn_perm(c[3], c[2], 0x07060302u) & ~m1;
-            r.v[i][1].z = __builtin_amdgcn_perm(c[5], c[4], 0x07060302u) & ~m1; r.v[i][1].w = __builtin_amdgcn_perm(c[7], c[6], 0x07060302u) & ~m1;
+            r.v[i][1].x = __builtin_amdgcn_perm(c[1], c[0], sel1) & ~m1; r.v[i][1].y = __builtin_amdgcn_perm(c[3], c[2], sel1) & ~m1;
+            r.v[i][1].z = __builtin_amdgcn_perm(c[5], c[4], sel1) & ~m1; r.v[i][1].w = __builtin_amdgcn_perm(c[7], c[6], sel1) & ~m1;
         }
     }
     template <int T>
