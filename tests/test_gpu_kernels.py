@@ -648,6 +648,43 @@ def test_conv_results_do_not_depend_on_the_run(ctx):
     assert np.array_equal(gpu_conv_bwd_bias(ctx, g, dy, w[:, 0, 0, 0], np.float32(1.0)), gpu_conv_bwd_bias(ctx, g, dy, w[:, 0, 0, 0], np.float32(1.0)))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n,k,p,q", [(3, 5, 1, 1), (5, 7, 1, 3), (2, 3, 1, 4), (3, 4, 1, 7), (4, 3, 2, 4), (3, 2, 3, 3), (300, 3, 13, 13),
+                                     (2, 70, 31, 33), (33, 96, 55, 55)])
+def test_bias_gradients_at_any_plane_and_alignment(ctx, n, k, p, q, bf16):
+    """Planes of less than one access, of one, of one and a remainder; one workgroup per channel and several; a tensor one
+    element past an aligned address. The bias gradients of convolution and fully connected layers against sums in
+    64 bits: at most log2-deep trees and chains of n p q / 256 additions, each within 2^-24 of the sum of magnitudes."""
+    rng = np.random.default_rng(n * 1000 + k + p * q)
+    dy = rng.standard_normal((n, k, p, q)).astype(np.float32)
+    if bf16:
+        dy = (dy.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    flat = np.concatenate([np.full(1, 1e30, np.float32), dy.ravel(), np.full(8, 1e30, np.float32)])
+    bias = rng.standard_normal(k).astype(np.float32)
+    alpha = np.float32(-0.37)
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, int(bf16)))
+    try:
+        with Dev(ctx) as d:
+            src = d.up((flat.view(np.uint32) >> 16).astype(np.uint16), np.uint16) if bf16 else d.up(flat)
+            at = src.ptr + (2 if bf16 else 4)
+            b, db, fb = d.up(bias), d.empty((k,)), d.empty((k * p * q,))
+            g = be.shape(n, 3, p, q, k, 1, 1, 0, 0, 1, 1)
+            announce("bias gradient", (n, k, p, q), "bf16" if bf16 else "f32")
+            check(lib.vdnn_conv_bwd_bias_sgd(ctx.handle, None, g, at, b.ptr, alpha))
+            check(lib.vdnn_conv_bwd_bias(ctx.handle, None, g, at, db.ptr))
+            check(lib.vdnn_fc_bwd_bias(ctx.handle, None, n, k * p * q, at, fb.ptr))
+            got_b, got_db, got_fb = b.download((k,)), db.download((k,)), fb.download((k * p * q,))
+    finally:
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+    d64 = dy.astype(np.float64)
+    want, mag = d64.sum(axis=(0, 2, 3)), np.abs(d64).sum(axis=(0, 2, 3))
+    depth = 2.0 ** -24 * (20 + n * p * q / 256)
+    assert np.all(np.abs(got_db - want) <= depth * mag)
+    assert np.all(np.abs(got_b - (bias + np.float64(alpha) * want)) <= depth * mag + 2.0 ** -23 * np.abs(bias))
+    want, mag = d64.sum(axis=0).ravel(), np.abs(d64).sum(axis=0).ravel()
+    assert np.all(np.abs(got_fb - want) <= 2.0 ** -24 * (20 + n / 16) * mag)
+
+
 def _fc_all(ctx, x, w, b, dy, alpha):
     n, cin = x.shape
     cout = w.shape[0]
