@@ -394,6 +394,47 @@ def test_conv_bf16_tensors_at_odd_element_offsets(ctx):
         assert_close(gw.download(w.shape), oracle.conv_bwd_filter_sgd(og, x, dy, np.zeros_like(w), 1.0), 1e-4, "bwd filter")
 
 
+@pytest.mark.parametrize("geom", [
+    (2, 5, 4, 4, 3, 3, 3, 1, 1, 1, 1),        # one group a row, four groups a plane: several samples per slice
+    (9, 33, 5, 7, 70, 3, 3, 1, 1, 1, 1),      # rows of 4 + 3 pixels
+    (3, 8, 6, 9, 130, 3, 5, 0, 2, 1, 1),      # no padding above, two columns beside
+    (2, 12, 13, 13, 65, 5, 5, 2, 2, 1, 1),
+    (2, 7, 11, 6, 33, 6, 6, 5, 5, 1, 1),      # a window as wide as the image, padding wider than a group
+    (2, 20, 27, 3, 40, 3, 3, 1, 2, 1, 1),     # an image narrower than a group: element by element
+    (3, 70, 21, 19, 130, 3, 3, 1, 1, 2, 2),   # strided
+    (2, 6, 16, 23, 66, 3, 1, 1, 0, 1, 3),     # strided in the columns only
+    (2, 9, 17, 17, 24, 11, 11, 0, 0, 1, 1),
+])
+def test_bwd_filter_on_padded_rows(ctx, geom):
+    """Backward filter of planes that are no whole groups of pixels, against sums in double of the same bfloat16 values: the
+    products are exact, so the error is that of the float sums (TOL of the float engine). An infinite input element
+    reaches exactly the filter elements whose window covers it."""
+    n, c, h, w_, k, r, s, ph, pw, sh, sw = geom
+    p, q = (h + 2 * ph - r) // sh + 1, (w_ + 2 * pw - s) // sw + 1
+    g, og = be.shape(*geom), oracle.shape(*geom)
+    rng = np.random.default_rng(sum(geom))
+    x, dy = rnd(rng, (n, c, h, w_)), rnd(rng, (n, k, p, q))
+    w = np.zeros((k, c, r, s), np.float32)
+    announce("bwd filter on padded rows", geom)
+    with Dev(ctx) as d:
+        a, b, out = d.act(x), d.act(dy), d.raw(w.nbytes)
+        check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, a.ptr, b.ptr, out.ptr, None, 0))
+        assert_close(out.download(w.shape), oracle.conv_bwd_filter_sgd(og, x, dy, w, 1.0), 1e-5, "dW")
+        # the last element of a row in the last sample: beside the groups that run past the row's end
+        xi = x.copy()
+        xi[n - 1, c - 1, h // 2, w_ - 1] = np.inf
+        a2 = d.act(xi)
+        check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, a2.ptr, b.ptr, out.ptr, None, 0))
+        got = out.download(w.shape)
+    covered = np.zeros((r, s), bool)
+    for i in range(r):
+        for j in range(s):
+            pp, qq = h // 2 + ph - i, w_ - 1 + pw - j
+            covered[i, j] = pp % sh == 0 and qq % sw == 0 and 0 <= pp // sh < p and 0 <= qq // sw < q
+    assert np.all(np.isfinite(got[:, : c - 1]))
+    assert np.array_equal(np.isfinite(got[:, c - 1]), np.broadcast_to(~covered, (k, r, s)))
+
+
 def test_pixel_pair_loads_stay_inside_the_tensors(ctx):
     """A pair of neighbouring pixels is one 32-bit load. Beside the first image row of a tensor such a pair lies before the
     tensor's first element, which need not be mapped: tensors of their own (device allocations of 11 MB, each at the start

@@ -1293,6 +1293,35 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
             }
         }
     }
+    if constexpr (sizeof(E) == 2) {
+        // every other plane of at least four pixels a row: output rows padded to groups of four pixels
+        const PixelGroupStep step = PixelGroupStep::make(g.P, g.Q);
+        const long Kpad = (long)g.N * g.P * step.QG * 4, per = 4l * g.P * step.QG;
+        const bool unit = g.sw == 1 && g.W >= 4;
+        if (g.Q >= 4 && Kpad < (1l << 31) - 4 * KH) {
+            long caph = (Kpad + 4 * KH - 1) / (4 * KH); // at least four slices per split
+            if (caph > by_mem) caph = by_mem;
+            const int wanth = choose_splits(tiles, Kpad, caph, ctx->num_cu, out_bytes, 2.0 * TM * TN * KB);
+            const GemmDims dh = make_dims(M, N, (int)Kpad, TM, TN, wanth, KH);
+            const long nspanh = dh.kchunk / per + 2 + KH / per; // a slice past the end of a range is fetched and not used
+            if (nspanh * g.K * PQ * 2 < (long)MAX_SUM_RANGE && nspanh * g.C * g.H * g.W * 2 < (long)MAX_SUM_RANGE) {
+                const LoadDyRowH al{dy, g.N, g.K, g.P, g.Q, dh.kchunk, dh.K, step};
+                int rch;
+#define VDNN_WGRAD_ROW_H(UNIT)                                                                                              \
+                do {                                                                                                        \
+                    const LoadIm2colRowH<UNIT> bl{x, g.N, g.C, g.H, g.W, g.R, g.S, g.P, g.Q, g.ph, g.pw, g.sh, g.sw, N, dh.kchunk, dh.K, dRS, dS, step}; \
+                    rch = narrow ? launch_igemm<64, 256, LoadDyRowH, LoadIm2colRowH<UNIT>, StoreDense<float>, true>(ctx, st, kBwdFilterHalfNames.t64, al, bl, ep, dh) \
+                                 : launch_igemm<128, 128, LoadDyRowH, LoadIm2colRowH<UNIT>, StoreDense<float>, true>(ctx, st, kBwdFilterHalfNames.t128, al, bl, ep, dh); \
+                } while (0)
+                if (unit) VDNN_WGRAD_ROW_H(true);
+                else VDNN_WGRAD_ROW_H(false);
+#undef VDNN_WGRAD_ROW_H
+                if (rch != VDNN_OK) return rch;
+                if (dh.splits > 1) return launch_reduce_splits(ctx, st, w, staging, (size_t)M * N, dh.splits, alpha, accumulate, nullptr, 0);
+                return VDNN_OK;
+            }
+        }
+    }
     if constexpr (sizeof(E) == 4) {
         // 3x3, stride 1, padding 1: one filter row and 64 input channels per workgroup, one fetch for three taps
         if (wgrad3x3_f32_ok(g)) { // loads of four pixels take any alignment of the tensors

@@ -727,3 +727,156 @@ struct LoadIm2colPixTapH2 {
 };
 
 } // namespace vdnn
+
+namespace vdnn {
+
+// ---- backward filter of any plane: the reduction runs over output rows padded to groups of four pixels ----------
+// Planes of odd extent (AlexNet's 55, 27 and 13) and strided layers ran on the float engine, whose matrix rate bounded
+// them at a sixteenth of this one's. Here the reduction index is (n, p, group, pixel) with ceil(Q/4) groups per output row,
+// so a group never leaves its row: the padding costs work (Q = 27: 4 %, Q = 13: 23 %) but no branches. A group's four
+// elements are one 64-bit load. Where they reach past an end of the image row the load is moved to the nearest
+// position inside it and the value shifted back, which brings zeros in where the padding was; pixels past Q are masked in
+// both operands (an infinity in x beside a zero in dy would be a NaN). So only elements of the tensors are read.
+// 64 x 96 x 27 x 27, 256 filters of 5 x 5: 579 -> 141 us for this kernel (99 -> 406 TFLOP/s).
+struct PixelGroups { // position in (n, p, group) and the step of one slice (KH / 4 groups)
+    int n, p, g;
+    __device__ __forceinline__ void init(int k_begin, int lane_group, int P, int QG, int n_first) {
+        const int i = k_begin / 4 + lane_group;
+        const int row = i / QG;
+        g = i - row * QG;
+        n = row / P;
+        p = row - n * P;
+        n -= n_first;
+    }
+    __device__ __forceinline__ void advance(int P, int QG, int dn, int dp, int dg) {
+        g += dg;
+        const bool row = g >= QG;
+        g -= row ? QG : 0;
+        p += dp + (row ? 1 : 0);
+        const bool sample = p >= P;
+        p -= sample ? P : 0;
+        n += dn + (sample ? 1 : 0);
+    }
+};
+// how far one slice moves, found on the host: dn samples, dp rows, dg groups
+struct PixelGroupStep {
+    int QG, dn, dp, dg;
+    static PixelGroupStep make(int P, int Q) {
+        const int QG = (Q + 3) / 4, groups = KH / 4, rows = groups / QG;
+        return PixelGroupStep{QG, rows / P, rows % P, groups % QG};
+    }
+};
+// the first `count` (0 .. 4) elements of a group, as a mask
+__device__ __forceinline__ unsigned long long group_mask(int count) { return count >= 4 ? ~0ull : (1ull << (16 * count)) - 1ull; }
+
+// dy as A[k][(n, p, group, pixel)]: thread t fetches group t%8 of rows t/8 + 32*i. Q >= 4.
+struct LoadDyRowH {
+    const bf16_t* dy;
+    int N, K, P, Q;
+    int kchunk, Ktot;
+    PixelGroupStep step;
+    template <int T> struct Regs { uintx2 v[T / 32]; int shift; };
+    template <int T> struct State { int mrow[T / 32]; PixelGroups at; __amdgpu_buffer_rsrc_t rsrc; };
+    template <int T>
+    __device__ __forceinline__ void init(State<T>& st, int row0, int tid, int, int k_begin) const {
+        const int per = 4 * P * step.QG, PQ = P * Q;
+        const int n_first = k_begin / per;
+        int k_last = k_begin + kchunk; if (k_last > Ktot) k_last = Ktot;
+        const int n_last = k_last > k_begin ? (k_last - 1) / per : n_first;
+        st.rsrc = make_rsrc(dy + (long)n_first * K * PQ, clamp_range((long)(n_last - n_first + 1) * K * PQ * 2));
+        st.at.init(k_begin, tid & 7, P, step.QG, n_first);
+#pragma unroll
+        for (int i = 0; i < T / 32; i++) { const int m = row0 + (tid >> 3) + 32 * i; st.mrow[i] = m < K ? m * PQ * 2 : SENT; }
+    }
+    template <int T>
+    __device__ __forceinline__ void load(State<T>& st, int, int, int, Regs<T>& r) const {
+        const int q = 4 * st.at.g, from = min(q, Q - 4);
+        const int off = (st.at.n * K * P * Q + st.at.p * Q + from) * 2;
+        r.shift = 16 * (q - from); // the row's last group: the elements that belong to the group before go out at the bottom
+#pragma unroll
+        for (int i = 0; i < T / 32; i++) r.v[i] = __builtin_bit_cast(uintx2, __builtin_amdgcn_raw_buffer_load_b64(st.rsrc, st.mrow[i] + off, 0, 0));
+        st.at.advance(P, step.QG, step.dn, step.dp, step.dg);
+    }
+    template <int T>
+    __device__ static __forceinline__ void store(unsigned short* lds, int tid, const Regs<T>& r) {
+#pragma unroll
+        for (int i = 0; i < T / 32; i++)
+            *(unsigned long long*)(lds + ((tid >> 3) + 32 * i) * HSTRIDE + 4 * (tid & 7)) = __builtin_bit_cast(unsigned long long, r.v[i]) >> r.shift;
+    }
+};
+
+// im2col operand B[(c,r,s)][(n, p, group, pixel)] in the filter's own column order: thread t fetches group t%8 of columns
+// t/8 + 32*i, each through its own tap. UNIT: column stride 1 and W >= 4; otherwise the four elements one by one.
+template <bool UNIT>
+struct LoadIm2colRowH {
+    const bf16_t* x;
+    int N, C, H, W, R, S, P, Q, ph, pw, sh, sw;
+    int ncols; // C*R*S
+    int kchunk, Ktot;
+    FastDiv divRS, divS;
+    PixelGroupStep step;
+    template <int T> struct Regs { uintx2 v[T / 32]; int shift[UNIT ? T / 32 : 1]; unsigned long long live; };
+    template <int T> struct State {
+        int coloff[T / 32]; // byte offset of (c, r, s), SENT past the last column
+        int tap[T / 32];    // r << 16 | s
+        PixelGroups at;
+        __amdgpu_buffer_rsrc_t rsrc;
+    };
+    template <int T>
+    __device__ __forceinline__ void init(State<T>& st, int j0, int tid, int, int k_begin) const {
+        const int per = 4 * P * step.QG;
+        const long chw = (long)C * H * W;
+        const int n_first = k_begin / per;
+        int k_last = k_begin + kchunk; if (k_last > Ktot) k_last = Ktot;
+        const int n_last = k_last > k_begin ? (k_last - 1) / per : n_first;
+        st.rsrc = make_rsrc(x + (long)n_first * chw, clamp_range((long)(n_last - n_first + 1) * chw * 2));
+        st.at.init(k_begin, tid & 7, P, step.QG, n_first);
+#pragma unroll
+        for (int i = 0; i < T / 32; i++) {
+            const int j = j0 + (tid >> 3) + 32 * i;
+            const int c = divRS.div(j), rs = j - c * (R * S);
+            const int r = divS.div(rs), s = rs - r * S;
+            st.coloff[i] = j < ncols ? (c * H + r) * W * 2 : SENT;
+            st.tap[i] = (r << 16) | s;
+        }
+    }
+    template <int T>
+    __device__ __forceinline__ void load(State<T>& st, int, int, int, Regs<T>& r) const {
+        const int q = 4 * st.at.g;
+        const int ih0 = st.at.p * sh - ph, iw0 = q * sw - pw;
+        const int base = (st.at.n * C * H * W + ih0 * W) * 2;
+        r.live = group_mask(Q - q);
+#pragma unroll
+        for (int i = 0; i < T / 32; i++) {
+            const int iw = iw0 + (st.tap[i] & 0xFFFF);
+            const bool row_ok = (unsigned)(ih0 + (st.tap[i] >> 16)) < (unsigned)H;
+            const int off = base + st.coloff[i];
+            if constexpr (UNIT) {
+                const int from = max(0, min(iw, W - 4)), by = iw - from;
+                const bool ok = row_ok && (unsigned)(by + 3) <= 6u;
+                r.shift[i] = 16 * max(-3, min(by, 3));
+                r.v[i] = __builtin_bit_cast(uintx2, __builtin_amdgcn_raw_buffer_load_b64(st.rsrc, ok ? off + 2 * from : SENT, 0, 0));
+            } else {
+                unsigned h[4];
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const bool ok = row_ok && (unsigned)(iw + e * sw) < (unsigned)W;
+                    h[e] = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(st.rsrc, ok ? off + 2 * (iw + e * sw) : SENT, 0, 0);
+                }
+                r.v[i].x = h[0] | (h[1] << 16); r.v[i].y = h[2] | (h[3] << 16);
+            }
+        }
+        st.at.advance(P, step.QG, step.dn, step.dp, step.dg);
+    }
+    template <int T>
+    __device__ static __forceinline__ void store(unsigned short* lds, int tid, const Regs<T>& r) {
+#pragma unroll
+        for (int i = 0; i < T / 32; i++) {
+            unsigned long long v = __builtin_bit_cast(unsigned long long, r.v[i]);
+            if constexpr (UNIT) v = (v >> max(r.shift[i], 0)) << max(-r.shift[i], 0);
+            *(unsigned long long*)(lds + ((tid >> 3) + 32 * i) * HSTRIDE + 4 * (tid & 7)) = v & r.live;
+        }
+    }
+};
+
+} // namespace vdnn
