@@ -100,3 +100,43 @@ def test_conv3x3_sweep_bfloat16(ctx, geom):
             assert_close(gw.download(w.shape), oracle.conv_bwd_filter_sgd(og, x, dy, np.zeros_like(w), 1.0), 1e-4, "bwd filter")
     finally:
         check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
+# The 64x64 tile: one row or column short of a tile and one past it, reductions of one slice and of many splits, 260 and
+# 516 tiles for 256 units (only the tiles behind whole rounds are split), taps shared by a tile's columns (channels in
+# 64s and 32s) and not, planes that are no whole groups of pixels.
+@pytest.mark.parametrize("geom", [
+    (1, 16, 5, 13, 63, 3, 3, 1, 1, 1, 1), (1, 17, 9, 7, 65, 3, 3, 0, 0, 1, 1), (2, 64, 8, 8, 64, 1, 1, 0, 0, 1, 1), (3, 5, 1, 21, 7, 1, 1, 0, 0, 1, 1),
+    (4, 32, 52, 80, 64, 3, 3, 1, 1, 1, 1), (2, 96, 129, 64, 64, 3, 3, 1, 1, 1, 1), (5, 33, 11, 11, 129, 5, 5, 2, 2, 1, 1), (2, 64, 12, 12, 66, 5, 5, 2, 2, 1, 1),
+    (3, 32, 9, 12, 130, 4, 4, 1, 1, 1, 1), (2, 128, 13, 13, 192, 3, 3, 1, 1, 1, 1)], ids=lambda g: "x".join(map(str, g)))
+def test_conv_small_tile(ctx, geom):
+    rng = np.random.default_rng(sum((i + 1) * v for i, v in enumerate(geom)))
+    g, og = be.shape(*geom), oracle.shape(*geom)
+    x = rng.standard_normal((g.n, g.c, g.h, g.w)).astype(np.float32)
+    w = (rng.standard_normal((g.k, g.c, g.r, g.s)) * np.sqrt(2.0 / (g.c * g.r * g.s))).astype(np.float32)
+    b = rng.standard_normal(g.k).astype(np.float32)
+    want_y = oracle.conv_fwd(og, x, w, b)
+    announce("conv small tile", geom)
+    assert_close(gpu_conv_fwd(ctx, g, x, w, b), want_y, TOL, "fwd")
+    dy = rng.standard_normal(want_y.shape).astype(np.float32)
+    assert_close(gpu_conv_bwd_data(ctx, g, dy, w), oracle.conv_bwd_data(og, dy, w), TOL, "bwd data")
+    zero = np.zeros_like(w)
+    assert_close(gpu_conv_bwd_filter(ctx, g, x, dy, zero, np.float32(1.0)), oracle.conv_bwd_filter_sgd(og, x, dy, zero, 1.0), TOL, "bwd filter")
+
+
+@pytest.mark.parametrize("n,cin,cout", [(1, 64, 1), (63, 17, 65), (65, 192, 64), (3, 193, 129), (64, 1028, 260), (130, 5, 7)])
+def test_fc_small_tile(ctx, n, cin, cout):
+    rng = np.random.default_rng(n * 7 + cin * 3 + cout)
+    x, w = rng.standard_normal((n, cin)).astype(np.float32), (rng.standard_normal((cout, cin)) / np.sqrt(cin)).astype(np.float32)
+    b, dy = rng.standard_normal(cout).astype(np.float32), rng.standard_normal((n, cout)).astype(np.float32)
+    announce("fc small tile", n, cin, cout)
+    with Dev(ctx) as d:
+        dx_, dw, db, ddy = d.f32(x), d.f32(w), d.f32(b), d.f32(dy)
+        y, gx = d.f32(np.zeros((n, cout))), d.f32(np.zeros((n, cin)))
+        check(lib.vdnn_fc_fwd(ctx.handle, None, n, cin, cout, dx_.ptr, dw.ptr, db.ptr, y.ptr))
+        check(lib.vdnn_fc_bwd_data(ctx.handle, None, n, cin, cout, ddy.ptr, dw.ptr, gx.ptr))
+        gw = d.f32(np.zeros_like(w))
+        check(lib.vdnn_fc_bwd_weight(ctx.handle, None, n, cin, cout, dx_.ptr, ddy.ptr, gw.ptr))
+        assert_close(y.download((n, cout)), oracle.fc_fwd(x, w, b), TOL, "fwd")
+        assert_close(gx.download((n, cin)), oracle.fc_bwd_data(dy, w), TOL, "bwd data")
+        assert_close(gw.download(w.shape), dy.astype(np.float64).T @ x.astype(np.float64), TOL, "bwd weight")

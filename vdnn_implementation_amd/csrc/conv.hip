@@ -63,12 +63,12 @@ static GemmDims make_dims(int M, int N, int K, int TM, int TN, int splits, int d
 }
 
 // names of the kernel classes in the timing report: {pass}_{tile}
-struct PassNames { const char* t64; const char* t128; };
-static const PassNames kFwdNames{"conv_fwd_64x256", "conv_fwd_128x128"};
-static const PassNames kBwdDataNames{"conv_bwd_data_64x256", "conv_bwd_data_128x128"};
-static const PassNames kBwdFilterNames{"conv_bwd_filter_64x256", "conv_bwd_filter_128x128"};
-static const PassNames kFwdPackedNames{"conv_fwd_packed_64x256", "conv_fwd_packed_128x128"};
-static const PassNames kBwdDataPackedNames{"conv_bwd_data_packed_64x256", "conv_bwd_data_packed_128x128"};
+struct PassNames { const char* t64; const char* t128; const char* t64s = ""; };
+static const PassNames kFwdNames{"conv_fwd_64x256", "conv_fwd_128x128", "conv_fwd_64x64"};
+static const PassNames kBwdDataNames{"conv_bwd_data_64x256", "conv_bwd_data_128x128", "conv_bwd_data_64x64"};
+static const PassNames kBwdFilterNames{"conv_bwd_filter_64x256", "conv_bwd_filter_128x128", "conv_bwd_filter_64x64"};
+static const PassNames kFwdPackedNames{"conv_fwd_packed_64x256", "conv_fwd_packed_128x128", "conv_fwd_packed_64x64"};
+static const PassNames kBwdDataPackedNames{"conv_bwd_data_packed_64x256", "conv_bwd_data_packed_128x128", "conv_bwd_data_packed_64x64"};
 static const PassNames kFwdHalfNames{"conv_fwd_bf16mfma_64x256", "conv_fwd_bf16mfma_128x128"};
 static const PassNames kBwdDataHalfNames{"conv_bwd_data_bf16mfma_64x256", "conv_bwd_data_bf16mfma_128x128"};
 static const PassNames kFwdWin3Names{"conv_fwd_bf16win_64x256", "conv_fwd_bf16win_64x256"};
@@ -104,9 +104,15 @@ int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, float* out, con
 int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, const float* partial, size_t count, int splits,
                               const float* bias, int opix, int channels, int relu, const bf16_t* gate);
 
+// What a loader's address work costs the 64x64 and the large tile (estimates of mfma_gemm.h), against the loaders whose
+// tap is a per-slice value; the others work it out for every element, a strided backward data with two divisions.
+template <class BL> struct LoadCost { static constexpr double SMALL = 1.25, LARGE = 1.15; };
+template <int MODE, class E> struct LoadCost<LoadIm2colPixTap<MODE, E>> { static constexpr double SMALL = 1.0, LARGE = 1.0; };
+template <bool BIG, class E> struct LoadCost<LoadIm2colPix<2, BIG, E>> { static constexpr double SMALL = 4.0, LARGE = 2.0; };
+
 // Forward / backward data. Tile shape by output-row count: 64-row tiles for narrow layers, 128
-// otherwise. A grid that cannot fill the chip (few output pixels: the fully connected layers written
-// as convolutions) splits its reduction; the partial sums go to the staging area and are added in split
+// otherwise; 64x64 where the estimates of mfma_gemm.h find it faster (float engine). A grid that cannot fill
+// the chip (few output pixels: the fully connected layers written as convolutions) splits its reduction; the partial sums go to the staging area and are added in split
 // order, with the bias, by a second kernel. The split count depends on the shape only.
 // HALF: the bfloat16 engine (32-deep slices); partial_bytes: room behind ep.partial (the context's staging
 // area unless part of it is taken by something else).
@@ -125,6 +131,19 @@ static int launch_by_m(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names
         const long by_mem = (long)(partial_bytes / out_bytes);
         if (cap > by_mem) cap = by_mem;
         splits = choose_splits(tiles, K, cap, ctx->num_cu, out_bytes, 2.0 * TM * TN * KB);
+    }
+    if constexpr (!HALF) {
+        const SmallTilePlan plan = small_tile_plan(M, N, K, ctx->reduce_scratch && ep.partial ? partial_bytes : 0, ctx->num_cu, 4, true, LoadCost<BL>::SMALL);
+        if (K <= kShortReduction || (2.0 * M * (double)N * K <= kSmallTileOps && plan.us < 0.9 * large_tile_us(M, N, K, TM, TN, splits, ctx->num_cu, false, LoadCost<BL>::LARGE))) {
+            GemmDims ds = make_dims(M, N, K, 64, 64, plan.splits);
+            const int tail = plan.full_tiles > 0 && ds.splits > 1 ? (int)((long)ds.mtiles * ds.ntiles - plan.full_tiles) : 0;
+            if (tail > 0) ds.full_tiles = (int)plan.full_tiles;
+            const int rcs = launch_igemm<64, 64, AL, BL, StoreNCHW<E>>(ctx, stream, names.t64s, al, bl, ep, ds, flops);
+            if (rcs != VDNN_OK || ds.splits == 1) return rcs;
+            if (tail > 0)
+                return launch_reduce_tail_nchw(ctx, stream, ep.out, ep.partial, tail, ds.splits, 64, 64, M, N, ds.mtiles, ds.full_tiles, ep.bias, ep.opix, ep.relu, ep.gate);
+            return launch_reduce_splits_nchw(ctx, stream, ep.out, ep.partial, (size_t)M * N, ds.splits, ep.bias, ep.opix, M, ep.relu, ep.gate);
+        }
     }
     GemmDims d = make_dims(M, N, K, TM, TN, splits, DEPTH);
     // Tail mode: when the tiles make whole rounds of resident workgroups (three per compute unit) plus a
@@ -229,9 +248,17 @@ static int conv_fwd_with(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const 
 }
 
 template <class AL, class BL>
-static int conv_wgrad_with(vdnn_ctx* ctx, hipStream_t st, const AL& al, const BL& bl, const StoreDense<float>& ep, const GemmDims& d, bool narrow) {
+static int conv_wgrad_with(vdnn_ctx* ctx, hipStream_t st, const AL& al, const BL& bl, const StoreDense<float>& ep, const GemmDims& d, bool narrow, bool small) {
+    if (small) return launch_igemm<64, 64>(ctx, st, kBwdFilterNames.t64s, al, bl, ep, d);
     return narrow ? launch_igemm<64, 256>(ctx, st, kBwdFilterNames.t64, al, bl, ep, d)
                   : launch_igemm<128, 128>(ctx, st, kBwdFilterNames.t128, al, bl, ep, d);
+}
+
+// NTAP: taps that share a 64x64 tile's columns
+template <int NTAP, class E>
+static int launch_wgrad_tap_small(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const LoadDyRedInc<E>& al, const E* x, const StoreFilterTap& ep, const GemmDims& d, FastDiv dS) {
+    const LoadIm2colRedTap<NTAP, E> bl{x, g.N, g.C, g.H, g.W, g.R, g.S, g.P, g.Q, g.ph, g.pw, g.sh, g.sw, d.N, d.kchunk, d.K, FastDiv::make(g.C), dS};
+    return launch_igemm<64, 64>(ctx, st, kBwdFilterNames.t64s, al, bl, ep, d);
 }
 
 // Workspace planning has no context at hand: it assumes the 256 compute units of the target part.
@@ -1228,14 +1255,24 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
     const long by_mem = staging ? (long)(staging_bytes / out_bytes) : 1;
     if (cap > by_mem) cap = by_mem;
     const int want = choose_splits(tiles, Kred, cap, ctx->num_cu, out_bytes, 2.0 * TM * TN * KB);
-    GemmDims d = make_dims(M, N, (int)Kred, TM, TN, want);
+    const bool vec = PQ % 4 == 0 && aligned16(dy); // bf16: four elements are 8 bytes, covered by the same test
+    const bool tap_planes = vec && PQ >= KB && 2 * g.Q >= KB; // planes the tap-major loaders take
+    // the 64x64 tile; its loaders have a column's tap to work out per element unless a tile's columns share it
+    const bool small_tap = tap_planes && g.C % 32 == 0;
+    const SmallTilePlan plan = small_tile_plan(M, N, Kred, staging ? staging_bytes : 0, ctx->num_cu, 2, false, tap_planes && g.C % 64 == 0 ? 1.05 : 1.9);
     // one split's samples of dy and of x are addressed through one descriptor with summed offsets
-    const long nspan = d.kchunk / PQ + 2;
-    VDNN_REQUIRE(nspan * g.K * PQ * (long)sizeof(E) < (long)MAX_SUM_RANGE && nspan * g.C * g.H * g.W * (long)sizeof(E) < (long)MAX_SUM_RANGE,
-                 "samples of one reduction split too large for one descriptor");
+    auto span_ok = [&](int kchunk) {
+        const long nspan = kchunk / PQ + 2;
+        return nspan * g.K * PQ * (long)sizeof(E) < (long)MAX_SUM_RANGE && nspan * g.C * g.H * g.W * (long)sizeof(E) < (long)MAX_SUM_RANGE;
+    };
+    const GemmDims d_small = make_dims(M, N, (int)Kred, 64, 64, plan.splits);
+    const bool small = (Kred <= kShortReduction || (2.0 * M * (double)N * (double)Kred <= kSmallTileOps &&
+                                                    plan.us < 0.9 * large_tile_us(M, N, Kred, TM, TN, want, ctx->num_cu, true, tap_planes && g.C % 32 == 0 ? 1.0 : 1.15))) &&
+                       span_ok(d_small.kchunk);
+    const GemmDims d = small ? d_small : make_dims(M, N, (int)Kred, TM, TN, want);
+    VDNN_REQUIRE(span_ok(d.kchunk), "samples of one reduction split too large for one descriptor");
     StoreDense<float> ep{w, staging, nullptr, (long)N, (long)M * N, alpha, accumulate};
     const FastDiv dRS = FastDiv::make(RS), dS = FastDiv::make(g.S), dQ = FastDiv::make(g.Q), dPQ = FastDiv::make(PQ);
-    const bool vec = PQ % 4 == 0 && aligned16(dy); // bf16: four elements are 8 bytes, covered by the same test
     // tap-major column order when the tile's columns fall into whole groups of channels with one tap each
     const int tile_n = narrow ? 256 : 128;
     const int ntap = g.C % tile_n == 0 ? 1 : (g.C % (tile_n / 2) == 0 ? 2 : (g.C % (tile_n / 4) == 0 ? 4 : 0));
@@ -1330,7 +1367,7 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
             if (taken || rcw != VDNN_OK) return rcw;
         }
     }
-    if (vec && ntap != 0 && PQ >= KB && 2 * g.Q >= KB) {
+    if (small ? small_tap : tap_planes && ntap != 0) {
         const FastDiv dC = FastDiv::make(g.C);
         StoreFilterTap ept{w, staging, g.C, RS, (long)M * N, alpha, accumulate, dC};
         LoadDyRedInc<E> al{dy, g.N, g.K, PQ, d.kchunk, d.K};
@@ -1341,7 +1378,11 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
             rc2 = narrow ? launch_igemm<64, 256>(ctx, st, kBwdFilterNames.t64, al, bl, ept, d)                               \
                          : launch_igemm<128, 128>(ctx, st, kBwdFilterNames.t128, al, bl, ept, d);                            \
         } while (0)
-        if (ntap == 1) VDNN_WGRAD_TAP(1);
+        if (small) {
+            if (g.C % 64 == 0) rc2 = launch_wgrad_tap_small<1, E>(ctx, st, g, al, x, ept, d, dS);
+            else rc2 = launch_wgrad_tap_small<2, E>(ctx, st, g, al, x, ept, d, dS);
+        }
+        else if (ntap == 1) VDNN_WGRAD_TAP(1);
         else if (ntap == 2) VDNN_WGRAD_TAP(2);
         else VDNN_WGRAD_TAP(4);
 #undef VDNN_WGRAD_TAP
@@ -1355,7 +1396,7 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
     do {                                                                                                                  \
         LoadDyRed<VEC, E> al{dy, g.N, g.K, PQ, d.kchunk, d.K, dPQ};                                                               \
         LoadIm2colRed<BIG, E> bl{x, g.N, g.C, g.H, g.W, g.R, g.S, g.P, g.Q, g.ph, g.pw, g.sh, g.sw, N, d.kchunk, d.K, dRS, dS, dQ, dPQ}; \
-        rc = conv_wgrad_with(ctx, st, al, bl, ep, d, narrow);                                                             \
+        rc = conv_wgrad_with(ctx, st, al, bl, ep, d, narrow, small);                                                             \
     } while (0)
     if (vec && !big) VDNN_WGRAD(true, false);
     else if (vec && big) VDNN_WGRAD(true, true);

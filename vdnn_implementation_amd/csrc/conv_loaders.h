@@ -360,18 +360,20 @@ struct StoreNCHW {
     const E* gate;     // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
     static constexpr bool TAIL = true;
     // tail mode: a split tile's sums go to partial[slot][row in tile][column in tile], slot = (tile, split)
-    __device__ __forceinline__ void store_tail(const floatx16 (&acc)[2][2], int wm0, int wn0, int lane, long slot, int TM, int TN) const {
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store_tail(const floatx16 (&acc)[MI][NJ], int wm0, int wn0, int lane, long slot, int TM, int TN) const {
         const int l32 = lane & 31, lk = lane >> 5;
         float* po = partial + slot * TM * TN;
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++)
+        for (int jt = 0; jt < NJ; jt++)
 #pragma unroll
-            for (int it = 0; it < 2; it++)
+            for (int it = 0; it < MI; it++)
 #pragma unroll
                 for (int v = 0; v < 16; v++)
                     po[(wm0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4)) * TN + wn0 + jt * 32 + l32] = acc[it][jt][v];
     }
-    __device__ __forceinline__ void store(const floatx16 (&acc)[2][2], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
         const int l32 = lane & 31, lk = lane >> 5;
         // Bias and gate values are read before the stores they feed, eight at a time: a load that follows a store
         // through a pointer it might share has to be issued behind it, and with the load's result needed for the next
@@ -379,7 +381,7 @@ struct StoreNCHW {
         // count against the three workgroups a compute unit holds. (A gate that *is* the output tensor - the gradient
         // written over the layer's own input - is read by the lane that overwrites it, before it does.)
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++) {
+        for (int jt = 0; jt < NJ; jt++) {
             const int j = j0 + jt * 32 + l32;
             if (j >= d.N) continue;
             const int n = j / opix, pix = j - n * opix;
@@ -387,7 +389,7 @@ struct StoreNCHW {
             E* o = out + base;
             float* po = partial + (size_t)ks * d.M * d.N + base;
 #pragma unroll
-            for (int it = 0; it < 2; it++)
+            for (int it = 0; it < MI; it++)
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     float bv[8], gt[8];

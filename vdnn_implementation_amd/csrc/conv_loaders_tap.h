@@ -195,17 +195,19 @@ struct StoreFilterTap {
     int accumulate;
     FastDiv divC;
     static constexpr bool TAIL = false;
-    __device__ __forceinline__ void store_tail(const floatx16 (&)[2][2], int, int, int, long, int, int) const {}
-    __device__ __forceinline__ void store(const floatx16 (&acc)[2][2], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store_tail(const floatx16 (&)[MI][NJ], int, int, int, long, int, int) const {}
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
         const int l32 = lane & 31, lk = lane >> 5;
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++) {
+        for (int jt = 0; jt < NJ; jt++) {
             const int j = j0 + jt * 32 + l32;
             if (j >= d.N) continue;
             const int tap = divC.div(j), c = j - tap * C;
             const long col = (long)c * RS + tap;
 #pragma unroll
-            for (int it = 0; it < 2; it++)
+            for (int it = 0; it < MI; it++)
 #pragma unroll
                 for (int v = 0; v < 16; v++) {
                     const int m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);

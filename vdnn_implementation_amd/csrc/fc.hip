@@ -23,12 +23,18 @@ template <class L> struct FilterOperand<L, bf16_t> { typedef RoundedToBf16<L> ty
 template <class AL, class BL, class EO>
 static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al, const BL& bl, int M, int N, int K,
                    EO* out, float alpha, int accumulate, const float* bias_j, int relu = 0, const EO* gate = nullptr) {
-    const int TM = M <= 64 ? 64 : 128, TN = M <= 64 ? 256 : 128;
+    int TM = M <= 64 ? 64 : 128, TN = M <= 64 ? 256 : 128;
     const long tiles = (long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     long cap = ((long)K + 8 * KB - 1) / (8 * KB); // at least eight slices per split
     const long by_mem = (long)(ctx->reduce_scratch_bytes / ((size_t)M * N * sizeof(float)));
     if (cap > by_mem) cap = by_mem;
     const long want = choose_splits(tiles, K, cap, ctx->num_cu, (size_t)M * N * sizeof(float), 2.0 * TM * TN * KB);
+    // The 64x64 tile (mfma_gemm.h) with the same splits: the same sums. Small products gain from more and shorter workgroups
+    // (64 rows, 4096 -> 1000: 23 -> 16 us forward; 128, 300 -> 100 backward data 24.5 -> 8.7), short reductions always
+    // (filter updates: a tile has as many slices as rows allow); larger ones break even at 4-8 GFLOP (128 rows, 4096 -> 4096:
+    // 47 -> 45 us, 256 rows 80 -> 81) and lose beyond (128 rows, 25088 -> 4096: 219 -> 236).
+    const bool small = K <= kShortReduction || 2.0 * M * (double)N * K <= 5e9;
+    if (small) TM = TN = 64;
     GemmDims d;
     d.M = M; d.N = N; d.K = K;
     d.mtiles = (M + TM - 1) / TM; d.ntiles = (N + TN - 1) / TN;
@@ -40,7 +46,8 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     StoreDense<EO> ep{out, ctx->reduce_scratch, d.splits > 1 ? nullptr : bias_j, (long)N, (long)M * N, alpha, accumulate, relu, gate};
     const long blocks = (long)d.mtiles * d.ntiles * d.splits;
     ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
-    if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
+    if (small) hipLaunchKernelGGL((igemm_kernel<64, 64, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
+    else if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     if (d.splits > 1) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, alpha, accumulate, bias_j, N, relu, gate);

@@ -189,9 +189,90 @@ static inline int choose_splits(long tiles, long K, long max_splits, int num_cu,
     return best_s;
 }
 
+// The 64x64 tile (wavefront tiles of 32x32): a quarter of the large tile's work per workgroup. A grid that leaves compute
+// units idle, or ends in a nearly empty round, is cut four times finer, and a workgroup's prologue and epilogue (address
+// set-up, the first slices' trip through memory, 16 stores per lane instead of 64, a kernel text a quarter as long to
+// fetch) are that much shorter, which is most of a small layer's time. Twice the operand loads and LDS reads per matrix
+// instruction make it 5-8 % slower where the grid fills the chip many times over.
+// One call, floats, before -> after: 1x64x56x56 with 128 filters of 3x3 forward 24.6 -> 17.7 us; 4x8x10x10, 12 filters of
+// 5x5 19.3 -> 8.9 us; 32x256x28x28, 256 filters of 3x3 304 -> 249 us (392 large tiles for 256 units); fully connected
+// 25088 -> 4096 at 64 rows, filter update (four slices a tile) 311 -> 241 us.
+// Which tile: the times of both are estimated, from 290 measured calls of 1 to 128 samples, 8 to 1024 channels, 1x1 to
+// 5x5, planes of 7 to 56 pixels a side; the choice is within 3 % of the better one in all but a few of them.
+// Products of more than kSmallTileOps operations keep the large tile whatever the estimates say: those of large training
+// steps, which are to give the same bits from one version of this file to the next, and whose grids seldom gain.
+struct SmallTilePlan {
+    int splits = 0;      // Splits of every tile, or (full_tiles > 0) of the tiles behind the first full_tiles
+    long full_tiles = 0;
+    double us = 0.0;
+};
+constexpr double kSmallTileOps = 3e10;
+constexpr long kShortReduction = 192; // up to here a large tile is mostly prologue and epilogue: 1.3-2.5x on every grid measured
+// load_cost: work of the loaders against those of the blocked tap-major order (1)
+static inline SmallTilePlan small_tile_plan(long M, long N, long K, size_t partial_bytes, int num_cu, long min_slices, bool tail_mode, double load_cost) {
+    constexpr double kSum = 4.0;                             // the second kernel of a split reduction, us
+    constexpr long kPrologue = 8;                            // prologue and epilogue, in slices
+    const double slice_us = 0.27 * load_cost;                // a unit's share of a 64x64x16 slice
+    // a workgroup has one wavefront per SIMD: one or two of them do not cover the latency of their loads
+    auto filled = [](long per_cu) { return per_cu <= 1 ? 0.66 : per_cu == 2 ? 0.86 : per_cu == 3 ? 0.97 : 1.0; };
+    const long tiles = ((M + 63) / 64) * ((N + 63) / 64), slices = (K + KB - 1) / KB;
+    const size_t out_bytes = (size_t)M * N * sizeof(float), tile_bytes = 64 * 64 * sizeof(float);
+    const long by_depth = slices / min_slices > 1 ? slices / min_slices : 1, full = tiles / num_cu * num_cu, rem = tiles - full;
+    SmallTilePlan best;
+    // every tile split
+    long cap = 8l * num_cu / tiles + 1;
+    if (cap > by_depth) cap = by_depth;
+    if (cap > (long)(partial_bytes / out_bytes)) cap = (long)(partial_bytes / out_bytes);
+    if (cap < 1) cap = 1;
+    for (long s = 1; s <= cap; s++) {
+        const long rounds = (tiles * s + num_cu - 1) / num_cu;
+        const double us = (double)rounds * (double)((slices + s - 1) / s + kPrologue) * slice_us / filled(rounds) +
+                          (s > 1 ? kSum + (double)s * (double)out_bytes * 0.6 / 4e6 : 0.0);
+        if (best.splits == 0 || us < best.us) { best.splits = (int)s; best.us = us; }
+    }
+    // only the tiles behind whole rounds split
+    if (tail_mode && full > 0 && rem > 0) {
+        long most = 4l * num_cu / rem + 1;
+        if (most > by_depth) most = by_depth;
+        if (most > (long)(partial_bytes / (rem * tile_bytes))) most = (long)(partial_bytes / (rem * tile_bytes));
+        for (long s = 2; s <= most; s++) {
+            const long f = full / num_cu, r = (rem * s + num_cu - 1) / num_cu;
+            const double us = ((double)f * (double)(slices + 2) / filled(f) + (double)r * (double)((slices + s - 1) / s + kPrologue)) * slice_us +
+                              kSum + (double)(s * rem) * (double)tile_bytes * 0.6 / 4e6;
+            if (us < best.us) { best.splits = (int)s; best.full_tiles = full; best.us = us; }
+        }
+    }
+    return best;
+}
+// The large tile's time on the same scale. whole_grids: the reduction is split whatever the number of tiles (backward
+// filter, fully connected layers); otherwise only a grid below two workgroups a unit is, and a remainder behind rounds of
+// three workgroups a unit runs in tail mode.
+static inline double large_tile_us(long M, long N, long K, int TM, int TN, int splits, int num_cu, bool whole_grids, double load_cost) {
+    constexpr double kSum = 4.0;
+    const double slice_us = 2.0 * TM * TN * KB / (118e6 / num_cu);
+    auto eff = [](long rounds) { return rounds == 1 ? 0.72 : rounds == 2 ? 0.92 : rounds == 4 ? 0.93 : rounds % 3 == 0 ? 1.0 : 0.97; };
+    const long tiles = ((M + TM - 1) / TM) * ((N + TN - 1) / TN), slices = (K + KB - 1) / KB;
+    if (whole_grids || tiles < 2l * num_cu) {
+        const long rounds = (tiles * splits + num_cu - 1) / num_cu;
+        return ((double)rounds * (double)((slices + splits - 1) / splits + 6) * slice_us / eff(rounds) + (splits > 1 ? (double)splits * (double)(M * N) * 8.0 / 4e6 : 0.0)) * 0.85 * load_cost +
+               (splits > 1 ? kSum : 0.0);
+    }
+    const long slots = 3l * num_cu, rem = tiles % slots;
+    const double us = (double)((tiles - rem) / num_cu) * (double)(slices + 2) * slice_us;
+    if (tiles > slots && rem > 0 && 2 * rem <= slots)
+        return (us + 3.0 * ((double)slices / (double)(slots / rem) + 6.0) * slice_us) * 0.88 * load_cost + kSum;
+    const long last = (rem + num_cu - 1) / num_cu;
+    return (us + (double)last * (double)(slices + 2) * slice_us / (last == 1 ? 0.72 : last == 2 ? 0.92 : 1.0)) * 0.88 * load_cost;
+}
+
+// Edge of a wavefront's square sub-tile: 64, or 32 in the 64x64 tile of grids that leave the chip idle.
+template <int TM, int TN> struct WaveTile { static constexpr int V = TM * TN == 64 * 64 ? 32 : 64; };
+
 template <int TM, int TN, class AL, class BL, class EP>
 __global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
-    static_assert(TM % 64 == 0 && TN % 64 == 0 && (TM / 64) * (TN / 64) == 4, "four 64x64 wave tiles");
+    constexpr int MI = WaveTile<TM, TN>::V / 32, NJ = MI; // MFMA tiles of a wavefront
+    constexpr int WAVES_M = TM / (32 * MI);
+    static_assert(TM % (32 * MI) == 0 && TN % (32 * NJ) == 0 && WAVES_M * (TN / (32 * NJ)) == 4, "four wave tiles");
     using LA = LdsTile<TM, AL::RED_MAJOR>;
     using LB = LdsTile<TN, BL::RED_MAJOR>;
     __shared__ __attribute__((aligned(16))) float As[2][LA::SIZE];
@@ -222,15 +303,15 @@ __global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, con
     al.template init<TM>(sa, m0, tid, d.M, k_begin);
     bl.template init<TN>(sb, j0, tid, d.N, k_begin);
 
-    floatx16 acc[2][2];
+    floatx16 acc[MI][NJ];
 #pragma unroll
-    for (int i = 0; i < 2; i++)
+    for (int i = 0; i < MI; i++)
 #pragma unroll
-        for (int j = 0; j < 2; j++)
+        for (int j = 0; j < NJ; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
 
-    const int wm0 = (wave % (TM / 64)) * 64, wn0 = (wave / (TM / 64)) * 64;
+    const int wm0 = (wave % WAVES_M) * 32 * MI, wn0 = (wave / WAVES_M) * 32 * NJ;
     typename AL::template Regs<TM> ra;
     typename BL::template Regs<TN> rb;
 
@@ -257,47 +338,47 @@ __global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, con
     al.template load<TM>(sa, k_begin + KB, k_end, tid, ra);
     bl.template load<TN>(sb, k_begin + KB, k_end, tid, rb);
     __syncthreads();
-    floatx4 a0[2], b0[2], a1[2], b1[2];
+    floatx4 a0[MI], b0[NJ], a1[MI], b1[NJ];
 #pragma unroll
-    for (int i = 0; i < 2; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[0] + a_off + i * A_TILE, l32, lk, 0);
+    for (int i = 0; i < MI; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[0] + a_off + i * A_TILE, l32, lk, 0);
 #pragma unroll
-    for (int j = 0; j < 2; j++) b0[j] = read_frag<TN, BL::RED_MAJOR>(Bs[0] + b_off + j * B_TILE, l32, lk, 0);
+    for (int j = 0; j < NJ; j++) b0[j] = read_frag<TN, BL::RED_MAJOR>(Bs[0] + b_off + j * B_TILE, l32, lk, 0);
     for (int s = 0; s < nslices; s++) {
         const int cur = s & 1, nxt = cur ^ 1;
 #pragma unroll
-        for (int i = 0; i < 2; i++) a1[i] = read_frag<TM, AL::RED_MAJOR>(As[cur] + a_off + i * A_TILE, l32, lk, 1);
+        for (int i = 0; i < MI; i++) a1[i] = read_frag<TM, AL::RED_MAJOR>(As[cur] + a_off + i * A_TILE, l32, lk, 1);
 #pragma unroll
-        for (int j = 0; j < 2; j++) b1[j] = read_frag<TN, BL::RED_MAJOR>(Bs[cur] + b_off + j * B_TILE, l32, lk, 1);
+        for (int j = 0; j < NJ; j++) b1[j] = read_frag<TN, BL::RED_MAJOR>(Bs[cur] + b_off + j * B_TILE, l32, lk, 1);
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+                for (int j = 0; j < NJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[i][e], b0[j][e], acc[i][j], 0, 0, 0);
         AL::template store<TM>(As[nxt], tid, ra);
         BL::template store<TN>(Bs[nxt], tid, rb);
         // issue order of the first half: every MFMA is followed by one LDS access
 #pragma unroll
-        for (int i = 0; i < 16; i++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x300, 2, 0); }
+        for (int i = 0; i < 4 * MI * NJ; i++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x300, 2, 0); }
         __syncthreads();
         const int kk0 = k_begin + (s + 2) * KB;
         al.template load<TM>(sa, kk0, k_end, tid, ra);
         bl.template load<TN>(sb, kk0, k_end, tid, rb);
 #pragma unroll
-        for (int i = 0; i < 2; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[nxt] + a_off + i * A_TILE, l32, lk, 0);
+        for (int i = 0; i < MI; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[nxt] + a_off + i * A_TILE, l32, lk, 0);
 #pragma unroll
-        for (int j = 0; j < 2; j++) b0[j] = read_frag<TN, BL::RED_MAJOR>(Bs[nxt] + b_off + j * B_TILE, l32, lk, 0);
+        for (int j = 0; j < NJ; j++) b0[j] = read_frag<TN, BL::RED_MAJOR>(Bs[nxt] + b_off + j * B_TILE, l32, lk, 0);
 #pragma unroll
         for (int e = 0; e < 4; e++)
 #pragma unroll
-            for (int i = 0; i < 2; i++)
+            for (int i = 0; i < MI; i++)
 #pragma unroll
-                for (int j = 0; j < 2; j++)
+                for (int j = 0; j < NJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[i][e], b1[j][e], acc[i][j], 0, 0, 0);
         // second half: every MFMA is followed by a global load and an LDS read
 #pragma unroll
-        for (int i = 0; i < 16; i++) {
+        for (int i = 0; i < 4 * MI * NJ; i++) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
@@ -434,8 +515,10 @@ struct StoreDense {
     int relu;      // rectify the result (after the bias)
     const E* gate; // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
     static constexpr bool TAIL = false;
-    __device__ __forceinline__ void store_tail(const floatx16 (&)[2][2], int, int, int, long, int, int) const {}
-    __device__ __forceinline__ void store(const floatx16 (&acc)[2][2], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store_tail(const floatx16 (&)[MI][NJ], int, int, int, long, int, int) const {}
+    template <int MI, int NJ>
+    __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
         const int l32 = lane & 31, lk = lane >> 5;
         // What the result is combined with is read sixteen elements ahead of the stores: a load issued after a store
         // through the same pointer would have to wait for it (the compiler cannot know that the rows differ), and
@@ -444,12 +527,12 @@ struct StoreDense {
         // workgroups a compute unit holds.
         const bool combine = !to_partial && (accumulate || gate != nullptr);
 #pragma unroll
-        for (int jt = 0; jt < 2; jt++) {
+        for (int jt = 0; jt < NJ; jt++) {
             const int j = j0 + jt * 32 + l32;
             if (j >= d.N) continue;
             const float bj = (!to_partial && bias_j) ? bias_j[j] : 0.0f;
 #pragma unroll
-            for (int it = 0; it < 2; it++) {
+            for (int it = 0; it < MI; it++) {
                 float aux[16]; // the old value (accumulate) or the gate: a call asks for one of the two at most
                 if (combine) {
 #pragma unroll
