@@ -140,3 +140,42 @@ def test_fc_small_tile(ctx, n, cin, cout):
         assert_close(y.download((n, cout)), oracle.fc_fwd(x, w, b), TOL, "fwd")
         assert_close(gx.download((n, cin)), oracle.fc_bwd_data(dy, w), TOL, "bwd data")
         assert_close(gw.download(w.shape), dy.astype(np.float64).T @ x.astype(np.float64), TOL, "bwd weight")
+
+
+# Backward data of strided layers by residue classes: strides per axis up to four classes, windows smaller than the stride
+# (classes that no tap reaches), padding up to the window, output channels that are no whole slices, planes smaller than
+# the window plus stride, one tile and many, enough filters for split reductions.
+STRIDED = [(2, 5, 9, 11, 7, 3, 3, 1, 1, 2, 2), (1, 17, 8, 8, 33, 1, 1, 0, 0, 2, 2), (3, 70, 13, 9, 130, 3, 3, 1, 1, 2, 2), (2, 6, 10, 7, 16, 4, 4, 3, 3, 2, 2),
+           (2, 64, 7, 30, 48, 5, 5, 2, 2, 2, 2), (1, 9, 12, 12, 5, 3, 3, 0, 0, 1, 2), (2, 9, 12, 13, 20, 3, 2, 0, 1, 3, 1), (1, 8, 17, 5, 40, 5, 3, 2, 0, 4, 1),
+           (1, 65, 3, 3, 600, 3, 3, 0, 0, 2, 2), (4, 40, 64, 66, 31, 3, 3, 1, 1, 2, 2), (1, 7, 20, 21, 18, 11, 11, 5, 5, 2, 2)]
+
+
+@pytest.mark.parametrize("geom", STRIDED, ids=lambda g: "x".join(map(str, g)))
+def test_strided_backward_data(ctx, geom):
+    rng = np.random.default_rng(sum((i + 1) * v for i, v in enumerate(geom)))
+    g, og = be.shape(*geom), oracle.shape(*geom)
+    w = (rng.standard_normal((g.k, g.c, g.r, g.s)) * np.sqrt(2.0 / (g.c * g.r * g.s))).astype(np.float32)
+    P, Q = lib.vdnn_out_dim(g.h, g.pad_h, g.r, g.stride_h), lib.vdnn_out_dim(g.w, g.pad_w, g.s, g.stride_w)
+    dy = rnd(rng, (g.n, g.k, P, Q))  # bfloat16 values: both element types see the same gradient
+    x = rnd(rng, (g.n, g.c, g.h, g.w))
+    announce("strided bwd data", geom)
+    want = oracle.conv_bwd_data(og, dy, w)
+    assert_close(gpu_conv_bwd_data(ctx, g, dy, w), want, TOL, "float")
+    with Dev(ctx) as d:
+        ddy, dw, dxx, gx = d.f32(dy), d.f32(w), d.f32(x), d.f32(np.zeros_like(x))
+        check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, dw.ptr, dxx.ptr, gx.ptr, None, 0))
+        assert_close(gx.download(x.shape), np.where(x > 0, want, 0), TOL, "float, gated")
+        if g.n > 1:  # what one sample holds reaches no other one
+            spoilt = dy.copy()
+            spoilt[1] = np.inf
+            b = d.f32(spoilt)
+            check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, b.ptr, dw.ptr, gx.ptr, None, 0))
+            assert_close(gx.download(x.shape)[0], want[0], TOL, "beside a sample of infinities")
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 1))
+    try:
+        with Dev(ctx) as d:
+            ddy, dw, dxx, gx = d.act(dy), d.f32(w), d.act(x), d.empty_act(x.shape)
+            check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, dw.ptr, dxx.ptr, gx.ptr, None, 0))
+            assert_close_bf16(get_act(gx, x.shape), np.where(x > 0, oracle.conv_bwd_data(og, dy, oracle.round_bf16(w)), 0), "bf16, gated")
+    finally:
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))

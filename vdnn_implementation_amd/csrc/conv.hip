@@ -18,6 +18,7 @@
 #include "conv_smallc.h"
 #include "conv_smallc_mfma.h"
 #include "winograd_f32.h"
+#include "conv_strided.h"
 
 namespace vdnn {
 
@@ -107,7 +108,7 @@ int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, co
 // What a loader's address work costs the 64x64 and the large tile (estimates of mfma_gemm.h), against the loaders whose
 // tap is a per-slice value; the others work it out for every element, a strided backward data with two divisions.
 template <class BL> struct LoadCost { static constexpr double SMALL = 1.25, LARGE = 1.15; };
-template <int MODE, class E> struct LoadCost<LoadIm2colPixTap<MODE, E>> { static constexpr double SMALL = 1.0, LARGE = 1.0; };
+template <int MODE, class E, bool PAD> struct LoadCost<LoadIm2colPixTap<MODE, E, PAD>> { static constexpr double SMALL = 1.0, LARGE = 1.0; };
 template <bool BIG, class E> struct LoadCost<LoadIm2colPix<2, BIG, E>> { static constexpr double SMALL = 4.0, LARGE = 2.0; };
 
 // Forward / backward data. Tile shape by output-row count: 64-row tiles for narrow layers, 128
@@ -892,6 +893,120 @@ static int launch_fwd_smallc3x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g,
     return VDNN_OK;
 }
 
+// Backward data of a strided layer by residue classes (conv_strided.h): as many samples at a time as the staging area
+// holds results of, 64x64 tiles, the reductions cut so that the workgroups of all classes together fill the chip.
+template <class E>
+static int launch_strided_bwd_data(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const E* dy, const float* w, E* dx, const E* gate, bool* taken) {
+    *taken = false;
+    const int classes = g.sh * g.sw;
+    // (samples that the one product's tiles could not address stay refused by the caller)
+    if (classes > kStridedClasses || !ctx->reduce_scratch || !pixel_tile_span_ok((long)g.K * g.P * g.Q, g.H * g.W, 256, (int)sizeof(E))) return VDNN_OK;
+    StridedGeo q{};
+    q.sh = g.sh; q.sw = g.sw; q.ph = g.ph; q.pw = g.pw;
+    q.C = g.C; q.H = g.H; q.W = g.W; q.R = g.R; q.S = g.S; q.K = g.K; q.Kpad = (g.K + KB - 1) / KB * KB;
+    long filter_elems = 0, most_slices = 0;
+    const long sample = (long)g.K * g.P * g.Q;
+    for (int a = 0; a < g.sh; a++)
+        for (int b = 0; b < g.sw; b++) {
+            StridedClassGeo& c = q.c[a * g.sw + b];
+            c.rows = a < g.R ? (g.R - a + g.sh - 1) / g.sh : 0;
+            c.cols = b < g.S ? (g.S - b + g.sw - 1) / g.sw : 0;
+            c.taps = c.rows * c.cols;
+            c.u0 = g.ph > a ? (g.ph - a + g.sh - 1) / g.sh : 0;
+            c.v0 = g.pw > b ? (g.pw - b + g.sw - 1) / g.sw : 0;
+            c.opix_h = g.H - 1 + g.ph >= a ? (g.H - 1 + g.ph - a) / g.sh - c.u0 + 1 : 0;
+            c.opix_w = g.W - 1 + g.pw >= b ? (g.W - 1 + g.pw - b) / g.sw - c.v0 + 1 : 0;
+            c.filter_first = filter_elems;
+            filter_elems += (long)g.C * q.Kpad * c.taps;
+            if (c.taps > 32) return VDNN_OK;
+            if (c.opix_h <= 0 || c.opix_w <= 0) { c.opix_h = c.opix_w = 0; continue; }
+            if (!pixel_tile_span_ok(sample, c.opix_h * c.opix_w, 64, (int)sizeof(E))) return VDNN_OK;
+            const long slices = (long)(q.Kpad / KB) * c.taps;
+            if (slices > most_slices) most_slices = slices;
+        }
+    if (most_slices == 0 || filter_elems * 4 >= 0x7FFF0000l) return VDNN_OK;
+    StagingCarve carve(ctx);
+    float* packed = packed_filter_place(ctx, carve, (size_t)filter_elems * sizeof(float));
+    if (!packed) return VDNN_OK;
+    const long per_sample = (long)g.C * g.H * g.W, room = (long)(ctx->reduce_scratch_bytes / sizeof(float));
+    const long nb = room / per_sample < g.N ? room / per_sample : g.N;
+    if (nb < 1 || nb * per_sample >= (1l << 31)) return VDNN_OK;
+    *taken = true;
+    {
+        ProfScope prof(ctx, st, "conv_pack_filter", 0.0, 8.0 * (double)filter_elems);
+        const dim3 grid((unsigned)((filter_elems + 255) / 256));
+        if (sizeof(E) == 2) hipLaunchKernelGGL(pack_filter_classes_kernel<true>, grid, dim3(256), 0, st, w, packed, q, filter_elems);
+        else hipLaunchKernelGGL(pack_filter_classes_kernel<false>, grid, dim3(256), 0, st, w, packed, q, filter_elems);
+        VDNN_LAUNCH_CHECK();
+    }
+    // slices per workgroup: the estimate of small_tile_plan over the tiles of all classes of the first (largest) chunk
+    auto class_splits = [&](const StridedClassGeo& c, long per) { return ((long)(q.Kpad / KB) * c.taps + per - 1) / per; };
+    auto tiles_of = [&](const StridedClassGeo& c, long n) { return (g.C + 63) / 64 * ((n * c.opix_h * c.opix_w + 63) / 64); };
+    long per = most_slices;
+    double best = 0.0;
+    for (long s = 1; s <= 32; s++) {
+        const long len = (most_slices + s - 1) / s;
+        if (s > 1 && len < 4) break;
+        long blocks = 0, elems = 0, work = 0;
+        for (int c = 0; c < classes; c++) {
+            if (q.c[c].opix_h == 0 || q.c[c].taps == 0) continue;
+            const long splits = class_splits(q.c[c], len), tiles = tiles_of(q.c[c], nb), slices = (long)(q.Kpad / KB) * q.c[c].taps;
+            blocks += tiles * splits;
+            work += tiles * (slices + 8 * splits);
+            elems += splits * nb * g.C * q.c[c].opix_h * q.c[c].opix_w;
+        }
+        if (elems > room) break;
+        // a round of workgroups lasts as long as its longest; beyond that the units share the work evenly
+        double us = 0.27 * (double)((work + ctx->num_cu - 1) / ctx->num_cu);
+        const double floor_us = 0.27 * (double)(len + 8) * (blocks <= ctx->num_cu ? 1.5 : 1.2);
+        if (us < floor_us) us = floor_us;
+        us += (double)elems * 2.4 / 4e6;
+        if (best == 0.0 || us < best) { best = us; per = len; }
+    }
+    const FastDiv one = FastDiv::make(1);
+    for (int n0 = 0; n0 < g.N; n0 += (int)nb) {
+        const int nc = g.N - n0 < nb ? g.N - n0 : (int)nb;
+        StridedLaunch<E> launch{};
+        long first = 0, blocks = 0;
+        for (int c = 0; c < classes; c++) {
+            StridedClassGeo& cg = q.c[c];
+            cg.result_first = first;
+            cg.splits = 0;
+            if (cg.opix_h == 0 || cg.taps == 0) continue;
+            const int opix = cg.opix_h * cg.opix_w, K = q.Kpad * cg.taps;
+            const GemmDims d = make_dims(g.C, nc * opix, K, 64, 64, (int)class_splits(cg, per));
+            cg.splits = d.splits;
+            float* out = ctx->reduce_scratch + first;
+            StridedClass<E> k{};
+            k.al = LoadDenseRed<true>{packed + cg.filter_first, (long)K, g.C, (unsigned)((long)g.C * K * 4)};
+            k.bl.base = LoadIm2colPix<1, false, E>{dy + (long)n0 * sample, g.P, g.Q, cg.opix_h, cg.opix_w, cg.rows, cg.cols, cg.u0, cg.v0, 1, 1, sample, nc, one, one};
+            k.bl.base.divRS = FastDiv::make(cg.taps); k.bl.base.divS = FastDiv::make(cg.cols);
+            k.bl.channels = g.K;
+            k.ep = StoreNCHW<float>{out, nullptr, opix, out, 0, nullptr};
+            k.d = d;
+            k.blocks = d.mtiles * d.ntiles * d.splits;
+            blocks += k.blocks;
+            first += (long)d.splits * nc * g.C * opix;
+            // the classes of most taps first
+            int at = launch.count++;
+            for (; at > 0 && launch.c[at - 1].d.kchunk < d.kchunk; at--) launch.c[at] = launch.c[at - 1];
+            launch.c[at] = k;
+        }
+        VDNN_REQUIRE(blocks < (1l << 31), "grid too large");
+        {
+            ProfScope prof(ctx, st, "conv_bwd_data_classes_64x64", 2.0 * nc * (double)g.K * g.C * g.R * g.S * g.P * g.Q, 0.0);
+            hipLaunchKernelGGL(igemm_classes_kernel<E>, dim3((unsigned)blocks), dim3(NT), 0, st, launch);
+            VDNN_LAUNCH_CHECK();
+        }
+        const long total = (long)nc * per_sample;
+        ProfScope prof(ctx, st, "conv_bwd_data_merge", 0.0, (double)first * 4.0 + (double)total * sizeof(E) * (gate ? 2.0 : 1.0));
+        hipLaunchKernelGGL(merge_classes_kernel<E>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, ctx->reduce_scratch, dx + (long)n0 * per_sample,
+                           gate ? gate + (long)n0 * per_sample : nullptr, q, nc, (unsigned)total);
+        VDNN_LAUNCH_CHECK();
+    }
+    return VDNN_OK;
+}
+
 // Backward filter of a bfloat16 3x3 / stride 1 / padding 1 layer with the vector loaders: picks the instantiation
 // for the number of taps per tile and the pixel group (combinations whose loads would mix taps do not exist).
 template <int TM, int TN, int NTAP, int G>
@@ -1017,6 +1132,11 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
     hipStream_t st = stream_of(ctx, stream);
     StagingCarve carve(ctx);
     const bool few_channels = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS && !gate; // the vector-ALU kernels have no gated store
+    if (!few_channels && (g.sh != 1 || g.sw != 1)) {
+        bool taken = false;
+        const int rc = launch_strided_bwd_data<E>(ctx, st, g, dy, w, dx, gate, &taken);
+        if (taken || rc != VDNN_OK) return rc;
+    }
     bool half_engine = false;
     if constexpr (sizeof(E) == 2) {
         half_engine = !few_channels && g.sh == 1 && g.sw == 1 && half_engine_ok(ctx, g.K, g.R * g.S, (size_t)g.K * g.C * g.R * g.S);

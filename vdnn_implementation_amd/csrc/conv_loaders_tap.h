@@ -56,11 +56,14 @@ struct LoadFilterTap {
 
 // ---- im2col operand, columns = output pixels, tap-major reduction ------------------------------------
 // MODE 0: forward gather from x; MODE 1: backward data at stride 1 (src = dy). At most 32 taps.
-template <int MODE, class E = float>
+// PAD: the last block of channels is a partial one; its channels from `channels` on read as zero (the other operand is zero
+// there, but a neighbouring sample's infinity times zero would not be).
+template <int MODE, class E = float, bool PAD = false>
 struct LoadIm2colPixTap {
     static constexpr bool RED_MAJOR = false;
     static constexpr int ES = ElemBytes<E>::V;
     LoadIm2colPix<MODE, false, E> base; // geometry and per-pixel state are those of the channel-major loader
+    int channels = 0;                   // PAD only
     template <int T> using Regs = typename LoadIm2colPix<MODE, false, E>::template Regs<T>;
     template <int T> using State = typename LoadIm2colPix<MODE, false, E>::template State<T>;
     template <int T>
@@ -78,7 +81,11 @@ struct LoadIm2colPixTap {
         const int chb = ch0 + __builtin_amdgcn_readfirstlane(tid / T);
         const int soff0 = (chb * plane + tapoff) * ES, step = (NT / T) * plane * ES;
 #pragma unroll
-        for (int i = 0; i < T * KB / NT; i++) r.s[i] = buf_load_e<E>(st.rsrc, voff, soff0 + i * step);
+        for (int i = 0; i < T * KB / NT; i++) {
+            int soff = soff0 + i * step;
+            if (PAD && chb + i * (NT / T) >= channels) soff = 0x7FFFFFF0;
+            r.s[i] = buf_load_e<E>(st.rsrc, voff, soff);
+        }
     }
     template <int T>
     __device__ static __forceinline__ void store(float* lds, int tid, const Regs<T>& r) {

@@ -269,7 +269,7 @@ static inline double large_tile_us(long M, long N, long K, int TM, int TN, int s
 template <int TM, int TN> struct WaveTile { static constexpr int V = TM * TN == 64 * 64 ? 32 : 64; };
 
 template <int TM, int TN, class AL, class BL, class EP>
-__global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
+__device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
     constexpr int MI = WaveTile<TM, TN>::V / 32, NJ = MI; // MFMA tiles of a wavefront
     constexpr int WAVES_M = TM / (32 * MI);
     static_assert(TM % (32 * MI) == 0 && TN % (32 * NJ) == 0 && WAVES_M * (TN / (32 * NJ)) == 4, "four wave tiles");
@@ -284,13 +284,13 @@ __global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, con
     const int ntiles_all = d.mtiles * d.ntiles;
     int tile, ks;
     bool whole;
-    if ((int)blockIdx.x < d.full_tiles) {
-        tile = xcd_remap(blockIdx.x, d.full_tiles); ks = 0; whole = true;
+    if (block < d.full_tiles) {
+        tile = xcd_remap(block, d.full_tiles); ks = 0; whole = true;
     } else if (d.full_tiles > 0) {
-        const int r = blockIdx.x - d.full_tiles, tl = ntiles_all - d.full_tiles;
+        const int r = block - d.full_tiles, tl = ntiles_all - d.full_tiles;
         tile = d.full_tiles + r % tl; ks = r / tl; whole = false;
     } else {
-        const int bid = xcd_remap(blockIdx.x, gridDim.x);
+        const int bid = xcd_remap(block, blocks);
         tile = bid % ntiles_all; ks = bid / ntiles_all; whole = d.splits == 1;
     }
     const int mt = tile % d.mtiles, nt = tile / d.mtiles;
@@ -389,6 +389,11 @@ __global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, con
         ep.store_tail(acc, wm0, wn0, lane, (long)(tile - d.full_tiles) * d.splits + ks, TM, TN);
     else
         ep.store(acc, m0 + wm0, j0 + wn0, lane, ks, d, !whole);
+}
+
+template <int TM, int TN, class AL, class BL, class EP>
+__global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
+    igemm_tile<TM, TN>(al, bl, ep, d, blockIdx.x, gridDim.x);
 }
 
 // ---- dense reduction-major operand: element (row, kk) at base[row*ld + kk] -------------------------
