@@ -179,3 +179,40 @@ def test_strided_backward_data(ctx, geom):
             assert_close_bf16(get_act(gx, x.shape), np.where(x > 0, oracle.conv_bwd_data(og, dy, oracle.round_bf16(w)), 0), "bf16, gated")
     finally:
         check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
+# Reduced channels (input channels forward, filters in backward data) that are no whole blocks of 16 or 32, through every
+# bfloat16 kernel that pads them (windowed 3x3; pixel pairs; single pixels, odd rows or strides) and the float engine: one
+# channel over and one short of a block, the smallest that pad. What a neighbouring sample holds must not reach a padded
+# channel: a sample of infinities leaves the others' results alone.
+@pytest.mark.parametrize("geom", [
+    (2, 33, 8, 18, 31, 3, 3, 1, 1, 1, 1), (3, 12, 6, 64, 13, 3, 3, 1, 1, 1, 1), (2, 95, 14, 14, 65, 3, 3, 1, 1, 1, 1), (2, 40, 9, 12, 20, 5, 5, 2, 2, 1, 1),
+    (2, 47, 7, 9, 49, 3, 3, 1, 1, 1, 1), (3, 15, 11, 13, 48, 3, 3, 0, 0, 1, 1), (2, 70, 13, 9, 130, 3, 3, 1, 1, 2, 2), (2, 129, 10, 16, 79, 1, 1, 0, 0, 1, 1),
+    (5, 300, 5, 5, 200, 1, 1, 0, 0, 1, 1)], ids=lambda g: "x".join(map(str, g)))
+def test_padded_channels(ctx, geom):
+    rng = np.random.default_rng(sum((i + 1) * v for i, v in enumerate(geom)))
+    g, og = be.shape(*geom), oracle.shape(*geom)
+    x = rnd(rng, (g.n, g.c, g.h, g.w))
+    w = oracle.round_bf16((rng.standard_normal((g.k, g.c, g.r, g.s)) * np.sqrt(2.0 / (g.c * g.r * g.s))).astype(np.float32))
+    want_y = oracle.conv_fwd(og, x, w, np.zeros(g.k, np.float32))
+    dy = rnd(rng, want_y.shape)
+    want_dx = oracle.conv_bwd_data(og, dy, w)
+    xi, dyi = x.copy(), dy.copy()
+    xi[1], dyi[1] = np.inf, -np.inf
+    announce("padded channels", geom)
+    for bf16 in (0, 1):
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, bf16))
+        try:
+            with Dev(ctx) as d:
+                up = d.act if bf16 else d.f32
+                get = (lambda b, s: get_act(b, s)) if bf16 else (lambda b, s: b.download(s))
+                close = assert_close_bf16 if bf16 else (lambda a, b, what: assert_close(a, b, TOL, what))
+                dw = d.f32(w)
+                for a, b, rows in ((x, dy, slice(None)), (xi, dyi, slice(0, 1))):
+                    y, dx = up(np.zeros_like(want_y)), up(np.zeros_like(x))
+                    check(lib.vdnn_conv_fwd(ctx.handle, None, g, 0, up(a).ptr, dw.ptr, None, y.ptr, None, 0))
+                    check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, up(b).ptr, dw.ptr, dx.ptr, None, 0))
+                    close(get(y, want_y.shape)[rows], want_y[rows], "fwd")
+                    close(get(dx, x.shape)[rows], want_dx[rows], "bwd data")
+        finally:
+            check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))

@@ -178,7 +178,7 @@ static int launch_by_m(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names
 // row of a channel block. Splits and tail mode as in launch_by_m. K counts 16-bit values of a row of the filter
 // operand (float layers: two per filter element).
 constexpr int kWin3SplitPerCU = 2;
-template <int MODE, class E>
+template <int MODE, class E, bool PAD = false>
 static int launch_win3x3(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names, const LoadPackedH& al, const Win3x3T<E>& geo, const StoreNCHW<E>& ep,
                          int M, int N, int K, double flops, size_t partial_bytes) {
     constexpr bool SPLIT = sizeof(E) == 4;
@@ -213,7 +213,7 @@ static int launch_win3x3(vdnn_ctx* ctx, hipStream_t stream, const PassNames& nam
     if (blocks <= 0 || blocks >= (1l << 31)) { set_error("conv3x3: grid of %ld workgroups out of range", blocks); return VDNN_EINVAL; }
     {
         ProfScope prof(ctx, stream, names.t64, flops, 0.0);
-        hipLaunchKernelGGL((conv3x3_bf16_kernel<MODE, E, SPLIT ? kWin3SplitPerCU : 3>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, geo, ep, d);
+        hipLaunchKernelGGL((conv3x3_bf16_kernel<MODE, E, SPLIT ? kWin3SplitPerCU : 3, PAD>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, geo, ep, d);
         VDNN_LAUNCH_CHECK();
     }
     if (d.splits == 1) return VDNN_OK;
@@ -272,6 +272,10 @@ constexpr size_t kMaxWgradWorkspace = (size_t)256 << 20;
 // spend R*S times the work on taps that fall outside the single output pixel.
 static bool is_dense(const ConvGeo& g) { return g.P == 1 && g.Q == 1 && g.ph == 0 && g.pw == 0 && g.R == g.H && g.S == g.W; }
 
+// Channel counts that are no whole blocks of 16 take the tap-major loaders with the last block padded where that multiplies at
+// most a quarter more: the others work out a tap per element, at half the rate (32 x 200 x 28 x 28, 300 of 3x3 forward
+// 356 -> 275 us; 64 x 130 x 13 x 13, 390 of 5x5 backward data 460 -> 352; 21 x 70 x 53 x 37, 130 of 3x3 forward 151 -> 121).
+static bool pad_pays(int channels) { return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels; }
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
 static bool packed_bwd_data_ok(const ConvGeo& g) {
     return g.C > 4 && g.sh == 1 && g.sw == 1 && g.R * g.S <= 32 && g.K % KB == 0;
@@ -526,15 +530,27 @@ static int launch_winograd_wgrad(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g
 
 // The bfloat16 engine's filter operand lives at the front of the staging area (rounded and re-laid-out by a
 // small kernel before every use: the master copy changes every step); what is left holds partial sums.
-static bool half_engine_ok(const vdnn_ctx* ctx, int reduced_channels, int RS, size_t filter_elems) {
-    return reduced_channels % KH == 0 && RS <= 32 && ctx->reduce_scratch && filter_elems * 2 + (16u << 20) <= ctx->reduce_scratch_bytes;
+// Channels that are no whole blocks of 32 are padded with zeros in the filter operand and not fetched in the other one. From
+// twelve channels on that is the faster route (the float engine with its per-element taps reaches 60-110 TFLOP/s, this
+// engine's 300-700 times the share of the block that is used):
+// 32 x 200 x 28 x 28, 300 filters of 3x3 forward 364 -> 48 us, backward data 338 -> 72; 64 x 130 x 13 x 13, 390 of 5x5 347 -> 127
+// and 468 -> 147; 16 x 12 x 112 x 112, 20 of 3x3 55 -> 25 and 83 -> 24.
+constexpr int kHalfMinChannels = 12;
+static bool half_engine_ok(const vdnn_ctx* ctx, int reduced_channels, int rows, int RS) {
+    if (RS > 32 || !ctx->reduce_scratch) return false;
+    const size_t elems = (size_t)rows * RS * reduced_channels, padded = (size_t)rows * RS * ((reduced_channels + KH - 1) / KH * KH);
+    if (padded * 2 + (16u << 20) > ctx->reduce_scratch_bytes || padded * 2 >= 0x7FFF0000ul) return false;
+    if (reduced_channels % KH == 0) return true;
+    // (a filter too large for the float route's rounded copy stays refused)
+    return reduced_channels >= kHalfMinChannels && elems * 4 + (8u << 20) <= ctx->reduce_scratch_bytes;
 }
 
 static int launch_pack_filter_bf16(vdnn_ctx* ctx, hipStream_t st, const float* w, unsigned short* packed, int rows, int Cred, int RS,
                                    int row_stride, int red_stride) {
-    const long total = (long)rows * Cred * RS;
+    const int Cpad = (Cred + KH - 1) / KH * KH;
+    const long total = (long)rows * Cpad * RS;
     ProfScope prof(ctx, st, "conv_pack_filter", 0.0, 6.0 * (double)total);
-    hipLaunchKernelGGL(pack_filter_tap_bf16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w, packed, rows, Cred, RS,
+    hipLaunchKernelGGL(pack_filter_tap_bf16_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w, packed, rows, Cred, Cpad, RS,
                        row_stride, red_stride, total);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
@@ -581,29 +597,37 @@ static const float* rounded_filter_copy(vdnn_ctx* ctx, hipStream_t st, StagingCa
     return wr;
 }
 
-// forward / backward data of a bfloat16 layer on the bfloat16 matrix cores; MODE as in LoadIm2colPixTapH
-template <int MODE>
-static int conv_half_engine(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const float* w, int rows, int Cred, int RS, int row_stride, int red_stride,
-                            const LoadIm2colPix<MODE, false, bf16_t>& pix, StoreNCHW<bf16_t> ep, int N, double flops) {
-    const size_t filter_elems = (size_t)rows * Cred * RS;
+// forward / backward data of a bfloat16 layer on the bfloat16 matrix cores; MODE as in LoadIm2colPixTapH, PAD: Cred is no
+// multiple of 32
+template <int MODE, bool PAD>
+static int conv_half_engine_with(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const float* w, int rows, int Cred, int RS, int row_stride, int red_stride,
+                                 const LoadIm2colPix<MODE, false, bf16_t>& pix, StoreNCHW<bf16_t> ep, int N, double flops) {
+    const int K = (Cred + KH - 1) / KH * KH * RS;
+    const size_t filter_elems = (size_t)rows * K;
     unsigned short* packed = (unsigned short*)ctx->reduce_scratch;
-    const size_t taken = (filter_elems * 2 + 255) / 256 * 256;
+    const size_t taken = (filter_elems * 2 + 255) / 256 * 256, left = ctx->reduce_scratch_bytes - taken;
     const int rc = launch_pack_filter_bf16(ctx, st, w, packed, rows, Cred, RS, row_stride, red_stride);
     if (rc != VDNN_OK) return rc;
     ep.partial = (float*)((char*)ctx->reduce_scratch + taken);
-    LoadPackedH al{packed, (long)Cred * RS, rows, (unsigned)(filter_elems * 2)};
+    LoadPackedH al{packed, (long)K, rows, (unsigned)(filter_elems * 2)};
     // 3x3 at stride 1 with padding 1: one staged window per filter row serves its three taps
     if (win3x3_ok(pix.R, pix.S, pix.ph, pix.pw, pix.sh, pix.sw, pix.Hs, pix.Ws, pix.OH, pix.OW, pix.sample_elems)) {
-        const Win3x3 geo{pix.src, pix.Hs, pix.Ws, pix.sample_elems, pix.sample_elems * pix.nsamples, pix.nsamples};
-        return launch_win3x3<MODE, bf16_t>(ctx, st, MODE == 0 ? kFwdWin3Names : kBwdDataWin3Names, al, geo, ep, rows, N, Cred * RS, flops, ctx->reduce_scratch_bytes - taken);
+        const Win3x3 geo{pix.src, pix.Hs, pix.Ws, pix.sample_elems, pix.sample_elems * pix.nsamples, pix.nsamples, Cred};
+        return launch_win3x3<MODE, bf16_t, PAD>(ctx, st, MODE == 0 ? kFwdWin3Names : kBwdDataWin3Names, al, geo, ep, rows, N, K, flops, left);
     }
     // a pixel pair per lane where the pairs of an output row are contiguous in the input
     if (pix.OW % 2 == 0 && pix.S <= 16 && pix.Ws >= pix.S && pix.Ws > pix.pw + 1 && (MODE == 1 || pix.sw == 1)) {
-        LoadIm2colPixTapH2<MODE> bl2{pix};
-        return launch_by_m<LoadPackedH, LoadIm2colPixTapH2<MODE>, bf16_t, true>(ctx, st, names, al, bl2, ep, rows, N, Cred * RS, flops, ctx->reduce_scratch_bytes - taken);
+        LoadIm2colPixTapH2<MODE, PAD> bl2{pix, Cred};
+        return launch_by_m<LoadPackedH, LoadIm2colPixTapH2<MODE, PAD>, bf16_t, true>(ctx, st, names, al, bl2, ep, rows, N, K, flops, left);
     }
-    LoadIm2colPixTapH<MODE> bl{pix};
-    return launch_by_m<LoadPackedH, LoadIm2colPixTapH<MODE>, bf16_t, true>(ctx, st, names, al, bl, ep, rows, N, Cred * RS, flops, ctx->reduce_scratch_bytes - taken);
+    LoadIm2colPixTapH<MODE, PAD> bl{pix, Cred};
+    return launch_by_m<LoadPackedH, LoadIm2colPixTapH<MODE, PAD>, bf16_t, true>(ctx, st, names, al, bl, ep, rows, N, K, flops, left);
+}
+template <int MODE>
+static int conv_half_engine(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const float* w, int rows, int Cred, int RS, int row_stride, int red_stride,
+                            const LoadIm2colPix<MODE, false, bf16_t>& pix, const StoreNCHW<bf16_t>& ep, int N, double flops) {
+    return Cred % KH == 0 ? conv_half_engine_with<MODE, false>(ctx, st, names, w, rows, Cred, RS, row_stride, red_stride, pix, ep, N, flops)
+                          : conv_half_engine_with<MODE, true>(ctx, st, names, w, rows, Cred, RS, row_stride, red_stride, pix, ep, N, flops);
 }
 
 // ---- perf-optimal mode, float layers: 3x3 / stride 1 / padding 1 on the bfloat16 matrix cores ------------------
@@ -690,9 +714,10 @@ static int launch_split_general(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g,
 
 static int launch_pack_filter(vdnn_ctx* ctx, hipStream_t st, const float* w, float* packed, int rows, int Cred, int RS,
                               int row_stride, int red_stride) {
-    const long total = (long)rows * Cred * RS;
+    const int Cpad = (Cred + KB - 1) / KB * KB;
+    const long total = (long)rows * Cpad * RS;
     ProfScope prof(ctx, st, "conv_pack_filter", 0.0, 8.0 * (double)total);
-    hipLaunchKernelGGL(pack_filter_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w, packed, rows, Cred, RS,
+    hipLaunchKernelGGL(pack_filter_tap_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, w, packed, rows, Cred, Cpad, RS,
                        row_stride, red_stride, total);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
@@ -1049,7 +1074,7 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
     const int K = g.C * g.R * g.S;
     const unsigned wbytes = (unsigned)((long)g.K * K * 4);
     if constexpr (sizeof(E) == 2) {
-        if (half_engine_ok(ctx, g.C, g.R * g.S, (size_t)g.K * K)) {
+        if (half_engine_ok(ctx, g.C, g.K, g.R * g.S)) {
             const int RS = g.R * g.S;
             LoadIm2colPix<0, false, bf16_t> pix{x, g.H, g.W, g.P, g.Q, g.R, g.S, g.ph, g.pw, g.sh, g.sw, (long)g.C * g.H * g.W, g.N,
                                                FastDiv::make(RS), FastDiv::make(g.S)};
@@ -1078,6 +1103,19 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
             }
             const int rc = launch_winograd(ctx, st, g, false, x, w, bias, y, relu, nullptr, workspace, workspace_bytes, &taken);
             if (taken || rc != VDNN_OK) return rc;
+        }
+    }
+    if (g.R * g.S <= 32 && g.C % KB != 0 && pad_pays(g.C)) {
+        // the same with the last block of channels filled up by zeros
+        const int RS = g.R * g.S, Kpad = (g.C + KB - 1) / KB * KB * RS;
+        const size_t bytes = (size_t)g.K * Kpad * 4;
+        if (float* packed = packed_filter_place(ctx, carve, bytes)) {
+            const int rc = launch_pack_filter(ctx, st, w, packed, g.K, g.C, RS, g.C * RS, RS);
+            if (rc != VDNN_OK) return rc;
+            LoadDenseRed<true> alp{packed, (long)Kpad, g.K, (unsigned)bytes};
+            LoadIm2colPixTap<0, E, true> bl{{x, g.H, g.W, g.P, g.Q, g.R, g.S, g.ph, g.pw, g.sh, g.sw, (long)g.C * g.H * g.W, g.N, FastDiv::make(RS), FastDiv::make(g.S)}, g.C};
+            StoreNCHW<E> ep{y, bias, g.P * g.Q, ctx->reduce_scratch, relu, nullptr};
+            return launch_by_m(ctx, st, kFwdNames, alp, bl, ep, g.K, g.N * g.P * g.Q, Kpad, 2.0 * g.K * (double)g.N * g.P * g.Q * K);
         }
     }
     if (g.R * g.S <= 32 && g.C % KB == 0) {
@@ -1139,7 +1177,7 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
     }
     bool half_engine = false;
     if constexpr (sizeof(E) == 2) {
-        half_engine = !few_channels && g.sh == 1 && g.sw == 1 && half_engine_ok(ctx, g.K, g.R * g.S, (size_t)g.K * g.C * g.R * g.S);
+        half_engine = !few_channels && g.sh == 1 && g.sw == 1 && half_engine_ok(ctx, g.K, g.C, g.R * g.S);
         if (!half_engine) {
             w = rounded_filter_copy(ctx, st, carve, w, (size_t)g.K * g.C * g.R * g.S);
             VDNN_REQUIRE(w != nullptr, "filter too large for the staging area (bfloat16 layer outside the bfloat16 engine)");
@@ -1255,6 +1293,18 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             }
             LoadFilterTap<true> alt{w, RS, g.C * RS, g.C, RS, wbytes, dRS};
             return launch_by_m(ctx, st, kBwdDataNames, alt, bl, ep, M, N, K, flops);
+        }
+        if (RS <= 32 && g.K % KB != 0 && pad_pays(g.K)) {
+            const int Kpad = (g.K + KB - 1) / KB * KB * RS;
+            const size_t bytes = (size_t)g.C * Kpad * 4;
+            if (float* packed = packed_filter_place(ctx, carve, bytes)) {
+                ep.partial = ctx->reduce_scratch;
+                const int rc = launch_pack_filter(ctx, st, w, packed, g.C, g.K, RS, RS, g.C * RS);
+                if (rc != VDNN_OK) return rc;
+                LoadDenseRed<true> alp{packed, (long)Kpad, g.C, (unsigned)bytes};
+                LoadIm2colPixTap<1, E, true> bl{{dy, g.P, g.Q, g.H, g.W, g.R, g.S, g.ph, g.pw, 1, 1, sample, g.N, dRS, dS}, g.K};
+                return launch_by_m(ctx, st, kBwdDataNames, alp, bl, ep, M, N, Kpad, flops);
+            }
         }
         if (RS <= 32) {
             LoadIm2colPix<1, false, E> bl{dy, g.P, g.Q, g.H, g.W, g.R, g.S, g.ph, g.pw, 1, 1, sample, g.N, dRS, dS};

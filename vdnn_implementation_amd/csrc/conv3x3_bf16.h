@@ -50,10 +50,12 @@ struct Win3x3T {
     long sample_elems;   // reduced channels * H * W
     long total_elems;    // samples * sample_elems
     int nsamples;
+    int channels = 0; // PAD only
 };
 typedef Win3x3T<bf16_t> Win3x3;
 
-template <int MODE, class E = bf16_t, int RESIDENT = 3>
+// PAD (bfloat16 layers): channels from geo.channels on (the rest of the last block) read as zero, as in LoadIm2colPixTap.
+template <int MODE, class E = bf16_t, int RESIDENT = 3, bool PAD = false>
 __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPackedH al, const Win3x3T<E> geo, const StoreNCHW<E> ep, const GemmDims d) {
     constexpr bool SPLIT = std::is_same<E, float>::value;
     constexpr int EB = (int)sizeof(E);
@@ -191,7 +193,7 @@ __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPa
                 const int soff = (ch * plane + rowoff + W + 2) * 2, step = plane * 2;
                 unsigned c[8];
 #pragma unroll
-                for (int e = 0; e < 8; e++) c[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, soff + e * step, 0);
+                for (int e = 0; e < 8; e++) c[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(rsrc, vo, PAD && ch + e >= geo.channels ? 0x7FFFFFF0 : soff + e * step, 0);
                 // 2 x 8 transpose of 16-bit values: the low halves are the first pixel's channels, the high halves the second's.
                 // wr[i][0] is the pixel this lane stores first: its first pixel in lanes 0-3 of every eight, its second in
                 // lanes 4-7 (store_window)
@@ -202,7 +204,8 @@ __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPa
             }
             if (wave == 0) {
                 const int soff = (cb * KH * plane + rowoff + W + 2) * 2;
-                f.hr = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rsrc, hoff | bit_to_all_ones(hrowinv, r), soff, 0);
+                const int past = PAD && cb * KH + lane % CH >= geo.channels ? OOB : 0;
+                f.hr = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(rsrc, hoff | bit_to_all_ones(hrowinv, r) | past, soff, 0);
             }
         }
     };

@@ -97,9 +97,11 @@ struct LoadPackedH {
 // MODE 0: forward gather from x; MODE 1: backward data at stride 1 (src = dy). A lane owns one pixel
 // (consecutive lanes, consecutive pixels: every 16-bit load of a wavefront covers one run of a plane) and
 // fetches eight consecutive channels of it per item, packed into one 128-bit LDS store.
-template <int MODE>
+// PAD: channels from `channels` on (the rest of the last block) read as zero, as in LoadIm2colPixTap.
+template <int MODE, bool PAD = false>
 struct LoadIm2colPixTapH {
     LoadIm2colPix<MODE, false, bf16_t> base; // geometry and per-pixel state of the float engine's loader
+    int channels = 0;                        // PAD only
     template <int T> struct Regs { uintx4 v[T / 64]; };
     template <int T> using State = typename LoadIm2colPix<MODE, false, bf16_t>::template State<T>;
     template <int T>
@@ -121,7 +123,7 @@ struct LoadIm2colPixTapH {
             const int soff = (ch * plane + tapoff) * 2, step = plane * 2;
             unsigned h[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) h[e] = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(st.rsrc, voff, soff + e * step, 0);
+            for (int e = 0; e < 8; e++) h[e] = (unsigned)(unsigned short)__builtin_amdgcn_raw_buffer_load_b16(st.rsrc, voff, PAD && ch + e >= channels ? 0x7FFFFFF0 : soff + e * step, 0);
             r.v[i].x = h[0] | (h[1] << 16); r.v[i].y = h[2] | (h[3] << 16);
             r.v[i].z = h[4] | (h[5] << 16); r.v[i].w = h[6] | (h[7] << 16);
         }
@@ -189,15 +191,16 @@ template <int MODE> struct SplitProducts<LoadIm2colPixTapS<MODE>> { static const
 // packed[row][(cb*RS + tap)*32 + l] = bf16(w[row*row_stride + (cb*32 + l)*red_stride + tap])
 //   forward:       rows = output channels, reduced channels = input channels:  row_stride = C*RS, red_stride = RS
 //   backward data: rows = input channels,  reduced channels = output channels: row_stride = RS,   red_stride = C*RS
+// Cpad: Cred in whole blocks of 32, zeros behind the last channel.
 static __global__ void __launch_bounds__(256) pack_filter_tap_bf16_kernel(const float* __restrict__ w, unsigned short* __restrict__ packed,
-                                                                   int rows, int Cred, int RS, int row_stride, int red_stride, long total) {
+                                                                   int rows, int Cred, int Cpad, int RS, int row_stride, int red_stride, long total) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
-    const int per_row = Cred * RS;
+    const int per_row = Cpad * RS;
     const int row = (int)(i / per_row), kk = (int)(i - (long)row * per_row);
     const int l = kk & 31, slice = kk >> 5;
     const int cb = slice / RS, tap = slice - cb * RS;
-    packed[i] = float_to_bf16_bits(w[(long)row * row_stride + (long)(cb * 32 + l) * red_stride + tap]);
+    packed[i] = cb * 32 + l < Cred ? float_to_bf16_bits(w[(long)row * row_stride + (long)(cb * 32 + l) * red_stride + tap]) : (unsigned short)0;
 }
 
 // Order of the tiles over the workgroup index: rows fastest unless the epilogue type says otherwise.
@@ -648,9 +651,10 @@ namespace vdnn {
 // inside is not fetched. (The elements beside an image row belong to its neighbours, but what lies before the first row
 // of the tensor belongs to somebody else, or to nobody: reading and masking it faulted where the tensor began a mapping.)
 // Needs an even output row length, unit column stride in forward, at most 16 taps per filter row.
-template <int MODE>
+template <int MODE, bool PAD = false>
 struct LoadIm2colPixTapH2 {
     LoadIm2colPix<MODE, false, bf16_t> base; // geometry only
+    int channels = 0;                        // PAD only
     template <int T> struct Regs { uintx4 v[T / 128][2]; }; // [item][pixel of the pair]
     template <int T> struct State {
         int vbase[T / 128];       // byte offset of the pair's first pixel from the descriptor base
@@ -708,7 +712,7 @@ struct LoadIm2colPixTapH2 {
             const int soff = (ch * plane + tapoff) * 2, step = plane * 2;
             unsigned c[8];
 #pragma unroll
-            for (int e = 0; e < 8; e++) c[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(st.rsrc, voff, soff + e * step, 0);
+            for (int e = 0; e < 8; e++) c[e] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(st.rsrc, voff, PAD && ch + e >= channels ? 0x7FFFFFF0 : soff + e * step, 0);
             r.v[i][0].x = __builtin_amdgcn_perm(c[1], c[0], sel0) & ~m0; r.v[i][0].y = __builtin_amdgcn_perm(c[3], c[2], sel0) & ~m0;
             r.v[i][0].z = __builtin_amdgcn_perm(c[5], c[4], sel0) & ~m0; r.v[i][0].w = __builtin_amdgcn_perm(c[7], c[6], sel0) & ~m0;
             r.v[i][1].x = __builtin_amdgcn_perm(c[1], c[0], sel1) & ~m1; r.v[i][1].y = __builtin_amdgcn_perm(c[3], c[2], sel1) & ~m1;
