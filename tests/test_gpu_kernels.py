@@ -795,6 +795,36 @@ def test_maxpool_is_exact(ctx, n, c, h, w, win, stride, ties):
     assert np.array_equal(gdx, oracle.maxpool_bwd(og, x, wy, dy))
 
 
+# 3x3 / stride 2 on planes in LDS: even and odd extents, the smallest plane, tensors that begin anywhere in their 16 bytes
+# (gradients beginning at the same place as the input and elsewhere).
+@pytest.mark.parametrize("bf16", [0, 1])
+@pytest.mark.parametrize("n,c,h,w", [(1, 1, 3, 3), (1, 5, 9, 4), (2, 37, 13, 13), (3, 7, 55, 55), (1, 3, 40, 57)])
+def test_maxpool_on_unaligned_runs(ctx, n, c, h, w, bf16):
+    rng = np.random.default_rng(h * 31 + w)
+    x = oracle.round_bf16(np.maximum(np.round(4 * rng.standard_normal((n, c, h, w))), -2).astype(np.float32))
+    g, og = be.shape(n, c, h, w, 0, 3, 3, 0, 0, 2, 2), oracle.shape(n, c, h, w, 0, 3, 3, 0, 0, 2, 2)
+    wy = oracle.maxpool_fwd(og, x)
+    dy = (rng.integers(-8, 9, wy.shape) / 4).astype(np.float32)  # sums of up to four are exact in both types
+    want = oracle.maxpool_bwd(og, x, wy, dy)
+    dtype, size = (np.uint16, 2) if bf16 else (np.float32, 4)
+    pack = (lambda a: (np.ascontiguousarray(a, np.float32).view(np.uint32) >> 16).astype(np.uint16)) if bf16 else (lambda a: a)
+    unpack = (lambda a: (a.astype(np.uint32) << 16).view(np.float32)) if bf16 else (lambda a: a)
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, bf16))
+    try:
+        with Dev(ctx) as d:
+            for ox, ody, odx in ((0, 0, 0), (1, 2, 1), (3, 1, 2)):
+                announce("maxpool unaligned", (n, c, h, w), bf16, (ox, ody, odx))
+                a, b = d.up(np.concatenate([np.zeros(ox, dtype), pack(x).ravel()]), dtype), d.up(np.concatenate([np.zeros(ody, dtype), pack(dy).ravel()]), dtype)
+                y, dx = d.empty((wy.size + 8,), dtype), d.empty((x.size + 8,), dtype)
+                check(lib.vdnn_maxpool_fwd(ctx.handle, None, g, a.ptr + ox * size, y.ptr))
+                check(lib.vdnn_maxpool_bwd(ctx.handle, None, g, a.ptr + ox * size, y.ptr, b.ptr + ody * size, dx.ptr + odx * size))
+                got_y, got = y.download((wy.size + 8,), dtype)[:wy.size], dx.download((x.size + 8,), dtype)[odx:odx + x.size]
+                assert np.array_equal(unpack(got_y).reshape(wy.shape), wy)
+                assert np.array_equal(unpack(got).reshape(x.shape), want)
+    finally:
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
 def test_maxpool_golden(ctx):
     for name in ("pool_3x3_s2", "pool_2x2_s2", "pool_2x2_s2_odd"):
         f = golden(name)

@@ -595,31 +595,84 @@ __global__ void __launch_bounds__(EB) maxpool_bwd_kernel(const E* __restrict__ x
     }
 }
 
-// Unpadded pooling with a compile-time window and stride (AlexNet's 3x3 / stride 2) on planes that fit LDS: a
-// workgroup stages `group` consecutive (n,c) planes - one contiguous run of memory - and writes their outputs, another
-// contiguous run. The general kernels address every element with 64-bit divisions by run-time extents and run-time
-// loop bounds, which cost more than the memory accesses; here every division is by a constant or a 32-bit multiply-high.
-// Same comparison, same order: the same bits.
-template <class E, int R, int S, int SH, int SW>
-__global__ void __launch_bounds__(EB) maxpool_fwd_planes_kernel(const E* __restrict__ x, E* __restrict__ y, int H, int W, int P, int Q,
-                                                                long planes, int group, FastDiv dPQ, FastDiv dQ) {
-    extern __shared__ float pool_lds[];
+// A contiguous run of `count` elements to LDS as floats, 16 bytes at a time, four accesses in flight per thread. A run may
+// begin anywhere (a plane of 55 x 55 floats does): element i lies at lds[run_shift + i], which keeps the 16-byte groups of
+// memory whole in LDS too. lds: 16-byte aligned, room for count + 16 / sizeof(E) floats.
+template <class E> __device__ __forceinline__ int run_shift(const E* p) { return (int)(((uintptr_t)p & 15) / sizeof(E)); }
+__device__ __forceinline__ void put_group(float* lds, uint4 v, const float*) { *(uint4*)lds = v; }
+__device__ __forceinline__ void put_group(float* lds, uint4 v, const bf16_t*) {
+    uint4 lo, hi;
+    lo.x = v.x << 16; lo.y = v.x & 0xFFFF0000u; lo.z = v.y << 16; lo.w = v.y & 0xFFFF0000u;
+    hi.x = v.z << 16; hi.y = v.z & 0xFFFF0000u; hi.z = v.w << 16; hi.w = v.w & 0xFFFF0000u;
+    *(uint4*)lds = lo; *(uint4*)(lds + 4) = hi;
+}
+template <class E>
+__device__ __forceinline__ void load_run(const E* __restrict__ src, int count, float* lds) {
+    constexpr int V = 16 / (int)sizeof(E);
+    const int shift = run_shift(src), head = shift ? (V - shift < count ? V - shift : count) : 0;
+    const int groups = (count - head) / V, tail = head + groups * V;
+    const uint4* g = (const uint4*)(src + head);
+    float* l = lds + shift + head; // a multiple of V if there is a group
+    for (int i0 = threadIdx.x; i0 < groups; i0 += 4 * EB) {
+        uint4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) if (i0 + k * EB < groups) v[k] = g[i0 + k * EB];
+#pragma unroll
+        for (int k = 0; k < 4; k++) if (i0 + k * EB < groups) put_group(l + V * (i0 + k * EB), v[k], src);
+    }
+    if ((int)threadIdx.x < head) lds[shift + threadIdx.x] = load_elem(src + threadIdx.x);
+    if ((int)threadIdx.x < count - tail) lds[shift + tail + threadIdx.x] = load_elem(src + tail + threadIdx.x);
+}
+__device__ __forceinline__ uint4 get_group(const float* lds, const float*) { return *(const uint4*)lds; }
+__device__ __forceinline__ uint4 get_group(const float* lds, const bf16_t*) {
+    const float4 a = *(const float4*)lds, b = *(const float4*)(lds + 4);
+    uint4 v;
+    v.x = pack2_bf16(a.x, a.y); v.y = pack2_bf16(a.z, a.w); v.z = pack2_bf16(b.x, b.y); v.w = pack2_bf16(b.z, b.w);
+    return v;
+}
+// the way back, from a run at lds[shift]; element by element where dst does not begin at the same place in its 16 bytes
+template <class E>
+__device__ __forceinline__ void store_run(E* __restrict__ dst, int count, const float* lds, int shift) {
+    constexpr int V = 16 / (int)sizeof(E);
+    if (run_shift(dst) != shift) {
+        for (int i = threadIdx.x; i < count; i += EB) store_elem(dst + i, lds[shift + i]);
+        return;
+    }
+    const int head = shift ? (V - shift < count ? V - shift : count) : 0;
+    const int groups = (count - head) / V, tail = head + groups * V;
+    for (int i = threadIdx.x; i < groups; i += EB) *(uint4*)(dst + head + V * i) = get_group(lds + shift + head + V * i, dst);
+    if ((int)threadIdx.x < head) store_elem(dst + threadIdx.x, lds[shift + threadIdx.x]);
+    if ((int)threadIdx.x < count - tail) store_elem(dst + tail + threadIdx.x, lds[shift + tail + threadIdx.x]);
+}
+constexpr int POOL_RUN_PAD = 8; // floats a run in LDS may be shifted by, as whole 16-byte groups
+
+// Unpadded 3x3 pooling at stride 2 (AlexNet's) on planes that fit LDS: a workgroup stages `group` consecutive (n,c)
+// planes - one contiguous run of memory - and writes their outputs, another contiguous run. The general kernels address
+// every element with 64-bit divisions by run-time extents and run-time loop bounds, which cost more than the memory
+// accesses; here every division is a 32-bit multiply-high. Same comparison, same order: the same bits.
+// 64 x 96 x 55 x 55 floats 21.3 -> 17.6 us (93 MB), 16 x 100 x 100 x 77 25 -> 13; a plane or two per workgroup of the smallest
+// batches pay up to a microsecond for the run's ends (8 x 300 x 40 x 31: 5.0 -> 5.6).
+template <class E>
+__global__ void __launch_bounds__(EB) maxpool3x3s2_fwd_planes_kernel(const E* __restrict__ x, E* __restrict__ y, int H, int W, int P, int Q,
+                                                                     long planes, int group, FastDiv dPQ, FastDiv dQ) {
+    extern __shared__ __attribute__((aligned(16))) float pool_lds[];
     const int HW = H * W, PQ = P * Q;
     const long plane0 = (long)blockIdx.x * group;
     const int here = (int)(planes - plane0 < group ? planes - plane0 : group);
     const E* xp = x + plane0 * HW;
-    for (int i = threadIdx.x; i < here * HW; i += EB) pool_lds[i] = load_elem(xp + i);
+    load_run(xp, here * HW, pool_lds);
+    const float* xs = pool_lds + run_shift(xp);
     __syncthreads();
     E* yp = y + plane0 * PQ;
     for (int o = threadIdx.x; o < here * PQ; o += EB) {
         const int pl = dPQ.div(o), pq = o - pl * PQ;
         const int p = dQ.div(pq), q = pq - p * Q;
-        const float* b = pool_lds + pl * HW + p * SH * W + q * SW;
+        const float* b = xs + pl * HW + 2 * p * W + 2 * q;
         float m = -FLT_MAX;
 #pragma unroll
-        for (int r = 0; r < R; r++)
+        for (int r = 0; r < 3; r++)
 #pragma unroll
-            for (int s_ = 0; s_ < S; s_++) {
+            for (int s_ = 0; s_ < 3; s_++) {
                 const float v = b[r * W + s_];
                 if (v > m) m = v;
             }
@@ -628,59 +681,82 @@ __global__ void __launch_bounds__(EB) maxpool_fwd_planes_kernel(const E* __restr
 }
 
 // The backward counterpart: x and dy of `group` planes in LDS, every window's winner found once (first strict maximum
-// in row-major order, the window's first element if nothing exceeds -FLT_MAX), then every input element adds up the dy
-// of the windows that contain it and chose it, windows in row-major order - the general kernels' rule and order.
-template <class E, int R, int S, int SH, int SW>
-__global__ void __launch_bounds__(EB) maxpool_bwd_planes_fixed_kernel(const E* __restrict__ x, const E* __restrict__ dy, E* __restrict__ dx,
-                                                                      int H, int W, int P, int Q, long planes, int group, int gate,
-                                                                      FastDiv dPQ, FastDiv dQ, FastDiv dHW, FastDiv dW) {
-    extern __shared__ float pool_lds[];
+// in row-major order, the window's first element if nothing exceeds -FLT_MAX). Then a thread takes two by two input
+// elements: together they lie in four windows, whose winners and dy it reads once; each element adds up the dy of those
+// that contain it and chose it, windows in row-major order - the general kernels' rule and order. The gradients take x's
+// place in LDS and leave in 16-byte groups. Element by element, with its own divisions and window bounds and 4-byte
+// accesses, 64 x 96 x 55 x 55 floats took 60 us; now 39 (186 MB). 16 x 100 x 100 x 77: 98 -> 33.
+template <class E>
+__global__ void __launch_bounds__(EB) maxpool3x3s2_bwd_planes_kernel(const E* __restrict__ x, const E* __restrict__ dy, E* __restrict__ dx,
+                                                                     int H, int W, int P, int Q, long planes, int group, int gate,
+                                                                     FastDiv dPQ, FastDiv dQ, FastDiv dBlocks, FastDiv dBW) {
+    extern __shared__ __attribute__((aligned(16))) float pool_lds[];
     const int HW = H * W, PQ = P * Q;
-    float* xs = pool_lds;                      // [group][HW]
-    float* dys = xs + group * HW;              // [group][PQ]
-    int* arg = (int*)(dys + group * PQ);       // [group][PQ] winner's index in its plane
+    const int xroom = (group * HW + 3) / 4 * 4 + POOL_RUN_PAD, dyroom = (group * PQ + 3) / 4 * 4 + POOL_RUN_PAD;
+    int* arg = (int*)(pool_lds + xroom + dyroom); // [group][PQ] winner's index in its plane
     const long plane0 = (long)blockIdx.x * group;
     const int here = (int)(planes - plane0 < group ? planes - plane0 : group);
     const E* xp = x + plane0 * HW;
     const E* dyp = dy + plane0 * PQ;
-    for (int i = threadIdx.x; i < here * HW; i += EB) xs[i] = load_elem(xp + i);
-    for (int i = threadIdx.x; i < here * PQ; i += EB) dys[i] = load_elem(dyp + i);
+    load_run(xp, here * HW, pool_lds);
+    load_run(dyp, here * PQ, pool_lds + xroom);
+    const int shift = run_shift(xp);
+    float* xs = pool_lds + shift;                             // [group][HW]
+    const float* dys = pool_lds + xroom + run_shift(dyp);     // [group][PQ]
     __syncthreads();
     for (int o = threadIdx.x; o < here * PQ; o += EB) {
         const int pl = dPQ.div(o), pq = o - pl * PQ;
         const int p = dQ.div(pq), q = pq - p * Q;
-        const int first = p * SH * W + q * SW;
+        const int first = 2 * p * W + 2 * q;
         const float* b = xs + pl * HW + first;
         float m = -FLT_MAX;
         int a = first;
 #pragma unroll
-        for (int r = 0; r < R; r++)
+        for (int r = 0; r < 3; r++)
 #pragma unroll
-            for (int s_ = 0; s_ < S; s_++) {
+            for (int s_ = 0; s_ < 3; s_++) {
                 const float v = b[r * W + s_];
                 if (v > m) { m = v; a = first + r * W + s_; }
             }
         arg[o] = a;
     }
     __syncthreads();
-    E* dxp = dx + plane0 * HW;
-    for (int i = threadIdx.x; i < here * HW; i += EB) {
-        const int pl = dHW.div(i), self = i - pl * HW;
-        const int h = dW.div(self), w = self - h * W;
-        // windows containing (h, w): p * SH <= h <= p * SH + R - 1
-        int p_lo = h - R + 1; p_lo = p_lo <= 0 ? 0 : (p_lo + SH - 1) / SH;
-        int p_hi = h / SH; if (p_hi > P - 1) p_hi = P - 1;
-        int q_lo = w - S + 1; q_lo = q_lo <= 0 ? 0 : (q_lo + SW - 1) / SW;
-        int q_hi = w / SW; if (q_hi > Q - 1) q_hi = Q - 1;
-        const int* ap = arg + pl * PQ;
-        const float* dp = dys + pl * PQ;
-        float acc = 0.0f;
-        for (int p = p_lo; p <= p_hi; p++)
-            for (int q = q_lo; q <= q_hi; q++)
-                if (ap[p * Q + q] == self) acc += dp[p * Q + q];
-        if (gate && !(xs[i] > 0.0f)) acc = 0.0f;
-        store_elem(dxp + i, acc);
+    const int BH = (H + 1) / 2, BW = (W + 1) / 2;
+    for (int i = threadIdx.x; i < here * BH * BW; i += EB) {
+        const int pl = dBlocks.div(i), bl = i - pl * BH * BW;
+        const int p = dBW.div(bl), q = bl - p * BW;
+        // the windows (p - 1 | p, q - 1 | q), row by row
+        int win[2][2];
+        float d[2][2];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int v = 0; v < 2; v++) {
+                const int wp = p - 1 + u, wq = q - 1 + v;
+                const bool ok = (unsigned)wp < (unsigned)P && (unsigned)wq < (unsigned)Q;
+                const int at = ok ? pl * PQ + wp * Q + wq : 0;
+                win[u][v] = ok ? arg[at] : -1;
+                d[u][v] = dys[at];
+            }
+#pragma unroll
+        for (int eh = 0; eh < 2; eh++)
+#pragma unroll
+            for (int ew = 0; ew < 2; ew++) {
+                const int h = 2 * p + eh, w = 2 * q + ew;
+                if (h >= H || w >= W) continue;
+                const int self = h * W + w;
+                float acc = 0.0f;
+#pragma unroll
+                for (int u = eh; u < 2; u++) // an odd row lies in window row p only
+#pragma unroll
+                    for (int v = ew; v < 2; v++) acc += win[u][v] == self ? d[u][v] : 0.0f;
+                float* at = xs + pl * HW + self;
+                if (gate && !(*at > 0.0f)) acc = 0.0f;
+                *at = acc;
+            }
     }
+    __syncthreads();
+    store_run(dx + plane0 * HW, here * HW, pool_lds, shift);
 }
 
 // Overlapping windows on planes that fit LDS (AlexNet's 3x3 stride 2): a workgroup stages `group` whole
@@ -1183,7 +1259,7 @@ static int maxpool_fwd_t(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
         const long planes = (long)g.N * g.C;
         const long blocks = (planes + group - 1) / group;
         VDNN_REQUIRE(blocks < (1l << 31), "grid too large");
-        hipLaunchKernelGGL((maxpool_fwd_planes_kernel<E, 3, 3, 2, 2>), dim3((unsigned)blocks), dim3(EB), group * per_plane, st, x, y, g.H, g.W, g.P, g.Q,
+        hipLaunchKernelGGL(maxpool3x3s2_fwd_planes_kernel<E>, dim3((unsigned)blocks), dim3(EB), group * per_plane + 4 * POOL_RUN_PAD, st, x, y, g.H, g.W, g.P, g.Q,
                            planes, group, FastDiv::make(g.P * g.Q), FastDiv::make(g.Q));
     } else {
         const size_t total = (size_t)g.N * g.C * g.P * g.Q;
@@ -1219,8 +1295,9 @@ static int maxpool_bwd_t(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
         const long blocks = (planes + group - 1) / group;
         VDNN_REQUIRE(blocks < (1l << 31), "grid too large");
         if (pool_is_3x3_s2(g))
-            hipLaunchKernelGGL((maxpool_bwd_planes_fixed_kernel<E, 3, 3, 2, 2>), dim3((unsigned)blocks), dim3(EB), group * per_plane, st, x, dy, dx,
-                               g.H, g.W, g.P, g.Q, planes, group, gate, FastDiv::make(g.P * g.Q), FastDiv::make(g.Q), FastDiv::make(g.H * g.W), FastDiv::make(g.W));
+            hipLaunchKernelGGL(maxpool3x3s2_bwd_planes_kernel<E>, dim3((unsigned)blocks), dim3(EB), group * per_plane + 4 * (2 * POOL_RUN_PAD + 8), st, x, dy, dx,
+                               g.H, g.W, g.P, g.Q, planes, group, gate, FastDiv::make(g.P * g.Q), FastDiv::make(g.Q),
+                               FastDiv::make(((g.H + 1) / 2) * ((g.W + 1) / 2)), FastDiv::make((g.W + 1) / 2));
         else
             hipLaunchKernelGGL(maxpool_bwd_planes_kernel<E>, dim3((unsigned)blocks), dim3(EB), group * per_plane, st, x, dy, dx, g, planes, group, gate);
     } else {
