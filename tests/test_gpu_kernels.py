@@ -795,6 +795,29 @@ def test_maxpool_is_exact(ctx, n, c, h, w, win, stride, ties):
     assert np.array_equal(gdx, oracle.maxpool_bwd(og, x, wy, dy))
 
 
+@pytest.mark.parametrize("bf16", [False, True])
+@pytest.mark.parametrize("n,cout", [(1, 1), (15, 17), (64, 4096), (127, 16), (128, 1000), (129, 33), (300, 5)])
+def test_fc_bias_gradient_adds_the_rows_in_order(ctx, n, cout, bf16):
+    """Rows of less than a chunk of 128, of one, of one and a remainder: float additions in ascending row order, to the bit."""
+    dy = np.random.default_rng(n + cout).standard_normal((n, cout)).astype(np.float32)
+    if bf16:
+        dy = (dy.view(np.uint32) & 0xFFFF0000).view(np.float32)
+    want = np.zeros(cout, np.float32)
+    for row in dy:
+        want = want + row
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, int(bf16)))
+    try:
+        with Dev(ctx) as d:
+            src = d.up((dy.view(np.uint32) >> 16).astype(np.uint16), np.uint16) if bf16 else d.up(dy)
+            out = d.empty((cout,))
+            announce("fc bias gradient", (n, cout), "bf16" if bf16 else "f32")
+            check(lib.vdnn_fc_bwd_bias(ctx.handle, None, n, cout, src.ptr, out.ptr))
+            got = out.download((cout,))
+    finally:
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+    assert np.array_equal(got, want)
+
+
 # 3x3 / stride 2 on planes in LDS: even and odd extents, the smallest plane, tensors that begin anywhere in their 16 bytes
 # (gradients beginning at the same place as the input and elsewhere).
 @pytest.mark.parametrize("bf16", [0, 1])
