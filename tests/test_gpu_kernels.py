@@ -685,6 +685,28 @@ def test_bias_gradients_at_any_plane_and_alignment(ctx, n, k, p, q, bf16):
     assert np.all(np.abs(got_fb - want) <= 2.0 ** -24 * (20 + n / 16) * mag)
 
 
+@pytest.mark.parametrize("bf16", [0, 1])
+def test_bias_gradient_of_few_channels_uses_the_chip(ctx, bf16):
+    """The same bytes as 8 planes of 56 x 56 a sample and as 512 of 7 x 7: few channels are no reason to leave the chip to
+    eight workgroups (that took 27 us against 6; in two stages 8)."""
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, bf16))
+    try:
+        with Dev(ctx) as d:
+            dy, b = d.empty((128, 8, 56, 56), np.uint16 if bf16 else np.float32), d.empty((512,))
+            check(lib.vdnn_fill(ctx.handle, None, 128 * 8 * 56 * 56, 0.5, dy.ptr))
+            best = {}
+            for k, hw in ((8, 56), (512, 7)) * 8:
+                g = be.shape(128, 3, hw, hw, k, 1, 1, 0, 0, 1, 1)
+                announce("bias gradient of few channels", k, hw, bf16)
+                be.profile_enable(ctx.handle, 1)
+                check(lib.vdnn_conv_bwd_bias(ctx.handle, None, g, dy.ptr, b.ptr))
+                best[k] = min(best.get(k, 1e9), be.profile_collect(ctx.handle)["conv_bwd_bias"]["ms"])
+    finally:
+        be.profile_enable(ctx.handle, 0)
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+    assert best[8] < 2.5 * best[512], best
+
+
 def _fc_all(ctx, x, w, b, dy, alpha):
     n, cin = x.shape
     cout = w.shape[0]

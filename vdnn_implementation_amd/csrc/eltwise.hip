@@ -1130,15 +1130,17 @@ int vdnn::launch_bias_grad_final(vdnn_ctx* ctx, hipStream_t st, const float* par
     return VDNN_OK;
 }
 
-// `splits`, `per`: from bias_grad_splits. Where a channel has less than one trip of a workgroup per split to read (four
-// accesses a thread), one workgroup takes the channel whole and writes the bias itself: the second launch costs more
-// (3 us) than the wider grid gives.
+// `splits`, `per`: from bias_grad_splits. A channel that a single workgroup reads in a few trips (four accesses a thread
+// each) is left to one, which writes the bias itself: the second launch costs 2-3 us, a trip 0.4 us. 750 calls of 2 to 600
+// channels, one workgroup against two stages: 3.1 against 5.3 us at one trip, 4.2 against 5.7 at four, 4.9 against 5.7 at
+// six, even at seven or eight, 12 against 5.3 at twenty and 27 against 5.4 at fifty (few channels: the other units idle).
+constexpr int BIAS_GRAD_TRIPS = 6;
 template <class E>
 static int bias_grad_launch(hipStream_t st, const E* dy, float* bias, float* partials, int N, int K, int PQ, int splits, int per,
                             float alpha, int accumulate) {
     constexpr int V = 16 / (int)sizeof(E);
     const int pqv = (PQ + V - 1) / V;
-    if ((long)N * pqv < 4l * EB * splits) { splits = 1; per = N; }
+    if ((long)N * pqv <= BIAS_GRAD_TRIPS * 4l * EB && (long)N * pqv < 4l * EB * splits) { splits = 1; per = N; }
     const BiasGradWalk walk{pqv, EB / pqv, EB % pqv};
     hipLaunchKernelGGL(bias_grad_partial_kernel<E>, dim3(K * splits), dim3(EB), 0, st, dy, splits == 1 ? bias : partials, N, K, PQ, splits, per, walk, alpha, accumulate);
     VDNN_LAUNCH_CHECK();
