@@ -818,9 +818,10 @@ def test_maxpool_is_exact(ctx, n, c, h, w, win, stride, ties):
 
 
 @pytest.mark.parametrize("bf16", [False, True])
-@pytest.mark.parametrize("n,cout", [(1, 1), (15, 17), (64, 4096), (127, 16), (128, 1000), (129, 33), (300, 5)])
+@pytest.mark.parametrize("n,cout", [(1, 1), (2, 300), (11, 257), (12, 256), (15, 17), (64, 4096), (127, 16), (128, 1000), (129, 33), (300, 5)])
 def test_fc_bias_gradient_adds_the_rows_in_order(ctx, n, cout, bf16):
-    """Rows of less than a chunk of 128, of one, of one and a remainder: float additions in ascending row order, to the bit."""
+    """A handful of rows, on both sides of the rule that tells them; rows of less than a chunk of 128, of one, of one and a
+    remainder: float additions in ascending row order, to the bit."""
     dy = np.random.default_rng(n + cout).standard_normal((n, cout)).astype(np.float32)
     if bf16:
         dy = (dy.view(np.uint32) & 0xFFFF0000).view(np.float32)

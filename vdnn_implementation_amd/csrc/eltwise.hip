@@ -512,6 +512,18 @@ __global__ void __launch_bounds__(EB) fc_bias_grad_kernel(const E* __restrict__ 
     bias[o] = accumulate ? __fmaf_rn(alpha, s, bias[o]) : alpha * s;
 }
 
+// The same with a handful of rows: one thread per column. Up to eleven rows the walk is shorter than the way through LDS
+// (1-4 rows of 18 to 4200 columns 2.1 against 2.6 us, 8 rows 2.4 against 2.6, 11 rows even, 16 rows 3.5 against 2.7).
+constexpr int FBG_FEW_ROWS = 11;
+template <class E>
+__global__ void __launch_bounds__(EB) fc_bias_grad_few_rows_kernel(const E* __restrict__ dy, float* __restrict__ bias, int N, int Cout, float alpha, int accumulate) {
+    const int o = blockIdx.x * EB + threadIdx.x;
+    if (o >= Cout) return;
+    float s = 0.0f;
+    for (int n = 0; n < N; n++) s += load_elem(dy + (size_t)n * Cout + o);
+    bias[o] = accumulate ? __fmaf_rn(alpha, s, bias[o]) : alpha * s;
+}
+
 // ---- max pooling --------------------------------------------------------------------------------
 struct PoolGeo { int N, C, H, W, R, S, P, Q, ph, pw, sh, sw; };
 
@@ -1226,7 +1238,10 @@ template <class E>
 static int fc_bwd_bias_impl(vdnn_ctx* ctx, vdnn_stream_t stream, int n, int c_out, const void* dy, float* bias, float alpha, int accumulate) {
     VDNN_KERNEL_PROLOGUE(ctx);
     VDNN_REQUIRE(dy && bias && n > 0 && c_out > 0, "bad argument");
-    hipLaunchKernelGGL(fc_bias_grad_kernel<E>, dim3((c_out + FBG_COLS - 1) / FBG_COLS), dim3(EB), 0, stream_of(ctx, stream), (const E*)dy, bias, n, c_out, alpha, accumulate);
+    if (n <= FBG_FEW_ROWS)
+        hipLaunchKernelGGL(fc_bias_grad_few_rows_kernel<E>, dim3((c_out + EB - 1) / EB), dim3(EB), 0, stream_of(ctx, stream), (const E*)dy, bias, n, c_out, alpha, accumulate);
+    else
+        hipLaunchKernelGGL(fc_bias_grad_kernel<E>, dim3((c_out + FBG_COLS - 1) / FBG_COLS), dim3(EB), 0, stream_of(ctx, stream), (const E*)dy, bias, n, c_out, alpha, accumulate);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
 }
