@@ -650,7 +650,7 @@ def test_conv_results_do_not_depend_on_the_run(ctx):
 
 @pytest.mark.parametrize("bf16", [False, True])
 @pytest.mark.parametrize("n,k,p,q", [(3, 5, 1, 1), (5, 7, 1, 3), (2, 3, 1, 4), (3, 4, 1, 7), (4, 3, 2, 4), (3, 2, 3, 3), (300, 3, 13, 13),
-                                     (2, 70, 31, 33), (33, 96, 55, 55)])
+                                     (37, 6, 40, 40), (2, 70, 31, 33), (33, 96, 55, 55)])
 def test_bias_gradients_at_any_plane_and_alignment(ctx, n, k, p, q, bf16):
     """Planes of less than one access, of one, of one and a remainder; one workgroup per channel and several; a tensor one
     element past an aligned address. The bias gradients of convolution and fully connected layers against sums in
