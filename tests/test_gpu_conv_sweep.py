@@ -124,6 +124,24 @@ def test_conv_small_tile(ctx, geom):
     assert_close(gpu_conv_bwd_filter(ctx, g, x, dy, zero, np.float32(1.0)), oracle.conv_bwd_filter_sgd(og, x, dy, zero, 1.0), TOL, "bwd filter")
 
 
+@pytest.mark.parametrize("geom", [(4, 64, 16, 16, 64, 5, 5, 2, 2, 1, 1), (16, 64, 14, 14, 128, 1, 1, 0, 0, 1, 1), (8, 128, 12, 12, 192, 5, 5, 2, 2, 1, 1),
+                                  (32, 96, 16, 16, 70, 1, 1, 0, 0, 1, 1), (2, 64, 28, 28, 256, 5, 5, 2, 2, 1, 1)], ids=lambda g: "x".join(map(str, g)))
+def test_backward_filter_bits_do_not_depend_on_the_address(ctx, geom):
+    """dy at a 16-byte boundary and one element past it: other loaders, the same tile and splits, so the same sums."""
+    rng = np.random.default_rng(sum(geom))
+    g = be.shape(*geom)
+    x, dy = rng.standard_normal((g.n, g.c, g.h, g.w)).astype(np.float32), rng.standard_normal((g.n, g.k, g.h, g.w)).astype(np.float32)
+    announce("backward filter, dy aligned and not", geom)
+    with Dev(ctx) as d:
+        xx, out = d.f32(x), [d.f32(np.zeros((g.k, g.c, g.r, g.s))) for _ in range(2)]
+        for shift, dw in enumerate(out):
+            b = d.f32(np.concatenate([np.zeros(shift, np.float32), dy.ravel()]))
+            assert b.ptr % 16 == 0
+            check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, xx.ptr, b.ptr + 4 * shift, dw.ptr, None, 0))
+        got = [dw.download((g.k, g.c, g.r, g.s)) for dw in out]
+    assert np.array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("n,cin,cout", [(1, 64, 1), (63, 17, 65), (65, 192, 64), (3, 193, 129), (64, 1028, 260), (130, 5, 7)])
 def test_fc_small_tile(ctx, n, cin, cout):
     rng = np.random.default_rng(n * 7 + cin * 3 + cout)

@@ -1435,9 +1435,10 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
     const int want = choose_splits(tiles, Kred, cap, ctx->num_cu, out_bytes, 2.0 * TM * TN * KB);
     const bool vec = PQ % 4 == 0 && aligned16(dy); // bf16: four elements are 8 bytes, covered by the same test
     const bool tap_planes = vec && PQ >= KB && 2 * g.Q >= KB; // planes the tap-major loaders take
-    // the 64x64 tile; its loaders have a column's tap to work out per element unless a tile's columns share it
-    const bool small_tap = tap_planes && g.C % 32 == 0;
-    const SmallTilePlan plan = small_tile_plan(M, N, Kred, staging ? staging_bytes : 0, ctx->num_cu, 2, false, tap_planes && g.C % 64 == 0 ? 1.05 : 1.9);
+    // the 64x64 tile; its loaders have a column's tap to work out per element unless a tile's columns share it. Tile and
+    // splits go by the shape alone (an aligned dy): they decide the order of the sums, which is not to change with an address
+    const bool small_tap = tap_planes && g.C % 32 == 0, tap_shape = PQ % 4 == 0 && PQ >= KB && 2 * g.Q >= KB;
+    const SmallTilePlan plan = small_tile_plan(M, N, Kred, staging ? staging_bytes : 0, ctx->num_cu, 2, false, tap_shape && g.C % 64 == 0 ? 1.05 : 1.9);
     // one split's samples of dy and of x are addressed through one descriptor with summed offsets
     auto span_ok = [&](int kchunk) {
         const long nspan = kchunk / PQ + 2;
@@ -1445,7 +1446,7 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
     };
     const GemmDims d_small = make_dims(M, N, (int)Kred, 64, 64, plan.splits);
     const bool small = (Kred <= kShortReduction || (2.0 * M * (double)N * (double)Kred <= kSmallTileOps &&
-                                                    plan.us < 0.9 * large_tile_us(M, N, Kred, TM, TN, want, ctx->num_cu, true, tap_planes && g.C % 32 == 0 ? 1.0 : 1.15))) &&
+                                                    plan.us < 0.9 * large_tile_us(M, N, Kred, TM, TN, want, ctx->num_cu, true, tap_shape && g.C % 32 == 0 ? 1.0 : 1.15))) &&
                        span_ok(d_small.kchunk);
     const GemmDims d = small ? d_small : make_dims(M, N, (int)Kred, TM, TN, want);
     VDNN_REQUIRE(span_ok(d.kchunk), "samples of one reduction split too large for one descriptor");
