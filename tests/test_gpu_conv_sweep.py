@@ -206,7 +206,10 @@ def test_strided_backward_data(ctx, geom):
 @pytest.mark.parametrize("geom", [
     (2, 33, 8, 18, 31, 3, 3, 1, 1, 1, 1), (3, 12, 6, 64, 13, 3, 3, 1, 1, 1, 1), (2, 95, 14, 14, 65, 3, 3, 1, 1, 1, 1), (2, 40, 9, 12, 20, 5, 5, 2, 2, 1, 1),
     (2, 47, 7, 9, 49, 3, 3, 1, 1, 1, 1), (3, 15, 11, 13, 48, 3, 3, 0, 0, 1, 1), (2, 70, 13, 9, 130, 3, 3, 1, 1, 2, 2), (2, 129, 10, 16, 79, 1, 1, 0, 0, 1, 1),
-    (5, 300, 5, 5, 200, 1, 1, 0, 0, 1, 1)], ids=lambda g: "x".join(map(str, g)))
+    (5, 300, 5, 5, 200, 1, 1, 0, 0, 1, 1),
+    # large enough for the bfloat16 engine in both directions
+    (2, 33, 40, 58, 31, 3, 3, 1, 1, 1, 1), (6, 12, 52, 64, 13, 3, 3, 1, 1, 1, 1), (4, 95, 26, 14, 65, 3, 3, 1, 1, 1, 1), (4, 40, 40, 40, 20, 5, 5, 2, 2, 1, 1),
+    (11, 47, 31, 29, 49, 3, 3, 1, 1, 1, 1), (18, 15, 43, 45, 48, 3, 3, 0, 0, 1, 1), (12, 129, 40, 46, 79, 1, 1, 0, 0, 1, 1)], ids=lambda g: "x".join(map(str, g)))
 def test_padded_channels(ctx, geom):
     rng = np.random.default_rng(sum((i + 1) * v for i, v in enumerate(geom)))
     g, og = be.shape(*geom), oracle.shape(*geom)
@@ -234,3 +237,41 @@ def test_padded_channels(ctx, geom):
                     close(get(dx, x.shape)[rows], want_dx[rows], "bwd data")
         finally:
             check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
+def kernels_of(ctx, g, which, bf16):
+    """Names of the kernels of one call on zeros."""
+    P, Q = lib.vdnn_out_dim(g.h, g.pad_h, g.r, g.stride_h), lib.vdnn_out_dim(g.w, g.pad_w, g.s, g.stride_w)
+    x, y, w = (g.n, g.c, g.h, g.w), (g.n, g.k, P, Q), (g.k, g.c, g.r, g.s)
+    check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, int(bf16)))
+    try:
+        with Dev(ctx) as d:
+            act = lambda shape: d.act(np.zeros(shape, np.float32)) if bf16 else d.f32(np.zeros(shape, np.float32))
+            a, b, f = act(x), act(y), d.f32(np.zeros(w, np.float32))
+            be.profile_enable(ctx.handle, 1)
+            if which == "fwd":
+                check(lib.vdnn_conv_fwd(ctx.handle, None, g, 0, a.ptr, f.ptr, None, b.ptr, None, 0))
+            elif which == "bwd data":
+                check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, b.ptr, f.ptr, a.ptr, None, 0))
+            else:
+                check(lib.vdnn_conv_bwd_filter(ctx.handle, None, g, 0, a.ptr, b.ptr, f.ptr, None, 0))
+            return set(be.profile_collect(ctx.handle))
+    finally:
+        be.profile_enable(ctx.handle, 0)
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
+# Which route a layer takes is decided by its size: on a grid of a few tiles the routes made for large layers were up to
+# 2.9 times slower than those they replaced. (pass, bfloat16, geometry, part of the kernel's name, taken or not; both sides of
+# each rule, by a factor of two or more)
+@pytest.mark.parametrize("which,bf16,geom,name,taken", [
+    # padded channels on the bfloat16 engine: windowed, pairs, single pixels
+    ("fwd", 1, (1, 18, 8, 8, 16, 3, 3, 1, 1, 1, 1), "bf16", False), ("fwd", 1, (4, 95, 40, 40, 65, 3, 3, 1, 1, 1, 1), "bf16win", True),
+    ("fwd", 1, (8, 12, 4, 4, 64, 1, 1, 0, 0, 1, 1), "bf16", False), ("fwd", 1, (12, 129, 60, 60, 79, 1, 1, 0, 0, 1, 1), "bf16mfma", True),
+    ("bwd data", 1, (11, 57, 5, 5, 45, 2, 2, 1, 1, 1, 1), "bf16", False), ("bwd data", 1, (22, 47, 31, 29, 49, 3, 3, 1, 1, 1, 1), "bf16mfma", True),
+    ("bwd data", 1, (27, 73, 95, 95, 16, 1, 1, 0, 0, 1, 1), "bf16", False),  # a reduction of half a block, however large the layer
+], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
+def test_route_by_size(ctx, which, bf16, geom, name, taken):
+    announce("route", which, bf16, geom)
+    names = kernels_of(ctx, be.shape(*geom), which, bf16)
+    assert any(name in n for n in names) == taken, names

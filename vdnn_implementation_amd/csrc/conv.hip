@@ -19,6 +19,7 @@
 #include "conv_smallc_mfma.h"
 #include "winograd_f32.h"
 #include "conv_strided.h"
+#include <cmath>
 
 namespace vdnn {
 
@@ -528,21 +529,44 @@ static int launch_winograd_wgrad(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g
     return VDNN_OK;
 }
 
-// The bfloat16 engine's filter operand lives at the front of the staging area (rounded and re-laid-out by a
-// small kernel before every use: the master copy changes every step); what is left holds partial sums.
-// Channels that are no whole blocks of 32 are padded with zeros in the filter operand and not fetched in the other one. From
-// twelve channels on that is the faster route (the float engine with its per-element taps reaches 60-110 TFLOP/s, this
-// engine's 300-700 times the share of the block that is used):
+// The bfloat16 engine's kernels for a geometry: the windowed one (one staged window per filter row serves the three taps of a
+// 3x3 at stride 1 with padding 1), a pixel pair per lane where the pairs of an output row are contiguous in the input, or a
+// pixel per lane.
+enum class HalfKernel { WINDOWED, PAIRS, SINGLE };
+template <int MODE>
+static HalfKernel half_kernel(const LoadIm2colPix<MODE, false, bf16_t>& pix) {
+    if (win3x3_ok(pix.R, pix.S, pix.ph, pix.pw, pix.sh, pix.sw, pix.Hs, pix.Ws, pix.OH, pix.OW, pix.sample_elems)) return HalfKernel::WINDOWED;
+    const bool pairs = pix.OW % 2 == 0 && pix.S <= 16 && pix.Ws >= pix.S && pix.Ws > pix.pw + 1 && (MODE == 1 || pix.sw == 1);
+    return pairs ? HalfKernel::PAIRS : HalfKernel::SINGLE;
+}
+
+// Channels that are no whole blocks of 32 are padded with zeros in the filter operand and not fetched in the other one: from
+// twelve channels on, where the layer is large enough. This engine has tiles of 128x128 and 64x256 only; on a grid that such
+// tiles leave mostly idle the float engine's 64x64 ones are faster, although it multiplies at a sixteenth of the rate (8 x 12 x 4
+// x 4, 64 filters of 1x1 forward 18.8 us here, 7.8 there; 11 x 57 x 5 x 5, 45 of 2x2 backward data 35.7 and 12.4). The lines
+// are those of least loss over 3200 calls of 12 to 600 channels, timed on both: operations, with few rows counting for more
+// (a tile has 64 of them whatever the layer has). By them the choice is 1.2 % behind the better route's time in the mean; with
+// this engine for all of them it was 15 % behind.
 // 32 x 200 x 28 x 28, 300 filters of 3x3 forward 364 -> 48 us, backward data 338 -> 72; 64 x 130 x 13 x 13, 390 of 5x5 347 -> 127
 // and 468 -> 147; 16 x 12 x 112 x 112, 20 of 3x3 55 -> 25 and 83 -> 24.
 constexpr int kHalfMinChannels = 12;
-static bool half_engine_ok(const vdnn_ctx* ctx, int reduced_channels, int rows, int RS) {
+static bool half_pad_pays(HalfKernel kernel, int rows, long N, int reduced_channels, int RS) {
+    const double weighed = 2.0 * N * (double)reduced_channels * RS * std::sqrt(64.0 * rows);
+    if (kernel == HalfKernel::WINDOWED) return weighed >= 1e8;
+    return reduced_channels * RS > KH && weighed >= (kernel == HalfKernel::PAIRS ? 3e8 : 4e8);
+}
+
+// The bfloat16 engine's filter operand lives at the front of the staging area (rounded and re-laid-out by a
+// small kernel before every use: the master copy changes every step); what is left holds partial sums.
+template <int MODE>
+static bool half_engine_ok(const vdnn_ctx* ctx, const LoadIm2colPix<MODE, false, bf16_t>& pix, int reduced_channels, int rows, int RS) {
     if (RS > 32 || !ctx->reduce_scratch) return false;
     const size_t elems = (size_t)rows * RS * reduced_channels, padded = (size_t)rows * RS * ((reduced_channels + KH - 1) / KH * KH);
     if (padded * 2 + (16u << 20) > ctx->reduce_scratch_bytes || padded * 2 >= 0x7FFF0000ul) return false;
     if (reduced_channels % KH == 0) return true;
     // (a filter too large for the float route's rounded copy stays refused)
-    return reduced_channels >= kHalfMinChannels && elems * 4 + (8u << 20) <= ctx->reduce_scratch_bytes;
+    return reduced_channels >= kHalfMinChannels && elems * 4 + (8u << 20) <= ctx->reduce_scratch_bytes &&
+           half_pad_pays(half_kernel(pix), rows, (long)pix.nsamples * pix.OH * pix.OW, reduced_channels, RS);
 }
 
 static int launch_pack_filter_bf16(vdnn_ctx* ctx, hipStream_t st, const float* w, unsigned short* packed, int rows, int Cred, int RS,
@@ -610,13 +634,12 @@ static int conv_half_engine_with(vdnn_ctx* ctx, hipStream_t st, const PassNames&
     if (rc != VDNN_OK) return rc;
     ep.partial = (float*)((char*)ctx->reduce_scratch + taken);
     LoadPackedH al{packed, (long)K, rows, (unsigned)(filter_elems * 2)};
-    // 3x3 at stride 1 with padding 1: one staged window per filter row serves its three taps
-    if (win3x3_ok(pix.R, pix.S, pix.ph, pix.pw, pix.sh, pix.sw, pix.Hs, pix.Ws, pix.OH, pix.OW, pix.sample_elems)) {
+    const HalfKernel kernel = half_kernel(pix);
+    if (kernel == HalfKernel::WINDOWED) {
         const Win3x3 geo{pix.src, pix.Hs, pix.Ws, pix.sample_elems, pix.sample_elems * pix.nsamples, pix.nsamples, Cred};
         return launch_win3x3<MODE, bf16_t, PAD>(ctx, st, MODE == 0 ? kFwdWin3Names : kBwdDataWin3Names, al, geo, ep, rows, N, K, flops, left);
     }
-    // a pixel pair per lane where the pairs of an output row are contiguous in the input
-    if (pix.OW % 2 == 0 && pix.S <= 16 && pix.Ws >= pix.S && pix.Ws > pix.pw + 1 && (MODE == 1 || pix.sw == 1)) {
+    if (kernel == HalfKernel::PAIRS) {
         LoadIm2colPixTapH2<MODE, PAD> bl2{pix, Cred};
         return launch_by_m<LoadPackedH, LoadIm2colPixTapH2<MODE, PAD>, bf16_t, true>(ctx, st, names, al, bl2, ep, rows, N, K, flops, left);
     }
@@ -1074,10 +1097,10 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
     const int K = g.C * g.R * g.S;
     const unsigned wbytes = (unsigned)((long)g.K * K * 4);
     if constexpr (sizeof(E) == 2) {
-        if (half_engine_ok(ctx, g.C, g.K, g.R * g.S)) {
-            const int RS = g.R * g.S;
-            LoadIm2colPix<0, false, bf16_t> pix{x, g.H, g.W, g.P, g.Q, g.R, g.S, g.ph, g.pw, g.sh, g.sw, (long)g.C * g.H * g.W, g.N,
-                                               FastDiv::make(RS), FastDiv::make(g.S)};
+        const int RS = g.R * g.S;
+        const LoadIm2colPix<0, false, bf16_t> pix{x, g.H, g.W, g.P, g.Q, g.R, g.S, g.ph, g.pw, g.sh, g.sw, (long)g.C * g.H * g.W, g.N,
+                                                 FastDiv::make(RS), FastDiv::make(g.S)};
+        if (half_engine_ok(ctx, pix, g.C, g.K, RS)) {
             StoreNCHW<bf16_t> ep{y, bias, g.P * g.Q, nullptr, relu, nullptr};
             return conv_half_engine<0>(ctx, st, kFwdHalfNames, w, g.K, g.C, RS, g.C * RS, RS, pix, ep, g.N * g.P * g.Q,
                                        2.0 * g.N * (double)g.K * K * g.P * g.Q);
@@ -1176,8 +1199,9 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
         if (taken || rc != VDNN_OK) return rc;
     }
     bool half_engine = false;
+    const LoadIm2colPix<1, false, E> pix{dy, g.P, g.Q, g.H, g.W, g.R, g.S, g.ph, g.pw, 1, 1, (long)g.K * g.P * g.Q, g.N, FastDiv::make(g.R * g.S), FastDiv::make(g.S)};
     if constexpr (sizeof(E) == 2) {
-        half_engine = !few_channels && g.sh == 1 && g.sw == 1 && half_engine_ok(ctx, g.K, g.C, g.R * g.S);
+        half_engine = !few_channels && g.sh == 1 && g.sw == 1 && half_engine_ok(ctx, pix, g.K, g.C, g.R * g.S);
         if (!half_engine) {
             w = rounded_filter_copy(ctx, st, carve, w, (size_t)g.K * g.C * g.R * g.S);
             VDNN_REQUIRE(w != nullptr, "filter too large for the staging area (bfloat16 layer outside the bfloat16 engine)");
@@ -1278,7 +1302,6 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
     const double flops = 2.0 * g.N * (double)g.K * g.C * RS * g.P * g.Q;
     if constexpr (sizeof(E) == 2) {
         if (half_engine) {
-            LoadIm2colPix<1, false, bf16_t> pix{dy, g.P, g.Q, g.H, g.W, g.R, g.S, g.ph, g.pw, 1, 1, sample, g.N, dRS, dS};
             return conv_half_engine<1>(ctx, st, kBwdDataHalfNames, w, g.C, g.K, RS, RS, g.C * RS, pix, ep, N, flops);
         }
     }
