@@ -404,6 +404,16 @@ def test_conv_bf16_tensors_at_odd_element_offsets(ctx):
     (3, 70, 21, 19, 130, 3, 3, 1, 1, 2, 2),   # strided
     (2, 6, 16, 23, 66, 3, 1, 1, 0, 1, 3),     # strided in the columns only
     (2, 9, 17, 17, 24, 11, 11, 0, 0, 1, 1),
+    # the same, large enough for the bfloat16 engine
+    (211, 60, 4, 4, 50, 3, 3, 1, 1, 1, 1),
+    (59, 33, 15, 7, 70, 3, 3, 1, 1, 1, 1),
+    (23, 20, 26, 9, 130, 3, 5, 0, 2, 1, 1),
+    (12, 22, 13, 13, 165, 5, 5, 2, 2, 1, 1),
+    (13, 7, 31, 6, 133, 6, 6, 5, 5, 1, 1),
+    (23, 60, 27, 3, 160, 3, 3, 1, 2, 1, 1),
+    (14, 70, 41, 19, 130, 3, 3, 1, 1, 2, 2),
+    (31, 66, 26, 23, 266, 3, 1, 1, 0, 1, 3),
+    (11, 19, 21, 21, 24, 11, 11, 0, 0, 1, 1),
 ])
 def test_bwd_filter_on_padded_rows(ctx, geom):
     """Backward filter of planes that are no whole groups of pixels, against sums in double of the same bfloat16 values: the

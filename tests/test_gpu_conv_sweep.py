@@ -270,6 +270,9 @@ def kernels_of(ctx, g, which, bf16):
     ("fwd", 1, (8, 12, 4, 4, 64, 1, 1, 0, 0, 1, 1), "bf16", False), ("fwd", 1, (12, 129, 60, 60, 79, 1, 1, 0, 0, 1, 1), "bf16mfma", True),
     ("bwd data", 1, (11, 57, 5, 5, 45, 2, 2, 1, 1, 1, 1), "bf16", False), ("bwd data", 1, (22, 47, 31, 29, 49, 3, 3, 1, 1, 1, 1), "bf16mfma", True),
     ("bwd data", 1, (27, 73, 95, 95, 16, 1, 1, 0, 0, 1, 1), "bf16", False),  # a reduction of half a block, however large the layer
+    # padded rows on the bfloat16 engine: groups of four pixels, single pixels (strided)
+    ("bwd filter", 1, (2, 12, 13, 13, 65, 5, 5, 2, 2, 1, 1), "bf16", False), ("bwd filter", 1, (24, 22, 13, 13, 165, 5, 5, 2, 2, 1, 1), "bf16", True),
+    ("bwd filter", 1, (5, 26, 32, 32, 5, 3, 3, 1, 1, 2, 2), "bf16", False), ("bwd filter", 1, (28, 70, 41, 19, 130, 3, 3, 1, 1, 2, 2), "bf16", True),
 ], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_route_by_size(ctx, which, bf16, geom, name, taken):
     announce("route", which, bf16, geom)
