@@ -165,7 +165,10 @@ def test_fc_small_tile(ctx, n, cin, cout):
 # the window plus stride, one tile and many, enough filters for split reductions.
 STRIDED = [(2, 5, 9, 11, 7, 3, 3, 1, 1, 2, 2), (1, 17, 8, 8, 33, 1, 1, 0, 0, 2, 2), (3, 70, 13, 9, 130, 3, 3, 1, 1, 2, 2), (2, 6, 10, 7, 16, 4, 4, 3, 3, 2, 2),
            (2, 64, 7, 30, 48, 5, 5, 2, 2, 2, 2), (1, 9, 12, 12, 5, 3, 3, 0, 0, 1, 2), (2, 9, 12, 13, 20, 3, 2, 0, 1, 3, 1), (1, 8, 17, 5, 40, 5, 3, 2, 0, 4, 1),
-           (1, 65, 3, 3, 600, 3, 3, 0, 0, 2, 2), (4, 40, 64, 66, 31, 3, 3, 1, 1, 2, 2), (1, 7, 20, 21, 18, 11, 11, 5, 5, 2, 2)]
+           (1, 65, 3, 3, 600, 3, 3, 0, 0, 2, 2), (4, 40, 64, 66, 31, 3, 3, 1, 1, 2, 2), (1, 7, 20, 21, 18, 11, 11, 5, 5, 2, 2),
+           # the small ones above again, large enough for the classes in both element types
+           (20, 25, 39, 21, 27, 3, 3, 1, 1, 2, 2), (8, 67, 28, 28, 333, 1, 1, 0, 0, 2, 2), (8, 36, 30, 27, 40, 4, 4, 3, 3, 2, 2), (3, 49, 32, 42, 65, 3, 3, 0, 0, 1, 2),
+           (4, 39, 32, 33, 130, 3, 2, 0, 1, 3, 1), (2, 28, 57, 15, 40, 5, 3, 2, 0, 4, 1), (6, 65, 7, 7, 600, 3, 3, 0, 0, 2, 2)]
 
 
 @pytest.mark.parametrize("geom", STRIDED, ids=lambda g: "x".join(map(str, g)))
@@ -273,6 +276,10 @@ def kernels_of(ctx, g, which, bf16):
     # padded rows on the bfloat16 engine: groups of four pixels, single pixels (strided)
     ("bwd filter", 1, (2, 12, 13, 13, 65, 5, 5, 2, 2, 1, 1), "bf16", False), ("bwd filter", 1, (24, 22, 13, 13, 165, 5, 5, 2, 2, 1, 1), "bf16", True),
     ("bwd filter", 1, (5, 26, 32, 32, 5, 3, 3, 1, 1, 2, 2), "bf16", False), ("bwd filter", 1, (28, 70, 41, 19, 130, 3, 3, 1, 1, 2, 2), "bf16", True),
+    # strided backward data by residue classes
+    ("bwd data", 0, (8, 96, 55, 55, 8, 2, 2, 1, 1, 2, 2), "classes", False), ("bwd data", 0, (8, 40, 64, 66, 64, 3, 3, 1, 1, 2, 2), "classes", True),
+    ("bwd data", 0, (1, 17, 8, 8, 33, 3, 3, 1, 1, 2, 2), "classes", False), ("bwd data", 1, (4, 358, 40, 19, 4, 2, 2, 0, 0, 1, 3), "classes", False),
+    ("bwd data", 1, (2, 34, 16, 16, 66, 3, 3, 1, 1, 2, 2), "classes", True),
 ], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_route_by_size(ctx, which, bf16, geom, name, taken):
     announce("route", which, bf16, geom)

@@ -941,6 +941,21 @@ static int launch_fwd_smallc3x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g,
     return VDNN_OK;
 }
 
+// Backward data by residue classes saves matrix work and pays with float results in the staging area, read again by the
+// merge: it loses where a pixel of dx has few products (32 x 128 x 94 x 94, 2 filters of 3x3 at stride 3x1: 106 us in one
+// product, 282 by classes; 57 x 121 x 89 x 89 bfloat16, 7 of 1x1 at stride 2: 103 and 232). Both times are estimated, from 4900
+// calls timed on both routes: launches, matrix work (by classes at 94 TFLOP/s; in one product, with per-element taps, at
+// 58, a bfloat16 layer at 66 with its filter to round first), and what moving the elements of dx adds. The choice is 0.6 %
+// (floats) and 0.4 % (bfloat16) behind the better route in the mean.
+static bool classes_pay(const ConvGeo& g, int elem_bytes, bool gated) {
+    const double reduction = (double)g.K * g.R * g.S, pixels = (double)g.N * g.H * g.W, elems = 1e-6 * pixels * g.C;
+    const double rows = (g.C + 63) / 64 * 64, padded = (double)((g.K + KB - 1) / KB * KB) * g.R * g.S;
+    const double classes_us = 14.1 + 1.07e-8 * 2.0 * padded * rows * pixels / (g.sh * g.sw) + (gated ? 4.6 : 3.9) * elems;
+    const double one_us = elem_bytes == 2 ? 11.2 + 0.31 * std::sqrt(reduction) + 1.52e-8 * 2.0 * reduction * rows * pixels + (gated ? 2.8 : 1.7) * elems
+                                          : 7.7 + 0.28 * std::sqrt(reduction) + 1.72e-8 * 2.0 * reduction * rows * pixels + (gated ? 1.7 : 1.3) * elems;
+    return classes_us < one_us;
+}
+
 // Backward data of a strided layer by residue classes (conv_strided.h): as many samples at a time as the staging area
 // holds results of, 64x64 tiles, the reductions cut so that the workgroups of all classes together fill the chip.
 template <class E>
@@ -948,7 +963,7 @@ static int launch_strided_bwd_data(vdnn_ctx* ctx, hipStream_t st, const ConvGeo&
     *taken = false;
     const int classes = g.sh * g.sw;
     // (samples that the one product's tiles could not address stay refused by the caller)
-    if (classes > kStridedClasses || !ctx->reduce_scratch || !pixel_tile_span_ok((long)g.K * g.P * g.Q, g.H * g.W, 256, (int)sizeof(E))) return VDNN_OK;
+    if (classes > kStridedClasses || !classes_pay(g, (int)sizeof(E), gate != nullptr) || !ctx->reduce_scratch || !pixel_tile_span_ok((long)g.K * g.P * g.Q, g.H * g.W, 256, (int)sizeof(E))) return VDNN_OK;
     StridedGeo q{};
     q.sh = g.sh; q.sw = g.sw; q.ph = g.ph; q.pw = g.pw;
     q.C = g.C; q.H = g.H; q.W = g.W; q.R = g.R; q.S = g.S; q.K = g.K; q.Kpad = (g.K + KB - 1) / KB * KB;

@@ -12,7 +12,8 @@
 //   merge_classes_kernel        dx from them: ordered sum of the splits, gate, whole rows of dx per store
 // One call, before -> after (floats): 21 x 70 x 53 x 37, 130 filters of 3x3, stride 2: 197 -> 64 us; 32 x 256 x 28 x 28, 512
 // of 3x3: 937 -> 187; 128 x 64 x 112 x 112, 64 of 3x3: 1955 -> 919; 1 x 64 x 56 x 56, 128 of 3x3: 41 -> 17; 64 x 128 x 56 x 56,
-// 128 of 1x1 (a quarter of the pixels have a tap): 141 -> 134.
+// 128 of 1x1 (a quarter of the pixels have a tap): 141 -> 134. Layers of short reductions stay with the one product (classes_pay
+// in conv.hip).
 #pragma once
 #include "conv_loaders_tap.h"
 
