@@ -280,6 +280,8 @@ def kernels_of(ctx, g, which, bf16):
     ("bwd data", 0, (8, 96, 55, 55, 8, 2, 2, 1, 1, 2, 2), "classes", False), ("bwd data", 0, (8, 40, 64, 66, 64, 3, 3, 1, 1, 2, 2), "classes", True),
     ("bwd data", 0, (1, 17, 8, 8, 33, 3, 3, 1, 1, 2, 2), "classes", False), ("bwd data", 1, (4, 358, 40, 19, 4, 2, 2, 0, 0, 1, 3), "classes", False),
     ("bwd data", 1, (2, 34, 16, 16, 66, 3, 3, 1, 1, 2, 2), "classes", True),
+    # one product of a strided layer: short reductions on 64x64 tiles, up to a size
+    ("bwd data", 0, (2, 128, 128, 128, 2, 7, 7, 3, 3, 2, 2), "64x64", True), ("bwd data", 0, (22, 128, 128, 128, 2, 7, 7, 3, 3, 2, 2), "64x64", False),
 ], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))
 def test_route_by_size(ctx, which, bf16, geom, name, taken):
     announce("route", which, bf16, geom)

@@ -108,9 +108,13 @@ int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, co
 
 // What a loader's address work costs the 64x64 and the large tile (estimates of mfma_gemm.h), against the loaders whose
 // tap is a per-slice value; the others work it out for every element, a strided backward data with two divisions.
-template <class BL> struct LoadCost { static constexpr double SMALL = 1.25, LARGE = 1.15; };
-template <int MODE, class E, bool PAD> struct LoadCost<LoadIm2colPixTap<MODE, E, PAD>> { static constexpr double SMALL = 1.0, LARGE = 1.0; };
-template <bool BIG, class E> struct LoadCost<LoadIm2colPix<2, BIG, E>> { static constexpr double SMALL = 4.0, LARGE = 2.0; };
+// SHORT_OPS: operations up to which a short reduction (kShortReduction) takes the 64x64 tile whatever the estimates say. A
+// strided backward data fetches four times as many elements through its divisions there as in a large tile and is bound by
+// that once the chip is full: 13 x 213 x 111 x 111, 13 filters of 3x3 at stride 2 216 us against 170, 16 x 600 x 75 x 75, 36 of 2x2 323
+// against 251; over 2400 calls the two are even at 3e9 to 6e9 operations.
+template <class BL> struct LoadCost { static constexpr double SMALL = 1.25, LARGE = 1.15, SHORT_OPS = 1e30; };
+template <int MODE, class E, bool PAD> struct LoadCost<LoadIm2colPixTap<MODE, E, PAD>> { static constexpr double SMALL = 1.0, LARGE = 1.0, SHORT_OPS = 1e30; };
+template <bool BIG, class E> struct LoadCost<LoadIm2colPix<2, BIG, E>> { static constexpr double SMALL = 4.0, LARGE = 2.0, SHORT_OPS = 4e9; };
 
 // Forward / backward data. Tile shape by output-row count: 64-row tiles for narrow layers, 128
 // otherwise; 64x64 where the estimates of mfma_gemm.h find it faster (float engine). A grid that cannot fill
@@ -136,7 +140,9 @@ static int launch_by_m(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names
     }
     if constexpr (!HALF) {
         const SmallTilePlan plan = small_tile_plan(M, N, K, ctx->reduce_scratch && ep.partial ? partial_bytes : 0, ctx->num_cu, 4, true, LoadCost<BL>::SMALL);
-        if (K <= kShortReduction || (2.0 * M * (double)N * K <= kSmallTileOps && plan.us < 0.9 * large_tile_us(M, N, K, TM, TN, splits, ctx->num_cu, false, LoadCost<BL>::LARGE))) {
+        const double ops = 2.0 * M * (double)N * K;
+        if ((K <= kShortReduction && ops <= LoadCost<BL>::SHORT_OPS) ||
+            (ops <= kSmallTileOps && plan.us < 0.9 * large_tile_us(M, N, K, TM, TN, splits, ctx->num_cu, false, LoadCost<BL>::LARGE))) {
             GemmDims ds = make_dims(M, N, K, 64, 64, plan.splits);
             const int tail = plan.full_tiles > 0 && ds.splits > 1 ? (int)((long)ds.mtiles * ds.ntiles - plan.full_tiles) : 0;
             if (tail > 0) ds.full_tiles = (int)plan.full_tiles;
