@@ -168,7 +168,7 @@ STRIDED = [(2, 5, 9, 11, 7, 3, 3, 1, 1, 2, 2), (1, 17, 8, 8, 33, 1, 1, 0, 0, 2, 
            (1, 65, 3, 3, 600, 3, 3, 0, 0, 2, 2), (4, 40, 64, 66, 31, 3, 3, 1, 1, 2, 2), (1, 7, 20, 21, 18, 11, 11, 5, 5, 2, 2),
            # the small ones above again, large enough for the classes in both element types
            (20, 25, 39, 21, 27, 3, 3, 1, 1, 2, 2), (8, 67, 28, 28, 333, 1, 1, 0, 0, 2, 2), (8, 36, 30, 27, 40, 4, 4, 3, 3, 2, 2), (3, 49, 32, 42, 65, 3, 3, 0, 0, 1, 2),
-           (4, 39, 32, 33, 130, 3, 2, 0, 1, 3, 1), (2, 28, 57, 15, 40, 5, 3, 2, 0, 4, 1), (6, 65, 7, 7, 600, 3, 3, 0, 0, 2, 2)]
+           (4, 39, 32, 33, 130, 3, 2, 0, 1, 3, 1), (9, 28, 57, 15, 40, 5, 3, 2, 0, 4, 1), (6, 65, 7, 7, 600, 3, 3, 0, 0, 2, 2)]
 
 
 @pytest.mark.parametrize("geom", STRIDED, ids=lambda g: "x".join(map(str, g)))

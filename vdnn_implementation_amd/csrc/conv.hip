@@ -950,15 +950,19 @@ static int launch_fwd_smallc3x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g,
 // Backward data by residue classes saves matrix work and pays with float results in the staging area, read again by the
 // merge: it loses where a pixel of dx has few products (32 x 128 x 94 x 94, 2 filters of 3x3 at stride 3x1: 106 us in one
 // product, 282 by classes; 57 x 121 x 89 x 89 bfloat16, 7 of 1x1 at stride 2: 103 and 232). Both times are estimated, from 4900
-// calls timed on both routes: launches, matrix work (by classes at 94 TFLOP/s; in one product, with per-element taps, at
-// 58, a bfloat16 layer at 66 with its filter to round first), and what moving the elements of dx adds. The choice is 0.6 %
-// (floats) and 0.4 % (bfloat16) behind the better route in the mean.
+// calls timed on both routes: launches, matrix work (by classes at 105 TFLOP/s; in one product, with a tap to work out per
+// element, at 50 up to 4 GFLOP, on the 64x64 tile, and 85 beyond, on the large ones; a bfloat16 layer's filter is rounded first),
+// and what moving the elements of dx adds, with the gate and beyond what the caches hold. The choice is 0.4 % (floats) and 0.7 %
+// (bfloat16) behind the better route in the mean.
 static bool classes_pay(const ConvGeo& g, int elem_bytes, bool gated) {
+    const bool half = elem_bytes == 2;
     const double reduction = (double)g.K * g.R * g.S, pixels = (double)g.N * g.H * g.W, elems = 1e-6 * pixels * g.C;
     const double rows = (g.C + 63) / 64 * 64, padded = (double)((g.K + KB - 1) / KB * KB) * g.R * g.S;
-    const double classes_us = 14.1 + 1.07e-8 * 2.0 * padded * rows * pixels / (g.sh * g.sw) + (gated ? 4.6 : 3.9) * elems;
-    const double one_us = elem_bytes == 2 ? 11.2 + 0.31 * std::sqrt(reduction) + 1.52e-8 * 2.0 * reduction * rows * pixels + (gated ? 2.8 : 1.7) * elems
-                                          : 7.7 + 0.28 * std::sqrt(reduction) + 1.72e-8 * 2.0 * reduction * rows * pixels + (gated ? 1.7 : 1.3) * elems;
+    const double classes_ops = 2e-8 * padded * rows * pixels / (g.sh * g.sw), one_ops = 2e-8 * reduction * rows * pixels;
+    const double small = one_ops < 40.0 ? one_ops : 40.0, uncached = elems > 12.0 ? elems - 12.0 : 0.0;
+    const double classes_us = 14.2 + 0.95 * classes_ops + (gated ? 4.55 : 4.05) * elems + (!gated ? 0.15 : half ? 0.75 : 1.75) * uncached;
+    const double one_us = half ? 10.5 + 0.23 * std::sqrt(reduction) + 2.0 * small + 1.2 * (one_ops - small) + (gated ? 2.1 : 1.2) * elems
+                               : 8.8 + 0.09 * std::sqrt(reduction) + 2.0 * small + 1.17 * (one_ops - small) + (gated ? 1.45 : 1.05) * elems;
     return classes_us < one_us;
 }
 
