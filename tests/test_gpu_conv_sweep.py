@@ -212,7 +212,9 @@ def test_strided_backward_data(ctx, geom):
     (5, 300, 5, 5, 200, 1, 1, 0, 0, 1, 1),
     # large enough for the bfloat16 engine in both directions
     (2, 33, 40, 58, 31, 3, 3, 1, 1, 1, 1), (6, 12, 52, 64, 13, 3, 3, 1, 1, 1, 1), (4, 95, 26, 14, 65, 3, 3, 1, 1, 1, 1), (4, 40, 40, 40, 20, 5, 5, 2, 2, 1, 1),
-    (11, 47, 31, 29, 49, 3, 3, 1, 1, 1, 1), (18, 15, 43, 45, 48, 3, 3, 0, 0, 1, 1), (12, 129, 40, 46, 79, 1, 1, 0, 0, 1, 1)], ids=lambda g: "x".join(map(str, g)))
+    (11, 47, 31, 29, 49, 3, 3, 1, 1, 1, 1), (18, 15, 43, 45, 48, 3, 3, 0, 0, 1, 1), (12, 129, 40, 46, 79, 1, 1, 0, 0, 1, 1),
+    # large enough for the float engine's padded loaders forward
+    (13, 47, 31, 29, 149, 3, 3, 1, 1, 1, 1), (18, 70, 53, 37, 130, 3, 3, 1, 1, 2, 2)], ids=lambda g: "x".join(map(str, g)))
 def test_padded_channels(ctx, geom):
     rng = np.random.default_rng(sum((i + 1) * v for i, v in enumerate(geom)))
     g, og = be.shape(*geom), oracle.shape(*geom)
@@ -280,6 +282,9 @@ def kernels_of(ctx, g, which, bf16):
     ("bwd data", 0, (8, 96, 55, 55, 8, 2, 2, 1, 1, 2, 2), "classes", False), ("bwd data", 0, (8, 40, 64, 66, 64, 3, 3, 1, 1, 2, 2), "classes", True),
     ("bwd data", 0, (1, 17, 8, 8, 33, 3, 3, 1, 1, 2, 2), "classes", False), ("bwd data", 1, (4, 358, 40, 19, 4, 2, 2, 0, 0, 1, 3), "classes", False),
     ("bwd data", 1, (2, 34, 16, 16, 66, 3, 3, 1, 1, 2, 2), "classes", True),
+    # padded channels of float layers: the filter re-laid-out or read as it is
+    ("fwd", 0, (1, 46, 29, 29, 48, 2, 2, 0, 0, 1, 1), "pack", False), ("fwd", 0, (12, 200, 28, 28, 300, 3, 3, 1, 1, 1, 1), "pack", True),
+    ("bwd data", 0, (2, 30, 12, 5, 46, 2, 2, 0, 0, 1, 1), "pack", False), ("bwd data", 0, (18, 95, 26, 14, 65, 3, 3, 1, 1, 1, 1), "pack", True),
     # one product of a strided layer: short reductions on 64x64 tiles, up to a size
     ("bwd data", 0, (2, 128, 128, 128, 2, 7, 7, 3, 3, 2, 2), "64x64", True), ("bwd data", 0, (22, 128, 128, 128, 2, 7, 7, 3, 3, 2, 2), "64x64", False),
 ], ids=lambda v: "x".join(map(str, v)) if isinstance(v, tuple) else str(v))

@@ -280,9 +280,15 @@ constexpr size_t kMaxWgradWorkspace = (size_t)256 << 20;
 static bool is_dense(const ConvGeo& g) { return g.P == 1 && g.Q == 1 && g.ph == 0 && g.pw == 0 && g.R == g.H && g.S == g.W; }
 
 // Channel counts that are no whole blocks of 16 take the tap-major loaders with the last block padded where that multiplies at
-// most a quarter more: the others work out a tap per element, at half the rate (32 x 200 x 28 x 28, 300 of 3x3 forward
-// 356 -> 275 us; 64 x 130 x 13 x 13, 390 of 5x5 backward data 460 -> 352; 21 x 70 x 53 x 37, 130 of 3x3 forward 151 -> 121).
-static bool pad_pays(int channels) { return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels; }
+// most a quarter more and the layer is large enough: the others work out a tap per element, at half the rate in large grids
+// (32 x 200 x 28 x 28, 300 of 3x3 forward 356 -> 275 us; 64 x 130 x 13 x 13, 390 of 5x5 backward data 460 -> 352; 21 x 70 x 53 x 37, 130 of 3x3
+// forward 151 -> 121), but need no launch for a re-laid-out filter (1 x 46 x 29 x 29, 48 of 2x2 forward 13.1 with it, 8.5 without). The
+// lines, operations with the rows in whole tiles, are those of least loss over 1200 calls timed on both: 1.2 % and 0.7 %
+// behind the better one in the mean.
+static bool pad_pays(int channels, int M, long N, int RS, double least_ops) {
+    return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels && 2.0 * ((M + 63) / 64 * 64) * (double)N * channels * RS >= least_ops;
+}
+constexpr double kPadFwdOps = 1.5e9, kPadBwdDataOps = 4e8;
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
 static bool packed_bwd_data_ok(const ConvGeo& g) {
     return g.C > 4 && g.sh == 1 && g.sw == 1 && g.R * g.S <= 32 && g.K % KB == 0;
@@ -1153,7 +1159,7 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
             if (taken || rc != VDNN_OK) return rc;
         }
     }
-    if (g.R * g.S <= 32 && g.C % KB != 0 && pad_pays(g.C)) {
+    if (g.R * g.S <= 32 && g.C % KB != 0 && pad_pays(g.C, g.K, (long)g.N * g.P * g.Q, g.R * g.S, kPadFwdOps)) {
         // the same with the last block of channels filled up by zeros
         const int RS = g.R * g.S, Kpad = (g.C + KB - 1) / KB * KB * RS;
         const size_t bytes = (size_t)g.K * Kpad * 4;
@@ -1347,7 +1353,7 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             LoadFilterTap<true> alt{w, RS, g.C * RS, g.C, RS, wbytes, dRS};
             return launch_by_m(ctx, st, kBwdDataNames, alt, bl, ep, M, N, K, flops);
         }
-        if (RS <= 32 && g.K % KB != 0 && pad_pays(g.K)) {
+        if (RS <= 32 && g.K % KB != 0 && pad_pays(g.K, M, N, RS, kPadBwdDataOps)) {
             const int Kpad = (g.K + KB - 1) / KB * KB * RS;
             const size_t bytes = (size_t)g.C * Kpad * 4;
             if (float* packed = packed_filter_place(ctx, carve, bytes)) {
