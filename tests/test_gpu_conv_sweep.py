@@ -102,6 +102,17 @@ def test_conv3x3_sweep_bfloat16(ctx, geom):
         check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
 
 
+# Layers of up to three input channels that leave the chip idle: backward data walks strips of two rows up, backward filter
+# splits of one slice of 64 pixels up. Strips that do not divide the rows, a last strip of one row, several column blocks,
+# reductions that are no whole slices, one and several tiles of filters.
+@pytest.mark.parametrize("geom", [(4, 3, 20, 20, 8, 3, 3, 1, 1, 1, 1), (1, 3, 21, 20, 8, 3, 3, 1, 1, 1, 1), (1, 1, 5, 16, 4, 3, 3, 1, 1, 1, 1), (2, 2, 7, 64, 33, 3, 3, 1, 1, 1, 1),
+                                  (3, 3, 33, 36, 70, 3, 3, 1, 1, 1, 1), (1, 3, 50, 224, 64, 3, 3, 1, 1, 1, 1), (8, 3, 101, 40, 16, 3, 3, 1, 1, 1, 1)],
+                         ids=lambda g: "x".join(map(str, g[:5])))
+def test_few_channels_on_an_idle_chip(ctx, geom):
+    test_conv3x3_sweep_float(ctx, geom)
+    test_conv3x3_sweep_bfloat16(ctx, geom)
+
+
 # The 64x64 tile: one row or column short of a tile and one past it, reductions of one slice and of many splits, 260 and
 # 516 tiles for 256 units (only the tiles behind whole rounds are split), taps shared by a tile's columns (channels in
 # 64s and 32s) and not, planes that are no whole groups of pixels.
@@ -200,6 +211,37 @@ def test_strided_backward_data(ctx, geom):
             assert_close_bf16(get_act(gx, x.shape), np.where(x > 0, oracle.conv_bwd_data(og, dy, oracle.round_bf16(w)), 0), "bf16, gated")
     finally:
         check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
+
+
+def test_strided_backward_data_in_chunks_of_samples(ctx):
+    """Results of five samples of 3.8 million elements do not fit the staging area of 16 million: four samples, then one, each
+    with its own splits. Gated and not, both element types."""
+    geom = (5, 24, 400, 400, 33, 3, 3, 1, 1, 2, 2)
+    rng = np.random.default_rng(5)
+    g, og = be.shape(*geom), oracle.shape(*geom)
+    w = (rng.standard_normal((33, 24, 3, 3)) * 0.1).astype(np.float32)
+    dy, x = rnd(rng, (5, 33, 200, 200)), rnd(rng, (5, 24, 400, 400))
+    for bf16 in (0, 1):
+        want = oracle.conv_bwd_data(og, dy, oracle.round_bf16(w) if bf16 else w)
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, bf16))
+        try:
+            with Dev(ctx) as d:
+                up = d.act if bf16 else d.f32
+                ddy, dxx, dw, gx = up(dy), up(x), d.f32(w), up(np.zeros_like(x))
+                for gate in (False, True):
+                    announce("strided bwd data in chunks", bf16, gate)
+                    be.profile_enable(ctx.handle, 1)
+                    if gate:
+                        check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, dw.ptr, dxx.ptr, gx.ptr, None, 0))
+                    else:
+                        check(lib.vdnn_conv_bwd_data(ctx.handle, None, g, 0, ddy.ptr, dw.ptr, gx.ptr, None, 0))
+                    assert be.profile_collect(ctx.handle)["conv_bwd_data_merge"]["launches"] == 2
+                    got, ref = (get_act(gx, x.shape) if bf16 else gx.download(x.shape)), np.where(x > 0, want, 0) if gate else want
+                    for n in range(5):
+                        (assert_close_bf16(got[n], ref[n], "sample %d" % n) if bf16 else assert_close(got[n], ref[n], TOL, "sample %d" % n))
+        finally:
+            be.profile_enable(ctx.handle, 0)
+            check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 0))
 
 
 # Reduced channels (input channels forward, filters in backward data) that are no whole blocks of 16 or 32, through every

@@ -653,8 +653,9 @@ def test_conv_results_do_not_depend_on_the_run(ctx):
                                      (37, 6, 40, 40), (2, 70, 31, 33), (33, 96, 55, 55)])
 def test_bias_gradients_at_any_plane_and_alignment(ctx, n, k, p, q, bf16):
     """Planes of less than one access, of one, of one and a remainder; one workgroup per channel and several; a tensor one
-    element past an aligned address. The bias gradients of convolution and fully connected layers against sums in
-    64 bits: at most log2-deep trees and chains of n p q / 256 additions, each within 2^-24 of the sum of magnitudes."""
+    element past an aligned address. A convolution's against sums in 64 bits: at most log2-deep trees and chains of
+    n p q / 256 additions, each within 2^-24 of the sum of magnitudes. A fully connected layer's, which adds its rows in one
+    ascending chain, to the bit."""
     rng = np.random.default_rng(n * 1000 + k + p * q)
     dy = rng.standard_normal((n, k, p, q)).astype(np.float32)
     if bf16:
@@ -681,8 +682,10 @@ def test_bias_gradients_at_any_plane_and_alignment(ctx, n, k, p, q, bf16):
     depth = 2.0 ** -24 * (20 + n * p * q / 256)
     assert np.all(np.abs(got_db - want) <= depth * mag)
     assert np.all(np.abs(got_b - (bias + np.float64(alpha) * want)) <= depth * mag + 2.0 ** -23 * np.abs(bias))
-    want, mag = d64.sum(axis=0).ravel(), np.abs(d64).sum(axis=0).ravel()
-    assert np.all(np.abs(got_fb - want) <= 2.0 ** -24 * (20 + n / 16) * mag)
+    chain = np.zeros(k * p * q, np.float32)
+    for row in dy.reshape(n, -1):
+        chain = chain + row
+    assert np.array_equal(got_fb, chain)
 
 
 @pytest.mark.parametrize("bf16", [0, 1])
