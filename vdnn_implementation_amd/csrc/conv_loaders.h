@@ -57,7 +57,10 @@ struct LoadIm2colPix {
         const int n = jj / opix, pix = jj - n * opix;
         const int oh = pix / OW, ow = pix - oh * OW;
         const long first = (long)n_first * sample_elems;
-        long shift; // descriptor base relative to the first sample, in elements (<= 0)
+        // Descriptor base relative to the first sample, in elements: not above it in MODE 0; in MODE 1 above it where the padding
+        // reaches beyond the window (ph >= R, pw >= S: a residue class of a strided layer), and only elements from there on
+        // are read then.
+        long shift;
         int ih0, iw0;
         if (MODE == 0) {
             shift = -((long)ph * Ws + pw);

@@ -199,8 +199,12 @@ static inline int choose_splits(long tiles, long K, long max_splits, int num_cu,
 // 25088 -> 4096 at 64 rows, filter update (four slices a tile) 311 -> 241 us.
 // Which tile: the times of both are estimated, from 290 measured calls of 1 to 128 samples, 8 to 1024 channels, 1x1 to
 // 5x5, planes of 7 to 56 pixels a side; the choice is within 3 % of the better one in all but a few of them.
-// Products of more than kSmallTileOps operations keep the large tile whatever the estimates say: those of large training
-// steps, which are to give the same bits from one version of this file to the next, and whose grids seldom gain.
+// Products of more than kSmallTileOps operations keep the large tile whatever the estimates say: their grids seldom gain (the
+// 64x64 tile is 5-8 % slower on a full chip), and large training steps keep the order of their sums. Reductions of up to
+// kShortReduction are the exception: they take the 64x64 tile at any size, because a large tile is mostly prologue and
+// epilogue there (strided backward data up to 4e9 operations, LoadCost in conv.hip). Their splits are this plan's,
+// so a remainder behind whole rounds may be summed in another order than the large tile's; fully connected layers, whose rule
+// is in fc.hip, keep the large tile's splits and with them its bits.
 struct SmallTilePlan {
     int splits = 0;      // Splits of every tile, or (full_tiles > 0) of the tiles behind the first full_tiles
     long full_tiles = 0;
