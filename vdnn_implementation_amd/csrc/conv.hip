@@ -12,6 +12,7 @@
 #include "conv_loaders_tap.h"
 #include "mfma_bf16.h"
 #include "conv3x3_bf16.h"
+#include "conv_launch.h"
 #include "wgrad3x3_bf16.h"
 #include "wgrad3x3_f32.h"
 #include "wgrad3x3_split.h"
@@ -41,27 +42,6 @@ static bool geo_from_shape(const vdnn_shape_t* s, ConvGeo& g) {
     // the filter bank is addressed through one descriptor with summed offsets
     if ((long)g.K * g.C * g.R * g.S * 4 >= (long)MAX_SUM_RANGE) return false;
     return true;
-}
-
-// samples one tile of `tile` pixels can touch, times the sample size: must stay below 2 GiB so that
-// per-lane byte offsets are positive ints and the exhausted-range scalar offset is out of range
-static bool pixel_tile_span_ok(long sample_elems, int opix, int tile, int elem_bytes) {
-    const long span = (long)(tile / opix + 2) * sample_elems * elem_bytes;
-    return span < 0x7FFF0000l;
-}
-
-static GemmDims make_dims(int M, int N, int K, int TM, int TN, int splits, int depth = KB) {
-    GemmDims d;
-    d.M = M; d.N = N; d.K = K;
-    d.mtiles = (M + TM - 1) / TM;
-    d.ntiles = (N + TN - 1) / TN;
-    if (splits < 1) splits = 1;
-    int kchunk = (K + splits - 1) / splits;
-    kchunk = (kchunk + depth - 1) / depth * depth;
-    d.kchunk = kchunk;
-    d.splits = (K + kchunk - 1) / kchunk;
-    d.full_tiles = 0;
-    return d;
 }
 
 // names of the kernel classes in the timing report: {pass}_{tile}
@@ -94,17 +74,6 @@ static int launch_igemm(vdnn_ctx* ctx, hipStream_t stream, const char* name, con
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
 }
-
-int launch_reduce_tail_nchw(vdnn_ctx* ctx, hipStream_t stream, float* out, const float* partial, int tail_tiles, int splits, int TM, int TN,
-                            int M, int N, int mtiles, int full_tiles, const float* bias, int opix, int relu, const float* gate);
-int launch_reduce_tail_nchw(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, const float* partial, int tail_tiles, int splits, int TM, int TN,
-                            int M, int N, int mtiles, int full_tiles, const float* bias, int opix, int relu, const bf16_t* gate);
-int launch_reduce_splits_tap(vdnn_ctx* ctx, hipStream_t stream, float* out, const float* partial, size_t count, int splits,
-                             float alpha, int accumulate, int C, int RS);
-int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, float* out, const float* partial, size_t count, int splits,
-                              const float* bias, int opix, int channels, int relu, const float* gate);
-int launch_reduce_splits_nchw(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, const float* partial, size_t count, int splits,
-                              const float* bias, int opix, int channels, int relu, const bf16_t* gate);
 
 // What a loader's address work costs the 64x64 and the large tile (estimates of mfma_gemm.h), against the loaders whose
 // tap is a per-slice value; the others work it out for every element, a strided backward data with two divisions.
@@ -236,11 +205,6 @@ static bool win3x3_ok(const int R, const int S, int ph, int pw, int sh, int sw, 
            pixel_tile_span_ok(sample_elems, OH * OW, W3_TN, elem_bytes);
 }
 
-static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
-
-int launch_reduce_splits(vdnn_ctx* ctx, hipStream_t stream, float* out, const float* partial, size_t count,
-                         int splits, float alpha, int accumulate, const float* bias_j, int ncols, int relu = 0, const float* gate = nullptr);
-
 // forward with the given A loader (128-bit or 32-bit filter loads)
 template <class AL, class E>
 static int conv_fwd_with(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const AL& al, const E* x, const float* bias, E* y, int relu) {
@@ -292,24 +256,6 @@ constexpr double kPadFwdOps = 1.5e9, kPadBwdDataOps = 4e8;
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
 static bool packed_bwd_data_ok(const ConvGeo& g) {
     return g.C > 4 && g.sh == 1 && g.sw == 1 && g.R * g.S <= 32 && g.K % KB == 0;
-}
-
-int launch_bias_grad_final(vdnn_ctx* ctx, hipStream_t st, const float* partial, float* bias, int K, int splits, float alpha, int accumulate);
-
-// The bias gradient as a by-product of backward filter (cudnnConvolutionBackwardBias, layer.cu:631-637, reads the same dy
-// as cudnnConvolutionBackwardFilter, :651-660): where the filter-gradient kernel of a shape can add up the dy values it
-// streams, it leaves per-channel partial sums in the context's bias staging area and `done` is set; the caller runs the
-// ordered final sum. out = (accumulate ? out : 0) + alpha * sum over n, p, q of dy.
-struct BiasOut {
-    float* out = nullptr;
-    float alpha = 1.0f;
-    int accumulate = 0;
-    bool done = false;
-    bool wanted() const { return out != nullptr; }
-};
-// room for K x parts partial sums in the bias staging area?
-static bool bias_parts_fit(const vdnn_ctx* ctx, int K, long parts) {
-    return ctx->bias_scratch && parts > 0 && (size_t)K * (size_t)parts * sizeof(float) <= ctx->bias_scratch_bytes;
 }
 
 // ---- Winograd F(4x4, 3x3): the perf-optimal mode's forward / backward data of wide 3x3 layers (winograd_f32.h) -----
@@ -592,32 +538,6 @@ static int launch_pack_filter_bf16(vdnn_ctx* ctx, hipStream_t st, const float* w
     return VDNN_OK;
 }
 
-// Takes bytes from the front of the context's staging area for as long as the object lives; everything that
-// uses the staging area meanwhile (partial sums, intermediate products) sees the remainder.
-struct StagingCarve {
-    vdnn_ctx* ctx;
-    float* base = nullptr;
-    size_t total = 0;
-    bool taken = false;
-    explicit StagingCarve(vdnn_ctx* c) : ctx(c) {}
-    void* take(size_t bytes) {
-        base = ctx->reduce_scratch; total = ctx->reduce_scratch_bytes; taken = true;
-        const size_t t = (bytes + 255) / 256 * 256;
-        ctx->reduce_scratch = (float*)((char*)base + t);
-        ctx->reduce_scratch_bytes = total - t;
-        return base;
-    }
-    ~StagingCarve() { if (taken) { ctx->reduce_scratch = base; ctx->reduce_scratch_bytes = total; } }
-};
-
-// Room for a re-laid-out filter bank at the front of the staging area: only if nothing was taken from it yet and at
-// least half of it stays for the partial sums of split reductions (the largest need of a layer is a round of partial
-// tiles: 768 x 64 KB). Null otherwise.
-static float* packed_filter_place(vdnn_ctx* ctx, StagingCarve& carve, size_t bytes) {
-    if (carve.taken || !ctx->reduce_scratch || 2 * ((bytes + 255) / 256 * 256) > ctx->reduce_scratch_bytes) return nullptr;
-    return (float*)carve.take(bytes);
-}
-
 __global__ void __launch_bounds__(256) round_filter_bf16_kernel(const float* __restrict__ w, float* __restrict__ out, long count) {
     const long i = (long)blockIdx.x * 256 + threadIdx.x;
     if (i < count) out[i] = round_to_bf16_value(w[i]);
@@ -863,11 +783,6 @@ static int launch_wgrad3x3_split(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g
 
 // Workgroups of wgrad3x3_f32_kernel that are resident on a compute unit (its launch bounds; three, at 167 registers, measured 10 % slower).
 constexpr int kWgrad3FPerCU = 2;
-
-static bool wgrad3x3_f32_ok(const ConvGeo& g) {
-    return g.R == 3 && g.S == 3 && g.ph == 1 && g.pw == 1 && g.sh == 1 && g.sw == 1 && g.P == g.H && g.Q == g.W &&
-           g.W % 2 == 0 && g.W >= 14 && (g.H * g.W) % 4 == 0 && g.C % WG3F_CH == 0; // a slice wraps at most two image rows
-}
 
 // The float counterpart of launch_wgrad3x3.
 static int launch_wgrad3x3_f32(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const float* x, const float* dy, float* w, float alpha, int accumulate,
@@ -1159,6 +1074,11 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
             if (taken || rc != VDNN_OK) return rc;
         }
     }
+    if constexpr (sizeof(E) == 4) {
+        bool taken = false;
+        const int rc = launch_same_x3_fwd(ctx, st, carve, g, x, w, bias, y, relu, &taken);
+        if (taken || rc != VDNN_OK) return rc;
+    }
     if (g.R * g.S <= 32 && g.C % KB != 0 && pad_pays(g.C, g.K, (long)g.N * g.P * g.Q, g.R * g.S, kPadFwdOps)) {
         // the same with the last block of channels filled up by zeros
         const int RS = g.R * g.S, Kpad = (g.C + KB - 1) / KB * KB * RS;
@@ -1323,6 +1243,11 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             const int rc = launch_winograd(ctx, st, g, true, dy, w, nullptr, dx, 0, gate, workspace, workspace_bytes, &taken);
             if (taken || rc != VDNN_OK) return rc;
         }
+    }
+    if constexpr (sizeof(E) == 4) {
+        bool taken = false;
+        const int rc = launch_same_x3_bwd_data(ctx, st, carve, g, dy, w, dx, gate, &taken);
+        if (taken || rc != VDNN_OK) return rc;
     }
     const int RS = g.R * g.S;
     LoadFilterT al{w, g.C, RS, (unsigned)((long)g.K * g.C * RS * 4), FastDiv::make(RS)};

@@ -24,7 +24,7 @@
 
 namespace vdnn {
 
-constexpr int WG3F_CH = 64; // input channels of a workgroup's tile
+constexpr int WG3F_CH = 64; // input channels of a workgroup's tile (wgrad3x3_f32_ok)
 
 struct Wgrad3x3F {
     const float* dy;
