@@ -1523,6 +1523,11 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
         }
     }
     if constexpr (sizeof(E) == 4) {
+        bool taken = false;
+        const int rcs = launch_wgrad_same_x3(ctx, st, g, x, dy, w, alpha, accumulate, staging, staging_bytes, &taken, bias);
+        if (taken || rcs != VDNN_OK) return rcs;
+    }
+    if constexpr (sizeof(E) == 4) {
         // 3x3, stride 1, padding 1: one filter row and 64 input channels per workgroup, one fetch for three taps
         if (wgrad3x3_f32_ok(g)) { // loads of four pixels take any alignment of the tensors
             bool taken = false;
@@ -1584,7 +1589,7 @@ static int conv_bwd_filter_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
 }
 
 // Does backward filter of this shape add up the bias gradient inside its own kernel? (The shapes' dispatch above: the
-// Winograd variant - float activations only -, the first-layer kernel, the filter-row kernels.)
+// Winograd variant - float activations only -, the first-layer kernel, the filter-row kernels and wgrad_same.h's.)
 static bool bwd_filter_sums_bias(const ConvGeo& g, int algo_mode, int dtype) {
     if (is_dense(g)) return false;
     const bool f32 = dtype == VDNN_DTYPE_F32;
@@ -1592,7 +1597,7 @@ static bool bwd_filter_sums_bias(const ConvGeo& g, int algo_mode, int dtype) {
     if (g.C <= 3 && g.R == 3 && g.S == 3 && g.ph == 1 && g.pw == 1 && g.sh == 1 && g.sw == 1 && g.P == g.H && g.Q == g.W && g.W % 4 == 0 && g.W >= KB &&
         g.P * g.Q >= WSC_SLICE)
         return true;
-    return g.C > 4 && (f32 ? wgrad3x3_f32_ok(g) : wgrad3x3_ok(g));
+    return g.C > 4 && (f32 ? wgrad3x3_f32_ok(g) || wgrad_same_x3_ok(g) : wgrad3x3_ok(g));
 }
 
 extern "C" {

@@ -97,4 +97,8 @@ static inline bool wgrad3x3_f32_ok(const ConvGeo& g) {
 int launch_same_x3_fwd(vdnn_ctx* ctx, hipStream_t st, StagingCarve& carve, const ConvGeo& g, const float* x, const float* w, const float* bias, float* y, int relu, bool* taken);
 int launch_same_x3_bwd_data(vdnn_ctx* ctx, hipStream_t st, StagingCarve& carve, const ConvGeo& g, const float* dy, const float* w, float* dx, const float* gate, bool* taken);
 
+bool wgrad_same_x3_ok(const ConvGeo& g);
+int launch_wgrad_same_x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const float* x, const float* dy, float* w, float alpha, int accumulate,
+                         float* staging, size_t staging_bytes, bool* taken, BiasOut* bias);
+
 } // namespace vdnn

@@ -1,6 +1,7 @@
 // Launchers of the float convolutions on the bfloat16 matrix cores at float precision (conv_same_f32x3.h).
 #include "conv_launch.h"
 #include "conv_same_f32x3.h"
+#include "wgrad_same.h"
 
 namespace vdnn {
 
@@ -107,6 +108,84 @@ int launch_same_x3_fwd(vdnn_ctx* ctx, hipStream_t st, StagingCarve& carve, const
 }
 int launch_same_x3_bwd_data(vdnn_ctx* ctx, hipStream_t st, StagingCarve& carve, const ConvGeo& g, const float* dy, const float* w, float* dx, const float* gate, bool* taken) {
     return launch_same_x3<1>(ctx, st, carve, g, dy, w, StoreNCHW<float>{dx, nullptr, g.H * g.W, nullptr, 0, gate}, taken);
+}
+
+// ---- backward filter of the same layers (wgrad_same.h) --------------------------------------------------------------
+static bool wgrad_same_ok(const ConvGeo& g) {
+    if (!x3_layer(g) || g.C % 8 != 0 || g.K % 8 != 0) return false;
+    const int WP = g.W + g.S / 2;
+    return g.H > WS_SLICE / WP && (long)g.N * g.H * WP < (1l << 30); // a slice reaches at most one sample further
+}
+// ... and pays: the tiles count 64 channels of each operand and S/2 slots more than pixels per row; beyond three times the
+// products the float engine's tiles are faster, as on small layers (4 x 64 x 30 x 31, 64 of 3x3 16.7 us there, 22.0 here; 112 x 8 x 20 x 119, 320
+// of 3x3 293 and 430; 1 x 64 x 56 x 56, 128 of 3x3 33.6 and 22.5). Of 500 calls timed on both, those beyond the lines gained 19.1 ms
+// together and lost 0.03.
+constexpr double kWgradX3LeastOps = 6e8, kWgradX3MostWaste = 3.0;
+bool wgrad_same_x3_ok(const ConvGeo& g) {
+    if (!wgrad_same_ok(g)) return false;
+    const double products = (double)g.C * g.K * g.W, padded = (double)((g.C + 63) / 64 * 64) * ((g.K + 63) / 64 * 64) * (g.W + g.S / 2);
+    return padded <= kWgradX3MostWaste * products && 2.0 * products * g.N * g.H * g.R * g.S >= kWgradX3LeastOps;
+}
+
+template <class E, int PARTS, int S, int RB, bool LOW>
+static void launch_wgrad_same_one(hipStream_t st, unsigned blocks, const WgradSame<E>& geo, const GemmDims& d) {
+    hipLaunchKernelGGL((wgrad_same_kernel<E, PARTS, S, RB, LOW>), dim3(blocks), dim3(NT), 0, st, geo, d);
+}
+
+// Splits of the reduction. A compute unit takes a slice of one workgroup in kAlone us, of two together in kPair (S = 3; measured on
+// 64 x 128 x 112 x 112), prologue and epilogue are about four slices.
+static long wgrad_same_splits(long tiles, long slices, size_t out_bytes, size_t room, int S, int num_cu) {
+    constexpr double kAlone = 1.35, kPair = 2.05, kEnds = 4.0, kSum = 5.0, kBytes = 4e6;
+    double best_us = 0.0;
+    long best = 1;
+    for (long s = 1; s <= slices / 4 || s == 1; s++) {
+        if (s > 1 && (s * out_bytes > room || tiles * s > 8l * num_cu)) break;
+        const long per_cu = (tiles * s + num_cu - 1) / num_cu;
+        const double us = ((double)(per_cu / 2) * kPair + (double)(per_cu % 2) * kAlone) * S / 3.0 * ((double)((slices + s - 1) / s) + kEnds) +
+                          (s > 1 ? kSum + 1.2 * (double)s * (double)out_bytes / kBytes : 0.0);
+        if (s == 1 || us < best_us) { best = s; best_us = us; }
+    }
+    return best;
+}
+
+template <class E>
+static int launch_wgrad_same(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const E* x, const E* dy, float* w, float alpha, int accumulate,
+                             float* staging, size_t staging_bytes, bool* taken, BiasOut* bias) {
+    *taken = false;
+    const int S = g.S, M = g.K, N = g.C * S * S, WP = g.W + S / 2, HW = g.H * g.W;
+    const int Kred = g.N * g.H * WP;
+    constexpr int TM = 64;
+    const int mtiles = (M + TM - 1) / TM, ntiles = S * ((g.C + WS_CH - 1) / WS_CH);
+    const long tiles = (long)mtiles * ntiles;
+    const long splits = wgrad_same_splits(tiles, (Kred + WS_SLICE - 1) / WS_SLICE, (size_t)M * N * sizeof(float), staging ? staging_bytes : 0, S, ctx->num_cu);
+    GemmDims d = make_dims(M, N, Kred, TM, S * WS_CH, (int)splits, WS_SLICE);
+    d.mtiles = mtiles; d.ntiles = ntiles;
+    const long nspan = d.kchunk / (g.H * WP) + 3;
+    if (nspan * g.K * HW * (long)sizeof(E) >= (long)MAX_SUM_RANGE || nspan * g.C * HW * (long)sizeof(E) >= (long)MAX_SUM_RANGE) return VDNN_OK; // not taken
+    const long blocks = tiles * d.splits;
+    if (blocks <= 0 || blocks >= (1l << 31)) return VDNN_OK;
+    *taken = true;
+    const bool with_bias = bias && bias->wanted() && bias_parts_fit(ctx, g.K, d.splits);
+    const WgradSame<E> geo{dy, x, g.N, g.K, g.C, g.H, g.W, w, staging, (long)M * N, alpha, accumulate, with_bias ? ctx->bias_scratch : nullptr, d.splits,
+                           Kred, WS_SLICE / WP, WS_SLICE % WP};
+    {
+        ProfScope prof(ctx, st, S == 3 ? "conv_bwd_filter_x3_3x3" : "conv_bwd_filter_x3_5x5", 2.0 * M * (double)N * (double)g.N * HW, 0.0);
+        if (S == 5) launch_wgrad_same_one<E, 3, 5, 1, true>(st, (unsigned)blocks, geo, d);
+        else launch_wgrad_same_one<E, 3, 3, 1, true>(st, (unsigned)blocks, geo, d);
+        VDNN_LAUNCH_CHECK();
+    }
+    if (with_bias) {
+        const int rc = launch_bias_grad_final(ctx, st, ctx->bias_scratch, bias->out, g.K, d.splits, bias->alpha, bias->accumulate);
+        if (rc != VDNN_OK) return rc;
+        bias->done = true;
+    }
+    if (d.splits > 1) return launch_reduce_splits_tap(ctx, st, w, staging, (size_t)M * N, d.splits, alpha, accumulate, g.C, S * S);
+    return VDNN_OK;
+}
+int launch_wgrad_same_x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const float* x, const float* dy, float* w, float alpha, int accumulate,
+                         float* staging, size_t staging_bytes, bool* taken, BiasOut* bias) {
+    *taken = false;
+    return wgrad_same_x3_ok(g) ? launch_wgrad_same<float>(ctx, st, g, x, dy, w, alpha, accumulate, staging, staging_bytes, taken, bias) : VDNN_OK;
 }
 
 } // namespace vdnn
