@@ -4,6 +4,7 @@
 #include "mfma_gemm.h"
 #include "fc_bf16.h"
 #include "fc_update.h"
+#include "fc_stream.h"
 
 namespace vdnn {
 
@@ -21,15 +22,19 @@ template <class L> struct FilterOperand<L, bf16_t> { typedef RoundedToBf16<L> ty
 
 // Out[M][N] (dense, row stride N) = alpha * A*B (+ Out) (+ bias per column); the reduction is split into
 // ordered partial sums when the tile grid alone cannot fill the chip.
-template <class AL, class BL, class EO>
-static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al, const BL& bl, int M, int N, int K,
-                   EO* out, float alpha, int accumulate, const float* bias_j, int relu = 0, const EO* gate = nullptr) {
-    int TM = M <= 64 ? 64 : 128, TN = M <= 64 ? 256 : 128;
+static int fc_splits(const vdnn_ctx* ctx, int M, int N, int K, int TM, int TN) {
     const long tiles = (long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
     long cap = ((long)K + 8 * KB - 1) / (8 * KB); // at least eight slices per split
     const long by_mem = (long)(ctx->reduce_scratch_bytes / ((size_t)M * N * sizeof(float)));
     if (cap > by_mem) cap = by_mem;
-    const long want = choose_splits(tiles, K, cap, ctx->num_cu, (size_t)M * N * sizeof(float), 2.0 * TM * TN * KB);
+    return choose_splits(tiles, K, cap, ctx->num_cu, (size_t)M * N * sizeof(float), 2.0 * TM * TN * KB);
+}
+
+template <class AL, class BL, class EO>
+static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al, const BL& bl, int M, int N, int K,
+                   EO* out, float alpha, int accumulate, const float* bias_j, int relu = 0, const EO* gate = nullptr) {
+    int TM = M <= 64 ? 64 : 128, TN = M <= 64 ? 256 : 128;
+    const long want = fc_splits(ctx, M, N, K, TM, TN);
     // The 64x64 tile (mfma_gemm.h) with the same splits: the same sums. Small products gain from more and shorter workgroups
     // (64 rows, 4096 -> 1000: 23 -> 16 us forward; 128, 300 -> 100 backward data 24.5 -> 8.7), short reductions always
     // (filter updates: a tile has as many slices as rows allow); larger ones break even at 4-8 GFLOP (128 rows, 4096 -> 4096:
@@ -52,6 +57,35 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     if (d.splits > 1) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, alpha, accumulate, bias_j, N, relu, gate);
+    return VDNN_OK;
+}
+
+// Forward (BWD false) and backward data of float layers through fc_stream.h, with fc_gemm's splits. Up to 32 rows of a filter that is far larger
+// than them: sixteen rows, 1024 -> 1024 forward 9.1 us on the tile engine and 13.6 there, 4096 -> 4096 26 and 22; forward of the largest
+// filters gains with few rows only (25088 -> 4096 one row 114 and 100, sixteen 119 and 116, 32 rows 119 and 132).
+static bool fc_stream_pays(int M, int N, int K, bool bwd) {
+    const long filter = (long)N * K;
+    return M <= 32 && K % KB == 0 && filter >= 3l << 22 && (bwd || M <= 16 || filter <= 1l << 26);
+}
+template <bool BWD>
+static int fc_stream(vdnn_ctx* ctx, hipStream_t st, const char* name, const float* rows, const float* w, int M, int N, int K, float* out, const float* bias_j, int relu, const float* gate) {
+    constexpr int TM = 64, TN = 256; // fc_gemm's, for its splits
+    GemmDims d;
+    d.M = M; d.N = N; d.K = K;
+    const int want = fc_splits(ctx, M, N, K, TM, TN);
+    d.kchunk = ((K + want - 1) / want + KB - 1) / KB * KB;
+    d.splits = (K + d.kchunk - 1) / d.kchunk;
+    d.full_tiles = 0;
+    d.mtiles = 1; d.ntiles = (N + TN - 1) / TN;
+    const StoreDense<float> ep{out, ctx->reduce_scratch, d.splits > 1 ? nullptr : bias_j, (long)N, (long)M * N, 1.0f, 0, relu, gate};
+    const FcStream g{rows, w, (unsigned)((long)M * K * 4), (unsigned)((long)N * K * 4)};
+    const dim3 grid((unsigned)((long)d.ntiles * d.splits));
+    {
+        ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
+        hipLaunchKernelGGL((fc_stream_kernel<BWD>), grid, dim3(NT), 0, st, g, ep, d);
+        VDNN_LAUNCH_CHECK();
+    }
+    if (d.splits > 1) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, 1.0f, 0, bias_j, N, relu, gate);
     return VDNN_OK;
 }
 
@@ -119,6 +153,9 @@ static int fc_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, int n, int c_in, int
         }
     }
     if (c_in % 4 == 0 && fc_aligned16(x) && fc_aligned16(w)) {
+        if constexpr (!IsBf16<E>::V) {
+            if (fc_stream_pays(n, c_out, c_in, false)) return fc_stream<false>(ctx, st, "fc_fwd", x, w, n, c_out, c_in, y, bias, relu, nullptr);
+        }
         LoadDenseRed<true, E> al{x, (long)c_in, n, xb};
         typename FilterOperand<LoadDenseRed<true>, E>::type bl{{w, (long)c_in, c_out, wb}};
         return fc_gemm(ctx, st, "fc_fwd", al, bl, n, c_out, c_in, y, 1.0f, 0, bias, relu);
@@ -146,6 +183,9 @@ static int fc_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, int n, int c_in
     }
     typename FilterOperand<LoadDenseRow<float>, E>::type bl{{w, (long)c_in, c_in, wb}};
     if (c_out % 4 == 0 && fc_aligned16(dy)) {
+        if constexpr (!IsBf16<E>::V) {
+            if (fc_stream_pays(n, c_in, c_out, true)) return fc_stream<true>(ctx, st, "fc_bwd_data", dy, w, n, c_in, c_out, dx, nullptr, 0, gate);
+        }
         LoadDenseRed<true, E> al{dy, (long)c_out, n, db};
         return fc_gemm(ctx, st, "fc_bwd_data", al, bl, n, c_in, c_out, dx, 1.0f, 0, nullptr, 0, gate);
     }
