@@ -17,15 +17,19 @@ constexpr int kX3LeastDepth = 288;
 static bool x3_pays(const ConvGeo& g, int rows, int reduced) {
     return reduced * g.R * g.S >= kX3LeastDepth && 2.0 * rows * (double)g.N * g.H * g.W * reduced * g.R * g.S >= kX3LeastOps;
 }
+// Layers of more than kSmallTileOps operations keep the order of their sums, as on the tile engine (mfma_gemm.h): OverFeat at batch 128, whose
+// steps take 103 ms here for 118, saturates its softmax, and in one of ten drawn steps its parameters came out 3.6e-5 from the float
+// instruction's.
+//
 // Layers of the float filter-row kernel (3x3, even rows of fourteen pixels or more, input channels in blocks of 64: every layer of VGG16
 // but the first) keep the float instruction in all three passes, where they run at 0.8 to 0.9 of its peak, although these kernels take
 // 0.6 to 0.65 of the time there too (64 x 256 x 56 x 56, 256 filters, forward 1755 and 1074 us, backward data 1765 and 1083, backward
 // filter 1845 and 1190): deep stacks of such layers train to other parameters in the last places when the order of any sum changes.
 // A pre-activation that falls on the other side of zero opens or shuts a unit for a sample; with backward data and filter alone
 // on these kernels, in 7 of 34 drawn pairs of VGG16 steps at batch 128 a weight of the fully connected layers moved by 2.5e-5 to 8e-5
-// of itself against the float instruction's step (AlexNet and OverFeat: 1.9e-5 at most in 28).
+// of itself against the float instruction's step (AlexNet at batches of 7 and 32, OverFeat at 24: 1.9e-5 at most in 18).
 static bool x3_layer(const ConvGeo& g) {
-    return (g.R == 3 || g.R == 5) && g.S == g.R && g.ph == g.R / 2 && g.pw == g.ph && g.sh == 1 && g.sw == 1 && !wgrad3x3_f32_ok(g);
+    return 2.0 * g.K * (double)g.N * g.H * g.W * g.C * g.R * g.S <= kSmallTileOps && (g.R == 3 || g.R == 5) && g.S == g.R && g.ph == g.R / 2 && g.pw == g.ph && g.sh == 1 && g.sw == 1 && !wgrad3x3_f32_ok(g);
 }
 
 static bool same_x3_ok(const ConvGeo& g, int mode) {
@@ -127,11 +131,6 @@ bool wgrad_same_x3_ok(const ConvGeo& g) {
     return padded <= kWgradX3MostWaste * products && 2.0 * products * g.N * g.H * g.R * g.S >= kWgradX3LeastOps;
 }
 
-template <class E, int PARTS, int S, int RB, bool LOW>
-static void launch_wgrad_same_one(hipStream_t st, unsigned blocks, const WgradSame<E>& geo, const GemmDims& d) {
-    hipLaunchKernelGGL((wgrad_same_kernel<E, PARTS, S, RB, LOW>), dim3(blocks), dim3(NT), 0, st, geo, d);
-}
-
 // Splits of the reduction. A compute unit takes a slice of one workgroup in kAlone us, of two together in kPair (S = 3; measured on
 // 64 x 128 x 112 x 112), prologue and epilogue are about four slices.
 static long wgrad_same_splits(long tiles, long slices, size_t out_bytes, size_t room, int S, int num_cu) {
@@ -148,10 +147,10 @@ static long wgrad_same_splits(long tiles, long slices, size_t out_bytes, size_t 
     return best;
 }
 
-template <class E>
-static int launch_wgrad_same(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const E* x, const E* dy, float* w, float alpha, int accumulate,
-                             float* staging, size_t staging_bytes, bool* taken, BiasOut* bias) {
+int launch_wgrad_same_x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const float* x, const float* dy, float* w, float alpha, int accumulate,
+                         float* staging, size_t staging_bytes, bool* taken, BiasOut* bias) {
     *taken = false;
+    if (!wgrad_same_x3_ok(g)) return VDNN_OK;
     const int S = g.S, M = g.K, N = g.C * S * S, WP = g.W + S / 2, HW = g.H * g.W;
     const int Kred = g.N * g.H * WP;
     constexpr int TM = 64;
@@ -161,17 +160,17 @@ static int launch_wgrad_same(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, co
     GemmDims d = make_dims(M, N, Kred, TM, S * WS_CH, (int)splits, WS_SLICE);
     d.mtiles = mtiles; d.ntiles = ntiles;
     const long nspan = d.kchunk / (g.H * WP) + 3;
-    if (nspan * g.K * HW * (long)sizeof(E) >= (long)MAX_SUM_RANGE || nspan * g.C * HW * (long)sizeof(E) >= (long)MAX_SUM_RANGE) return VDNN_OK; // not taken
+    if (nspan * g.K * HW * 4 >= (long)MAX_SUM_RANGE || nspan * g.C * HW * 4 >= (long)MAX_SUM_RANGE) return VDNN_OK; // not taken
     const long blocks = tiles * d.splits;
     if (blocks <= 0 || blocks >= (1l << 31)) return VDNN_OK;
     *taken = true;
     const bool with_bias = bias && bias->wanted() && bias_parts_fit(ctx, g.K, d.splits);
-    const WgradSame<E> geo{dy, x, g.N, g.K, g.C, g.H, g.W, w, staging, (long)M * N, alpha, accumulate, with_bias ? ctx->bias_scratch : nullptr, d.splits,
+    const WgradSame geo{dy, x, g.N, g.K, g.C, g.H, g.W, w, staging, (long)M * N, alpha, accumulate, with_bias ? ctx->bias_scratch : nullptr, d.splits,
                            Kred, WS_SLICE / WP, WS_SLICE % WP};
     {
         ProfScope prof(ctx, st, S == 3 ? "conv_bwd_filter_x3_3x3" : "conv_bwd_filter_x3_5x5", 2.0 * M * (double)N * (double)g.N * HW, 0.0);
-        if (S == 5) launch_wgrad_same_one<E, 3, 5, 1, true>(st, (unsigned)blocks, geo, d);
-        else launch_wgrad_same_one<E, 3, 3, 1, true>(st, (unsigned)blocks, geo, d);
+        if (S == 5) hipLaunchKernelGGL(wgrad_same_kernel<5>, dim3((unsigned)blocks), dim3(NT), 0, st, geo, d);
+        else hipLaunchKernelGGL(wgrad_same_kernel<3>, dim3((unsigned)blocks), dim3(NT), 0, st, geo, d);
         VDNN_LAUNCH_CHECK();
     }
     if (with_bias) {
@@ -182,10 +181,4 @@ static int launch_wgrad_same(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, co
     if (d.splits > 1) return launch_reduce_splits_tap(ctx, st, w, staging, (size_t)M * N, d.splits, alpha, accumulate, g.C, S * S);
     return VDNN_OK;
 }
-int launch_wgrad_same_x3(vdnn_ctx* ctx, hipStream_t st, const ConvGeo& g, const float* x, const float* dy, float* w, float alpha, int accumulate,
-                         float* staging, size_t staging_bytes, bool* taken, BiasOut* bias) {
-    *taken = false;
-    return wgrad_same_x3_ok(g) ? launch_wgrad_same<float>(ctx, st, g, x, dy, w, alpha, accumulate, staging, staging_bytes, taken, bias) : VDNN_OK;
-}
-
 } // namespace vdnn
