@@ -1424,8 +1424,12 @@ static int conv_bwd_filter_core(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_
         return nspan * g.K * PQ * (long)sizeof(E) < (long)MAX_SUM_RANGE && nspan * g.C * g.H * g.W * (long)sizeof(E) < (long)MAX_SUM_RANGE;
     };
     const GemmDims d_small = make_dims(M, N, (int)Kred, 64, 64, plan.splits);
+    // Rows that end in the first half of a 128-row tile leave a 64-row tile less to multiply for nothing than the estimates see
+    // (21 x 70 x 53 x 37, 130 of 3x3 at stride 2 54 -> 50 us, 16 x 100 x 40 x 40 51 -> 46, 10 x 33 x 60 x 60, 150 of 5x5 62 -> 57); small
+    // products go by the estimates, which are right there (2 x 16 x 8 x 8, 275 of 3x3 10.7 us, 12.5 in the other tile).
+    const bool half_tile = !narrow && M % TM != 0 && M % TM <= 64 && 2.0 * M * (double)N * (double)Kred >= 5e8;
     const bool small = (Kred <= kShortReduction || (2.0 * M * (double)N * (double)Kred <= kSmallTileOps &&
-                                                    plan.us < 0.9 * large_tile_us(M, N, Kred, TM, TN, want, ctx->num_cu, true, tap_shape && g.C % 32 == 0 ? 1.0 : 1.15))) &&
+                                                    plan.us < (half_tile ? 1.12 : 0.9) * large_tile_us(M, N, Kred, TM, TN, want, ctx->num_cu, true, tap_shape && g.C % 32 == 0 ? 1.0 : 1.15))) &&
                        span_ok(d_small.kchunk);
     const GemmDims d = small ? d_small : make_dims(M, N, (int)Kred, TM, TN, want);
     VDNN_REQUIRE(span_ok(d.kchunk), "samples of one reduction split too large for one descriptor");
