@@ -14,7 +14,8 @@
 // without gaps, in the order in which the packing teams claimed their place (an atomic cursor), so the
 // stream is as long as its content and its length is known on the device only.
 //
-// Offload. The packing kernel reads the tensor at HBM speed. Bytes of the stream below `staging_bytes` go to
+// Offload. The packing kernel reads the tensor at HBM speed (zvc_pack_rows_kernel; without a staging buffer
+// zvc_pack_kernel stores everything into host memory). Bytes of the stream below `staging_bytes` go to
 // a staging buffer in device memory, which the copy engine then moves to the pinned host buffer like any
 // other offload; bytes beyond it are stored by the kernel straight into the host buffer through the device's
 // mapping of pinned memory. The caller sizes the staging buffer from the length the same tensor had the step
@@ -23,6 +24,8 @@
 // beside a kernel that wrote the whole stream that way), loads from host memory do not: so the way out
 // goes through the copy engine, and the way back is a kernel that reads the host buffer and expands as it goes.
 #include "backend_internal.h"
+
+#include <algorithm>
 
 namespace vdnn {
 
@@ -37,6 +40,10 @@ static constexpr int kZvcPad = 8;           // elements of zero fill behind the 
 // workgroups cost few places.
 static constexpr int kZvcTeams = 4;
 static constexpr int kZvcThreads = 256 * kZvcTeams;
+// Workgroups per compute unit of zvc_pack_rows_kernel. One leaves the convolution beside it alone but takes twice as long by itself
+// (a pooling layer has no matrix work to hide it behind): a step of VGG16 at batch 128 in bfloat16 22.4 ms with one, 21.9 with two
+// and four, 21.8 with three, 22.0 with eight.
+static constexpr int kZvcPackPerCu = 3;
 static constexpr int kZvcCursors = 64;      // offloads that may be in flight at once
 
 __host__ __device__ inline size_t zvc_table_bytes(size_t chunks) { return (chunks * 4 + 15) / 16 * 16; }
@@ -51,31 +58,152 @@ struct alignas(16) ZvcRecord {
     E kept[kZvcChunk + kZvcPad];
 };
 
-__global__ void zvc_begin_kernel(unsigned long long* cursor, unsigned long long table_bytes) { *cursor = table_bytes; }
+// Where an offload's claims stand: the bytes of records claimed so far, and the workgroups that are done. Both words are zero
+// between offloads: the workgroup that is done last puts them back, so no launch before the packing kernel clears them and
+// none behind it reads them (they were two launches of 5 us each, one after the other with the packing kernel, per tensor).
+struct ZvcCursor {
+    unsigned long long claimed;
+    unsigned long long done;
+};
 
+// The end of a packing workgroup, by one of its threads, whose claims have all returned.
 // total: length of the stream. link: bytes that cross the link for it (the copy engine moves `staging_bytes`
-// whatever the stream's length; with staging_bytes = ~0 the block stays on the device and only what did not fit
-// crossed the link - the caller passes the block's size in `kept_bytes` then).
-__global__ void zvc_end_kernel(const unsigned long long* cursor, unsigned long long staging_bytes, unsigned long long kept_bytes,
-                               unsigned long long* total_host, unsigned long long* link_bytes) {
-    const unsigned long long total = *cursor;
+// whatever the stream's length; with keep the block stays on the device and only what did not fit crosses the link).
+__device__ __forceinline__ void zvc_finish(ZvcCursor* cursor, unsigned long long table_bytes, unsigned long long staging_bytes, bool keep,
+                                           unsigned long long* total_host, unsigned long long* link_bytes) {
+    if (atomicAdd(&cursor->done, 1ull) != gridDim.x - 1) return;
+    const unsigned long long total = table_bytes + atomicExch(&cursor->claimed, 0ull);
+    atomicExch(&cursor->done, 0ull);
     if (total_host) *total_host = total;
-    if (staging_bytes == ~0ull) atomicAdd(link_bytes, total > kept_bytes ? total - kept_bytes : 0ull);
+    if (keep) atomicAdd(link_bytes, total > staging_bytes ? total - staging_bytes : 0ull);
     else atomicAdd(link_bytes, total > staging_bytes ? total : staging_bytes);
 }
 
-// E is the element as raw bits (uint32_t for float, uint16_t for bfloat16).
+struct ZvcReport {
+    unsigned long long* total_host;
+    unsigned long long* link_bytes;
+    int keep;
+};
+
+// Packing into a staging buffer in device memory. A wavefront has a chunk to itself: it holds the chunk's 4096 elements in registers (a lane
+// a map word as well), a workgroup of four claims the place of its records together (a claim is an atomic on one word for the
+// whole device, 3.5 ns apiece), and every row of 64 elements leaves with one masked store of its kept elements, which lie one
+// behind the other. No element goes through LDS and a wavefront meets the others of its workgroup twice per chunk.
+// Alone it is bound by memory: 411 MB of floats, half of them zero, in 149 us (4.2 TB/s read and written; a large copy
+// reaches 4.7), of bfloat16 in 197 us (151 and 212 through LDS). In a training step it runs beside a convolution, and
+// what counts is the room it takes there: workgroups of sixteen wavefronts with 35 to 68 KB of LDS waited for a place
+// until the convolution's first round was over and ended behind it (64 channels of 112 x 112, batch 128, bfloat16: 715 us beside a
+// convolution of 536); this one starts at once, 53 (bfloat16) or 88 registers a wavefront, and takes 254 to 316 us there.
+template <class E>
+__global__ __launch_bounds__(256) void zvc_pack_rows_kernel(const E* __restrict__ src, size_t count, size_t chunks,
+                                                            unsigned char* __restrict__ staging, size_t staging_bytes,
+                                                            unsigned char* __restrict__ host, ZvcCursor* __restrict__ cursor, ZvcReport report) {
+    constexpr int V = 16 / int(sizeof(E));   // elements per 128-bit load
+    constexpr int kBlocks = kZvcChunk / (64 * V);
+    __shared__ unsigned wave_bytes[4];
+    __shared__ unsigned long long place;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const bool aligned = (reinterpret_cast<uintptr_t>(src) & 15) == 0;   // (chunks start at multiples of 16 bytes)
+    const size_t table_bytes = zvc_table_bytes(chunks);
+    // every wavefront of a workgroup makes the same number of trips, so that the barriers meet
+    for (size_t first_chunk = size_t(blockIdx.x) * 4; first_chunk < chunks; first_chunk += size_t(gridDim.x) * 4) {
+        const size_t chunk = first_chunk + wave;
+        const bool live = chunk < chunks;
+        const size_t base = chunk * kZvcChunk + size_t(lane) * V;
+        v4u q[kBlocks];   // q[b]: this lane's V elements of block b
+        if (live && aligned && (chunk + 1) * kZvcChunk <= count) {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) q[b] = *reinterpret_cast<const v4u*>(src + base + size_t(b) * 64 * V);
+        } else {
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b) {
+                const size_t idx = base + size_t(b) * 64 * V;
+                unsigned w[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int j = 0; j < V; ++j)
+                    if (live && idx + j < count) w[j * int(sizeof(E)) / 4] |= unsigned(src[idx + j]) << (j * int(sizeof(E)) % 4 * 8);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) q[b][j] = w[j];
+            }
+        }
+        auto element = [&](int b, int j) -> E { return E(q[b][j * int(sizeof(E)) / 4] >> (j * int(sizeof(E)) % 4 * 8)); };
+        unsigned long long word = 0;   // word `lane` of the map
+        unsigned kept = 0;
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+            for (int j = 0; j < V; ++j) {
+                const unsigned long long m = __ballot(element(b, j) != 0);
+                word = lane == b * V + j ? m : word;
+                kept += __popcll(m);
+            }
+        const unsigned bytes = live ? kZvcMapBytes + (kept * unsigned(sizeof(E)) + 15u) / 16u * 16u : 0u;
+        if (lane == 0) wave_bytes[wave] = bytes;
+        __syncthreads();
+        if (threadIdx.x == 0) place = atomicAdd(&cursor->claimed, (unsigned long long)(wave_bytes[0] + wave_bytes[1] + wave_bytes[2] + wave_bytes[3]));
+        unsigned ahead = 0;   // (read between the barriers: behind the second one the next trip's sizes may come in)
+#pragma unroll
+        for (int w = 0; w < 3; ++w) ahead += w < wave ? wave_bytes[w] : 0u;
+        __syncthreads();
+        size_t at = table_bytes + place + ahead;
+        if (!live) continue;   // (in the last trip only)
+        at = (size_t)__builtin_amdgcn_readfirstlane(unsigned(at)) | (size_t)__builtin_amdgcn_readfirstlane(unsigned(at >> 32)) << 32;
+        if (lane == 0) {
+            const size_t entry = chunk * 4;
+            *reinterpret_cast<unsigned*>((entry < staging_bytes ? staging : host) + entry) = unsigned(at / 16);
+        }
+        const unsigned fill = (bytes - kZvcMapBytes) / unsigned(sizeof(E)) - kept;   // elements of zero fill
+        if (at + bytes <= staging_bytes) {
+            unsigned char* p = staging + at;
+            reinterpret_cast<unsigned long long*>(p)[lane] = word;
+            p += kZvcMapBytes;
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    const E e = element(b, j);
+                    const unsigned long long m = __ballot(e != 0);
+                    const unsigned to = __builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0u));
+                    if (e != 0) reinterpret_cast<E*>(p)[to] = e;
+                    p += size_t(__popcll(m)) * sizeof(E);
+                }
+            if (unsigned(lane) < fill) reinterpret_cast<E*>(p)[lane] = E(0);
+        } else {
+            // the record ends behind the staging buffer: each piece goes where its place lies
+            auto target = [&](size_t o) { return (o < staging_bytes ? staging : host) + o; };
+            *reinterpret_cast<unsigned long long*>(target(at + size_t(lane) * 8)) = word;
+            size_t o = at + kZvcMapBytes;
+#pragma unroll
+            for (int b = 0; b < kBlocks; ++b)
+#pragma unroll
+                for (int j = 0; j < V; ++j) {
+                    const E e = element(b, j);
+                    const unsigned long long m = __ballot(e != 0);
+                    const unsigned to = __builtin_amdgcn_mbcnt_hi(unsigned(m >> 32), __builtin_amdgcn_mbcnt_lo(unsigned(m), 0u));
+                    if (e != 0) *reinterpret_cast<E*>(target(o + to * sizeof(E))) = e;
+                    o += size_t(__popcll(m)) * sizeof(E);
+                }
+            if (unsigned(lane) < fill) *reinterpret_cast<E*>(target(o + lane * sizeof(E))) = E(0);
+            // a wavefront has one record on its way to host memory at a time: stores that pile up ahead of the link
+            // hold up the stores of the kernels on the other streams behind them
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        }
+    }
+    if (threadIdx.x == 0) zvc_finish(cursor, table_bytes, staging_bytes, report.keep != 0, report.total_host, report.link_bytes);
+}
+
+// Packing straight into host memory. The records go through LDS, so that what crosses the link are whole 16-byte pieces side by
+// side, and few workgroups share the link. E is the element as raw bits (uint32_t for float, uint16_t for bfloat16).
 template <class E>
 __global__ __launch_bounds__(kZvcThreads) void zvc_pack_kernel(const E* __restrict__ src, size_t count, size_t chunks,
-                                                               unsigned char* __restrict__ staging, size_t staging_bytes,
-                                                               unsigned char* __restrict__ host, unsigned long long* __restrict__ cursor) {
+                                                               unsigned char* __restrict__ host, ZvcCursor* __restrict__ cursor, ZvcReport report) {
     __shared__ ZvcRecord<E> rec[kZvcTeams];
     __shared__ unsigned wave_total[kZvcTeams][4];
     __shared__ unsigned long long place[kZvcTeams];
     const int team = threadIdx.x >> 8, tid = threadIdx.x & 255;
     const int lane = tid & 63, wave = tid >> 6;
     const unsigned long long below = (1ull << lane) - 1ull;
-    const size_t stride = size_t(gridDim.x) * kZvcTeams;
+    const size_t stride = size_t(gridDim.x) * kZvcTeams, table_bytes = zvc_table_bytes(chunks);
     const bool aligned = (reinterpret_cast<uintptr_t>(src) & 15) == 0;   // (chunks start at multiples of 16 bytes)
     // every team makes the same number of trips, so that the barriers meet; a team past the end idles through them
     for (size_t first_chunk = size_t(blockIdx.x) * kZvcTeams; first_chunk < chunks; first_chunk += stride) {
@@ -113,8 +241,7 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_pack_kernel(const E* __restri
         for (int w = 0; w < 4; ++w) { const unsigned t = wave_total[team][w]; pos += w < wave ? t : 0u; total += t; }
         const unsigned units = kZvcMapBytes / 16 + (total * unsigned(sizeof(E)) + 15u) / 16u;   // 16-byte units of the record
         if (threadIdx.x == 0) {
-            // one claim for the workgroup's records: every claim is an atomic on the same word, and the device does
-            // about one of those in 3.5 ns (a quarter of this kernel's time on a float tensor, half on a bfloat16 one)
+            // one claim for the workgroup's records: every claim is an atomic on the same word
             unsigned bytes[kZvcTeams], all = 0;
 #pragma unroll
             for (int t = 0; t < kZvcTeams; ++t) {
@@ -124,7 +251,7 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_pack_kernel(const E* __restri
                 bytes[t] = first_chunk + t < chunks ? kZvcMapBytes + (n * unsigned(sizeof(E)) + 15u) / 16u * 16u : 0u;
                 all += bytes[t];
             }
-            unsigned long long at = atomicAdd(cursor, (unsigned long long)all);
+            unsigned long long at = table_bytes + atomicAdd(&cursor->claimed, (unsigned long long)all);
 #pragma unroll
             for (int t = 0; t < kZvcTeams; ++t) { place[t] = at; at += bytes[t]; }
         }
@@ -137,21 +264,16 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_pack_kernel(const E* __restri
         __syncthreads();
         if (live) {
             const size_t at = place[team];
-            if (tid == 0) {
-                const size_t entry = chunk * 4;
-                *reinterpret_cast<unsigned*>((entry < staging_bytes ? staging : host) + entry) = unsigned(at / 16);
-            }
+            if (tid == 0) *reinterpret_cast<unsigned*>(host + chunk * 4) = unsigned(at / 16);
             const v4u* in = reinterpret_cast<const v4u*>(&rec[team]);
-            for (unsigned u = tid; u < units; u += 256) {
-                const size_t o = at + size_t(u) * 16;
-                *reinterpret_cast<v4u*>((o < staging_bytes ? staging : host) + o) = in[u];
-            }
+            for (unsigned u = tid; u < units; u += 256) *reinterpret_cast<v4u*>(host + at + size_t(u) * 16) = in[u];
             // a team has one record on its way to host memory at a time: stores that pile up ahead of the link
             // hold up the stores of the kernels on the other streams behind them
-            if (at + size_t(units) * 16 > staging_bytes) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         }
         __syncthreads();
     }
+    if (threadIdx.x == 0) zvc_finish(cursor, table_bytes, 0, report.keep != 0, report.total_host, report.link_bytes);
 }
 
 // The stream's bytes below `device_bytes` are read from `device` (a staging block that was kept), the rest from `host`.
@@ -222,9 +344,10 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_unpack_kernel(const unsigned 
 
 static int zvc_ensure_counters(vdnn_ctx* ctx) {
     if (ctx->zvc_counters) return VDNN_OK;
-    // [0]: bytes over the link; [1 .. kZvcCursors]: stream cursors, one per offload in flight
-    VDNN_HIP(hipMalloc((void**)&ctx->zvc_counters, sizeof(unsigned long long) * (1 + kZvcCursors)));
-    VDNN_HIP(hipMemset(ctx->zvc_counters, 0, sizeof(unsigned long long) * (1 + kZvcCursors)));
+    // [0], [1]: bytes over the link; then the stream cursors, one per offload in flight
+    const size_t bytes = sizeof(unsigned long long) * 2 + sizeof(ZvcCursor) * kZvcCursors;
+    VDNN_HIP(hipMalloc((void**)&ctx->zvc_counters, bytes));
+    VDNN_HIP(hipMemset(ctx->zvc_counters, 0, bytes));
     return VDNN_OK;
 }
 
@@ -248,24 +371,22 @@ static int zvc_offload(vdnn_ctx* ctx, void* dst_host, void* staging_dev, size_t 
     VDNN_REQUIRE(staging_bytes <= vdnn_zvc_buffer_bytes(count, elem_bytes), "staging buffer longer than the longest stream");
     if (int rc = zvc_ensure_counters(ctx)) return rc;
     const size_t chunks = (count + kZvcChunk - 1) / kZvcChunk;
-    unsigned long long* cursor = ctx->zvc_counters + 1 + (ctx->zvc_next_cursor++ % kZvcCursors);
-    // with a staging buffer the kernel works at HBM speed and should be gone soon; without one it is bound by
-    // the link and by how many stores it may have in flight
-    const size_t need = (chunks + kZvcTeams - 1) / kZvcTeams;
-    const size_t cap = staging_bytes ? size_t(ctx->num_cu) * 2 : size_t(ctx->num_cu) / 8;
-    const int grid = int(need < cap ? need : cap);
+    ZvcCursor* cursor = reinterpret_cast<ZvcCursor*>(ctx->zvc_counters + 2) + ctx->zvc_next_cursor++ % kZvcCursors;
+    const ZvcReport report{total_host, ctx->zvc_counters, keep_on_device};
+    auto grid = [&](size_t per_workgroup, size_t cap) { return int(std::min((chunks + per_workgroup - 1) / per_workgroup, cap)); };
     {
         ProfScope prof(ctx, ps, staging_bytes ? "offload_zvc_pack" : "offload_zvc", 0.0, (double)(count * elem_bytes));
-        zvc_begin_kernel<<<1, 1, 0, ps>>>(cursor, zvc_table_bytes(chunks));
-        if (elem_bytes == 4)
-            zvc_pack_kernel<uint32_t><<<grid, kZvcThreads, 0, ps>>>((const uint32_t*)src_dev, count, chunks, (unsigned char*)staging_dev, staging_bytes,
-                                                                     (unsigned char*)dst_host, cursor);
-        else
-            zvc_pack_kernel<uint16_t><<<grid, kZvcThreads, 0, ps>>>((const uint16_t*)src_dev, count, chunks, (unsigned char*)staging_dev, staging_bytes,
-                                                                     (unsigned char*)dst_host, cursor);
-        VDNN_HIP(hipGetLastError());
-        zvc_end_kernel<<<1, 1, 0, ps>>>(cursor, keep_on_device ? ~0ull : (unsigned long long)staging_bytes, (unsigned long long)staging_bytes, total_host,
-                                     ctx->zvc_counters);
+        auto pack = [&](auto element) {
+            using E = decltype(element);
+            if (staging_bytes)
+                zvc_pack_rows_kernel<E><<<grid(4, size_t(ctx->num_cu) * kZvcPackPerCu), 256, 0, ps>>>((const E*)src_dev, count, chunks, (unsigned char*)staging_dev,
+                                                                                          staging_bytes, (unsigned char*)dst_host, cursor, report);
+            else   // bound by the link and by how many stores it may have in flight
+                zvc_pack_kernel<E><<<grid(kZvcTeams, size_t(ctx->num_cu) / 8), kZvcThreads, 0, ps>>>((const E*)src_dev, count, chunks, (unsigned char*)dst_host,
+                                                                                               cursor, report);
+        };
+        if (elem_bytes == 4) pack(uint32_t(0));
+        else pack(uint16_t(0));
         VDNN_HIP(hipGetLastError());
     }
     if (packed) {
