@@ -70,6 +70,7 @@ static int launch_igemm(vdnn_ctx* ctx, hipStream_t stream, const char* name, con
     // unpadded layer multiplies taps that fall outside the output; they are not counted)
     ProfScope prof(ctx, stream, name, flops > 0.0 ? flops : 2.0 * d.M * (double)d.N * d.K, 0.0);
     if constexpr (HALF) hipLaunchKernelGGL((igemm_bf16_kernel<TM, TN, AL, BL, EP>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
+    else if constexpr (TM == 64 && TN == 64) launch_igemm64((unsigned)blocks, stream, al, bl, ep, d);
     else hipLaunchKernelGGL((igemm_kernel<TM, TN, AL, BL, EP>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
@@ -979,7 +980,8 @@ static int launch_strided_bwd_data(vdnn_ctx* ctx, hipStream_t st, const ConvGeo&
         VDNN_REQUIRE(blocks < (1l << 31), "grid too large");
         {
             ProfScope prof(ctx, st, "conv_bwd_data_classes_64x64", 2.0 * nc * (double)g.K * g.C * g.R * g.S * g.P * g.Q, 0.0);
-            hipLaunchKernelGGL(igemm_classes_kernel<E>, dim3((unsigned)blocks), dim3(NT), 0, st, launch);
+            if (small_tile_ahead(launch.c[launch.count - 1].d, blocks)) hipLaunchKernelGGL((igemm_classes_kernel<E, kSmallTileAhead>), dim3((unsigned)blocks), dim3(NT), 0, st, launch);
+            else hipLaunchKernelGGL((igemm_classes_kernel<E, 1>), dim3((unsigned)blocks), dim3(NT), 0, st, launch);
             VDNN_LAUNCH_CHECK();
         }
         const long total = (long)nc * per_sample;

@@ -70,6 +70,7 @@ __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPa
     constexpr int NJ = CW / 32;          // 32-column blocks of a wavefront
     __shared__ __attribute__((aligned(16))) unsigned short As[2][TM * HSTRIDE];
     __shared__ __attribute__((aligned(16))) unsigned short Bw[2][(W3_ROWS + 1) * HSTRIDE]; // the window and a row of zeros
+    __shared__ __attribute__((aligned(16))) float bias_rows[SPLIT ? 4 : TM]; // read before the reduction: behind it, a round trip to memory per row
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
@@ -163,6 +164,9 @@ __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPa
         }
     }
     if (tid < HSTRIDE) { Bw[0][W3_ROWS * HSTRIDE + tid] = 0; Bw[1][W3_ROWS * HSTRIDE + tid] = 0; }
+    if constexpr (!SPLIT) {
+        if (ep.bias && tid < TM) bias_rows[tid] = ep.bias[min(m0 + tid, d.M - 1)];
+    }
 
     // Two windows are in flight: the one fetched for the row step after the next, and the one for the step after
     // that. [item][pixel of the pair]: eight channels each, ready for LDS; the halo element of this lane (wavefront 0).
@@ -373,20 +377,25 @@ __global__ void __launch_bounds__(NT, RESIDENT) conv3x3_bf16_kernel(const LoadPa
             __syncthreads(); // every wavefront has read its last fragments
             unsigned short* stg = &Bw[0][0] + wave * (64 * STG);
 #pragma unroll
-            for (int it = 0; it < 2; it++)
+            for (int it = 0; it < 2; it++) {
+                floatx4 bv[4];
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int row = it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                    const int m = m0 + row;
-                    const float b = (ep.bias && m < d.M) ? ep.bias[m] : 0.0f;
+                for (int q = 0; q < 4; q++) bv[q] = *(const floatx4*)(bias_rows + it * 32 + 8 * q + 4 * lk);
 #pragma unroll
-                    for (int jt = 0; jt < 2; jt++) {
-                        float r = acc[0][it][jt][v];
-                        if (ep.bias) r += b;
-                        if (ep.relu) r = relu_value(r);
-                        stg[row * STG + jt * 32 + l32] = float_to_bf16_bits(r);
+                for (int jt = 0; jt < 2; jt++) {
+                    floatx16 r = acc[0][it][jt];
+                    if (ep.bias) {
+#pragma unroll
+                        for (int v = 0; v < 16; v++) r[v] += bv[v / 4][v % 4];
                     }
+                    if (ep.relu) {
+#pragma unroll
+                        for (int v = 0; v < 16; v++) r[v] = relu_value(r[v]);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 16; v++) stg[(it * 32 + result_row(v, lk)) * STG + jt * 32 + l32] = float_to_bf16_bits(r[v]);
                 }
+            }
             __builtin_amdgcn_wave_barrier(); // the block is read by other lanes of the same wavefront: LDS keeps a wavefront's order
             if (j < d.N) {
 #pragma unroll

@@ -21,6 +21,14 @@ __device__ __forceinline__ unsigned valid_window_bits(int origin, int window, in
     return ((1u << hi) - 1u) & ~((1u << lo) - 1u);
 }
 
+// ... with 0 <= origin - t < extent
+__device__ __forceinline__ unsigned valid_mirrored_bits(int origin, int window, int extent) {
+    int lo = origin - extent + 1; if (lo < 0) lo = 0;
+    int hi = origin + 1; if (hi > window) hi = window;
+    if (hi <= lo) return 0u;
+    return ((1u << hi) - 1u) & ~((1u << lo) - 1u);
+}
+
 // ---- im2col operand, columns = output pixels (row-major in LDS: lanes run along pixels) ---------
 // MODE 0: forward gather from x.          src[n, ch, oh*sh-ph+r, ow*sw-pw+s]
 // MODE 1: backward data, stride 1.        src[n, ch, oh+ph-r,    ow+pw-s]          (src = dy)
@@ -82,19 +90,13 @@ struct LoadIm2colPix {
         if (n_last > nsamples - 1) n_last = nsamples - 1;
         st.rsrc = make_rsrc(src + first + shift, clamp_range(((long)(n_last - n_first + 1) * sample_elems - shift) * ES));
         unsigned vrow = 0, vcol = 0; // valid taps
-        for (int r = 0; r < R; r++) {
-            bool ok;
-            if (MODE == 0) ok = (unsigned)(ih0 + r) < (unsigned)Hs;
-            else if (MODE == 1) ok = (unsigned)(ih0 - r) < (unsigned)Hs;
-            else { const int t = ih0 - r; ok = t >= 0 && t % sh == 0 && t / sh < Hs; }
-            if (ok) vrow |= 1u << r;
-        }
-        for (int s = 0; s < S; s++) {
-            bool ok;
-            if (MODE == 0) ok = (unsigned)(iw0 + s) < (unsigned)Ws;
-            else if (MODE == 1) ok = (unsigned)(iw0 - s) < (unsigned)Ws;
-            else { const int t = iw0 - s; ok = t >= 0 && t % sw == 0 && t / sw < Ws; }
-            if (ok) vcol |= 1u << s;
+        if (MODE == 0) {
+            vrow = valid_window_bits(ih0, R, Hs); vcol = valid_window_bits(iw0, S, Ws);
+        } else if (MODE == 1) {
+            vrow = valid_mirrored_bits(ih0, R, Hs); vcol = valid_mirrored_bits(iw0, S, Ws);
+        } else {
+            for (int r = 0; r < R; r++) { const int t = ih0 - r; if (t >= 0 && t % sh == 0 && t / sh < Hs) vrow |= 1u << r; }
+            for (int s = 0; s < S; s++) { const int t = iw0 - s; if (t >= 0 && t % sw == 0 && t / sw < Ws) vcol |= 1u << s; }
         }
         if (!valid) { vrow = 0; vcol = 0; }
         st.invrow = ~vrow; st.invcol = ~vcol;
@@ -130,6 +132,8 @@ struct LoadIm2colPix {
         for (int i = 0; i < T * KB / NT; i++) lds[(tid / T + (NT / T) * i) * T + tid % T] = r.s[i];
     }
 };
+
+template <bool BIGWIN, class E> struct FetchesAhead<LoadIm2colPix<2, BIGWIN, E>> { static constexpr bool V = false; };
 
 // ---- filter bank as the A operand of backward data: A[c][(k,r,s)] = w[k,c,r,s] ------------------
 // a gather (runs of R*S contiguous values): 32-bit loads, thread t: kk t%16 of rows t/16 + 16*i
@@ -362,6 +366,45 @@ struct StoreNCHW {
     int relu;          // rectify the result (after the bias)
     const E* gate;     // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
     static constexpr bool TAIL = true;
+    // The gate or the bias (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; rows and columns past the end
+    // read some element inside. (A gate that is the output tensor - the gradient written over the layer's own input - is read by
+    // the lane that overwrites it, before it does.)
+    __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
+        const int lk = lane >> 5;
+        if (to_partial) return;
+        if (gate) {
+            const int j = min(j0 + (lane & 31), d.N - 1), n = j / opix, pix = j - n * opix;
+            const E* from = gate + (size_t)n * d.M * opix + pix;
+#pragma unroll
+            for (int v = 0; v < 16; v++) aux[v] = load_elem(from + (size_t)min(m0 + result_row(v, lk), d.M - 1) * opix);
+        } else if (bias) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) aux[v] = bias[min(m0 + result_row(v, lk), d.M - 1)];
+        }
+    }
+    __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+        const int j = j0 + (lane & 31), lk = lane >> 5;
+        if (j >= d.N) return;
+        const int n = j / opix, pix = j - n * opix;
+        const size_t first = (size_t)n * d.M * opix + pix + (size_t)(m0 + 4 * lk) * opix;
+        if (to_partial) {
+            store_rows(partial + (size_t)ks * d.M * d.N + first, acc, opix, m0, lk, d.M);
+            return;
+        }
+        if (bias) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] += aux[v];
+        }
+        if (relu) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = relu_value(acc[v]);
+        }
+        if (gate) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = aux[v] > 0.0f ? acc[v] : 0.0f;
+        }
+        store_rows(out + first, acc, opix, m0, lk, d.M);
+    }
     // tail mode: a split tile's sums go to partial[slot][row in tile][column in tile], slot = (tile, split)
     template <int MI, int NJ>
     __device__ __forceinline__ void store_tail(const floatx16 (&acc)[MI][NJ], int wm0, int wn0, int lane, long slot, int TM, int TN) const {
@@ -375,56 +418,21 @@ struct StoreNCHW {
                 for (int v = 0; v < 16; v++)
                     po[(wm0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4)) * TN + wn0 + jt * 32 + l32] = acc[it][jt][v];
     }
+    // Blocks of 32 x 32, branches on what is uniform once per block (store_rows). What a block is combined with is read before its first
+    // store, sixteen elements at a time: a load that follows a store through a pointer it might share has to be issued behind it, and
+    // with the load's result needed for the next store that is one round trip to memory per element. Sixteen, not the whole tile: the
+    // registers they wait in count against the three workgroups a compute unit holds.
     template <int MI, int NJ>
     __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
-        const int l32 = lane & 31, lk = lane >> 5;
-        // Bias and gate values are read before the stores they feed, eight at a time: a load that follows a store
-        // through a pointer it might share has to be issued behind it, and with the load's result needed for the next
-        // store that is one round trip to memory per element. Eight, not the whole tile: the registers they wait in
-        // count against the three workgroups a compute unit holds. (A gate that *is* the output tensor - the gradient
-        // written over the layer's own input - is read by the lane that overwrites it, before it does.)
 #pragma unroll
-        for (int jt = 0; jt < NJ; jt++) {
-            const int j = j0 + jt * 32 + l32;
-            if (j >= d.N) continue;
-            const int n = j / opix, pix = j - n * opix;
-            const size_t base = (size_t)n * d.M * opix + pix;
-            E* o = out + base;
-            float* po = partial + (size_t)ks * d.M * d.N + base;
+        for (int it = 0; it < MI; it++) {
+            float aux[16]; // the bias is the same for a row of blocks
+            read_aux(aux, m0 + it * 32, j0, lane, d, to_partial);
 #pragma unroll
-            for (int it = 0; it < MI; it++)
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    float bv[8], gt[8];
-                    if (!to_partial && bias) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const int v = 8 * h + u, m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                            bv[u] = m < d.M ? bias[m] : 0.0f;
-                        }
-                    }
-                    if (!to_partial && gate) {
-#pragma unroll
-                        for (int u = 0; u < 8; u++) {
-                            const int v = 8 * h + u, m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                            gt[u] = m < d.M ? load_elem(gate + base + (size_t)m * opix) : 1.0f;
-                        }
-                    }
-#pragma unroll
-                    for (int u = 0; u < 8; u++) {
-                        const int v = 8 * h + u, m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                        if (m >= d.M) continue;
-                        float r = acc[it][jt][v];
-                        if (to_partial) {
-                            po[(size_t)m * opix] = r;
-                        } else {
-                            if (bias) r += bv[u];
-                            if (relu) r = relu_value(r);
-                            if (gate) r = gt[u] > 0.0f ? r : 0.0f;
-                            store_elem(o + (size_t)m * opix, r);
-                        }
-                    }
-                }
+            for (int jt = 0; jt < NJ; jt++) {
+                if (jt > 0 && gate) read_aux(aux, m0 + it * 32, j0 + jt * 32, lane, d, to_partial);
+                store32(acc[it][jt], aux, m0 + it * 32, j0 + jt * 32, lane, ks, d, to_partial);
+            }
         }
     }
 };

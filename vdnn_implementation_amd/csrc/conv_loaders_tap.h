@@ -202,28 +202,36 @@ struct StoreFilterTap {
     int accumulate;
     FastDiv divC;
     static constexpr bool TAIL = false;
+    // The old values of a lane's sixteen results of a 32x32 block
+    __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
+        if (to_partial || !accumulate) return;
+        const int j = min(j0 + (lane & 31), d.N - 1), lk = lane >> 5, tap = divC.div(j);
+        const float* from = out + (long)(j - tap * C) * RS + tap;
+#pragma unroll
+        for (int v = 0; v < 16; v++) aux[v] = from[(long)min(m0 + result_row(v, lk), d.M - 1) * d.N];
+    }
+    __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+        const int j = j0 + (lane & 31), lk = lane >> 5;
+        if (j >= d.N) return;
+        const long row = (long)(m0 + 4 * lk) * d.N;
+        if (to_partial) {
+            store_rows(partial + (long)ks * partial_stride + row + j, acc, d.N, m0, lk, d.M);
+            return;
+        }
+        const int tap = divC.div(j);
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = accumulate ? __fmaf_rn(alpha, acc[v], aux[v]) : alpha * acc[v];
+        store_rows(out + row + (long)(j - tap * C) * RS + tap, acc, d.N, m0, lk, d.M);
+    }
     template <int MI, int NJ>
     __device__ __forceinline__ void store_tail(const floatx16 (&)[MI][NJ], int, int, int, long, int, int) const {}
     template <int MI, int NJ>
     __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
-        const int l32 = lane & 31, lk = lane >> 5;
 #pragma unroll
-        for (int jt = 0; jt < NJ; jt++) {
-            const int j = j0 + jt * 32 + l32;
-            if (j >= d.N) continue;
-            const int tap = divC.div(j), c = j - tap * C;
-            const long col = (long)c * RS + tap;
-#pragma unroll
-            for (int it = 0; it < MI; it++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                    if (m >= d.M) continue;
-                    const long idx = (long)m * d.N + col;
-                    const float a = acc[it][jt][v];
-                    if (to_partial) partial[(long)ks * partial_stride + (long)m * d.N + j] = a;
-                    else out[idx] = accumulate ? __fmaf_rn(alpha, a, out[idx]) : alpha * a;
-                }
+        for (int b = 0; b < MI * NJ; b++) {
+            float aux[16];
+            read_aux(aux, m0 + b / NJ * 32, j0 + b % NJ * 32, lane, d, to_partial);
+            store32(acc[b / NJ][b % NJ], aux, m0 + b / NJ * 32, j0 + b % NJ * 32, lane, ks, d, to_partial);
         }
     }
 };

@@ -154,6 +154,9 @@ __device__ __forceinline__ floatx4 read_frag(const float* tile, int l32, int lk,
     }
 }
 
+// row of a 32x32 result tile that register v of a lane holds (l >> 5 = lk)
+__device__ __forceinline__ int result_row(int v, int lk) { return 8 * (v / 4) + 4 * lk + v % 4; }
+
 // Launch geometry of one igemm call. Split s covers reduction indices [s*kchunk, min(K, (s+1)*kchunk)).
 // full_tiles > 0 (tail mode): the first full_tiles tiles are computed whole by one workgroup each, only the
 // remaining tiles - the ones that would start a nearly empty last round - are split.
@@ -269,12 +272,34 @@ static inline double large_tile_us(long M, long N, long K, int TM, int TN, int s
     return (us + (double)last * (double)(slices + 2) * slice_us / (last == 1 ? 0.72 : last == 2 ? 0.92 : 1.0)) * 0.88 * load_cost;
 }
 
-// Edge of a wavefront's square sub-tile: 64, or 32 in the 64x64 tile of grids that leave the chip idle.
-template <int TM, int TN> struct WaveTile { static constexpr int V = TM * TN == 64 * 64 ? 32 : 64; };
+// The tile and the part of the reduction that a workgroup computes.
+struct TilePlace {
+    int tile, ks, m0, j0, k_begin, k_end;
+    bool whole; // the whole reduction
+};
+__device__ __forceinline__ TilePlace tile_place(const GemmDims& d, int block, int blocks, int TM, int TN) {
+    // m-tile fastest: workgroups that share a B tile (the large operand) are neighbours
+    const int ntiles_all = d.mtiles * d.ntiles;
+    TilePlace p;
+    if (block < d.full_tiles) {
+        p.tile = xcd_remap(block, d.full_tiles); p.ks = 0; p.whole = true;
+    } else if (d.full_tiles > 0) {
+        const int r = block - d.full_tiles, tl = ntiles_all - d.full_tiles;
+        p.tile = d.full_tiles + r % tl; p.ks = r / tl; p.whole = false;
+    } else {
+        const int bid = xcd_remap(block, blocks);
+        p.tile = bid % ntiles_all; p.ks = bid / ntiles_all; p.whole = d.splits == 1;
+    }
+    p.m0 = p.tile % d.mtiles * TM;
+    p.j0 = p.tile / d.mtiles * TN;
+    p.k_begin = p.whole ? 0 : p.ks * d.kchunk;
+    p.k_end = p.whole ? d.K : min(d.K, p.k_begin + d.kchunk);
+    return p;
+}
 
 template <int TM, int TN, class AL, class BL, class EP>
 __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
-    constexpr int MI = WaveTile<TM, TN>::V / 32, NJ = MI; // MFMA tiles of a wavefront
+    constexpr int MI = 2, NJ = 2; // MFMA tiles of a wavefront
     constexpr int WAVES_M = TM / (32 * MI);
     static_assert(TM % (32 * MI) == 0 && TN % (32 * NJ) == 0 && WAVES_M * (TN / (32 * NJ)) == 4, "four wave tiles");
     using LA = LdsTile<TM, AL::RED_MAJOR>;
@@ -284,23 +309,9 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
 
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6;
-    // m-tile fastest: workgroups that share a B tile (the large operand) are neighbours
-    const int ntiles_all = d.mtiles * d.ntiles;
-    int tile, ks;
-    bool whole;
-    if (block < d.full_tiles) {
-        tile = xcd_remap(block, d.full_tiles); ks = 0; whole = true;
-    } else if (d.full_tiles > 0) {
-        const int r = block - d.full_tiles, tl = ntiles_all - d.full_tiles;
-        tile = d.full_tiles + r % tl; ks = r / tl; whole = false;
-    } else {
-        const int bid = xcd_remap(block, blocks);
-        tile = bid % ntiles_all; ks = bid / ntiles_all; whole = d.splits == 1;
-    }
-    const int mt = tile % d.mtiles, nt = tile / d.mtiles;
-    const int m0 = mt * TM, j0 = nt * TN;
-    const int k_begin = whole ? 0 : ks * d.kchunk;
-    const int k_end = whole ? d.K : min(d.K, k_begin + d.kchunk);
+    const TilePlace at = tile_place(d, block, blocks, TM, TN);
+    const int tile = at.tile, ks = at.ks, m0 = at.m0, j0 = at.j0, k_begin = at.k_begin, k_end = at.k_end;
+    const bool whole = at.whole;
 
     typename AL::template State<TM> sa;
     typename BL::template State<TN> sb;
@@ -396,8 +407,139 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
 }
 
 template <int TM, int TN, class AL, class BL, class EP>
-__global__ void __launch_bounds__(NT) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
+__global__ void __launch_bounds__(NT, 3) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
     igemm_tile<TM, TN>(al, bl, ep, d, blockIdx.x, gridDim.x);
+}
+
+// The 64x64 tile. A workgroup has one wavefront per SIMD and a few to some tens of slices, and where it is taken most of the chip
+// has one or two workgroups a unit: what counts is the latency of every step (1 x 64 x 112 x 112, 64 filters of 3x3, 36 slices on 196
+// lone workgroups, clocked inside the kernel). Against igemm_tile's pipeline:
+// - AHEAD slices are on their way from memory (four, or one where there are few), so that a slice's values are there when they are
+//   written to LDS: operands that another kernel has just written 0.37 -> 0.33 us a slice. (0.21 are the matrix instructions; with
+//   one wavefront per SIMD the rest is the issue of some hundred instructions and the barrier.)
+// - What the result is combined with (bias, gate, old values) is read before the loop, and the epilogue branches on what is
+//   uniform only, once per tile: 2.7 -> 0.9 us.
+// One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
+// four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 102.7.
+template <int AHEAD, class AL, class BL, class EP>
+__device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
+    constexpr int T = 64;
+    using LA = LdsTile<T, AL::RED_MAJOR>;
+    using LB = LdsTile<T, BL::RED_MAJOR>;
+    __shared__ __attribute__((aligned(16))) float As[2][LA::SIZE];
+    __shared__ __attribute__((aligned(16))) float Bs[2][LB::SIZE];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63, wave = tid >> 6;
+    const TilePlace at = tile_place(d, block, blocks, T, T);
+    const int k_begin = at.k_begin, k_end = at.k_end;
+
+    typename AL::template State<T> sa;
+    typename BL::template State<T> sb;
+    al.template init<T>(sa, at.m0, tid, d.M, k_begin);
+    bl.template init<T>(sb, at.j0, tid, d.N, k_begin);
+
+    typename AL::template Regs<T> fa, ra[AHEAD];
+    typename BL::template Regs<T> fb, rb[AHEAD];
+    al.template load<T>(sa, k_begin, k_end, tid, fa);
+    bl.template load<T>(sb, k_begin, k_end, tid, fb);
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+        al.template load<T>(sa, k_begin + (u + 1) * KB, k_end, tid, ra[u]);
+        bl.template load<T>(sb, k_begin + (u + 1) * KB, k_end, tid, rb[u]);
+    }
+
+    const int nslices = (k_end - k_begin + KB - 1) / KB;
+    const int l32 = lane & 31, lk = lane >> 5;
+    const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
+    float aux[16];
+    ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, !at.whole);
+    floatx16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = 0.0f;
+
+    const int a_off = wm0 * LA::ROW_STRIDE, b_off = wn0 * LB::ROW_STRIDE;
+    AL::template store<T>(As[0], tid, fa);
+    BL::template store<T>(Bs[0], tid, fb);
+    __syncthreads();
+    floatx4 a0 = read_frag<T, AL::RED_MAJOR>(As[0] + a_off, l32, lk, 0), b0 = read_frag<T, BL::RED_MAJOR>(Bs[0] + b_off, l32, lk, 0);
+    // Slice s: write slice s+1 to the other LDS buffer, read the second group's fragments, multiply the first group; barrier; fetch
+    // slice s+1+AHEAD into the registers just written, read the first group's fragments of s+1, multiply the second group.
+    // All reads of a buffer precede the barrier after which it is overwritten. Fetches past the end of the range read as zero or
+    // are never used: buffer loads cannot fault.
+    auto slice = [&](int s, int cur, typename AL::template Regs<T>& na, typename BL::template Regs<T>& nb) {
+        const int nxt = cur ^ 1;
+        const floatx4 a1 = read_frag<T, AL::RED_MAJOR>(As[cur] + a_off, l32, lk, 1), b1 = read_frag<T, BL::RED_MAJOR>(Bs[cur] + b_off, l32, lk, 1);
+        AL::template store<T>(As[nxt], tid, na);
+        BL::template store<T>(Bs[nxt], tid, nb);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[e], b0[e], acc, 0, 0, 0);
+        if constexpr (AHEAD > 1) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x300, 16, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 3, 0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; i++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x300, 2, 0); }
+        }
+        __syncthreads();
+        const int kk0 = k_begin + (s + 1 + AHEAD) * KB;
+        al.template load<T>(sa, kk0, k_end, tid, na);
+        bl.template load<T>(sb, kk0, k_end, tid, nb);
+        a0 = read_frag<T, AL::RED_MAJOR>(As[nxt] + a_off, l32, lk, 0);
+        b0 = read_frag<T, BL::RED_MAJOR>(Bs[nxt] + b_off, l32, lk, 0);
+#pragma unroll
+        for (int e = 0; e < 4; e++) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a1[e], b1[e], acc, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
+        }
+    };
+    if constexpr (AHEAD == 1) {
+        for (int s = 0; s < nslices; s++) slice(s, s & 1, ra[0], rb[0]);
+    } else {
+        static_assert(AHEAD % 2 == 0, "a round of slices ends in the LDS buffer it began with");
+        int s = 0;
+        for (; s + AHEAD <= nslices; s += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) slice(s + u, u & 1, ra[u], rb[u]);
+        }
+#pragma unroll
+        for (int u = 0; u + 1 < AHEAD; u++) {
+            if (s + u >= nslices) break;
+            slice(s + u, u & 1, ra[u], rb[u]);
+        }
+    }
+
+    if (EP::TAIL && d.full_tiles > 0 && !at.whole) {
+        const floatx16 tail[1][1] = {{acc}};
+        ep.store_tail(tail, wm0, wn0, lane, (long)(at.tile - d.full_tiles) * d.splits + at.ks, T, T);
+    } else {
+        ep.store32(acc, aux, at.m0 + wm0, at.j0 + wn0, lane, at.ks, d, !at.whole);
+    }
+}
+// Slices ahead: four where the shortest reduction of a workgroup is long enough for them
+constexpr int kSmallTileAhead = 4;
+constexpr long kSmallTileLone = 1024; // workgroups: four on each of 256 compute units, what the registers of that variant leave room for
+static inline bool small_tile_ahead(const GemmDims& d, long blocks) { return d.kchunk >= (kSmallTileAhead + 2) * KB && blocks <= kSmallTileLone; }
+// ... and where the loader's address work does not count for more than the latency (LoadIm2colPix<2>: two divisions per element)
+template <class L> struct FetchesAhead { static constexpr bool V = true; };
+
+template <class AL, class BL, class EP, int AHEAD>
+__global__ void __launch_bounds__(NT) igemm64_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
+    igemm_small_tile<AHEAD>(al, bl, ep, d, blockIdx.x, gridDim.x);
+}
+template <class AL, class BL, class EP>
+static inline void launch_igemm64(unsigned blocks, hipStream_t stream, const AL& al, const BL& bl, const EP& ep, const GemmDims& d) {
+    if constexpr (FetchesAhead<BL>::V) {
+        if (small_tile_ahead(d, blocks)) {
+            hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, kSmallTileAhead>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, 1>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
 }
 
 // ---- dense reduction-major operand: element (row, kk) at base[row*ld + kk] -------------------------
@@ -510,6 +652,22 @@ struct RoundedToBf16 : L {
     }
 };
 
+// A lane's sixteen results of a 32x32 block, `to` at row m0 + 4 lk, rows from M on left out. The test per row is for the blocks at the
+// lower edge only: with a branch on each of a tile's 64 rows, and one each on bias, gate and rectifier, a tile's epilogue took 2.7 us per
+// 32x32 block of a wavefront, most of it the fetch of its text. Forward 9 x 448 x 189 x 189, 576 of 1x1 in bfloat16 631 -> 418 us; 29 x 32 x 30 x 30, 289
+// of 3x3 30 -> 22; backward 11 x 486 x 71 x 71, 64 of 3x3 246 -> 184; floats at two bfloat16 parts, 122 x 80 x 23 x 23, 528 of 3x3 216 -> 198.
+template <class E, class L>
+__device__ __forceinline__ void store_rows(E* to, const floatx16& acc, L stride, int m0, int lk, int M) {
+    if (m0 + 32 <= M) {
+#pragma unroll
+        for (int v = 0; v < 16; v++) store_elem(to + (long)(8 * (v / 4) + v % 4) * stride, acc[v]);
+    } else {
+#pragma unroll
+        for (int v = 0; v < 16; v++)
+            if (m0 + result_row(v, lk) < M) store_elem(to + (long)(8 * (v / 4) + v % 4) * stride, acc[v]);
+    }
+}
+
 // ---- dense result: out[m*ld_m + j] = alpha*acc (+ old if accumulate) (+ bias[j]); or a split's
 //      partial sums to scratch[ks][m*ld_m + j] ------------------------------------------------------
 template <class E = float>
@@ -523,53 +681,58 @@ struct StoreDense {
     int accumulate;
     int relu;      // rectify the result (after the bias)
     const E* gate; // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
+    // The old values or the gate (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; rows and
+    // columns past the end read some element inside.
+    __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
+        if (to_partial || !(accumulate || gate)) return;
+        const int j = min(j0 + (lane & 31), d.N - 1), lk = lane >> 5;
+        const E* from = accumulate ? out : gate;
+#pragma unroll
+        for (int v = 0; v < 16; v++) aux[v] = load_elem(from + (long)min(m0 + result_row(v, lk), d.M - 1) * ld_m + j);
+    }
+    __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
+        const int j = j0 + (lane & 31), lk = lane >> 5;
+        if (j >= d.N) return;
+        const long first = (long)(m0 + 4 * lk) * ld_m + j;
+        if (to_partial) {
+            store_rows(partial + (long)ks * partial_stride + first, acc, ld_m, m0, lk, d.M);
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = accumulate ? __fmaf_rn(alpha, acc[v], aux[v]) : alpha * acc[v];
+        if (bias_j) {
+            const float bj = bias_j[j];
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] += bj;
+        }
+        if (relu) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = relu_value(acc[v]);
+        }
+        if (gate) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[v] = aux[v] > 0.0f ? acc[v] : 0.0f;
+        }
+        store_rows(out + first, acc, ld_m, m0, lk, d.M);
+    }
     static constexpr bool TAIL = false;
     template <int MI, int NJ>
     __device__ __forceinline__ void store_tail(const floatx16 (&)[MI][NJ], int, int, int, long, int, int) const {}
+    // What a block is combined with is read sixteen elements ahead of its stores: a load issued after a store
+    // through the same pointer would have to wait for it (the compiler cannot know that the rows differ), and
+    // sixty-four round trips to memory in a row are the kernel's whole time when the output is large (the filter of
+    // a fully connected layer, updated in place). Sixteen, not more: the registers they wait in count against the
+    // workgroups a compute unit holds.
     template <int MI, int NJ>
     __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
-        const int l32 = lane & 31, lk = lane >> 5;
-        // What the result is combined with is read sixteen elements ahead of the stores: a load issued after a store
-        // through the same pointer would have to wait for it (the compiler cannot know that the rows differ), and
-        // sixty-four round trips to memory in a row are the kernel's whole time when the output is large (the filter of
-        // a fully connected layer, updated in place). Sixteen, not more: the registers they wait in count against the
-        // workgroups a compute unit holds.
-        const bool combine = !to_partial && (accumulate || gate != nullptr);
 #pragma unroll
-        for (int jt = 0; jt < NJ; jt++) {
-            const int j = j0 + jt * 32 + l32;
-            if (j >= d.N) continue;
-            const float bj = (!to_partial && bias_j) ? bias_j[j] : 0.0f;
+        for (int jt = 0; jt < NJ; jt++)
 #pragma unroll
             for (int it = 0; it < MI; it++) {
-                float aux[16]; // the old value (accumulate) or the gate: a call asks for one of the two at most
-                if (combine) {
-#pragma unroll
-                    for (int v = 0; v < 16; v++) {
-                        const int m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                        const long idx = (long)m * ld_m + j;
-                        aux[v] = m < d.M ? (accumulate ? load_elem(out + idx) : load_elem(gate + idx)) : 0.0f;
-                    }
-                }
-#pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const int m = m0 + it * 32 + 8 * (v / 4) + 4 * lk + (v % 4);
-                    if (m >= d.M) continue;
-                    const long idx = (long)m * ld_m + j;
-                    const float a = acc[it][jt][v];
-                    if (to_partial) {
-                        partial[(long)ks * partial_stride + idx] = a;
-                    } else {
-                        // one fused multiply-add: every route to "out += alpha * sum" rounds the same way
-                        float r = accumulate ? __fmaf_rn(alpha, a, aux[v]) : alpha * a;
-                        if (bias_j) r += bj;
-                        if (relu) r = relu_value(r);
-                        if (gate) r = (accumulate ? load_elem(gate + idx) : aux[v]) > 0.0f ? r : 0.0f;
-                        store_elem(out + idx, r);
-                    }
-                }
+                float aux[16];
+                read_aux(aux, m0 + it * 32, j0 + jt * 32, lane, d, to_partial);
+                store32(acc[it][jt], aux, m0 + it * 32, j0 + jt * 32, lane, ks, d, to_partial);
             }
-        }
     }
 };
 
