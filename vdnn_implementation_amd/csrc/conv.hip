@@ -1135,7 +1135,20 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
                     : vdnn_fc_bwd_data(ctx, stream, g.N, g.C * g.H * g.W, g.K, dy, w, dx);
     hipStream_t st = stream_of(ctx, stream);
     StagingCarve carve(ctx);
-    const bool few_channels = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS && !gate; // the vector-ALU kernels have no gated store
+    // Up to four input channels. As a product of C rows the reduction over (k, r, s) fills 3 of a tile's 64 rows (and of a strided layer 16 of
+    // 121 taps); the products w * dy of all taps as rows of a 1x1 convolution fill C*R*S of them, each computed once, and a second kernel adds
+    // them up and gates. Whole gated backward passes of 3 channels, product of C rows -> here: 23 x 176 x 176, 160 filters of 11x11 at stride 4 27.7 ms ->
+    // 0.19; 14 x 128 x 128, 594 of 5x5 3.69 -> 0.81; 25 x 86 x 86, 64 of 3x3 222 us -> 140; bfloat16 8 x 87 x 87, 323 of 11x11 at stride 4 5.5 ms -> 0.06.
+    // Gated layers that keep the product of C rows: 1x1 windows (nothing to save: 108 x 20 x 20, 512 filters 73 us, 97 here) and bfloat16 at
+    // stride 1, where that product runs on the bfloat16 matrix cores (10 x 132 x 132, 26 of 3x3 57 us, 66 here; 28 x 141 x 141, 128 373, 317).
+    const bool rows3 = g.C <= 3 && g.K <= 64 && g.R == 3 && g.S == 3 && g.ph == 1 && g.pw == 1 && g.sh == 1 && g.sw == 1 && (long)g.K * g.P * g.Q * (long)sizeof(E) < (long)MAX_SUM_RANGE;
+    // (the rounded filter of a bfloat16 layer lies in the staging area too; a gated layer whose filter does not fit keeps the other route)
+    const size_t filter_bytes = (size_t)g.K * g.C * g.R * g.S * sizeof(float), rounded_bytes = sizeof(E) == 2 ? (filter_bytes + 255) / 256 * 256 : 0;
+    const bool products = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS && ctx->reduce_scratch &&
+                          ctx->reduce_scratch_bytes >= rounded_bytes + (size_t)g.C * g.R * g.S * g.P * g.Q * sizeof(float) &&
+                          (!gate || !rounded_bytes || filter_bytes + (8u << 20) <= ctx->reduce_scratch_bytes) &&
+                          pixel_tile_span_ok((long)g.K * g.P * g.Q, g.P * g.Q, 256, (int)sizeof(E));
+    const bool few_channels = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS && (!gate || (g.R * g.S > 1 && (sizeof(E) == 4 || g.sh > 1 || g.sw > 1) && (rows3 || products)));
     if (!few_channels && (g.sh != 1 || g.sw != 1)) {
         bool taken = false;
         const int rc = launch_strided_bwd_data<E>(ctx, st, g, dy, w, dx, gate, &taken);
@@ -1152,16 +1165,15 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
         }
     }
     if (few_channels) {
-        if ((g.sh != 1 || g.sw != 1) && ctx->reduce_scratch && ctx->reduce_scratch_bytes >= (size_t)g.C * g.R * g.S * g.P * g.Q * sizeof(float) &&
-                 pixel_tile_span_ok((long)g.K * g.P * g.Q, g.P * g.Q, 256, (int)sizeof(E))) {
-            // Strided layer with few input channels (the 11x11 stride-4 first layers): its three or four
-            // output rows cannot fill a matrix tile, so the products are formed once, as a 1x1 convolution
-            // with C*R*S output channels over dy on the matrix cores, into the staging area, and gathered
-            // into dx by a second kernel; as many samples at a time as the staging area holds.
+        const bool s1 = g.sh == 1 && g.sw == 1;
+        if (products && (s1 ? gate && !rows3 : true)) {
+            // The products once, into the staging area, gathered into dx by a second kernel; as many samples at a time as the
+            // staging area holds.
             const int RS = g.R * g.S, CRS = g.C * RS, PQ = g.P * g.Q;
             const size_t per_sample = (size_t)CRS * PQ * sizeof(float);
             int nb = (int)(ctx->reduce_scratch_bytes / per_sample);
             if (nb > g.N) nb = g.N;
+            if (nb > (1l << 31) / ((long)g.C * g.H * g.W)) nb = (int)((1l << 31) / ((long)g.C * g.H * g.W)); // (32-bit indexes in the second kernel)
             float* T = ctx->reduce_scratch;
             LoadFilterT alt{w, CRS, 1, (unsigned)((long)g.K * CRS * 4), FastDiv::make(1)};
             for (int n0 = 0; n0 < g.N; n0 += nb) {
@@ -1172,10 +1184,10 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
                 const int rc = launch_by_m(ctx, st, kBwdDataNames, alt, bl, ept, CRS, nc * PQ, g.K, 2.0 * nc * (double)g.K * CRS * PQ);
                 if (rc != VDNN_OK) return rc;
                 ConvGeo gc = g; gc.N = nc;
-                const long total = (long)nc * g.C * g.H * g.W;
-                ProfScope gather(ctx, st, "conv_bwd_data_gather", 0.0, (double)per_sample * nc + (double)total * sizeof(E));
+                const long total = (long)nc * g.C * g.H * g.W, first = (long)n0 * g.C * g.H * g.W;
+                ProfScope gather(ctx, st, "conv_bwd_data_gather", 0.0, (double)per_sample * nc + (double)total * sizeof(E) * (gate ? 2.0 : 1.0));
                 hipLaunchKernelGGL(conv_bwd_data_gather_taps_kernel<E>, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st,
-                                   T, dx + (long)n0 * g.C * g.H * g.W, gc, total);
+                                   T, dx + first, gate ? gate + first : nullptr, gc, (unsigned)total);
                 VDNN_LAUNCH_CHECK();
             }
             return VDNN_OK;
@@ -1186,8 +1198,7 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
         ProfScope prof(ctx, st, "conv_bwd_data_smallc", 2.0 * g.C * (double)g.N * g.P * g.Q * g.K * g.R * g.S, 0.0);
         const bool s1_3x3 = g.sh == 1 && g.sw == 1 && g.R == 3 && g.S == 3;
         // 3x3, padding 1, at most three input and 64 output channels: the products once, on the matrix cores, row by row
-        if (s1_3x3 && g.C <= 3 && g.K <= 64 && g.ph == 1 && g.pw == 1 && g.P == g.H && g.Q == g.W &&
-            (long)g.K * g.P * g.Q * (long)sizeof(E) < (long)MAX_SUM_RANGE) {
+        if (rows3) {
             // about three workgroups per compute unit, strips of at least eight image rows
             const int cblocks = (g.W + BDS_EMIT - 1) / BDS_EMIT;
             int strips = (int)((3l * ctx->num_cu + (long)g.N * cblocks - 1) / ((long)g.N * cblocks));
@@ -1201,9 +1212,9 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             if (rows > g.H) rows = g.H;
             strips = (g.H + rows - 1) / rows;
             const dim3 grid((unsigned)(g.N * strips * cblocks));
-            if (g.C == 1) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<1, E>), grid, dim3(256), 0, st, dy, w, dx, g.N, g.K, g.H, g.W, rows);
-            else if (g.C == 2) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<2, E>), grid, dim3(256), 0, st, dy, w, dx, g.N, g.K, g.H, g.W, rows);
-            else hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<3, E>), grid, dim3(256), 0, st, dy, w, dx, g.N, g.K, g.H, g.W, rows);
+            if (g.C == 1) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<1, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);
+            else if (g.C == 2) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<2, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);
+            else hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<3, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);
             VDNN_LAUNCH_CHECK();
             return VDNN_OK;
         }

@@ -125,34 +125,29 @@ __global__ void __launch_bounds__(256) conv_bwd_data_smallc_strided_kernel(const
     if (g.C > 3) store_elem(o + 3 * plane, acc.w);
 }
 
-// Second stage of the strided few-channel backward data on the matrix cores. The first stage is a 1x1
+// Second stage of the few-channel backward data on the matrix cores. The first stage is a 1x1
 // convolution T[n][(c,r,s)][p][q] = sum_k w[k,c,r,s] * dy[n,k,p,q] (every product the layer needs, once);
 // here an input pixel adds up the entries whose tap lands on it: dx[n,c,h,x] = sum over taps (r,s) with
-// (h+ph-r) = p*sh and (x+pw-s) = q*sw of T[n][(c,r,s)][p][q], taps in ascending (r,s) order.
+// (h+ph-r) = p*sh and (x+pw-s) = q*sw of T[n][(c,r,s)][p][q], taps in ascending (r,s) order. Bound by T's trip through memory; a launch
+// covers no more elements than the staging area holds (2^24), so that 32-bit indexes and divisions do. gate: optional, laid out as dx.
 template <class E>
-__global__ void __launch_bounds__(256) conv_bwd_data_gather_taps_kernel(const float* __restrict__ T, E* __restrict__ dx, const ConvGeo g, long total) {
-    const long i = (long)blockIdx.x * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) conv_bwd_data_gather_taps_kernel(const float* __restrict__ T, E* __restrict__ dx, const E* __restrict__ gate, const ConvGeo g, unsigned total) {
+    const unsigned i = blockIdx.x * 256 + threadIdx.x;
     if (i >= total) return;
-    const int x = (int)(i % g.W);
-    long t = i / g.W;
-    const int h = (int)(t % g.H); t /= g.H;
-    const int c = (int)(t % g.C);
-    const long n = t / g.C;
-    const int PQ = g.P * g.Q;
-    const float* Tc = T + (n * g.C + c) * (long)g.R * g.S * PQ;
+    const unsigned row = i / (unsigned)g.W, plane = row / (unsigned)g.H; // plane: n * C + c
+    const int x = (int)(i - row * (unsigned)g.W) + g.pw, h = (int)(row - plane * (unsigned)g.H) + g.ph;
+    const int PQ = g.P * g.Q, p0 = h / g.sh, q0 = x / g.sw, r0 = h - p0 * g.sh, s0 = x - q0 * g.sw;
+    const float keep = gate ? load_elem(gate + i) : 1.0f;
+    const float* Tc = T + (long)plane * g.R * g.S * PQ;
     float acc = 0.0f;
-    for (int r = (h + g.ph) % g.sh; r < g.R; r += g.sh) {
-        const int p = (h + g.ph - r) / g.sh;
-        if (h + g.ph - r < 0) break;
+    for (int r = r0, p = p0; r < g.R && p >= 0; r += g.sh, p--) {
         if (p >= g.P) continue;
-        for (int s = (x + g.pw) % g.sw; s < g.S; s += g.sw) {
-            const int q = (x + g.pw - s) / g.sw;
-            if (x + g.pw - s < 0) break;
+        for (int s = s0, q = q0; s < g.S && q >= 0; s += g.sw, q--) {
             if (q >= g.Q) continue;
             acc += Tc[(long)(r * g.S + s) * PQ + p * g.Q + q];
         }
     }
-    store_elem(dx + i, acc);
+    store_elem(dx + i, keep > 0.0f ? acc : 0.0f);
 }
 
 // The same, for a compile-time window at stride 1 (VGG's 3x3): fully unrolled and branch-free. Taps

@@ -394,7 +394,7 @@ constexpr int BDS_COLS = 128;          // T columns of a workgroup
 constexpr int BDS_EMIT = BDS_COLS - 2; // dx columns of a workgroup
 template <int CC, class E>
 __global__ void __launch_bounds__(256) conv_bwd_data_smallc3x3_mfma_kernel(const E* __restrict__ dy, const float* __restrict__ w, E* __restrict__ dx,
-                                                                            int N, int K, int H, int W, int strip_rows) {
+                                                                            const E* __restrict__ gate, int N, int K, int H, int W, int strip_rows) {
     constexpr int NROW = 9 * CC, ES = ElemBytes<E>::V, KS = 32; // up to 64 output channels
     constexpr int WP = BDS_COLS + 1, TROW = NROW * WP;          // odd row stride: the nine reads of a value fall on different banks
     static_assert(NROW <= 32, "one block of 32 rows");
@@ -456,7 +456,9 @@ __global__ void __launch_bounds__(256) conv_bwd_data_smallc3x3_mfma_kernel(const
 #pragma unroll
                     for (int s = 0; s < 3; s++) sum += row[s * WP - s];
                 }
-                store_elem(dx + ((long)n * CC + c) * PQ + (long)ih * W + e0 + ew, sum);
+                const long at = ((long)n * CC + c) * PQ + (long)ih * W + e0 + ew;
+                if (gate) sum = load_elem(gate + at) > 0.0f ? sum : 0.0f;
+                store_elem(dx + at, sum);
             }
         }
         __syncthreads();
