@@ -60,6 +60,11 @@ int vdnn_ctx_create(vdnn_ctx** out, int device, int flags) {
             delete ctx;
             return VDNN_EDEVICE;
         }
+        if (hipMalloc((void**)&ctx->tile_counters, kTileCounters * sizeof(unsigned)) != hipSuccess ||
+            hipMemset(ctx->tile_counters, 0, kTileCounters * sizeof(unsigned)) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->tile_counters = nullptr; // (split reductions are added up by a second kernel then)
+        }
         if (noalloc_prepare_current_device() != VDNN_OK) {
             delete ctx;
             return VDNN_EDEVICE;
@@ -86,6 +91,7 @@ int vdnn_ctx_destroy(vdnn_ctx* ctx) {
         for (auto& r : ctx->prof_records) { (void)hipEventDestroy(r.start); (void)hipEventDestroy(r.stop); }
         for (auto e : ctx->prof_free_events) (void)hipEventDestroy(e);
         if (ctx->zvc_counters) (void)hipFree(ctx->zvc_counters);
+        if (ctx->tile_counters) (void)hipFree(ctx->tile_counters);
         if (ctx->compute) (void)hipStreamDestroy(ctx->compute);
         if (ctx->d2h) (void)hipStreamDestroy(ctx->d2h);
         if (ctx->h2d) (void)hipStreamDestroy(ctx->h2d);

@@ -23,6 +23,9 @@ struct vdnn_ctx {
     // on another stream beside the kernels that keep their partial sums in the rest.
     float* bias_scratch = nullptr;
     size_t bias_scratch_bytes = 0;
+    // Zero between launches: how many workgroups of a split tile are done (sum_splits in mfma_gemm.h). Shared by the kernels that share the
+    // staging area, which their partial sums lie in.
+    unsigned* tile_counters = nullptr;
     int num_cu = 256;
     int act_dtype = VDNN_DTYPE_F32;   // element type of activation tensors handed to the kernels
     // per-kernel timing (vdnn_profile_*)
@@ -45,6 +48,8 @@ namespace vdnn {
 
 static constexpr size_t kReduceScratchBytes = size_t(64) << 20;
 static constexpr size_t kBiasScratchBytes = size_t(1) << 20;     // its last part: the convolution bias gradient's partial sums
+
+static constexpr int kTileCounters = 4096;
 
 void set_error(const char* fmt, ...);
 

@@ -109,8 +109,9 @@ static int launch_by_m(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names
             GemmDims ds = make_dims(M, N, K, 64, 64, plan.splits);
             const int tail = plan.full_tiles > 0 && ds.splits > 1 ? (int)((long)ds.mtiles * ds.ntiles - plan.full_tiles) : 0;
             if (tail > 0) ds.full_tiles = (int)plan.full_tiles;
+            const bool fused = fuse_split_sums(ctx, ds, partial_bytes);
             const int rcs = launch_igemm<64, 64, AL, BL, StoreNCHW<E>>(ctx, stream, names.t64s, al, bl, ep, ds, flops);
-            if (rcs != VDNN_OK || ds.splits == 1) return rcs;
+            if (rcs != VDNN_OK || ds.splits == 1 || fused) return rcs;
             if (tail > 0)
                 return launch_reduce_tail_nchw(ctx, stream, ep.out, ep.partial, tail, ds.splits, 64, 64, M, N, ds.mtiles, ds.full_tiles, ep.bias, ep.opix, ep.relu, ep.gate);
             return launch_reduce_splits_nchw(ctx, stream, ep.out, ep.partial, (size_t)M * N, ds.splits, ep.bias, ep.opix, M, ep.relu, ep.gate);
@@ -243,6 +244,10 @@ static bool is_dense(const ConvGeo& g) { return g.P == 1 && g.Q == 1 && g.ph == 
 static bool pad_pays(int channels, int M, long N, int RS, double least_ops) {
     return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels && 2.0 * ((M + 63) / 64 * 64) * (double)N * channels * RS >= least_ops;
 }
+// A filter re-laid-out for the tap-major loaders costs a launch and saves three of four loads of it; small layers read it as it lies (19 x 32 x 7 x 7, 13
+// filters of 3x3 forward 11.1 -> 8.9 us; 2 x 16 x 53 x 53, 80 of 3x3, 1.3e8 operations, 9.8 -> 9.1; 15 x 16 x 17 x 17, 176 of 5x5, 3.6e8, 14.9 -> 19.4).
+constexpr double kPackOps = 1.5e8;
+static bool pack_pays(double ops) { return ops >= kPackOps; }
 constexpr double kPadFwdOps = 1.5e9, kPadBwdDataOps = 4e8;
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
 static bool packed_bwd_data_ok(const ConvGeo& g) {
@@ -1093,7 +1098,12 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
         // master copy's order a slice's sixteen channels of one tap lie R*S floats apart). Perf-optimal: in the
         // workspace. Memory-optimal: at the front of the context's staging area, where it leaves room for the partial sums.
         const bool in_workspace = algo_mode == 1 && workspace && workspace_bytes >= wbytes && aligned16(workspace);
-        float* packed = in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes);
+        if (RS == 1 && aligned16(w)) { // one tap: the filter is laid out as it is packed
+            StoreNCHW<E> ep{y, bias, g.P * g.Q, ctx->reduce_scratch, relu, nullptr};
+            LoadDenseRed<true> al{w, (long)K, g.K, wbytes};
+            return launch_by_m(ctx, st, in_workspace ? kFwdPackedNames : kFwdNames, al, bl, ep, g.K, g.N * g.P * g.Q, K);
+        }
+        float* packed = pack_pays(2.0 * g.K * (double)g.N * g.P * g.Q * K) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr;
         StoreNCHW<E> ep{y, bias, g.P * g.Q, ctx->reduce_scratch, relu, nullptr};
         if (packed) {
             const int rc = launch_pack_filter(ctx, st, w, packed, g.K, g.C, RS, g.C * RS, RS);
@@ -1270,7 +1280,11 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             const unsigned wbytes = (unsigned)((long)g.K * g.C * RS * 4);
             LoadIm2colPixTap<1, E> bl{{dy, g.P, g.Q, g.H, g.W, g.R, g.S, g.ph, g.pw, 1, 1, sample, g.N, dRS, dS}};
             const bool in_workspace = algo_mode == 1 && workspace && workspace_bytes >= wbytes && aligned16(workspace);
-            float* packed = in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes); // [c][(kb*RS + tap)*16 + l]
+            if (RS == 1) { // one tap: the filter read as it lies, lanes along the input channels
+                LoadDenseRow<float> alr{w, (long)g.C, g.C, wbytes};
+                return launch_by_m(ctx, st, in_workspace ? kBwdDataPackedNames : kBwdDataNames, alr, bl, ep, M, N, K, flops);
+            }
+            float* packed = pack_pays(2.0 * M * (double)N * K) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr; // [c][(kb*RS + tap)*16 + l]
             if (packed) {
                 ep.partial = ctx->reduce_scratch; // (behind the filter bank, if that lies in the staging area)
                 const int rc = launch_pack_filter(ctx, st, w, packed, g.C, g.K, RS, RS, g.C * RS);

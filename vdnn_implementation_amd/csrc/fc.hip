@@ -5,11 +5,10 @@
 #include "fc_bf16.h"
 #include "fc_update.h"
 #include "fc_stream.h"
+#include "conv_launch.h"
 
 namespace vdnn {
 
-int launch_reduce_splits(vdnn_ctx* ctx, hipStream_t stream, float* out, const float* partial, size_t count,
-                         int splits, float alpha, int accumulate, const float* bias_j, int ncols, int relu, const float* gate);
 int launch_reduce_splits(vdnn_ctx* ctx, hipStream_t stream, bf16_t* out, const float* partial, size_t count,
                          int splits, float alpha, int accumulate, const float* bias_j, int ncols, int relu, const bf16_t* gate);
 
@@ -49,14 +48,15 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     d.kchunk = kchunk;
     d.splits = (K + kchunk - 1) / kchunk;
     d.full_tiles = 0;
-    StoreDense<EO> ep{out, ctx->reduce_scratch, d.splits > 1 ? nullptr : bias_j, (long)N, (long)M * N, alpha, accumulate, relu, gate};
+    const bool fused = small && fuse_split_sums(ctx, d, ctx->reduce_scratch_bytes);
+    StoreDense<EO> ep{out, ctx->reduce_scratch, d.splits > 1 && !fused ? nullptr : bias_j, (long)N, (long)M * N, alpha, accumulate, relu, gate};
     const long blocks = (long)d.mtiles * d.ntiles * d.splits;
     ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
     if (small) launch_igemm64((unsigned)blocks, st, al, bl, ep, d);
     else if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
-    if (d.splits > 1) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, alpha, accumulate, bias_j, N, relu, gate);
+    if (d.splits > 1 && !fused) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, alpha, accumulate, bias_j, N, relu, gate);
     return VDNN_OK;
 }
 

@@ -164,6 +164,7 @@ struct GemmDims {
     int M, N, K;
     int mtiles, ntiles, splits, kchunk;
     int full_tiles;
+    unsigned* counters = nullptr; // the 64x64 tile: splits are added up by the workgroup that ends last (sum_splits), one counter a split tile
 };
 
 // Number of reduction splits for a grid of `tiles` output tiles over a reduction of K, at most
@@ -421,6 +422,56 @@ __global__ void __launch_bounds__(NT, 3) igemm_kernel(const AL al, const BL bl, 
 //   uniform only, once per tile: 2.7 -> 0.9 us.
 // One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
 // four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 102.7.
+// Split reductions of the 64x64 tile without a second kernel. Every workgroup of a tile leaves its sums in the staging area and counts
+// itself; the one that counts last adds them up in split order - the sums a second kernel would form - and writes the result. The
+// counters are zero between launches: the last workgroup puts its tile's back.
+// The eight L2s are not coherent with each other. The sums are therefore stored and loaded at device scope (sc1: through the L2, as
+// relaxed atomics at that scope are), and a workgroup counts only when every wavefront has waited for its stores to complete. A
+// release and an acquire of everything would write back and invalidate the whole L2, per workgroup: with them a layer of 10 x 192 x 13 x 13,
+// 256 filters of 3x3 at stride 2 took 23 us, with a second kernel 18.
+typedef unsigned word4 __attribute__((ext_vector_type(4)));
+constexpr int kDeviceScope = 16; // cache policy of a buffer access: sc1
+__device__ __forceinline__ bool sum_splits(floatx16& acc, float* staging, const GemmDims& d, int slot_tile, int ks, int tid) {
+    __shared__ int last;
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(staging + (long)slot_tile * d.splits * (64 * 64), (unsigned)d.splits * (64 * 64 * 4));
+#pragma unroll
+    for (int q = 0; q < 4; q++)
+        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(word4, floatx4{acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]}), rs,
+                                               tid * 16 + q * (NT * 16), ks * (64 * 64 * 4), kDeviceScope);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned before = __hip_atomic_fetch_add(d.counters + slot_tile, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = before == (unsigned)d.splits - 1;
+        if (last) __hip_atomic_store(d.counters + slot_tile, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last) return false;
+    auto load = [&](int q, int s) { return __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rs, tid * 16 + q * (NT * 16), s * (64 * 64 * 4), kDeviceScope)); };
+    floatx4 sum[4];
+#pragma unroll
+    for (int q = 0; q < 4; q++) sum[q] = load(q, 0);
+    // two splits on their way at once: with more, these registers would be the kernel's most
+    int s = 1;
+    for (; s + 2 <= d.splits; s += 2) {
+        floatx4 v[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) v[u][q] = load(q, s + u);
+#pragma unroll
+        for (int u = 0; u < 2; u++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) sum[q] += v[u][q];
+    }
+    for (; s < d.splits; s++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) sum[q] += load(q, s);
+#pragma unroll
+    for (int v = 0; v < 16; v++) acc[v] = sum[v / 4][v % 4];
+    return true;
+}
+
 template <int AHEAD, class AL, class BL, class EP>
 __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
     constexpr int T = 64;
@@ -513,7 +564,11 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
         }
     }
 
-    if (EP::TAIL && d.full_tiles > 0 && !at.whole) {
+    if (!at.whole && d.counters) {
+        if (!sum_splits(acc, ep.partial, d, at.tile - d.full_tiles, at.ks, tid)) return;
+        ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, false);
+        ep.store32(acc, aux, at.m0 + wm0, at.j0 + wn0, lane, 0, d, false);
+    } else if (EP::TAIL && d.full_tiles > 0 && !at.whole) {
         const floatx16 tail[1][1] = {{acc}};
         ep.store_tail(tail, wm0, wn0, lane, (long)(at.tile - d.full_tiles) * d.splits + at.ks, T, T);
     } else {
