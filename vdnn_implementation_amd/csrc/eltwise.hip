@@ -876,6 +876,106 @@ __global__ void __launch_bounds__(EB) maxpool2x2_bwd_kernel(const E* x, const E*
     }
 }
 
+// A pair of neighbouring elements that begins at any element, as floats
+typedef float float2_any __attribute__((ext_vector_type(2), aligned(4)));
+typedef unsigned pair_any __attribute__((aligned(2)));
+__device__ __forceinline__ float2 pair_at(const float* p) { const float2_any v = *(const float2_any*)p; float2 r; r.x = v.x; r.y = v.y; return r; }
+__device__ __forceinline__ float2 pair_at(const bf16_t* p) {
+    const unsigned v = *(const pair_any*)p;
+    float2 r; r.x = bf16_bits_to_float(v & 0xFFFFu); r.y = bf16_bits_to_float(v >> 16);
+    return r;
+}
+__device__ __forceinline__ void put_pair(float* p, float a, float b) { float2_any v; v.x = a; v.y = b; *(float2_any*)p = v; }
+__device__ __forceinline__ void put_pair(bf16_t* p, float a, float b) { *(pair_any*)p = pack2_bf16(a, b); }
+
+// Backward of unpadded 2x2 pooling at stride 2 on planes of any extents: one thread per 2x2 cell of the plane, the cells that an odd last
+// row or column leaves behind the windows included (zero there). Bound by memory: whole blocks of layers with it, 24 x 15 x 123 x 123 bfloat16 60 -> 28 us,
+// 28 x 186 x 18 x 18 bfloat16 26 -> 13.5, 32 x 21 x 54 x 173 floats 73 -> 40; the gather over all windows of an element took 172 us for 4 x 125 x 221 x 221
+// floats, whole planes in LDS 7 us for 16 x 12 x 11 x 11.
+template <class E>
+__global__ void __launch_bounds__(EB) maxpool2x2_bwd_any_kernel(const E* __restrict__ x, const E* __restrict__ dy, E* __restrict__ dx,
+                                                                int H, int W, int P, int Q, unsigned cells, int gate) {
+    const unsigned i = blockIdx.x * EB + threadIdx.x;
+    if (i >= cells) return;
+    const unsigned CW = (unsigned)(W + 1) / 2, CH = (unsigned)(H + 1) / 2;
+    const unsigned t = i / CW, nc = t / CH;
+    const int q = (int)(i - t * CW), p = (int)(t - nc * CH);
+    const size_t off = ((size_t)nc * H + 2 * p) * W + 2 * q;
+    if (p < P && q < Q) {
+        const float2 a = pair_at(x + off), b = pair_at(x + off + W);
+        float d = load_elem(dy + ((size_t)nc * P + p) * Q + q);
+        int s = 0; float m = -FLT_MAX;   // the first strict maximum wins
+        if (a.x > m) { m = a.x; s = 0; } if (a.y > m) { m = a.y; s = 1; }
+        if (b.x > m) { m = b.x; s = 2; } if (b.y > m) { m = b.y; s = 3; }
+        if (gate) d = m > 0.0f ? d : 0.0f;
+        put_pair(dx + off, s == 0 ? d : 0.0f, s == 1 ? d : 0.0f);
+        put_pair(dx + off + W, s == 2 ? d : 0.0f, s == 3 ? d : 0.0f);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            if (2 * p + e / 2 < H && 2 * q + e % 2 < W) store_elem(dx + off + (e / 2) * W + e % 2, 0.0f);
+    }
+}
+
+// Backward of unpadded 3x3 pooling at stride 2 on planes that do not fit LDS. A wavefront owns 63 of the 2x2 blocks of two rows, the elements (2p,
+// 2q) .. (2p + 1, 2q + 1), which the windows (p - 1 | p, q - 1 | q) cover: a lane finds the winners of windows (p - 1, q) and (p, q) and has
+// those of column q - 1 from the lane before it; lane 0 makes that column only. Same winners, windows row by row: the same bits as the
+// kernel on whole planes. 44 x 10 x 118 x 118 bfloat16 with rectifier and normalisation 211 -> 68 us (the gather: 150).
+constexpr int POOL_ROW_BLOCKS = 63;
+template <class E>
+__global__ void __launch_bounds__(EB) maxpool3x3s2_bwd_rows_kernel(const E* __restrict__ x, const E* __restrict__ dy, E* __restrict__ dx,
+                                                                   int H, int W, int P, int Q, int strips, long waves, int gate) {
+    const int lane = threadIdx.x & 63;
+    const long id = (long)blockIdx.x * (EB / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (id >= waves) return;
+    const int BH = (H + 1) / 2;
+    const long t = id / strips, nc = t / BH;
+    const int p = (int)(t - nc * BH), q = (int)(id - t * strips) * POOL_ROW_BLOCKS + lane - 1;
+    const E* xp = x + nc * H * W;
+    float v[5][3]; // rows 2p - 2 .. 2p + 2, columns 2q .. 2q + 2; outside the plane some element inside, which no window below takes
+#pragma unroll
+    for (int r = 0; r < 5; r++) {
+        const E* row = xp + (long)min(max(2 * p - 2 + r, 0), H - 1) * W;
+#pragma unroll
+        for (int c = 0; c < 3; c++) v[r][c] = load_elem(row + min(max(2 * q + c, 0), W - 1));
+    }
+    int win[2][2];   // winner's index in the plane, of windows (p - 1 + u, q - 1 + v); -1: no such window
+    float d[2][2];
+#pragma unroll
+    for (int u = 0; u < 2; u++) {
+        const int wp = p - 1 + u;
+        const bool ok = (unsigned)wp < (unsigned)P && (unsigned)q < (unsigned)Q;
+        const int first = 2 * wp * W + 2 * q;
+        float m = -FLT_MAX;
+        int a = first;
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+#pragma unroll
+            for (int c = 0; c < 3; c++)
+                if (v[2 * u + r][c] > m) { m = v[2 * u + r][c]; a = first + r * W + c; }
+        win[u][1] = ok ? a : -1;
+        d[u][1] = load_elem(dy + nc * P * Q + (ok ? wp * Q + q : 0));
+        win[u][0] = __shfl_up(win[u][1], 1);
+        d[u][0] = __shfl_up(d[u][1], 1);
+    }
+    if (lane == 0) return;
+#pragma unroll
+    for (int eh = 0; eh < 2; eh++)
+#pragma unroll
+        for (int ew = 0; ew < 2; ew++) {
+            const int h = 2 * p + eh, w = 2 * q + ew;
+            if (h >= H || w >= W) continue;
+            const int self = h * W + w;
+            float acc = 0.0f;
+#pragma unroll
+            for (int u = eh; u < 2; u++) // an odd row lies in window row p only
+#pragma unroll
+                for (int c = ew; c < 2; c++) acc += win[u][c] == self ? d[u][c] : 0.0f;
+            if (gate && !(v[2 + eh][ew] > 0.0f)) acc = 0.0f;
+            store_elem(dx + nc * H * W + self, acc);
+        }
+}
+
 // ---- LRN across channels: window 5, alpha 1e-4, beta 0.75, k 2 -------------------------------------
 #define LRN_A5 (1e-4f / 5.0f)
 #define LRN_BETA 0.75f
@@ -894,22 +994,45 @@ __device__ __forceinline__ float lrn_pow_m075(float scale) {
     return r * __builtin_amdgcn_sqrtf(r);
 }
 
+// (sample, chunk, pixel) of a thread, pixel fastest, in 32-bit divisions where the numbers allow it
+struct LrnPlace { size_t n; int c0, pix; };
+__device__ __forceinline__ LrnPlace lrn_place(size_t i, int hw, int chunks, size_t total) {
+    LrnPlace p;
+    if (total <= 0xFFFFFFFFul) {
+        const unsigned j = (unsigned)i, t = j / (unsigned)hw, n = t / (unsigned)chunks;
+        p.pix = (int)(j - t * (unsigned)hw);
+        p.c0 = (int)(t - n * (unsigned)chunks) * LRN_CH;
+        p.n = n;
+    } else {
+        const size_t t = i / hw;
+        p.pix = (int)(i % hw);
+        p.c0 = (int)(t % chunks) * LRN_CH;
+        p.n = t / chunks;
+    }
+    return p;
+}
+// Element of a channel at `at`, zero outside the tensor. Two-byte elements are read from the nearest channel inside and dropped: behind a
+// branch each, their loads wait for one another (55 x 480 x 45 x 45 with rectifier and 2x2 pooling 756 -> 376 us, 117 x 14 x 172 x 172 440 -> 293). Floats
+// do not, and the channels read for nothing cost them up to 5 %.
+__device__ __forceinline__ float lrn_channel(const float* at, int c, int C, int hw) { return c >= 0 && c < C ? at[(size_t)c * hw] : 0.0f; }
+__device__ __forceinline__ float lrn_channel(const bf16_t* at, int c, int C, int hw) {
+    const float v = load_elem(at + (size_t)min(max(c, 0), C - 1) * hw);
+    return (unsigned)c < (unsigned)C ? v : 0.0f;
+}
+
 template <class E>
 __global__ void __launch_bounds__(EB) lrn_fwd_kernel(const E* __restrict__ x, E* __restrict__ y, int C, int hw, int chunks, size_t total) {
-    const size_t i = (size_t)blockIdx.x * EB + threadIdx.x; // (sample, chunk, pixel), pixel fastest
+    const size_t i = (size_t)blockIdx.x * EB + threadIdx.x;
     if (i >= total) return;
-    const int pix = (int)(i % hw);
-    const size_t t = i / hw;
-    const int chunk = (int)(t % chunks);
-    const size_t n = t / chunks;
-    const int c0 = chunk * LRN_CH;
+    const LrnPlace at = lrn_place(i, hw, chunks, total);
+    const size_t n = at.n;
+    const int c0 = at.c0, pix = at.pix;
     const E* xp = x + (n * C) * hw + pix;
     E* yp = y + (n * C) * hw + pix;
     float v[LRN_CH + 4]; // channels c0-2 .. c0+LRN_CH+1, zero outside the tensor
 #pragma unroll
     for (int k = 0; k < LRN_CH + 4; k++) {
-        const int c = c0 - 2 + k;
-        v[k] = (c >= 0 && c < C) ? load_elem(xp + (size_t)c * hw) : 0.0f;
+        v[k] = lrn_channel(xp, c0 - 2 + k, C, hw);
     }
 #pragma unroll
     for (int k = 0; k < LRN_CH; k++) {
@@ -927,12 +1050,9 @@ __global__ void __launch_bounds__(EB) lrn_bwd_kernel(const E* __restrict__ x, co
                                                      E* __restrict__ dx, int C, int hw, int chunks, size_t total) {
     const size_t i = (size_t)blockIdx.x * EB + threadIdx.x;
     if (i >= total) return;
-    const int pix = (int)(i % hw);
-    const size_t t_ = i / hw;
-    const int chunk = (int)(t_ % chunks);
-    const size_t n = t_ / chunks;
-    const int c0 = chunk * LRN_CH;
-    const size_t base = (n * C) * hw + pix;
+    const LrnPlace at = lrn_place(i, hw, chunks, total);
+    const int c0 = at.c0;
+    const size_t base = (at.n * C) * hw + at.pix;
     float xv[LRN_CH + 8];  // channels c0-4 .. c0+LRN_CH+3
     float term[LRN_CH + 4]; // dy*y/scale of channels c0-2 .. c0+LRN_CH+1
     float dyv[LRN_CH + 4];  // dy of the same channels: the thread's own sixteen are among them
@@ -940,15 +1060,13 @@ __global__ void __launch_bounds__(EB) lrn_bwd_kernel(const E* __restrict__ x, co
     float scale_own[LRN_CH];
 #pragma unroll
     for (int k = 0; k < LRN_CH + 8; k++) {
-        const int c = c0 - 4 + k;
-        xv[k] = (c >= 0 && c < C) ? load_elem(x + base + (size_t)c * hw) : 0.0f;
+        xv[k] = lrn_channel(x + base, c0 - 4 + k, C, hw);
     }
 #pragma unroll
     for (int k = 0; k < LRN_CH + 4; k++) { // every fetch is issued before the first value is used
         const int c = c0 - 2 + k;
-        const bool in = c >= 0 && c < C;
-        dyv[k] = in ? load_elem(dy + base + (size_t)c * hw) : 0.0f;
-        yv[k] = in ? load_elem(y + base + (size_t)c * hw) : 0.0f;
+        dyv[k] = lrn_channel(dy + base, c, C, hw);
+        yv[k] = lrn_channel(y + base, c, C, hw);
     }
 #pragma unroll
     for (int k = 0; k < LRN_CH + 4; k++) {
@@ -1271,6 +1389,11 @@ static bool pool_is_3x3_s2(const PoolGeo& g) {
            2 * (g.P - 1) + 3 <= g.H && 2 * (g.Q - 1) + 3 <= g.W;
 }
 
+// 2x2 / stride 2 without padding, every window inside the plane
+static bool pool_is_2x2_s2(const PoolGeo& g) {
+    return g.R == 2 && g.S == 2 && g.sh == 2 && g.sw == 2 && g.ph == 0 && g.pw == 0 && 2 * g.P <= g.H && 2 * g.Q <= g.W;
+}
+
 static bool pool_is_2x2_exact(const PoolGeo& g, const void* a, const void* b, const void* c) {
     return g.R == 2 && g.S == 2 && g.sh == 2 && g.sw == 2 && g.ph == 0 && g.pw == 0 && g.H % 2 == 0 && g.W % 4 == 0 &&
            aligned16(a) && aligned16(b) && (!c || aligned16(c));
@@ -1323,6 +1446,9 @@ static int maxpool_bwd_t(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
     if (pool_is_2x2_exact(g, x, dx, dy) && (g.W / 2) % 2 == 0) {
         const size_t pairs = (size_t)g.N * g.C * (g.H / 2) * (g.W / 4);
         hipLaunchKernelGGL(maxpool2x2_bwd_kernel<E>, dim3(grid_for(pairs, EB, 0x7FFFFFFF)), dim3(EB), 0, st, x, dy, dx, g.H, g.W, pairs, gate);
+    } else if (pool_is_2x2_s2(g) && (size_t)g.N * g.C * ((g.H + 1) / 2) * ((g.W + 1) / 2) <= 0x7FFFFFFFul) {
+        const size_t cells = (size_t)g.N * g.C * ((g.H + 1) / 2) * ((g.W + 1) / 2);
+        hipLaunchKernelGGL(maxpool2x2_bwd_any_kernel<E>, dim3(grid_for(cells, EB, 0x7FFFFFFF)), dim3(EB), 0, st, x, dy, dx, g.H, g.W, g.P, g.Q, (unsigned)cells, gate);
     } else if ((size_t)g.H * g.W * 4 + (size_t)g.P * g.Q * 8 <= 48 * 1024) {
         // whole planes in LDS: as many per workgroup as give every thread a few elements
         const size_t per_plane = (size_t)g.H * g.W * 4 + (size_t)g.P * g.Q * 8;
@@ -1338,6 +1464,11 @@ static int maxpool_bwd_t(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
                                FastDiv::make(((g.H + 1) / 2) * ((g.W + 1) / 2)), FastDiv::make((g.W + 1) / 2));
         else
             hipLaunchKernelGGL(maxpool_bwd_planes_kernel<E>, dim3((unsigned)blocks), dim3(EB), group * per_plane, st, x, dy, dx, g, planes, group, gate);
+    } else if (pool_is_3x3_s2(g) && (long)g.N * g.C < (1l << 31)) {
+        const int strips = ((g.W + 1) / 2 + POOL_ROW_BLOCKS - 1) / POOL_ROW_BLOCKS;
+        const long waves = (long)g.N * g.C * ((g.H + 1) / 2) * strips, blocks = (waves + EB / 64 - 1) / (EB / 64);
+        VDNN_REQUIRE(blocks < (1l << 31), "grid too large");
+        hipLaunchKernelGGL(maxpool3x3s2_bwd_rows_kernel<E>, dim3((unsigned)blocks), dim3(EB), 0, st, x, dy, dx, g.H, g.W, g.P, g.Q, strips, waves, gate);
     } else {
         const size_t total = (size_t)g.N * g.C * g.H * g.W;
         hipLaunchKernelGGL(maxpool_bwd_kernel<E>, dim3(grid_for(total, EB, 0x7FFFFFFF)), dim3(EB), 0, st, x, dy, dx, g, total, gate);
