@@ -38,6 +38,10 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     // (64 rows, 4096 -> 1000: 23 -> 16 us forward; 128, 300 -> 100 backward data 24.5 -> 8.7), short reductions always
     // (filter updates: a tile has as many slices as rows allow); larger ones break even at 4-8 GFLOP (128 rows, 4096 -> 4096:
     // 47 -> 45 us, 256 rows 80 -> 81) and lose beyond (128 rows, 25088 -> 4096: 219 -> 236).
+    // Larger ones keep two slices on their way beside the one in LDS: the filter comes from memory, every byte once, and one
+    // slice's MFMAs are shorter than that takes. Four passes, one slice ahead -> two, the same bits: 64 rows 25088 -> 4096
+    // 431 -> 418 us, 256 rows 9216 -> 4096 491 -> 477, 320 rows 3000 -> 5000 307 -> 298, 512 rows 4096 -> 4096 426 -> 413;
+    // four ahead 425 in the first.
     const bool small = K <= kShortReduction || 2.0 * M * (double)N * K <= 5e9;
     if (small) TM = TN = 64;
     GemmDims d;
@@ -53,8 +57,8 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     const long blocks = (long)d.mtiles * d.ntiles * d.splits;
     ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
     if (small) launch_igemm64((unsigned)blocks, st, al, bl, ep, d);
-    else if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
-    else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
+    else if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>, 2>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
+    else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>, 2>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     if (d.splits > 1 && !fused) return launch_reduce_splits(ctx, st, out, ctx->reduce_scratch, (size_t)M * N, d.splits, alpha, accumulate, bias_j, N, relu, gate);
     return VDNN_OK;

@@ -298,7 +298,8 @@ __device__ __forceinline__ TilePlace tile_place(const GemmDims& d, int block, in
     return p;
 }
 
-template <int TM, int TN, class AL, class BL, class EP>
+// AHEAD: slices on their way from memory beside the one in LDS and the one that is being multiplied.
+template <int TM, int TN, int AHEAD, class AL, class BL, class EP>
 __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
     constexpr int MI = 2, NJ = 2; // MFMA tiles of a wavefront
     constexpr int WAVES_M = TM / (32 * MI);
@@ -328,39 +329,52 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
             for (int v = 0; v < 16; v++) acc[i][j][v] = 0.0f;
 
     const int wm0 = (wave % WAVES_M) * 32 * MI, wn0 = (wave / WAVES_M) * 32 * NJ;
-    typename AL::template Regs<TM> ra;
-    typename BL::template Regs<TN> rb;
+    typename AL::template Regs<TM> ra[AHEAD];
+    typename BL::template Regs<TN> rb[AHEAD];
 
-    // Software pipeline, one barrier per slice - in the middle of it - and no branch in the loop.
+    // Software pipeline, one barrier per slice - in the middle of it - and no branch within a slice.
     // A slice's 32 MFMAs per wavefront run as two groups of 16 (reduction indices 0-7 and 8-15).
     //   first half of slice s:  read the fragments of (s, group 1) from LDS buffer s%2, multiply group 0
     //                           (fragments already in registers), write the registers holding slice s+1
-    //                           (fetched during slice s-1) to the other LDS buffer;
+    //                           (fetched during slice s-AHEAD) to the other LDS buffer;
     //   barrier;
-    //   second half:            issue the fetch of slice s+2 into the same registers, read the fragments
+    //   second half:            issue the fetch of slice s+1+AHEAD into the same registers, read the fragments
     //                           of (s+1, group 0) from the buffer just completed, multiply group 1.
     // Each group's fragments are thus read while the previous group is multiplied, across the barrier as
-    // well, so no wavefront waits for LDS; a global load has a full slice of MFMA time to return. All
+    // well, so no wavefront waits for LDS; a global load has AHEAD slices of MFMA time to return. All
     // reads of a buffer precede the barrier after which it may be overwritten. Fetches past the end of
     // the range read as zero or are never used: buffer loads cannot fault, the last rounds need no guard.
     const int nslices = (k_end - k_begin + KB - 1) / KB;
     const int l32 = lane & 31, lk = lane >> 5;
     constexpr int A_TILE = 32 * LA::ROW_STRIDE, B_TILE = 32 * LB::ROW_STRIDE;
     const int a_off = wm0 * LA::ROW_STRIDE, b_off = wn0 * LB::ROW_STRIDE;
-    al.template load<TM>(sa, k_begin, k_end, tid, ra);
-    bl.template load<TN>(sb, k_begin, k_end, tid, rb);
-    AL::template store<TM>(As[0], tid, ra);
-    BL::template store<TN>(Bs[0], tid, rb);
-    al.template load<TM>(sa, k_begin + KB, k_end, tid, ra);
-    bl.template load<TN>(sb, k_begin + KB, k_end, tid, rb);
+    {
+        typename AL::template Regs<TM> fa;
+        typename BL::template Regs<TN> fb;
+        al.template load<TM>(sa, k_begin, k_end, tid, fa);
+        bl.template load<TN>(sb, k_begin, k_end, tid, fb);
+        if constexpr (AHEAD == 1) {
+            AL::template store<TM>(As[0], tid, fa);
+            BL::template store<TN>(Bs[0], tid, fb);
+        }
+#pragma unroll
+        for (int u = 0; u < AHEAD; u++) {
+            al.template load<TM>(sa, k_begin + (u + 1) * KB, k_end, tid, ra[u]);
+            bl.template load<TN>(sb, k_begin + (u + 1) * KB, k_end, tid, rb[u]);
+        }
+        if constexpr (AHEAD > 1) {
+            AL::template store<TM>(As[0], tid, fa);
+            BL::template store<TN>(Bs[0], tid, fb);
+        }
+    }
     __syncthreads();
     floatx4 a0[MI], b0[NJ], a1[MI], b1[NJ];
 #pragma unroll
     for (int i = 0; i < MI; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[0] + a_off + i * A_TILE, l32, lk, 0);
 #pragma unroll
     for (int j = 0; j < NJ; j++) b0[j] = read_frag<TN, BL::RED_MAJOR>(Bs[0] + b_off + j * B_TILE, l32, lk, 0);
-    for (int s = 0; s < nslices; s++) {
-        const int cur = s & 1, nxt = cur ^ 1;
+    auto slice = [&](int s, int cur, typename AL::template Regs<TM>& na, typename BL::template Regs<TN>& nb) {
+        const int nxt = cur ^ 1;
 #pragma unroll
         for (int i = 0; i < MI; i++) a1[i] = read_frag<TM, AL::RED_MAJOR>(As[cur] + a_off + i * A_TILE, l32, lk, 1);
 #pragma unroll
@@ -372,15 +386,15 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
 #pragma unroll
                 for (int j = 0; j < NJ; j++)
                     acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a0[i][e], b0[j][e], acc[i][j], 0, 0, 0);
-        AL::template store<TM>(As[nxt], tid, ra);
-        BL::template store<TN>(Bs[nxt], tid, rb);
+        AL::template store<TM>(As[nxt], tid, na);
+        BL::template store<TN>(Bs[nxt], tid, nb);
         // issue order of the first half: every MFMA is followed by one LDS access
 #pragma unroll
         for (int i = 0; i < 4 * MI * NJ; i++) { __builtin_amdgcn_sched_group_barrier(0x008, 1, 0); __builtin_amdgcn_sched_group_barrier(0x300, 2, 0); }
         __syncthreads();
-        const int kk0 = k_begin + (s + 2) * KB;
-        al.template load<TM>(sa, kk0, k_end, tid, ra);
-        bl.template load<TN>(sb, kk0, k_end, tid, rb);
+        const int kk0 = k_begin + (s + 1 + AHEAD) * KB;
+        al.template load<TM>(sa, kk0, k_end, tid, na);
+        bl.template load<TN>(sb, kk0, k_end, tid, nb);
 #pragma unroll
         for (int i = 0; i < MI; i++) a0[i] = read_frag<TM, AL::RED_MAJOR>(As[nxt] + a_off + i * A_TILE, l32, lk, 0);
 #pragma unroll
@@ -399,6 +413,21 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
             __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         }
+    };
+    if constexpr (AHEAD == 1) {
+        for (int s = 0; s < nslices; s++) slice(s, s & 1, ra[0], rb[0]);
+    } else {
+        static_assert(AHEAD % 2 == 0, "a round of slices ends in the LDS buffer it began with");
+        int s = 0;
+        for (; s + AHEAD <= nslices; s += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; u++) slice(s + u, u & 1, ra[u], rb[u]);
+        }
+#pragma unroll
+        for (int u = 0; u + 1 < AHEAD; u++) {
+            if (s + u >= nslices) break;
+            slice(s + u, u & 1, ra[u], rb[u]);
+        }
     }
 
     if (EP::TAIL && d.full_tiles > 0 && !whole)
@@ -407,9 +436,9 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
         ep.store(acc, m0 + wm0, j0 + wn0, lane, ks, d, !whole);
 }
 
-template <int TM, int TN, class AL, class BL, class EP>
+template <int TM, int TN, class AL, class BL, class EP, int AHEAD = 1>
 __global__ void __launch_bounds__(NT, 3) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
-    igemm_tile<TM, TN>(al, bl, ep, d, blockIdx.x, gridDim.x);
+    igemm_tile<TM, TN, AHEAD>(al, bl, ep, d, blockIdx.x, gridDim.x);
 }
 
 // The 64x64 tile. A workgroup has one wavefront per SIMD and a few to some tens of slices, and where it is taken most of the chip
