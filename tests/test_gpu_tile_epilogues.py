@@ -13,7 +13,8 @@ pytestmark = pytest.mark.gpu
 
 # n, c, h, w, k, window: 1x1 layers have c / 16 slices forward, k / 16 backward
 CONVS = [(2, 16, 9, 7, 1, 1), (1, 80, 8, 8, 31, 1), (3, 96, 5, 13, 33, 1), (1, 112, 11, 3, 64, 1), (2, 128, 6, 6, 96, 1), (1, 144, 7, 9, 112, 1),
-         (2, 33, 10, 10, 65, 3), (1, 160, 17, 15, 130, 3), (40, 24, 33, 31, 40, 3), (7, 64, 54, 54, 190, 3)]
+         (2, 33, 10, 10, 65, 3), (1, 160, 17, 15, 130, 3), (40, 24, 33, 31, 40, 3), (7, 64, 54, 54, 190, 3),
+         (60, 33, 60, 60, 40, 3), (24, 66, 50, 50, 200, 3)]  # the larger tiles, odd and even counts of slices
 FCS = [(1, 16, 1), (5, 99, 33), (33, 96, 31), (64, 112, 64), (65, 128, 130), (100, 1000, 97), (130, 4096, 300),
        (61, 9010, 4700), (200, 5009, 2600)]  # the larger tiles, odd and even counts of slices in a split
 

@@ -62,6 +62,16 @@ static const PassNames kBwdFilterHalfNames{"conv_bwd_filter_bf16mfma_64x256", "c
 static const PassNames kBwdFilterWin3Names{"conv_bwd_filter_bf16win_64x192", "conv_bwd_filter_bf16win_128x192"};
 static const PassNames kBwdFilterRow3Names{"conv_bwd_filter_row_64x192", "conv_bwd_filter_row_128x192"};
 
+// Slices on their way from memory in the float engine: two where the registers hold them without spilling to memory (168, of
+// which a gather's address work takes most: dense backward filter and strided backward data keep one). Activations come
+// from memory or another die's cache, and three workgroups on a compute unit do not cover that with one slice each. Same
+// sums. Forward, one -> two: 32 x 448 x 71 x 71 -> 128 3x3 stride 2 390 -> 372 us, 62 x 128 x 54 x 54 -> 32 216 -> 205,
+// 13 x 256 x 137 x 137 -> 640 5150 -> 4975, 16 x 22 x 87 x 208 -> 160 5x5 658 -> 640; both backward passes of the last three
+// 352 -> 343, 11800 -> 11670, 1914 -> 1864. The tap by tap backward filter alone: 32 x 128 x 12 x 179 -> 208 backward 668 -> 658.
+template <class BL, class EP> struct SlicesAhead { static constexpr int V = 1; };
+template <class BL, class E> struct SlicesAhead<BL, StoreNCHW<E>> { static constexpr int V = FetchesAhead<BL>::V ? 2 : 1; };
+template <class BL> struct SlicesAhead<BL, StoreFilterTap> { static constexpr int V = 2; };
+
 template <int TM, int TN, class AL, class BL, class EP, bool HALF = false>
 static int launch_igemm(vdnn_ctx* ctx, hipStream_t stream, const char* name, const AL& al, const BL& bl, const EP& ep, const GemmDims& d, double flops = 0.0) {
     const long all_tiles = (long)d.mtiles * d.ntiles;
@@ -72,7 +82,7 @@ static int launch_igemm(vdnn_ctx* ctx, hipStream_t stream, const char* name, con
     ProfScope prof(ctx, stream, name, flops > 0.0 ? flops : 2.0 * d.M * (double)d.N * d.K, 0.0);
     if constexpr (HALF) hipLaunchKernelGGL((igemm_bf16_kernel<TM, TN, AL, BL, EP>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
     else if constexpr (TM == 64 && TN == 64) launch_igemm64((unsigned)blocks, stream, al, bl, ep, d);
-    else hipLaunchKernelGGL((igemm_kernel<TM, TN, AL, BL, EP>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
+    else hipLaunchKernelGGL((igemm_kernel<TM, TN, AL, BL, EP, SlicesAhead<BL, EP>::V>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;
 }
