@@ -60,10 +60,16 @@ int vdnn_ctx_create(vdnn_ctx** out, int device, int flags) {
             delete ctx;
             return VDNN_EDEVICE;
         }
-        if (hipMalloc((void**)&ctx->tile_counters, kTileCounters * sizeof(unsigned)) != hipSuccess ||
-            hipMemset(ctx->tile_counters, 0, kTileCounters * sizeof(unsigned)) != hipSuccess) {
+        // (split reductions are added up by a second kernel where there are no counters). The context's streams do not wait for the
+        // default one, and clearing returns before it is done.
+        if (hipMalloc((void**)&ctx->tile_counters, kTileCounters * sizeof(unsigned)) != hipSuccess) {
             (void)hipGetLastError();
-            ctx->tile_counters = nullptr; // (split reductions are added up by a second kernel then)
+            ctx->tile_counters = nullptr;
+        } else if (hipMemsetAsync(ctx->tile_counters, 0, kTileCounters * sizeof(unsigned), ctx->compute) != hipSuccess ||
+                   hipStreamSynchronize(ctx->compute) != hipSuccess) {
+            (void)hipGetLastError();
+            (void)hipFree(ctx->tile_counters);
+            ctx->tile_counters = nullptr;
         }
         if (noalloc_prepare_current_device() != VDNN_OK) {
             delete ctx;

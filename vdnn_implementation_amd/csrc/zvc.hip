@@ -346,8 +346,14 @@ static int zvc_ensure_counters(vdnn_ctx* ctx) {
     if (ctx->zvc_counters) return VDNN_OK;
     // [0], [1]: bytes over the link; then the stream cursors, one per offload in flight
     const size_t bytes = sizeof(unsigned long long) * 2 + sizeof(ZvcCursor) * kZvcCursors;
-    VDNN_HIP(hipMalloc((void**)&ctx->zvc_counters, bytes));
-    VDNN_HIP(hipMemset(ctx->zvc_counters, 0, bytes));
+    unsigned long long* counters = nullptr;
+    VDNN_HIP(hipMalloc((void**)&counters, bytes));
+    // the first launch finds them cleared: the context's streams do not wait for the default one, and clearing returns before it is done
+    hipError_t cleared = hipMemsetAsync(counters, 0, bytes, ctx->pack);
+    if (cleared == hipSuccess) cleared = hipStreamSynchronize(ctx->pack);
+    if (cleared != hipSuccess) (void)hipFree(counters);
+    VDNN_HIP(cleared);
+    ctx->zvc_counters = counters;
     return VDNN_OK;
 }
 
