@@ -43,6 +43,44 @@ def test_maxpool_backward(geom, bf16, gated):
         assert np.array_equal(get(gx.download(x.shape, dtype)), want)
 
 
+SPECIAL = [(2, 3, 7, 9, 2), (1, 5, 40, 31, 2), (3, 2, 2, 3, 2), (1, 3, 221, 190, 2), (1, 3, 117, 118, 3), (1, 2, 99, 254, 3), (5, 3, 21, 30, 3)]
+
+
+@pytest.mark.parametrize("gated", [False, True], ids=["plain", "gated"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["float", "bfloat16"])
+@pytest.mark.parametrize("geom", SPECIAL, ids=lambda g: "x".join(map(str, g)))
+def test_maxpool_backward_of_values_that_do_not_compare(geom, bf16, gated):
+    """NaN, infinities, the lowest value and both zeros in x, negative zeros in dy and gradients whose sums round: the checker's bits,
+    whose sums begin with +0 and run over the windows row by row."""
+    n, c, h, w, win = geom
+    rng = np.random.default_rng(h * w)
+    full = (n, c, h, w, 0, win, win, 0, 0, 2, 2)
+    g, og = be.shape(*full), oracle.shape(*full)
+    x = oracle.round_bf16(rng.standard_normal((n, c, h, w)).astype(np.float32))
+    lowest = np.uint32(0xFF7F0000).view(np.float32) if bf16 else np.finfo(np.float32).min
+    for value in (np.nan, np.inf, -np.inf, lowest, -0.0, 0.0):
+        x[rng.random(x.shape) < 0.12] = value
+    x[:, :, :2, :2] = -np.inf     # windows in which nothing exceeds the lowest value
+    y = oracle.maxpool_fwd(og, x)
+    dy = rng.standard_normal(y.shape).astype(np.float32)
+    if bf16:
+        dy = oracle.round_bf16(dy)
+    dy[rng.random(y.shape) < 0.3] = -0.0
+    want = oracle.maxpool_bwd(og, x, y, dy)
+    if gated:
+        want = np.where(x > 0, want, np.float32(0))
+    if bf16:
+        want = oracle.round_bf16(want)
+    with be.Context(pool_bytes=256 << 20) as ctx, Dev(ctx) as d:
+        if bf16:
+            check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 1))
+        dtype, put, get = (np.uint16, to_bf16_bits, from_bf16_bits) if bf16 else (np.float32, lambda a: a, lambda a: a)
+        dx_, dy_, ddy, gx = d.up(put(x), dtype), d.empty(y.shape, dtype), d.up(put(dy), dtype), d.up(put(np.full_like(x, 7)), dtype)
+        announce("pool of special values", geom, bf16, gated)
+        check((lib.vdnn_maxpool_bwd_relu if gated else lib.vdnn_maxpool_bwd)(ctx.handle, None, g, dx_.ptr, dy_.ptr, ddy.ptr, gx.ptr))
+        assert np.array_equal(get(gx.download(x.shape, dtype)).view(np.uint32), want.view(np.uint32))
+
+
 # n, c, h, w, k, pad, stride; the last is one chunk of fewer pixels than threads
 FILTERS = [(3, 3, 25, 25, 24, 1, 1), (9, 4, 31, 29, 8, 0, 1), (2, 1, 40, 37, 4, 1, 2), (30, 2, 45, 45, 12, 0, 2), (1, 3, 9, 11, 16, 1, 1)]
 

@@ -903,7 +903,7 @@ __global__ void __launch_bounds__(EB) maxpool2x2_bwd_any_kernel(const E* __restr
     const size_t off = ((size_t)nc * H + 2 * p) * W + 2 * q;
     if (p < P && q < Q) {
         const float2 a = pair_at(x + off), b = pair_at(x + off + W);
-        float d = load_elem(dy + ((size_t)nc * P + p) * Q + q);
+        float d = 0.0f + load_elem(dy + ((size_t)nc * P + p) * Q + q); // (a sum that begins with zero, as over several windows: -0 becomes +0)
         int s = 0; float m = -FLT_MAX;   // the first strict maximum wins
         if (a.x > m) { m = a.x; s = 0; } if (a.y > m) { m = a.y; s = 1; }
         if (b.x > m) { m = b.x; s = 2; } if (b.y > m) { m = b.y; s = 3; }
