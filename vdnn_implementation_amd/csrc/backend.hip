@@ -1,6 +1,7 @@
 // Context, pooled device memory, streams, events and copies of the device back end.
 #include "backend_internal.h"
 
+#include <algorithm>
 #include <cstring>
 
 namespace vdnn {
@@ -12,6 +13,40 @@ void set_error(const char* fmt, ...) {
     va_start(ap, fmt);
     vsnprintf(g_error, sizeof(g_error), fmt, ap);
     va_end(ap);
+}
+
+bool stream_is_captured(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
+}
+
+// Cleared on a stream of the context and waited for: the context's streams do not wait for the default one, and clearing returns
+// before it is done.
+void* zeroed_device_memory(vdnn_ctx* ctx, size_t bytes) {
+    void* p = nullptr;
+    if (hipMalloc(&p, bytes) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    if (hipMemsetAsync(p, 0, bytes, ctx->pack) != hipSuccess || hipStreamSynchronize(ctx->pack) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipFree(p);
+        return nullptr;
+    }
+    return p;
+}
+
+unsigned* tile_counters_of(vdnn_ctx* ctx, hipStream_t stream) {
+    if (!ctx->tile_counters || stream_is_captured(stream)) return nullptr;
+    auto& owners = ctx->tile_counter_streams;
+    const size_t set = size_t(std::find(owners.begin(), owners.end(), stream) - owners.begin());
+    if (set >= size_t(kTileCounterSets)) return nullptr;
+    if (set == owners.size()) owners.push_back(stream);
+    return ctx->tile_counters + set * kTileCounters;
 }
 
 hipEvent_t prof_take_event(vdnn_ctx* ctx) {
@@ -60,17 +95,8 @@ int vdnn_ctx_create(vdnn_ctx** out, int device, int flags) {
             delete ctx;
             return VDNN_EDEVICE;
         }
-        // (split reductions are added up by a second kernel where there are no counters). The context's streams do not wait for the
-        // default one, and clearing returns before it is done.
-        if (hipMalloc((void**)&ctx->tile_counters, kTileCounters * sizeof(unsigned)) != hipSuccess) {
-            (void)hipGetLastError();
-            ctx->tile_counters = nullptr;
-        } else if (hipMemsetAsync(ctx->tile_counters, 0, kTileCounters * sizeof(unsigned), ctx->compute) != hipSuccess ||
-                   hipStreamSynchronize(ctx->compute) != hipSuccess) {
-            (void)hipGetLastError();
-            (void)hipFree(ctx->tile_counters);
-            ctx->tile_counters = nullptr;
-        }
+        // (split reductions are added up by a second kernel where there are no counters)
+        ctx->tile_counters = (unsigned*)zeroed_device_memory(ctx, sizeof(unsigned) * kTileCounters * kTileCounterSets);
         if (noalloc_prepare_current_device() != VDNN_OK) {
             delete ctx;
             return VDNN_EDEVICE;

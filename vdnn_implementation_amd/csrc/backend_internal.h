@@ -23,9 +23,11 @@ struct vdnn_ctx {
     // on another stream beside the kernels that keep their partial sums in the rest.
     float* bias_scratch = nullptr;
     size_t bias_scratch_bytes = 0;
-    // Zero between launches: how many workgroups of a split tile are done (sum_splits in mfma_gemm.h). Shared by the kernels that share the
-    // staging area, which their partial sums lie in.
+    // How many workgroups of a split tile are done (sum_splits in mfma_gemm.h): a set of counters per stream, for the first kTileCounterSets
+    // streams that ask. Zero between the launches of a stream, which run one behind the other and each put theirs back; with one set for all
+    // streams, two calls that overlap would spoil not their own sums alone but, through counters left standing, every later call's.
     unsigned* tile_counters = nullptr;
+    std::vector<hipStream_t> tile_counter_streams;
     int num_cu = 256;
     int act_dtype = VDNN_DTYPE_F32;   // element type of activation tensors handed to the kernels
     // per-kernel timing (vdnn_profile_*)
@@ -49,11 +51,18 @@ namespace vdnn {
 static constexpr size_t kReduceScratchBytes = size_t(64) << 20;
 static constexpr size_t kBiasScratchBytes = size_t(1) << 20;     // its last part: the convolution bias gradient's partial sums
 
-static constexpr int kTileCounters = 4096;
+static constexpr int kTileCounters = 4096, kTileCounterSets = 8;
 
 void set_error(const char* fmt, ...);
 
 inline hipStream_t stream_of(vdnn_ctx* ctx, vdnn_stream_t s) { return s ? (hipStream_t)s : ctx->compute; }
+
+// whether launches on the stream are being recorded into a graph (which may then run on any stream)
+bool stream_is_captured(hipStream_t stream);
+// `bytes` of device memory, zero before the call returns; null (and no error left behind) where there is none
+void* zeroed_device_memory(vdnn_ctx* ctx, size_t bytes);
+// the counters of a stream's launches; null while it is captured, and for streams beyond the first kTileCounterSets
+unsigned* tile_counters_of(vdnn_ctx* ctx, hipStream_t stream);
 
 hipEvent_t prof_take_event(vdnn_ctx* ctx);
 // looks up the current device's copy of the scratch array of vdnn_conv_bwd_bias_sgd_noalloc (eltwise.hip)

@@ -120,7 +120,7 @@ static int launch_by_m(vdnn_ctx* ctx, hipStream_t stream, const PassNames& names
             GemmDims ds = make_dims(M, N, K, 64, 64, plan.splits);
             const int tail = plan.full_tiles > 0 && ds.splits > 1 ? (int)((long)ds.mtiles * ds.ntiles - plan.full_tiles) : 0;
             if (tail > 0) ds.full_tiles = (int)plan.full_tiles;
-            const bool fused = fuse_split_sums(ctx, ds, partial_bytes);
+            const bool fused = fuse_split_sums(ctx, stream, ds, partial_bytes);
             const int rcs = launch_igemm<64, 64, AL, BL, StoreNCHW<E>>(ctx, stream, names.t64s, al, bl, ep, ds, flops);
             if (rcs != VDNN_OK || ds.splits == 1 || fused) return rcs;
             if (tail > 0)

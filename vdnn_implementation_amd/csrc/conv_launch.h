@@ -32,11 +32,11 @@ static inline GemmDims make_dims(int M, int N, int K, int TM, int TN, int splits
 // 16.3 -> 15.3; 26 x 16 x 55 x 55, 64 of 3x3 27.4 -> 25.1; 5 x 144 x 54 x 54, 64 of 3x3 36.5 -> 30.8. Not for backward filter, whose
 // products fill the chip by their splits: 5 x 144 x 16 x 16, 128 of 3x3 backward 33.1 -> 35.2.
 constexpr int kFusedSplits = 6;
-static inline bool fuse_split_sums(const vdnn_ctx* ctx, GemmDims& d, size_t partial_bytes) {
+static inline bool fuse_split_sums(vdnn_ctx* ctx, hipStream_t stream, GemmDims& d, size_t partial_bytes) {
     const long tiles = (long)d.mtiles * d.ntiles - d.full_tiles;
-    if (d.splits < 2 || d.splits > kFusedSplits || !ctx->tile_counters || tiles > kTileCounters || (size_t)tiles * d.splits * 64 * 64 * sizeof(float) > partial_bytes) return false;
-    d.counters = ctx->tile_counters;
-    return true;
+    if (d.splits < 2 || d.splits > kFusedSplits || tiles > kTileCounters || (size_t)tiles * d.splits * 64 * 64 * sizeof(float) > partial_bytes) return false;
+    d.counters = tile_counters_of(ctx, stream);
+    return d.counters != nullptr;
 }
 
 // What is planned without a context at hand assumes the 256 compute units of the target part and the staging area as it is made.

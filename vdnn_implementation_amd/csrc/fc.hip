@@ -52,7 +52,7 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     d.kchunk = kchunk;
     d.splits = (K + kchunk - 1) / kchunk;
     d.full_tiles = 0;
-    const bool fused = small && fuse_split_sums(ctx, d, ctx->reduce_scratch_bytes);
+    const bool fused = small && fuse_split_sums(ctx, st, d, ctx->reduce_scratch_bytes);
     StoreDense<EO> ep{out, ctx->reduce_scratch, d.splits > 1 && !fused ? nullptr : bias_j, (long)N, (long)M * N, alpha, accumulate, relu, gate};
     const long blocks = (long)d.mtiles * d.ntiles * d.splits;
     ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
