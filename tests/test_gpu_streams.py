@@ -1,4 +1,5 @@
-"""State that outlives a launch: the counters with which a split product adds up its own sums (csrc/mfma_gemm.h, sum_splits). One set per stream, so that calls on several streams, overlapping or captured, leave nothing behind that a later call meets."""
+"""State that outlives a launch: the counters with which a split product adds up its own sums (csrc/mfma_gemm.h, sum_splits) and the packing
+kernels' cursors. One set per stream, so that calls on several streams, overlapping or captured, leave nothing behind that a later call meets."""
 import numpy as np
 import pytest
 import torch
@@ -6,6 +7,7 @@ import torch
 import oracle
 import vdnn_implementation_amd.backend as be
 from gpu_util import Dev, announce
+from test_gpu_zvc import Pinned, decode, tensor
 from vdnn_implementation_amd.backend import check, lib
 
 pytestmark = pytest.mark.gpu
@@ -142,3 +144,35 @@ def test_captured_product_beside_calls_of_its_stream(ctx):
             call(recording.cuda_stream, y2)
             ctx.synchronize()
             assert np.array_equal(y2.download(shape), want)
+
+
+@pytest.mark.parametrize("staged", [False, True], ids=["direct", "staged"])
+def test_many_offloads_in_flight_on_two_streams(ctx, staged):
+    """A hundred and forty packing kernels on two streams: one stream's long tensor packs while the other's short ones come and go."""
+    rng = np.random.default_rng(5)
+    big, small = tensor(rng, 3_000_000, np.uint32, 0.4), [tensor(rng, int(rng.integers(1, 20000)), np.uint16, 0.5) for _ in range(7)]
+    s1, s2 = other_streams(2)
+    with Dev(ctx) as d:
+        sources = [d.up(t, t.dtype) for t in [big] + small]
+        todo = []
+        for i in range(140):
+            which = 0 if i % 35 == 0 else 1 + i % 7
+            a = big if which == 0 else small[which - 1]
+            need = lib.vdnn_zvc_buffer_bytes(a.size, a.itemsize)
+            stage = d.empty((need,), np.uint8) if staged else None
+            todo.append((a, sources[which], Pinned(ctx, need), stage, need, (s1 if which == 0 else s2).cuda_stream, Pinned(ctx, 8)))
+        announce("offloads on two streams", staged)
+        for a, src, host, stage, need, s, word in todo:
+            if staged:
+                check(lib.vdnn_zvc_offload_staged_async(ctx.handle, host.ptr, stage.ptr, need, src.ptr, a.size, a.itemsize, word.ptr, None, s, None, 0))
+            else:
+                check(lib.vdnn_zvc_offload_async(ctx.handle, host.ptr, src.ptr, a.size, a.itemsize, s))
+        ctx.synchronize()
+        for a, _, host, stage, need, s, word in todo:
+            got, length = decode(host.view, a.size, a.dtype)
+            assert np.array_equal(got, a)
+            if staged:
+                assert int(word.view.view(np.uint64)[0]) == length
+        for _, _, host, _, _, _, word in todo:
+            host.free()
+            word.free()

@@ -123,6 +123,7 @@ int vdnn_ctx_destroy(vdnn_ctx* ctx) {
         for (auto& r : ctx->prof_records) { (void)hipEventDestroy(r.start); (void)hipEventDestroy(r.stop); }
         for (auto e : ctx->prof_free_events) (void)hipEventDestroy(e);
         if (ctx->zvc_counters) (void)hipFree(ctx->zvc_counters);
+        for (void* b : ctx->zvc_cursor_blocks) (void)hipFree(b);
         if (ctx->tile_counters) (void)hipFree(ctx->tile_counters);
         if (ctx->compute) (void)hipStreamDestroy(ctx->compute);
         if (ctx->d2h) (void)hipStreamDestroy(ctx->d2h);

@@ -39,11 +39,12 @@ struct vdnn_ctx {
     std::vector<ProfRecord> prof_records;
     std::vector<hipEvent_t> prof_free_events;
     unsigned long long prof_untimed = 0;   // launches since vdnn_profile_enable that ran beyond the limit
-    // zero-value compression of offloaded tensors: device words (bytes sent over the link, then the stream
-    // cursors of the offloads in flight) and bytes of the tensors that were packed
+    // zero-value compression of offloaded tensors: a device word (bytes sent over the link), bytes of the tensors that were packed, and
+    // the cursors in blocks of kZvcCursors, each owned by the stream at its index (null: by one captured call)
     unsigned long long* zvc_counters = nullptr;
     unsigned long long zvc_raw_bytes = 0;
-    unsigned zvc_next_cursor = 0;
+    std::vector<void*> zvc_cursor_blocks;
+    std::vector<hipStream_t> zvc_cursor_streams;
 };
 
 namespace vdnn {

@@ -44,7 +44,7 @@ static constexpr int kZvcThreads = 256 * kZvcTeams;
 // (a pooling layer has no matrix work to hide it behind): a step of VGG16 at batch 128 in bfloat16 22.4 ms with one, 21.9 with two
 // and four, 21.8 with three, 22.0 with eight.
 static constexpr int kZvcPackPerCu = 3;
-static constexpr int kZvcCursors = 64;      // offloads that may be in flight at once
+static constexpr int kZvcCursors = 64;      // cursors of a block
 
 __host__ __device__ inline size_t zvc_table_bytes(size_t chunks) { return (chunks * 4 + 15) / 16 * 16; }
 __host__ __device__ inline size_t zvc_record_bytes_max(int elem_bytes) { return size_t(kZvcMapBytes) + size_t(kZvcChunk) * elem_bytes; }
@@ -59,7 +59,7 @@ struct alignas(16) ZvcRecord {
 };
 
 // Where an offload's claims stand: the bytes of records claimed so far, and the workgroups that are done. Both words are zero
-// between offloads: the workgroup that is done last puts them back, so no launch before the packing kernel clears them and
+// between the offloads of a stream: the workgroup that is done last puts them back, so no launch before the packing kernel clears them and
 // none behind it reads them (they were two launches of 5 us each, one after the other with the packing kernel, per tensor).
 struct ZvcCursor {
     unsigned long long claimed;
@@ -343,18 +343,27 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_unpack_kernel(const unsigned 
 }
 
 static int zvc_ensure_counters(vdnn_ctx* ctx) {
-    if (ctx->zvc_counters) return VDNN_OK;
-    // [0], [1]: bytes over the link; then the stream cursors, one per offload in flight
-    const size_t bytes = sizeof(unsigned long long) * 2 + sizeof(ZvcCursor) * kZvcCursors;
-    unsigned long long* counters = nullptr;
-    VDNN_HIP(hipMalloc((void**)&counters, bytes));
-    // the first launch finds them cleared: the context's streams do not wait for the default one, and clearing returns before it is done
-    hipError_t cleared = hipMemsetAsync(counters, 0, bytes, ctx->pack);
-    if (cleared == hipSuccess) cleared = hipStreamSynchronize(ctx->pack);
-    if (cleared != hipSuccess) (void)hipFree(counters);
-    VDNN_HIP(cleared);
-    ctx->zvc_counters = counters;
+    if (!ctx->zvc_counters) ctx->zvc_counters = (unsigned long long*)zeroed_device_memory(ctx, sizeof(unsigned long long));
+    if (!ctx->zvc_counters) { set_error("no device memory for the offload's counter"); return VDNN_EDEVICE; }
     return VDNN_OK;
+}
+
+// The cursor of a packing kernel on `stream`. A stream's kernels run one behind the other and each leaves its cursor at zero, so one per
+// stream does for any number of offloads in flight; two that ran on one cursor at once would write into each other's records and past
+// the stream's end. A captured call, whose graph may run beside anything, has a cursor of its own.
+static ZvcCursor* zvc_cursor(vdnn_ctx* ctx, hipStream_t stream) {
+    auto& owners = ctx->zvc_cursor_streams;
+    const bool captured = stream_is_captured(stream);
+    size_t i = captured ? owners.size() : size_t(std::find(owners.begin(), owners.end(), stream) - owners.begin());
+    if (i == owners.size()) {
+        if (i == ctx->zvc_cursor_blocks.size() * kZvcCursors) {
+            void* block = zeroed_device_memory(ctx, sizeof(ZvcCursor) * kZvcCursors);
+            if (!block) return nullptr;
+            ctx->zvc_cursor_blocks.push_back(block);
+        }
+        owners.push_back(captured ? nullptr : stream);
+    }
+    return (ZvcCursor*)ctx->zvc_cursor_blocks[i / kZvcCursors] + i % kZvcCursors;
 }
 
 static int zvc_offload(vdnn_ctx* ctx, void* dst_host, void* staging_dev, size_t staging_bytes, const void* src_dev, size_t count,
@@ -377,7 +386,8 @@ static int zvc_offload(vdnn_ctx* ctx, void* dst_host, void* staging_dev, size_t 
     VDNN_REQUIRE(staging_bytes <= vdnn_zvc_buffer_bytes(count, elem_bytes), "staging buffer longer than the longest stream");
     if (int rc = zvc_ensure_counters(ctx)) return rc;
     const size_t chunks = (count + kZvcChunk - 1) / kZvcChunk;
-    ZvcCursor* cursor = reinterpret_cast<ZvcCursor*>(ctx->zvc_counters + 2) + ctx->zvc_next_cursor++ % kZvcCursors;
+    ZvcCursor* cursor = zvc_cursor(ctx, ps);
+    if (!cursor) { set_error("no device memory for the offload's cursor"); return VDNN_EDEVICE; }
     const ZvcReport report{total_host, ctx->zvc_counters, keep_on_device};
     auto grid = [&](size_t per_workgroup, size_t cap) { return int(std::min((chunks + per_workgroup - 1) / per_workgroup, cap)); };
     {
