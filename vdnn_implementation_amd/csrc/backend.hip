@@ -91,14 +91,14 @@ int vdnn_ctx_create(vdnn_ctx** out, int device, int flags) {
             hipStreamCreateWithFlags(&ctx->d2h, hipStreamNonBlocking) != hipSuccess ||
             hipStreamCreateWithFlags(&ctx->h2d, hipStreamNonBlocking) != hipSuccess ||
             hipStreamCreateWithFlags(&ctx->pack, hipStreamNonBlocking) != hipSuccess) {
+            vdnn_ctx_destroy(ctx);
             set_error("hipStreamCreate failed");
-            delete ctx;
             return VDNN_EDEVICE;
         }
         // (split reductions are added up by a second kernel where there are no counters)
         ctx->tile_counters = (unsigned*)zeroed_device_memory(ctx, sizeof(unsigned) * kTileCounters * kTileCounterSets);
         if (noalloc_prepare_current_device() != VDNN_OK) {
-            delete ctx;
+            vdnn_ctx_destroy(ctx);
             return VDNN_EDEVICE;
         }
     }
