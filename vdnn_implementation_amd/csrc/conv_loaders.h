@@ -356,6 +356,8 @@ struct LoadIm2colRed {
     }
 };
 
+template <class E> struct LargeTileResident<256, LoadIm2colRed<true, E>> { static constexpr int V = 2; };
+
 // ---- result of forward / backward data: out[n][m][pix] = acc (+ bias[m]) --------------------------
 template <class E = float>
 struct StoreNCHW {

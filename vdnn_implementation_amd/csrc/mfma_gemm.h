@@ -436,8 +436,13 @@ __device__ __forceinline__ void igemm_tile(const AL& al, const BL& bl, const EP&
         ep.store(acc, m0 + wm0, j0 + wn0, lane, ks, d, !whole);
 }
 
+// Workgroups of the large tiles that share a compute unit: three, for which 168 registers are left - two where a loader's address work takes more
+// (column operands of 256 with a window beyond 32 taps: 16 registers spilled in the loop at three, backward filter 4 x 49 x 138 x 138, 58 of
+// 7x7 at stride 3 72 us, 50 at two; 42 x 436 x 57 x 57, 16 of 7x7 479, 358).
+template <int TN, class BL> struct LargeTileResident { static constexpr int V = 3; };
+
 template <int TM, int TN, class AL, class BL, class EP, int AHEAD = 1>
-__global__ void __launch_bounds__(NT, 3) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
+__global__ void __launch_bounds__(NT, (LargeTileResident<TN, BL>::V)) igemm_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
     igemm_tile<TM, TN, AHEAD>(al, bl, ep, d, blockIdx.x, gridDim.x);
 }
 
