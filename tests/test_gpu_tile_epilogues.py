@@ -19,6 +19,12 @@ FCS = [(1, 16, 1), (5, 99, 33), (33, 96, 31), (64, 112, 64), (65, 128, 130), (10
        (61, 9010, 4700), (200, 5009, 2600)]  # the larger tiles, odd and even counts of slices in a split
 
 
+# rows around the eights that a block's result leaves in, forward (filters) and backward data (channels), in the 64x64 and the large tiles
+FEW_ROWS = [(2, 7, 30, 30, 9, 3), (3, 17, 21, 19, 8, 1), (2, 24, 13, 17, 25, 3), (1, 15, 40, 40, 16, 5), (30, 8, 90, 91, 1, 3), (40, 9, 80, 80, 7, 1), (9, 16, 90, 91, 24, 3),
+            (1, 300, 24, 23, 6, 1), (12, 150, 6, 5, 9, 3)]  # the last two with split sums
+FEW_ROWS_FC = [(1, 9, 61), (7, 33, 130), (8, 700, 40), (9, 3000, 129), (17, 640, 800), (25, 5893, 753)]
+
+
 @pytest.fixture(scope="module")
 def ctx():
     with be.Context(pool_bytes=512 << 20) as c:
@@ -30,7 +36,7 @@ def within(got, want, products):
     return error <= 2.0 ** -24 * max(np.sqrt(products / 2), 4)  # (a few products: the roundings of bias, update and result)
 
 
-@pytest.mark.parametrize("geom", CONVS, ids=lambda g: "x".join(map(str, g)))
+@pytest.mark.parametrize("geom", CONVS + FEW_ROWS, ids=lambda g: "x".join(map(str, g)))
 def test_convolution(ctx, geom):
     n, c, h, w, k, r = geom
     rng = np.random.default_rng(n + c + k)
@@ -61,7 +67,7 @@ def test_convolution(ctx, geom):
         assert np.array_equal(dx_.download(x.shape), np.where(x > 0, plain, 0))
 
 
-@pytest.mark.parametrize("sizes", FCS, ids=lambda s: "x".join(map(str, s)))
+@pytest.mark.parametrize("sizes", FCS + FEW_ROWS_FC, ids=lambda s: "x".join(map(str, s)))
 def test_fully_connected(ctx, sizes):
     n, ci, co = sizes
     rng = np.random.default_rng(n + ci + co)

@@ -368,9 +368,9 @@ struct StoreNCHW {
     int relu;          // rectify the result (after the bias)
     const E* gate;     // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
     static constexpr bool TAIL = true;
-    // The gate or the bias (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; rows and columns past the end
-    // read some element inside. (A gate that is the output tensor - the gradient written over the layer's own input - is read by
-    // the lane that overwrites it, before it does.)
+    // The gate or the bias (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; columns past the end, and
+    // rows past it in the eight that begins inside, read some element inside, other rows past it are not read. (A gate that is the
+    // output tensor - the gradient written over the layer's own input - is read by the lane that overwrites it, before it does.)
     __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
         const int lk = lane >> 5;
         if (to_partial) return;
@@ -378,10 +378,18 @@ struct StoreNCHW {
             const int j = min(j0 + (lane & 31), d.N - 1), n = j / opix, pix = j - n * opix;
             const E* from = gate + (size_t)n * d.M * opix + pix;
 #pragma unroll
-            for (int v = 0; v < 16; v++) aux[v] = load_elem(from + (size_t)min(m0 + result_row(v, lk), d.M - 1) * opix);
+            for (int q = 0; q < 4; q++) {
+                if (rows_behind(m0, q, d.M)) break;
+#pragma unroll
+                for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_elem(from + (size_t)min(m0 + result_row(v, lk), d.M - 1) * opix);
+            }
         } else if (bias) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) aux[v] = bias[min(m0 + result_row(v, lk), d.M - 1)];
+            for (int q = 0; q < 4; q++) {
+                if (rows_behind(m0, q, d.M)) break;
+#pragma unroll
+                for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = bias[min(m0 + result_row(v, lk), d.M - 1)];
+            }
         }
     }
     __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
@@ -428,7 +436,8 @@ struct StoreNCHW {
     __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
 #pragma unroll
         for (int it = 0; it < MI; it++) {
-            float aux[16]; // the bias is the same for a row of blocks
+            if (rows_behind(m0, 4 * it, d.M)) break;
+            float aux[16] = {}; // the bias is the same for a row of blocks
             read_aux(aux, m0 + it * 32, j0, lane, d, to_partial);
 #pragma unroll
             for (int jt = 0; jt < NJ; jt++) {

@@ -208,7 +208,11 @@ struct StoreFilterTap {
         const int j = min(j0 + (lane & 31), d.N - 1), lk = lane >> 5, tap = divC.div(j);
         const float* from = out + (long)(j - tap * C) * RS + tap;
 #pragma unroll
-        for (int v = 0; v < 16; v++) aux[v] = from[(long)min(m0 + result_row(v, lk), d.M - 1) * d.N];
+        for (int q = 0; q < 4; q++) {
+            if (rows_behind(m0, q, d.M)) break;
+#pragma unroll
+            for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = from[(long)min(m0 + result_row(v, lk), d.M - 1) * d.N];
+        }
     }
     __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
         const int j = j0 + (lane & 31), lk = lane >> 5;
@@ -229,7 +233,8 @@ struct StoreFilterTap {
     __device__ __forceinline__ void store(const floatx16 (&acc)[MI][NJ], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
 #pragma unroll
         for (int b = 0; b < MI * NJ; b++) {
-            float aux[16];
+            if (rows_behind(m0, 4 * (b / NJ), d.M)) break;
+            float aux[16] = {};
             read_aux(aux, m0 + b / NJ * 32, j0 + b % NJ * 32, lane, d, to_partial);
             store32(acc[b / NJ][b % NJ], aux, m0 + b / NJ * 32, j0 + b % NJ * 32, lane, ks, d, to_partial);
         }

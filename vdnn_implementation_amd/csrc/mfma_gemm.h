@@ -537,7 +537,7 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
     const int nslices = (k_end - k_begin + KB - 1) / KB;
     const int l32 = lane & 31, lk = lane >> 5;
     const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
-    float aux[16];
+    float aux[16] = {};
     ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, !at.whole);
     floatx16 acc;
 #pragma unroll
@@ -741,9 +741,12 @@ struct RoundedToBf16 : L {
     }
 };
 
+// The first of the eight rows from which a lane's registers 4 q .. 4 q + 3 are, past the last row or not; the same for the whole wavefront.
+__device__ __forceinline__ bool rows_behind(int m0, int q, int M) { return __builtin_amdgcn_readfirstlane(m0) + 8 * q >= M; }
+
 // A lane's sixteen results of a 32x32 block, `to` at row m0 + 4 lk, rows from M on left out. The test per row is for the blocks at the
-// lower edge only: with a branch on each of a tile's 64 rows, and one each on bias, gate and rectifier, a tile's epilogue took 2.7 us per
-// 32x32 block of a wavefront, most of it the fetch of its text. Forward 9 x 448 x 189 x 189, 576 of 1x1 in bfloat16 631 -> 418 us; 29 x 32 x 30 x 30, 289
+// lower edge only, and there for the rows of the eights that begin inside: with a branch on each of a tile's 64 rows, and one each on bias,
+// gate and rectifier, a tile's epilogue took 2.7 us per 32x32 block of a wavefront, most of it the fetch of its text. Forward 9 x 448 x 189 x 189, 576 of 1x1 in bfloat16 631 -> 418 us; 29 x 32 x 30 x 30, 289
 // of 3x3 30 -> 22; backward 11 x 486 x 71 x 71, 64 of 3x3 246 -> 184; floats at two bfloat16 parts, 122 x 80 x 23 x 23, 528 of 3x3 216 -> 198.
 template <class E, class L>
 __device__ __forceinline__ void store_rows(E* to, const floatx16& acc, L stride, int m0, int lk, int M) {
@@ -752,8 +755,12 @@ __device__ __forceinline__ void store_rows(E* to, const floatx16& acc, L stride,
         for (int v = 0; v < 16; v++) store_elem(to + (long)(8 * (v / 4) + v % 4) * stride, acc[v]);
     } else {
 #pragma unroll
-        for (int v = 0; v < 16; v++)
-            if (m0 + result_row(v, lk) < M) store_elem(to + (long)(8 * (v / 4) + v % 4) * stride, acc[v]);
+        for (int q = 0; q < 4; q++) {
+            if (rows_behind(m0, q, M)) break;
+#pragma unroll
+            for (int v = 4 * q; v < 4 * q + 4; v++)
+                if (m0 + result_row(v, lk) < M) store_elem(to + (long)(8 * q + v % 4) * stride, acc[v]);
+        }
     }
 }
 
@@ -770,14 +777,18 @@ struct StoreDense {
     int accumulate;
     int relu;      // rectify the result (after the bias)
     const E* gate; // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
-    // The old values or the gate (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; rows and
-    // columns past the end read some element inside.
+    // The old values or the gate (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; columns past the
+    // end, and rows past it in the eight that begins inside, read some element inside. What else is past it is not read (nor stored).
     __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
         if (to_partial || !(accumulate || gate)) return;
         const int j = min(j0 + (lane & 31), d.N - 1), lk = lane >> 5;
         const E* from = accumulate ? out : gate;
 #pragma unroll
-        for (int v = 0; v < 16; v++) aux[v] = load_elem(from + (long)min(m0 + result_row(v, lk), d.M - 1) * ld_m + j);
+        for (int q = 0; q < 4; q++) {
+            if (rows_behind(m0, q, d.M)) break;
+#pragma unroll
+            for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_elem(from + (long)min(m0 + result_row(v, lk), d.M - 1) * ld_m + j);
+        }
     }
     __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
         const int j = j0 + (lane & 31), lk = lane >> 5;
@@ -818,7 +829,8 @@ struct StoreDense {
         for (int jt = 0; jt < NJ; jt++)
 #pragma unroll
             for (int it = 0; it < MI; it++) {
-                float aux[16];
+                if (rows_behind(m0, 4 * it, d.M)) break;
+                float aux[16] = {};
                 read_aux(aux, m0 + it * 32, j0 + jt * 32, lane, d, to_partial);
                 store32(acc[it][jt], aux, m0 + it * 32, j0 + jt * 32, lane, ks, d, to_partial);
             }
