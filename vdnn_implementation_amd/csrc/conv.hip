@@ -81,7 +81,7 @@ static int launch_igemm(vdnn_ctx* ctx, hipStream_t stream, const char* name, con
     // unpadded layer multiplies taps that fall outside the output; they are not counted)
     ProfScope prof(ctx, stream, name, flops > 0.0 ? flops : 2.0 * d.M * (double)d.N * d.K, 0.0);
     if constexpr (HALF) hipLaunchKernelGGL((igemm_bf16_kernel<TM, TN, AL, BL, EP>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
-    else if constexpr (TM == 64 && TN == 64) launch_igemm64((unsigned)blocks, stream, al, bl, ep, d);
+    else if constexpr (TM == 64 && TN == 64) launch_igemm64<EP::TAIL>((unsigned)blocks, stream, al, bl, ep, d); // (forward and backward data)
     else hipLaunchKernelGGL((igemm_kernel<TM, TN, AL, BL, EP, SlicesAhead<BL, EP>::V>), dim3((unsigned)blocks), dim3(NT), 0, stream, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();
     return VDNN_OK;

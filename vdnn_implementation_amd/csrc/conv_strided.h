@@ -39,7 +39,7 @@ template <class E, int AHEAD>
 __global__ void __launch_bounds__(NT) igemm_classes_kernel(const StridedLaunch<E> s) {
     int c = 0, bid = blockIdx.x;
     while (c + 1 < s.count && bid >= s.c[c].blocks) bid -= s.c[c++].blocks;
-    igemm_small_tile<AHEAD>(s.c[c].al, s.c[c].bl, s.c[c].ep, s.c[c].d, bid, s.c[c].blocks);
+    igemm_small_tile<AHEAD, false>(s.c[c].al, s.c[c].bl, s.c[c].ep, s.c[c].d, bid, s.c[c].blocks);
 }
 
 // where a class's filter taps, pixels and partial sums lie

@@ -56,7 +56,7 @@ static int fc_gemm(vdnn_ctx* ctx, hipStream_t st, const char* name, const AL& al
     StoreDense<EO> ep{out, ctx->reduce_scratch, d.splits > 1 && !fused ? nullptr : bias_j, (long)N, (long)M * N, alpha, accumulate, relu, gate};
     const long blocks = (long)d.mtiles * d.ntiles * d.splits;
     ProfScope prof(ctx, st, name, 2.0 * M * (double)N * K, 0.0);
-    if (small) launch_igemm64((unsigned)blocks, st, al, bl, ep, d);
+    if (small) launch_igemm64<true>((unsigned)blocks, st, al, bl, ep, d);
     else if (TM == 64) hipLaunchKernelGGL((igemm_kernel<64, 256, AL, BL, StoreDense<EO>, 2>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     else hipLaunchKernelGGL((igemm_kernel<128, 128, AL, BL, StoreDense<EO>, 2>), dim3((unsigned)blocks), dim3(NT), 0, st, al, bl, ep, d);
     VDNN_LAUNCH_CHECK();

@@ -446,16 +446,6 @@ __global__ void __launch_bounds__(NT, (LargeTileResident<TN, BL>::V)) igemm_kern
     igemm_tile<TM, TN, AHEAD>(al, bl, ep, d, blockIdx.x, gridDim.x);
 }
 
-// The 64x64 tile. A workgroup has one wavefront per SIMD and a few to some tens of slices, and where it is taken most of the chip
-// has one or two workgroups a unit: what counts is the latency of every step (1 x 64 x 112 x 112, 64 filters of 3x3, 36 slices on 196
-// lone workgroups, clocked inside the kernel). Against igemm_tile's pipeline:
-// - AHEAD slices are on their way from memory (four, or one where there are few), so that a slice's values are there when they are
-//   written to LDS: operands that another kernel has just written 0.37 -> 0.33 us a slice. (0.21 are the matrix instructions; with
-//   one wavefront per SIMD the rest is the issue of some hundred instructions and the barrier.)
-// - What the result is combined with (bias, gate, old values) is read before the loop, and the epilogue branches on what is
-//   uniform only, once per tile: 2.7 -> 0.9 us.
-// One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
-// four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 102.7.
 // Split reductions of the 64x64 tile without a second kernel. Every workgroup of a tile leaves its sums in the staging area and counts
 // itself; the one that counts last adds them up in split order - the sums a second kernel would form - and writes the result. The
 // counters are zero between launches: the last workgroup puts its tile's back.
@@ -506,7 +496,17 @@ __device__ __forceinline__ bool sum_splits(floatx16& acc, float* staging, const 
     return true;
 }
 
-template <int AHEAD, class AL, class BL, class EP>
+// The 64x64 tile. A workgroup has one wavefront per SIMD and a few to some tens of slices, and where it is taken most of the chip
+// has one or two workgroups a unit: what counts is the latency of every step (1 x 64 x 112 x 112, 64 filters of 3x3, 36 slices on 196
+// lone workgroups, clocked inside the kernel). Against igemm_tile's pipeline:
+// - AHEAD slices are on their way from memory (four, or one where there are few), so that a slice's values are there when they are
+//   written to LDS: operands that another kernel has just written 0.37 -> 0.33 us a slice. (0.21 are the matrix instructions; with
+//   one wavefront per SIMD the rest is the issue of some hundred instructions and the barrier.)
+// - What the result is combined with (bias, gate, old values) is read before the loop, and the epilogue branches on what is
+//   uniform only, once per tile: 2.7 -> 0.9 us.
+// One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
+// four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 102.7.
+template <int AHEAD, bool SUMS, class AL, class BL, class EP>
 __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
     constexpr int T = 64;
     using LA = LdsTile<T, AL::RED_MAJOR>;
@@ -537,8 +537,9 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
     const int nslices = (k_end - k_begin + KB - 1) / KB;
     const int l32 = lane & 31, lk = lane >> 5;
     const int wm0 = (wave & 1) * 32, wn0 = (wave >> 1) * 32;
+    constexpr bool AUX_FIRST = AHEAD > 1 || SUMS; // (where the registers are there anyway; the others fill the chip, or are over at once)
     float aux[16] = {};
-    ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, !at.whole);
+    if constexpr (AUX_FIRST) ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, !at.whole);
     floatx16 acc;
 #pragma unroll
     for (int v = 0; v < 16; v++) acc[v] = 0.0f;
@@ -598,7 +599,7 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
         }
     }
 
-    if (!at.whole && d.counters) {
+    if (SUMS && !at.whole && d.counters) {
         if (!sum_splits(acc, ep.partial, d, at.tile - d.full_tiles, at.ks, tid)) return;
         ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, false);
         ep.store32(acc, aux, at.m0 + wm0, at.j0 + wn0, lane, 0, d, false);
@@ -606,6 +607,7 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
         const floatx16 tail[1][1] = {{acc}};
         ep.store_tail(tail, wm0, wn0, lane, (long)(at.tile - d.full_tiles) * d.splits + at.ks, T, T);
     } else {
+        if constexpr (!AUX_FIRST) ep.read_aux(aux, at.m0 + wm0, at.j0 + wn0, lane, d, !at.whole);
         ep.store32(acc, aux, at.m0 + wm0, at.j0 + wn0, lane, at.ks, d, !at.whole);
     }
 }
@@ -616,19 +618,27 @@ static inline bool small_tile_ahead(const GemmDims& d, long blocks) { return d.k
 // ... and where the loader's address work does not count for more than the latency (LoadIm2colPix<2>: two divisions per element)
 template <class L> struct FetchesAhead { static constexpr bool V = true; };
 
-template <class AL, class BL, class EP, int AHEAD>
+// SUMS: whether the instance can add up splits itself. That takes half of its registers (with one slice ahead eight wavefronts a SIMD become
+// four) and stands in the text that a lone workgroup fetches, so calls without take another.
+template <class AL, class BL, class EP, int AHEAD, bool SUMS>
 __global__ void __launch_bounds__(NT) igemm64_kernel(const AL al, const BL bl, const EP ep, const GemmDims d) {
-    igemm_small_tile<AHEAD>(al, bl, ep, d, blockIdx.x, gridDim.x);
+    igemm_small_tile<AHEAD, SUMS>(al, bl, ep, d, blockIdx.x, gridDim.x);
 }
-template <class AL, class BL, class EP>
+template <bool SUMS, class AL, class BL, class EP>
 static inline void launch_igemm64(unsigned blocks, hipStream_t stream, const AL& al, const BL& bl, const EP& ep, const GemmDims& d) {
-    if constexpr (FetchesAhead<BL>::V) {
-        if (small_tile_ahead(d, blocks)) {
-            hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, kSmallTileAhead>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
+    if constexpr (SUMS) {
+        if (!d.counters) {
+            launch_igemm64<false>(blocks, stream, al, bl, ep, d);
             return;
         }
     }
-    hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, 1>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
+    if constexpr (FetchesAhead<BL>::V) {
+        if (small_tile_ahead(d, blocks)) {
+            hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, kSmallTileAhead, SUMS>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
+            return;
+        }
+    }
+    hipLaunchKernelGGL((igemm64_kernel<AL, BL, EP, 1, SUMS>), dim3(blocks), dim3(NT), 0, stream, al, bl, ep, d);
 }
 
 // ---- dense reduction-major operand: element (row, kk) at base[row*ld + kk] -------------------------
