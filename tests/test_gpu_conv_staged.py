@@ -51,3 +51,30 @@ def test_against_oracle(geom, staged):
         be.profile_enable(ctx.handle, False)
         check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, df.ptr, dx_.ptr, gx.ptr, None, 0))
         assert np.array_equal(from_bf16_bits(gx.download(x.shape, np.uint16)), np.where(x > 0, plain, 0))
+        if lib.vdnn_conv_bwd_data_in_place_ok(g):
+            check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, df.ptr, dx_.ptr, dx_.ptr, None, 0))
+            assert np.array_equal(from_bf16_bits(dx_.download(x.shape, np.uint16)), np.where(x > 0, plain, 0))
+
+
+# n, c, h, w, k, window, pad, stride; whether forward takes the copy
+ROUTES = [((12, 96, 27, 27, 130, 5, 2, 1), True), ((24, 608, 45, 45, 80, 5, 2, 2), False),  # (no room left for eight splits)
+          ((2, 255, 120, 218, 3, 3, 0, 1), False),   # pairs of pixels, nine taps
+          ((20, 96, 40, 40, 192, 5, 2, 1), True),    # pairs, twenty-five taps
+          ((5, 202, 143, 143, 112, 2, 1, 1), False)]  # four taps
+
+
+@pytest.mark.parametrize("geom,staged", ROUTES, ids=lambda g: "x".join(map(str, g)) if isinstance(g, tuple) else "")
+def test_copies_only_where_they_pay(geom, staged):
+    n, c, h, w, k, r, pad, stride = geom
+    p, q = (h + 2 * pad - r) // stride + 1, (w + 2 * pad - r) // stride + 1
+    g = be.shape(n, c, h, w, k, r, r, pad, pad, stride, stride)
+    with be.Context(pool_bytes=512 << 20) as ctx, Dev(ctx) as d:
+        check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 1))
+        x, f, b, y = d.empty((n, c, h, w), np.uint16), d.empty((k, c, r, r)), d.empty((k,)), d.empty((n, k, p, q), np.uint16)
+        for buf, count in ((f, k * c * r * r), (b, k)):
+            buf.upload(np.zeros(count, np.float32))
+        x.upload(np.zeros((n, c, h, w), np.uint16))
+        be.profile_enable(ctx.handle, True)
+        announce("copy or not", geom)
+        check(lib.vdnn_conv_fwd(ctx.handle, None, g, 0, x.ptr, f.ptr, b.ptr, y.ptr, None, 0))
+        assert ("conv_stage_pixels" in be.profile_collect(ctx.handle)) == staged

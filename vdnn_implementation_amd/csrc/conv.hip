@@ -561,20 +561,28 @@ static const float* rounded_filter_copy(vdnn_ctx* ctx, hipStream_t st, StagingCa
 }
 
 // Forward (MODE 0) and backward data at stride 1 (MODE 1) from a copy of the source in `scratch` (conv_staged.h). al: the filter bank; K: its row.
-// Where the copy fits there at once, and the operations, rows in whole blocks of 64, are worth its trip through memory: a large source
-// is read from memory again tap by tap (43 x 304 x 131 x 131, 64 of 3x3 forward 664 us, 837 from a copy in nine parts; 118 x 64 x 131 x 131, 82 of
-// 5x5 1048, 1090), a 1x1 window reads it once anyway (6 x 64 x 105 x 105, 704 of 1x1 41, 44), and a small layer is over before the copy
-// is (7 x 576 x 10 x 10, 384 of 3x3 27.5, 29.7).
+// Where the copy fits there at once: a large source is read from memory again tap by tap (43 x 304 x 131 x 131, 64 of 3x3 forward 664 us, 837
+// from a copy in nine parts; 118 x 64 x 131 x 131, 82 of 5x5 1048, 1090), and a 1x1 window reads it once anyway (6 x 64 x 105 x 105, 704 of
+// 1x1 41, 44). Where the copy's trip through memory is less than what it saves of the product, rows in whole blocks of 64: much of a product that
+// fetches single values, little of one that fetches pairs, and less the fewer the taps. And where enough room stays behind the copy
+// for the splits of a grid that needs them (24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, eight splits before and one behind 59 MB: 150 us, 244).
+// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3028 take the copy: 1.22 times as fast in the mean, 28 of them more than 5 %
+// slower; by the operations alone, half of every product saved, 3668 did, 142 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
+// 3x3 forward 44, 52; 27 x 347 x 78 x 78, 80 of 2x2 gated 115, 156).
 template <int MODE>
 static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const LoadPackedH& al, int K, int rows, int Cred,
-                         const LoadIm2colPix<MODE, false, bf16_t>& pix, StoreNCHW<bf16_t> ep, double flops, char* scratch, size_t scratch_bytes, bool* taken) {
+                         const LoadIm2colPix<MODE, false, bf16_t>& pix, bool pairs, StoreNCHW<bf16_t> ep, double flops, char* scratch, size_t scratch_bytes, bool* taken) {
     *taken = false;
     const int blocks = (Cred + KH - 1) / KH, RS = pix.R * pix.S, opix = pix.OH * pix.OW;
     const long pixels = (long)pix.nsamples * pix.Hs * pix.Ws, N = (long)pix.nsamples * opix;
     // (the loader's descriptor starts ahead of the copy by less than the filter's rows and columns of pixels)
     const size_t lead = ((size_t)(pix.R * pix.Ws + pix.S) * blocks * 64 + 255) / 256 * 256, copy_bytes = ((size_t)pixels * blocks * 64 + 255) / 256 * 256;
     const double us = 2.0 * ((rows + 63) / 64 * 64) * (double)N * Cred * RS / 350e6, copy_us = (double)pixels * Cred * 4 / 3.5e6 + 4.0;
-    if (RS == 1 || lead + copy_bytes > scratch_bytes || 0.5 * us <= copy_us) return VDNN_OK;
+    const double saved = pairs ? (RS >= 16 ? 0.25 : RS >= 9 ? 0.1 : 0.0) : RS >= 16 ? 0.65 : RS >= 9 ? 0.5 : 0.12;
+    if (RS == 1 || lead + copy_bytes > scratch_bytes || saved * us <= copy_us) return VDNN_OK;
+    const int TM = rows <= 64 ? 64 : 128, TN = rows <= 64 ? 256 : 128;
+    const size_t room = scratch_bytes - lead - copy_bytes;
+    if (3 * pixel_product_splits(rows, (int)N, K, TM, TN, KH, room, ctx->num_cu) < pixel_product_splits(rows, (int)N, K, TM, TN, KH, scratch_bytes, ctx->num_cu)) return VDNN_OK;
     *taken = true;
     unsigned short* copy = (unsigned short*)(scratch + lead);
     ep.partial = (float*)(scratch + lead + copy_bytes);
@@ -586,7 +594,7 @@ static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, 
     constexpr bool MIRROR = MODE == 1;
     const LoadPixStaged<MIRROR> bl{copy, pix.Hs, pix.Ws, pix.OH, pix.OW, pix.R, pix.S, MIRROR ? pix.R - 1 - pix.ph : pix.ph, MIRROR ? pix.S - 1 - pix.pw : pix.pw,
                                    MIRROR ? 1 : pix.sh, MIRROR ? 1 : pix.sw, blocks * KH, pix.nsamples, FastDiv::make(RS), FastDiv::make(pix.S)};
-    return launch_by_m<LoadPackedH, LoadPixStaged<MIRROR>, bf16_t, true>(ctx, st, names, al, bl, ep, rows, (int)N, K, flops, scratch_bytes - lead - copy_bytes);
+    return launch_by_m<LoadPackedH, LoadPixStaged<MIRROR>, bf16_t, true>(ctx, st, names, al, bl, ep, rows, (int)N, K, flops, room);
 }
 
 // forward / backward data of a bfloat16 layer on the bfloat16 matrix cores; MODE as in LoadIm2colPixTapH, PAD: Cred is no
@@ -608,7 +616,7 @@ static int conv_half_engine_with(vdnn_ctx* ctx, hipStream_t st, const PassNames&
         return launch_win3x3<MODE, bf16_t, PAD>(ctx, st, MODE == 0 ? kFwdWin3Names : kBwdDataWin3Names, al, geo, ep, rows, N, K, flops, left);
     }
     bool staged = false;
-    const int rcs = launch_staged<MODE>(ctx, st, names, al, K, rows, Cred, pix, ep, flops, (char*)ctx->reduce_scratch + taken, left, &staged);
+    const int rcs = launch_staged<MODE>(ctx, st, names, al, K, rows, Cred, pix, kernel == HalfKernel::PAIRS, ep, flops, (char*)ctx->reduce_scratch + taken, left, &staged);
     if (staged || rcs != VDNN_OK) return rcs;
     if (kernel == HalfKernel::PAIRS) {
         LoadIm2colPixTapH2<MODE, PAD> bl2{pix, Cred};
