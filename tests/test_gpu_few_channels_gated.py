@@ -20,7 +20,9 @@ GEOMS = [
     (4, 4, 21, 18, 24, 3, 0, 2),
     (1, 1, 9, 9, 7, 5, 2, 2),
     (2, 3, 20, 21, 8, 2, 0, 3),      # pixels between the windows
-    (40, 3, 64, 64, 70, 5, 2, 1),    # more products than the staging area holds at a time
+    (40, 3, 64, 64, 70, 5, 2, 1),
+    (75, 3, 64, 64, 70, 5, 2, 1),    # more products than the staging area holds at a time: 53 samples, then 22
+    (47, 4, 150, 150, 33, 7, 3, 2),  # ... of a strided layer: 14 samples three times, then 5
     (2, 3, 12, 12, 9, 1, 0, 2),      # one tap
 ]
 
@@ -43,9 +45,42 @@ def test_gated_backward_data(geom, bf16):
             check(lib.vdnn_ctx_set_activation_dtype(ctx.handle, 1))
         dtype, put, get = (np.uint16, to_bf16_bits, from_bf16_bits) if bf16 else (np.float32, lambda a: a, lambda a: a)
         dx_, df, ddy, gx = d.up(put(x), dtype), d.up(f), d.up(put(dy), dtype), d.up(put(np.full_like(x, 7)), dtype)
+        be.profile_enable(ctx.handle, True)
         announce("few channels, gated", geom, bf16)
         check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, ddy.ptr, df.ptr, dx_.ptr, gx.ptr, None, 0))
         got = get(gx.download(x.shape, dtype)).astype(np.float64)
+        gathers = be.profile_collect(ctx.handle).get("conv_bwd_data_gather", {"launches": 0})["launches"]
+    if n > 40 and (stride > 1 or not bf16):
+        assert gathers == -(-n // (66060288 // (c * r * r * p * q * 4)))  # chunks of what 63 MB hold
     assert np.all(got[x <= 0] == 0)
     error = np.linalg.norm(got - want) / np.linalg.norm(want)
     assert error <= (2.0 ** -9 if bf16 else 2.0 ** -24 * max(np.sqrt(k * r * r / 2), 2))
+
+
+# n, c, h, w, k, window, pad, stride; whether the products are formed once (a float layer)
+ROUTES = [(3, 3, 60, 60, 96, 11, 5, 1, True), (20, 4, 54, 54, 1, 11, 5, 1, False), (8, 3, 62, 62, 2, 7, 3, 1, False), (25, 4, 110, 110, 3, 2, 1, 1, False),
+          (23, 3, 88, 88, 64, 11, 0, 4, True), (87, 3, 40, 40, 12, 3, 0, 2, True)]
+
+
+@pytest.mark.parametrize("geom", ROUTES, ids=lambda g: "x".join(map(str, g)))
+def test_products_only_where_they_pay(geom):
+    """Few filters at stride 1 read little as one product of C rows: the products of all taps and the gather took up to eleven times as long."""
+    n, c, h, w, k, r, pad, stride, products = geom
+    p, q = (h + 2 * pad - r) // stride + 1, (w + 2 * pad - r) // stride + 1
+    g = be.shape(n, c, h, w, k, r, r, pad, pad, stride, stride)
+    with be.Context(pool_bytes=256 << 20) as ctx, Dev(ctx) as d:
+        x, f, dy, dx = (d.up(np.ones(s, np.float32)) for s in ((n, c, h, w), (k, c, r, r), (n, k, p, q), (n, c, h, w)))
+        be.profile_enable(ctx.handle, True)
+        announce("products or not", geom)
+        check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, dy.ptr, f.ptr, x.ptr, dx.ptr, None, 0))
+        assert ("conv_bwd_data_gather" in be.profile_collect(ctx.handle)) == products
+
+
+@pytest.mark.parametrize("k,row_kernel", [(2, False), (64, True)])
+def test_row_kernel_only_where_it_pays(k, row_kernel):
+    g = be.shape(40, 3, 80, 80, k, 3, 3, 1, 1)
+    with be.Context(pool_bytes=256 << 20) as ctx, Dev(ctx) as d:
+        x, f, dy, dx = (d.up(np.ones(s, np.float32)) for s in ((40, 3, 80, 80), (k, 3, 3, 3), (40, k, 80, 80), (40, 3, 80, 80)))
+        be.profile_enable(ctx.handle, True)
+        check(lib.vdnn_conv_bwd_data_relu(ctx.handle, None, g, 0, dy.ptr, f.ptr, x.ptr, dx.ptr, None, 0))
+        assert ("conv_bwd_data_smallc" in be.profile_collect(ctx.handle)) == row_kernel

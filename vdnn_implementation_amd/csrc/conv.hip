@@ -566,8 +566,8 @@ static const float* rounded_filter_copy(vdnn_ctx* ctx, hipStream_t st, StagingCa
 // 1x1 41, 44). Where the copy's trip through memory is less than what it saves of the product, rows in whole blocks of 64: much of a product that
 // fetches single values, little of one that fetches pairs, and less the fewer the taps. And where enough room stays behind the copy
 // for the splits of a grid that needs them (24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, eight splits before and one behind 59 MB: 150 us, 244).
-// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3028 take the copy: 1.22 times as fast in the mean, 28 of them more than 5 %
-// slower; by the operations alone, half of every product saved, 3668 did, 142 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
+// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3124 take the copy: 1.22 times as fast in the mean, 31 of them more than 5 %
+// slower; by the operations alone, half of every product saved, 3668 did, 188 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
 // 3x3 forward 44, 52; 27 x 347 x 78 x 78, 80 of 2x2 gated 115, 156).
 template <int MODE>
 static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const LoadPackedH& al, int K, int rows, int Cred,
@@ -1180,6 +1180,55 @@ static bool conv_bwd_data_in_place_ok(const ConvGeo& g) {
     return g.sh == 1 && g.sw == 1 && g.C > 4 && !is_dense(g);
 }
 
+// The row kernel of 3x3 layers of up to three channels (conv_smallc_mfma.h): about three workgroups per compute unit, strips of at least eight image rows
+struct RowStrips { int rows, strips, cblocks; };
+static RowStrips row_strips(const ConvGeo& g, int num_cu) {
+    RowStrips r;
+    r.cblocks = (g.W + BDS_EMIT - 1) / BDS_EMIT;
+    const long per_row = (long)g.N * r.cblocks;
+    r.strips = (int)((3l * num_cu + per_row - 1) / per_row);
+    r.rows = (g.H + r.strips - 1) / r.strips;
+    // a strip forms the products of two rows beyond its own, so eight or more of its own - unless that leaves units idle:
+    // then the walk down a strip is the kernel's whole time (4 x 3 x 20 x 20, 8 filters: 20.8 -> 10.1 us with strips of two rows)
+    const int fill = (int)((per_row * g.H + num_cu - 1) / num_cu);
+    const int least = fill >= 8 ? 8 : fill < 2 ? 2 : fill;
+    if (r.rows < least) r.rows = least;
+    if (r.rows > g.H) r.rows = g.H;
+    r.strips = (g.H + r.rows - 1) / r.rows;
+    return r;
+}
+
+// Samples whose products of all taps the staging area holds at a time (32-bit indexes in the kernel that gathers them)
+static int gather_samples(const vdnn_ctx* ctx, const ConvGeo& g) {
+    const long fit = (long)(ctx->reduce_scratch_bytes / ((size_t)g.C * g.R * g.S * g.P * g.Q * sizeof(float))), indexes = (1l << 31) / ((long)g.C * g.H * g.W);
+    const long n = fit < indexes ? fit : indexes;
+    return (int)(n < g.N ? n : g.N);
+}
+
+// Gated backward data of up to four input channels: whether the products of all taps once and a gather (rows3: the row kernel) are faster than the
+// product of C rows over every (filter, tap), which wastes 61 of a tile's 64 rows but reads little when there are few filters. Estimates in us, by
+// that product's own (one) and least squares over 5174 drawn calls of 1 to 256 filters of 2x2 to 11x11, strides 1 to 4, timed both ways; the gather waits
+// for the taps that reach a pixel one after the other, 0.3 us each. Of 1422 calls at stride 1, 524 take the products, 2.7 times as fast as the
+// product of C rows in the mean (one more than 5 % slower; 753 where all of them took the products); of 258 for the row kernel 55, 2.2 times (none;
+// 146); of 3494 strided ones 3200, 3.5 times (21; 175). The choice is 1.1 %, 2.1 % and 0.4 % behind the faster route. Up to eight filters at
+// stride 1 never gained: 87 x 3 x 190 x 190, 2 of 11x11 1054 us, 5875 by the products; 75 x 2 x 138 x 5, 4 of 3x3 11.7, 88.6 by the row kernel.
+static bool gated_products_pay(const vdnn_ctx* ctx, const ConvGeo& g, bool rows3) {
+    const int RS = g.R * g.S, PQ = g.P * g.Q;
+    const bool s1 = g.sh == 1 && g.sw == 1;
+    if (s1 && g.K <= 8) return false;
+    const double one = pixel_product_us(g.C, g.N * g.H * g.W, g.K * RS, ctx->reduce_scratch_bytes, ctx->num_cu, s1 ? 1.25 : 4.0, s1 ? 1.15 : 2.0);
+    const double one_us = s1 ? 1.8 + 0.785 * one : RS < 9 ? 4.0 + 0.24 * one : RS <= 32 ? 2.7 + 0.36 * one : 0.67 * one;
+    if (rows3) {
+        const RowStrips r = row_strips(g, ctx->num_cu);
+        const long rounds = ((long)g.N * r.strips * r.cblocks + 3l * ctx->num_cu - 1) / (3l * ctx->num_cu);
+        return 2.55 * (double)rounds * (r.rows + 2) < 0.8 * one_us;
+    }
+    const int nb = gather_samples(ctx, g), chunks = (g.N + nb - 1) / nb;
+    const double products = pixel_product_us(g.C * RS, nb * PQ, g.K, 0, ctx->num_cu, 1.25, 1.15) * g.N / nb;
+    const double reach = (double)((g.R + g.sh - 1) / g.sh) * ((g.S + g.sw - 1) / g.sw), mb = 4e-6 * g.N * (double)g.C * RS * PQ;
+    return 0.575 * products + 0.05 * mb + chunks * (5.3 + 0.3 * reach) < (s1 ? 0.9 : 1.0) * one_us;
+}
+
 template <class E>
 static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t* shape, int algo_mode,
                               const E* dy, const float* w, E* dx,
@@ -1209,7 +1258,8 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
                           ctx->reduce_scratch_bytes >= rounded_bytes + (size_t)g.C * g.R * g.S * g.P * g.Q * sizeof(float) &&
                           (!gate || !rounded_bytes || filter_bytes + (8u << 20) <= ctx->reduce_scratch_bytes) &&
                           pixel_tile_span_ok((long)g.K * g.P * g.Q, g.P * g.Q, 256, (int)sizeof(E));
-    const bool few_channels = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS && (!gate || (g.R * g.S > 1 && (sizeof(E) == 4 || g.sh > 1 || g.sw > 1) && (rows3 || products)));
+    const bool few_channels = g.C <= 4 && g.R * g.S <= SMALLC_MAXTAPS &&
+                              (!gate || (g.R * g.S > 1 && (sizeof(E) == 4 || g.sh > 1 || g.sw > 1) && (rows3 || products) && gated_products_pay(ctx, g, rows3)));
     if (!few_channels && (g.sh != 1 || g.sw != 1)) {
         bool taken = false;
         const int rc = launch_strided_bwd_data<E>(ctx, st, g, dy, w, dx, gate, &taken);
@@ -1232,9 +1282,7 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
             // staging area holds.
             const int RS = g.R * g.S, CRS = g.C * RS, PQ = g.P * g.Q;
             const size_t per_sample = (size_t)CRS * PQ * sizeof(float);
-            int nb = (int)(ctx->reduce_scratch_bytes / per_sample);
-            if (nb > g.N) nb = g.N;
-            if (nb > (1l << 31) / ((long)g.C * g.H * g.W)) nb = (int)((1l << 31) / ((long)g.C * g.H * g.W)); // (32-bit indexes in the second kernel)
+            const int nb = gather_samples(ctx, g);
             float* T = ctx->reduce_scratch;
             LoadFilterT alt{w, CRS, 1, (unsigned)((long)g.K * CRS * 4), FastDiv::make(1)};
             for (int n0 = 0; n0 < g.N; n0 += nb) {
@@ -1260,19 +1308,9 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
         const bool s1_3x3 = g.sh == 1 && g.sw == 1 && g.R == 3 && g.S == 3;
         // 3x3, padding 1, at most three input and 64 output channels: the products once, on the matrix cores, row by row
         if (rows3) {
-            // about three workgroups per compute unit, strips of at least eight image rows
-            const int cblocks = (g.W + BDS_EMIT - 1) / BDS_EMIT;
-            int strips = (int)((3l * ctx->num_cu + (long)g.N * cblocks - 1) / ((long)g.N * cblocks));
-            int rows = (g.H + strips - 1) / strips;
-            // a strip forms the products of two rows beyond its own, so eight or more of its own - unless that leaves units idle:
-            // then the walk down a strip is the kernel's whole time (4 x 3 x 20 x 20, 8 filters: 20.8 -> 10.1 us with strips of two rows)
-            const long per_row = (long)g.N * cblocks;
-            const int fill = (int)((per_row * g.H + ctx->num_cu - 1) / ctx->num_cu);
-            const int least = fill >= 8 ? 8 : fill < 2 ? 2 : fill;
-            if (rows < least) rows = least;
-            if (rows > g.H) rows = g.H;
-            strips = (g.H + rows - 1) / rows;
-            const dim3 grid((unsigned)(g.N * strips * cblocks));
+            const RowStrips strip = row_strips(g, ctx->num_cu);
+            const int rows = strip.rows;
+            const dim3 grid((unsigned)(g.N * strip.strips * strip.cblocks));
             if (g.C == 1) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<1, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);
             else if (g.C == 2) hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<2, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);
             else hipLaunchKernelGGL((conv_bwd_data_smallc3x3_mfma_kernel<3, E>), grid, dim3(256), 0, st, dy, w, dx, gate, g.N, g.K, g.H, g.W, rows);

@@ -53,11 +53,12 @@ static inline int pixel_product_splits(int M, int N, int K, int TM, int TN, int 
     if (cap > by_mem) cap = by_mem;
     return choose_splits(tiles, K, cap, num_cu, out_bytes, 2.0 * TM * TN * KB);
 }
-// ... and what the tile engine takes for it in the tile it would choose, the filter re-laid out tap-major
-static inline double pixel_product_us(int M, int N, int K, size_t partial_bytes, int num_cu) {
+// ... and what the tile engine takes for it in the tile it would choose (small_cost, large_cost: the loaders' work, LoadCost in conv.hip; 1: the
+// filter re-laid out tap-major)
+static inline double pixel_product_us(int M, int N, int K, size_t partial_bytes, int num_cu, double small_cost = 1.0, double large_cost = 1.0) {
     const int TM = M <= 64 ? 64 : 128, TN = M <= 64 ? 256 : 128;
-    const double small = small_tile_plan(M, N, K, partial_bytes, num_cu, 4, true, 1.0).us;
-    const double large = large_tile_us(M, N, K, TM, TN, pixel_product_splits(M, N, K, TM, TN, KB, partial_bytes, num_cu), num_cu, false, 1.0);
+    const double small = small_tile_plan(M, N, K, partial_bytes, num_cu, 4, true, small_cost).us;
+    const double large = large_tile_us(M, N, K, TM, TN, pixel_product_splits(M, N, K, TM, TN, KB, partial_bytes, num_cu), num_cu, false, large_cost);
     return K <= kShortReduction || small < 0.9 * large ? small : large;
 }
 
