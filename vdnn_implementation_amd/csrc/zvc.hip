@@ -41,9 +41,9 @@ static constexpr int kZvcPad = 8;           // elements of zero fill behind the 
 static constexpr int kZvcTeams = 4;
 static constexpr int kZvcThreads = 256 * kZvcTeams;
 // Workgroups per compute unit of zvc_pack_rows_kernel. One leaves the convolution beside it alone but takes twice as long by itself
-// (a pooling layer has no matrix work to hide it behind): a step of VGG16 at batch 128 in bfloat16 22.4 ms with one, 21.9 with two
-// and four, 21.8 with three, 22.0 with eight.
-static constexpr int kZvcPackPerCu = 3;
+// (a pooling layer has no matrix work to hide it behind); beyond two, a step gains nothing (six steps of VGG16 at batch 128 in bfloat16
+// 129.1 ms with two, 129.4 with three) and the kernel alone loses (400 MB of bfloat16 167 us with two, 182 with three and four, 186 with six).
+static constexpr int kZvcPackPerCu = 2;
 static constexpr int kZvcCursors = 64;      // cursors of a block
 
 __host__ __device__ inline size_t zvc_table_bytes(size_t chunks) { return (chunks * 4 + 15) / 16 * 16; }
@@ -89,11 +89,13 @@ struct ZvcReport {
 // a map word as well), a workgroup of four claims the place of its records together (a claim is an atomic on one word for the
 // whole device, 3.5 ns apiece), and every row of 64 elements leaves with one masked store of its kept elements, which lie one
 // behind the other. No element goes through LDS and a wavefront meets the others of its workgroup twice per chunk.
-// Alone it is bound by memory: 411 MB of floats, half of them zero, in 149 us (4.2 TB/s read and written; a large copy
-// reaches 4.7), of bfloat16 in 197 us (151 and 212 through LDS). In a training step it runs beside a convolution, and
+// Alone it is bound by memory on large tensors and by the chain load, claim, store on those of one or two trips. With its launch, half of the
+// elements zero, against a kernel through LDS with one launch before and one behind it: 400 MB of floats 132 -> 122 us, of bfloat16 194 ->
+// 167; 6 MB 11 -> 11; 50 MB 24 -> 29 and 31 -> 34 (that kernel had four wavefronts on a chunk). What does not fit the staging buffer goes to
+// the host in rows as well, at the link's rate: half of 27 MB 254 -> 259 us. In a training step it runs beside a convolution, and
 // what counts is the room it takes there: workgroups of sixteen wavefronts with 35 to 68 KB of LDS waited for a place
 // until the convolution's first round was over and ended behind it (64 channels of 112 x 112, batch 128, bfloat16: 715 us beside a
-// convolution of 536); this one starts at once, 53 (bfloat16) or 88 registers a wavefront, and takes 254 to 316 us there.
+// convolution of 536); this one starts at once, 52 (bfloat16) or 86 registers a wavefront, and takes 254 to 316 us there.
 template <class E>
 __global__ __launch_bounds__(256) void zvc_pack_rows_kernel(const E* __restrict__ src, size_t count, size_t chunks,
                                                             unsigned char* __restrict__ staging, size_t staging_bytes,
@@ -127,16 +129,21 @@ __global__ __launch_bounds__(256) void zvc_pack_rows_kernel(const E* __restrict_
             }
         }
         auto element = [&](int b, int j) -> E { return E(q[b][j * int(sizeof(E)) / 4] >> (j * int(sizeof(E)) % 4 * 8)); };
-        unsigned long long word = 0;   // word `lane` of the map
+        unsigned word_lo = 0, word_hi = 0;   // word `lane` of the map
         unsigned kept = 0;
 #pragma unroll
         for (int b = 0; b < kBlocks; ++b)
 #pragma unroll
             for (int j = 0; j < V; ++j) {
                 const unsigned long long m = __ballot(element(b, j) != 0);
-                word = lane == b * V + j ? m : word;
+                // lane b V + j = m (two wait states after the comparison that wrote the mask)
+                asm("s_nop 1\n\tv_writelane_b32 %0, %2, %4\n\tv_writelane_b32 %1, %3, %4" : "+v"(word_lo), "+v"(word_hi) : "s"(unsigned(m)), "s"(unsigned(m >> 32)), "n"(b * V + j));
                 kept += __popcll(m);
             }
+        const unsigned long long word = (unsigned long long)word_hi << 32 | word_lo;
+        // (the stores below compare again: the masks of 64 rows kept from here would not fit the scalar registers)
+#pragma unroll
+        for (int b = 0; b < kBlocks; ++b) asm volatile("" : "+v"(q[b]));
         const unsigned bytes = live ? kZvcMapBytes + (kept * unsigned(sizeof(E)) + 15u) / 16u * 16u : 0u;
         if (lane == 0) wave_bytes[wave] = bytes;
         __syncthreads();
