@@ -128,8 +128,9 @@ __global__ void __launch_bounds__(256) conv_bwd_data_smallc_strided_kernel(const
 // Second stage of the few-channel backward data on the matrix cores. The first stage is a 1x1
 // convolution T[n][(c,r,s)][p][q] = sum_k w[k,c,r,s] * dy[n,k,p,q] (every product the layer needs, once);
 // here an input pixel adds up the entries whose tap lands on it: dx[n,c,h,x] = sum over taps (r,s) with
-// (h+ph-r) = p*sh and (x+pw-s) = q*sw of T[n][(c,r,s)][p][q], taps in ascending (r,s) order. Bound by T's trip through memory; a launch
-// covers no more elements than the staging area holds (2^24), so that 32-bit indexes and divisions do. gate: optional, laid out as dx.
+// (h+ph-r) = p*sh and (x+pw-s) = q*sw of T[n][(c,r,s)][p][q], taps in ascending (r,s) order. Bound by T's trip through memory. The
+// staging area bounds T alone, and dx is the larger one where the stride exceeds the window: the caller takes no more samples a launch than leave
+// total, dx's elements, at most 2^31 (gather_samples), so that 32-bit indexes and divisions do. gate: optional, laid out as dx.
 template <class E>
 __global__ void __launch_bounds__(256) conv_bwd_data_gather_taps_kernel(const float* __restrict__ T, E* __restrict__ dx, const E* __restrict__ gate, const ConvGeo g, unsigned total) {
     const unsigned i = blockIdx.x * 256 + threadIdx.x;

@@ -2,12 +2,13 @@
 //
 // One workgroup of 256 threads (4 wavefronts of 64) produces a TM x TN tile of
 //     Out[m][j] = sum_kk A[m][kk] * B[kk][j]
-// from KB-deep slices staged in LDS. Each wavefront owns a 64x64 sub-tile = 2x2 MFMA tiles of
-// v_mfma_f32_32x32x2_f32 (64 accumulator registers per lane). Operands come from "loader" policies:
+// from KB-deep slices staged in LDS. In the large tiles (igemm_tile) each wavefront owns a 64x64 sub-tile = 2x2 MFMA tiles of
+// v_mfma_f32_32x32x2_f32 (64 accumulator registers per lane), in the 64x64 tile (igemm_small_tile) one MFMA tile. Operands come from "loader" policies:
 // a loader says how element (row, kk) of its operand is fetched from global memory (a dense matrix,
 // a filter bank, or an im2col view of an NCHW tensor computed on the fly - the im2col matrix only
-// ever exists as LDS tiles). Global loads run two slices ahead in registers, LDS is double-buffered,
-// and the loop has one barrier per slice and no branch (see igemm_kernel).
+// ever exists as LDS tiles). Global loads run AHEAD slices ahead in registers beside the one in
+// LDS (one, two or four), LDS is double-buffered, and the loop has one barrier per slice and no branch but, with AHEAD > 1, those of
+// the slices that are left behind whole rounds of AHEAD.
 //
 // The matrix pipe and the vector ALU of a SIMD do not overlap well, so every vector instruction in
 // the loop costs MFMA time. The loaders therefore fetch through buffer descriptors: an element that
@@ -510,7 +511,7 @@ __device__ __forceinline__ bool sum_splits(floatx16& acc, float* staging, const 
 // - What the result is combined with (bias, gate, old values) is read before the loop, and the epilogue branches on what is
 //   uniform only, once per tile: 2.7 -> 0.9 us.
 // One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
-// four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 102.7.
+// four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 104.6.
 template <int AHEAD, bool SUMS, class AL, class BL, class EP>
 __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, const EP& ep, const GemmDims& d, int block, int blocks) {
     constexpr int T = 64;
@@ -619,7 +620,10 @@ __device__ __forceinline__ void igemm_small_tile(const AL& al, const BL& bl, con
 }
 // Slices ahead: four where the shortest reduction of a workgroup is long enough for them
 constexpr int kSmallTileAhead = 4;
-constexpr long kSmallTileLone = 1024; // workgroups: four on each of 256 compute units, what the registers of that variant leave room for
+// Workgroups up to which they are: four on each unit is what that variant's registers leave room for. (256 units, the target part: callers that plan
+// have no context at hand.) 4294 drawn float calls below the line, timed with four and with one: four are 1.2 % faster in the mean, more than 5 % in 473
+// and slower in 29; up to 2048 workgroups 1.1 % (68, 12), beyond nothing (59, 38).
+constexpr long kSmallTileLone = 1024;
 static inline bool small_tile_ahead(const GemmDims& d, long blocks) { return d.kchunk >= (kSmallTileAhead + 2) * KB && blocks <= kSmallTileLone; }
 // ... and where the loader's address work does not count for more than the latency (LoadIm2colPix<2>: two divisions per element)
 template <class L> struct FetchesAhead { static constexpr bool V = true; };

@@ -107,7 +107,7 @@ def from_rocprof(directory):
     out = []
     for k in kernels:
         a, b = int(k["Start_Timestamp"]), int(k["End_Timestamp"])
-        if b <= t0 or a >= t1 or "zvc_pack" in k["Kernel_Name"] or "zvc_begin" in k["Kernel_Name"] or "zvc_end" in k["Kernel_Name"]:
+        if b <= t0 or a >= t1 or "zvc_pack" in k["Kernel_Name"]:
             continue
         out.append(("compute", a, b))
     moved = {"d2h": 0, "h2d": 0}
