@@ -256,8 +256,10 @@ static bool pad_pays(int channels, int M, long N, int RS, double least_ops) {
     return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels && 2.0 * ((M + 63) / 64 * 64) * (double)N * channels * RS >= least_ops;
 }
 // A filter re-laid-out for the tap-major loaders costs a launch and saves three of four loads of it; small layers read it as it lies (19 x 32 x 7 x 7, 13
-// filters of 3x3 forward 11.1 -> 8.9 us; 2 x 16 x 53 x 53, 80 of 3x3, 1.3e8 operations, 9.8 -> 9.1; 15 x 16 x 17 x 17, 176 of 5x5, 3.6e8, 14.9 -> 19.4).
-constexpr double kPackOps = 1.5e8;
+// filters of 3x3 forward 11.1 -> 8.9 us; 15 x 16 x 17 x 17, 176 of 5x5, 3.6e8 operations, re-laid-out 14.9, else 19.4). The line is where the two break even
+// over 5000 drawn calls timed both ways: between 2e8 and 3e8 operations as it lies is 1.2 % faster in forward and 5.5 % in backward data, between 3e8 and 4e8
+// 1.2 % slower and level, from there on up to 19 % slower.
+constexpr double kPackOps = 3e8;
 static bool pack_pays(double ops) { return ops >= kPackOps; }
 constexpr double kPadFwdOps = 1.5e9, kPadBwdDataOps = 4e8;
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
