@@ -256,11 +256,11 @@ static bool pad_pays(int channels, int M, long N, int RS, double least_ops) {
     return 4 * ((channels + KB - 1) / KB * KB) <= 5 * channels && 2.0 * ((M + 63) / 64 * 64) * (double)N * channels * RS >= least_ops;
 }
 // A filter re-laid-out for the tap-major loaders costs a launch and saves three of four loads of it; small layers read it as it lies (19 x 32 x 7 x 7, 13
-// filters of 3x3 forward 11.1 -> 8.9 us; 15 x 16 x 17 x 17, 176 of 5x5, 3.6e8 operations, re-laid-out 14.9, else 19.4). The line is where the two break even
-// over 5000 drawn calls timed both ways: between 2e8 and 3e8 operations as it lies is 1.2 % faster in forward and 5.5 % in backward data, between 3e8 and 4e8
-// 1.2 % slower and level, from there on up to 19 % slower.
-constexpr double kPackOps = 3e8;
-static bool pack_pays(double ops) { return ops >= kPackOps; }
+// filters of 3x3 forward 11.1 -> 8.9 us; 15 x 16 x 17 x 17, 176 of 5x5, 3.6e8 operations, re-laid-out 14.9, else 19.4). As it lies, the elements of a tap are
+// a window apart, so that the line falls with the taps. Over 5727 drawn calls timed both ways, windows of 2x2 to 5x5, the choice is 0.3 % behind the better
+// way in the mean and 5 % in 44 (one line for all windows at 3e8 operations: 0.6 %, 145).
+constexpr double kPackOps = 4e9;
+static bool pack_pays(double ops, int taps) { return ops * taps >= kPackOps; }
 constexpr double kPadFwdOps = 1.5e9, kPadBwdDataOps = 4e8;
 static bool packed_fwd_ok(const ConvGeo& g) { return g.R * g.S <= 32 && g.C % KB == 0; }
 static bool packed_bwd_data_ok(const ConvGeo& g) {
@@ -1156,7 +1156,7 @@ static int conv_fwd_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_shape_t
             LoadDenseRed<true> al{w, (long)K, g.K, wbytes};
             return launch_by_m(ctx, st, in_workspace ? kFwdPackedNames : kFwdNames, al, bl, ep, g.K, g.N * g.P * g.Q, K);
         }
-        float* packed = pack_pays(2.0 * g.K * (double)g.N * g.P * g.Q * K) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr;
+        float* packed = pack_pays(2.0 * g.K * (double)g.N * g.P * g.Q * K, RS) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr;
         StoreNCHW<E> ep{y, bias, g.P * g.Q, ctx->reduce_scratch, relu, nullptr};
         if (packed) {
             const int rc = launch_pack_filter(ctx, st, w, packed, g.K, g.C, RS, g.C * RS, RS);
@@ -1375,7 +1375,7 @@ static int conv_bwd_data_impl(vdnn_ctx* ctx, vdnn_stream_t stream, const vdnn_sh
                 LoadDenseRow<float> alr{w, (long)g.C, g.C, wbytes};
                 return launch_by_m(ctx, st, in_workspace ? kBwdDataPackedNames : kBwdDataNames, alr, bl, ep, M, N, K, flops);
             }
-            float* packed = pack_pays(2.0 * M * (double)N * K) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr; // [c][(kb*RS + tap)*16 + l]
+            float* packed = pack_pays(2.0 * M * (double)N * K, RS) ? (in_workspace ? (float*)workspace : packed_filter_place(ctx, carve, wbytes)) : nullptr; // [c][(kb*RS + tap)*16 + l]
             if (packed) {
                 ep.partial = ctx->reduce_scratch; // (behind the filter bank, if that lies in the staging area)
                 const int rc = launch_pack_filter(ctx, st, w, packed, g.C, g.K, RS, RS, g.C * RS);
