@@ -60,6 +60,7 @@ def test_against_oracle(geom, staged):
 ROUTES = [((12, 96, 27, 27, 130, 5, 2, 1), True), ((24, 608, 45, 45, 80, 5, 2, 2), False),  # (no room left for eight splits)
           ((2, 255, 120, 218, 3, 3, 0, 1), False),   # pairs of pixels, nine taps
           ((20, 96, 40, 40, 192, 5, 2, 1), True),    # pairs, twenty-five taps
+          ((123, 16, 38, 38, 16, 5, 2, 1), True),    # pairs; sixteen channels are multiplied as a block of thirty-two
           ((5, 202, 143, 143, 112, 2, 1, 1), False)]  # four taps
 
 

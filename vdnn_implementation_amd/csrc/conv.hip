@@ -565,12 +565,14 @@ static const float* rounded_filter_copy(vdnn_ctx* ctx, hipStream_t st, StagingCa
 // Forward (MODE 0) and backward data at stride 1 (MODE 1) from a copy of the source in `scratch` (conv_staged.h). al: the filter bank; K: its row.
 // Where the copy fits there at once: a large source is read from memory again tap by tap (43 x 304 x 131 x 131, 64 of 3x3 forward 664 us, 837
 // from a copy in nine parts; 118 x 64 x 131 x 131, 82 of 5x5 1048, 1090), and a 1x1 window reads it once anyway (6 x 64 x 105 x 105, 704 of
-// 1x1 41, 44). Where the copy's trip through memory is less than what it saves of the product, rows in whole blocks of 64: much of a product that
-// fetches single values, little of one that fetches pairs, and less the fewer the taps. And where enough room stays behind the copy
-// for the splits of a grid that needs them (24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, eight splits before and one behind 59 MB: 150 us, 244).
-// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3124 take the copy: 1.22 times as fast in the mean, 31 of them more than 5 %
-// slower; by the operations alone, half of every product saved, 3668 did, 188 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
-// 3x3 forward 44, 52; 27 x 347 x 78 x 78, 80 of 2x2 gated 115, 156).
+// 1x1 41, 44). Where the copy's trip through memory is less than what it saves of the product, rows in whole blocks of 64 and channels in
+// whole blocks of 32, as both ways multiply them: much of a product that fetches single values, little of one that fetches pairs, and less the
+// fewer the taps. And where the room behind the copy leaves a fifth of the splits of a grid that needs them (with a half to a fifth still 1.2 to
+// 1.5 times as fast; 24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, eight splits before and one behind 59 MB: 150 us, 244).
+// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3704 take the copy: 1.2 times as fast in the mean, 63 of them more than 5 %
+// slower. By the operations alone, half of every product saved, 3668 did, 188 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
+// 3x3 forward 44, 52; 27 x 347 x 78 x 78, 80 of 2x2 gated 115, 156); with a part block of channels counted as it is stored, calls that gain were left
+// (93 x 16 x 38 x 38, 16 of 5x5 backward data 36, 50 without).
 template <int MODE>
 static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, const LoadPackedH& al, int K, int rows, int Cred,
                          const LoadIm2colPix<MODE, false, bf16_t>& pix, bool pairs, StoreNCHW<bf16_t> ep, double flops, char* scratch, size_t scratch_bytes, bool* taken) {
@@ -579,12 +581,12 @@ static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, 
     const long pixels = (long)pix.nsamples * pix.Hs * pix.Ws, N = (long)pix.nsamples * opix;
     // (the loader's descriptor starts ahead of the copy by less than the filter's rows and columns of pixels)
     const size_t lead = ((size_t)(pix.R * pix.Ws + pix.S) * blocks * 64 + 255) / 256 * 256, copy_bytes = ((size_t)pixels * blocks * 64 + 255) / 256 * 256;
-    const double us = 2.0 * ((rows + 63) / 64 * 64) * (double)N * Cred * RS / 350e6, copy_us = (double)pixels * Cred * 4 / 3.5e6 + 4.0;
-    const double saved = pairs ? (RS >= 16 ? 0.25 : RS >= 9 ? 0.1 : 0.0) : RS >= 16 ? 0.65 : RS >= 9 ? 0.5 : 0.12;
+    const double us = 2.0 * ((rows + 63) / 64 * 64) * (double)N * (blocks * KH) * RS / 350e6, copy_us = (double)pixels * (Cred + blocks * KH) * 2 / 3.5e6 + 4.0;
+    const double saved = pairs ? (RS >= 16 ? 0.35 : RS >= 9 ? 0.1 : 0.0) : RS >= 16 ? 0.65 : RS >= 9 ? 0.5 : 0.2;
     if (RS == 1 || lead + copy_bytes > scratch_bytes || saved * us <= copy_us) return VDNN_OK;
     const int TM = rows <= 64 ? 64 : 128, TN = rows <= 64 ? 256 : 128;
     const size_t room = scratch_bytes - lead - copy_bytes;
-    if (3 * pixel_product_splits(rows, (int)N, K, TM, TN, KH, room, ctx->num_cu) < pixel_product_splits(rows, (int)N, K, TM, TN, KH, scratch_bytes, ctx->num_cu)) return VDNN_OK;
+    if (5 * pixel_product_splits(rows, (int)N, K, TM, TN, KH, room, ctx->num_cu) < pixel_product_splits(rows, (int)N, K, TM, TN, KH, scratch_bytes, ctx->num_cu)) return VDNN_OK;
     *taken = true;
     unsigned short* copy = (unsigned short*)(scratch + lead);
     ep.partial = (float*)(scratch + lead + copy_bytes);
