@@ -368,7 +368,7 @@ struct StoreNCHW {
     int relu;          // rectify the result (after the bias)
     const E* gate;     // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
     static constexpr bool TAIL = true;
-    // The gate or the bias (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; columns past the end, and
+    // The gate, as it lies (load_raw), or the bias (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; columns past the end, and
     // rows past it in the eight that begins inside, read some element inside, other rows past it are not read. (A gate that is the
     // output tensor - the gradient written over the layer's own input - is read by the lane that overwrites it, before it does.)
     __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
@@ -381,7 +381,7 @@ struct StoreNCHW {
             for (int q = 0; q < 4; q++) {
                 if (rows_behind(m0, q, d.M)) break;
 #pragma unroll
-                for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_elem(from + (size_t)min(m0 + result_row(v, lk), d.M - 1) * opix);
+                for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_raw(from + (size_t)min(m0 + result_row(v, lk), d.M - 1) * opix);
             }
         } else if (bias) {
 #pragma unroll
@@ -411,7 +411,7 @@ struct StoreNCHW {
         }
         if (gate) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[v] = aux[v] > 0.0f ? acc[v] : 0.0f;
+            for (int v = 0; v < 16; v++) acc[v] = raw_value<E>(aux[v]) > 0.0f ? acc[v] : 0.0f;
         }
         store_rows(out + first, acc, opix, m0, lk, d.M);
     }

@@ -764,6 +764,19 @@ struct RoundedToBf16 : L {
 // The first of the eight rows from which a lane's registers 4 q .. 4 q + 3 are, past the last row or not; the same for the whole wavefront.
 __device__ __forceinline__ bool rows_behind(int m0, int q, int M) { return __builtin_amdgcn_readfirstlane(m0) + 8 * q >= M; }
 
+// An element as it lies in memory, in a float's place, and its value. What a block is combined with is read behind a branch for each eight of its
+// rows: with the conversion of a two-byte element in there every branch waits for its loads (7 x 160 x 170 x 170, 32 of 1x1
+// gated backward data in bfloat16 45 us, 59 so; 334 of 3290 drawn gated calls more than 5 % slower).
+__device__ __forceinline__ float load_raw(const float* p) { return *p; }
+__device__ __forceinline__ float load_raw(const bf16_t* p) { return __builtin_bit_cast(float, (unsigned)p->bits); }
+template <class E>
+__device__ __forceinline__ float raw_value(float raw) {
+    if constexpr (sizeof(E) == 2) {
+        asm("" : "+v"(raw)); // (the compiler would move the conversion up to the load)
+        return bf16_bits_to_float(__builtin_bit_cast(unsigned, raw));
+    } else return raw;
+}
+
 // A lane's sixteen results of a 32x32 block, `to` at row m0 + 4 lk, rows from M on left out. The test per row is for the blocks at the
 // lower edge only, and there for the rows of the eights that begin inside: with a branch on each of a tile's 64 rows, and one each on bias,
 // gate and rectifier, a tile's epilogue took 2.7 us per 32x32 block of a wavefront, most of it the fetch of its text. Forward 9 x 448 x 189 x 189, 576 of 1x1 in bfloat16 631 -> 418 us; 29 x 32 x 30 x 30, 289
@@ -797,7 +810,7 @@ struct StoreDense {
     int accumulate;
     int relu;      // rectify the result (after the bias)
     const E* gate; // optional, same layout as out: the result is kept where gate > 0 and zero elsewhere
-    // The old values or the gate (a call asks for one of the two at most) of a lane's sixteen results of a 32x32 block; columns past the
+    // The old values or the gate, as they lie (load_raw; a call asks for one of the two at most), of a lane's sixteen results of a 32x32 block; columns past the
     // end, and rows past it in the eight that begins inside, read some element inside. What else is past it is not read (nor stored).
     __device__ __forceinline__ void read_aux(float (&aux)[16], int m0, int j0, int lane, const GemmDims& d, bool to_partial) const {
         if (to_partial || !(accumulate || gate)) return;
@@ -807,7 +820,7 @@ struct StoreDense {
         for (int q = 0; q < 4; q++) {
             if (rows_behind(m0, q, d.M)) break;
 #pragma unroll
-            for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_elem(from + (long)min(m0 + result_row(v, lk), d.M - 1) * ld_m + j);
+            for (int v = 4 * q; v < 4 * q + 4; v++) aux[v] = load_raw(from + (long)min(m0 + result_row(v, lk), d.M - 1) * ld_m + j);
         }
     }
     __device__ __forceinline__ void store32(floatx16 acc, const float (&aux)[16], int m0, int j0, int lane, int ks, const GemmDims& d, bool to_partial) const {
@@ -818,8 +831,15 @@ struct StoreDense {
             store_rows(partial + (long)ks * partial_stride + first, acc, ld_m, m0, lk, d.M);
             return;
         }
+        float with[16]; // (converted behind one branch, not one for each row)
 #pragma unroll
-        for (int v = 0; v < 16; v++) acc[v] = accumulate ? __fmaf_rn(alpha, acc[v], aux[v]) : alpha * acc[v];
+        for (int v = 0; v < 16; v++) with[v] = aux[v];
+        if (sizeof(E) == 2 && (accumulate || gate)) {
+#pragma unroll
+            for (int v = 0; v < 16; v++) with[v] = raw_value<E>(aux[v]);
+        }
+#pragma unroll
+        for (int v = 0; v < 16; v++) acc[v] = accumulate ? __fmaf_rn(alpha, acc[v], with[v]) : alpha * acc[v];
         if (bias_j) {
             const float bj = bias_j[j];
 #pragma unroll
@@ -831,7 +851,7 @@ struct StoreDense {
         }
         if (gate) {
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[v] = aux[v] > 0.0f ? acc[v] : 0.0f;
+            for (int v = 0; v < 16; v++) acc[v] = with[v] > 0.0f ? acc[v] : 0.0f;
         }
         store_rows(out + first, acc, ld_m, m0, lk, d.M);
     }
