@@ -176,3 +176,35 @@ def test_many_offloads_in_flight_on_two_streams(ctx, staged):
         for _, _, host, _, _, _, word in todo:
             host.free()
             word.free()
+
+
+def test_captured_offloads_of_a_context_that_has_no_cursors_left():
+    """A hundred packing kernels recorded into one graph, the context's first call among them: cursors come in blocks of 64, so memory is taken
+    while a stream is captured. Replayed several times with calls outside the graph in between."""
+    rng = np.random.default_rng(6)
+    tensors = [tensor(rng, int(rng.integers(1, 20000)), np.uint32, 0.5) for _ in range(100)]
+    recording, other = other_streams(2)
+    with be.Context(pool_bytes=512 << 20) as ctx, Dev(ctx) as d:
+        sources = [d.up(t, t.dtype) for t in tensors]
+        hosts = [Pinned(ctx, lib.vdnn_zvc_buffer_bytes(t.size, t.itemsize)) for t in tensors]
+        call = lambda i, s: check(lib.vdnn_zvc_offload_async(ctx.handle, hosts[i].ptr, sources[i].ptr, tensors[i].size, tensors[i].itemsize, s))
+        ctx.synchronize()
+        torch.cuda.synchronize()
+        announce("captured offloads")
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=recording):
+            for i in range(len(tensors)):
+                call(i, recording.cuda_stream)
+        for _ in range(4):
+            for host in hosts:
+                host.view[:] = 0xAB
+            with torch.cuda.stream(other):
+                graph.replay()
+            torch.cuda.synchronize()
+            for t, host in zip(tensors, hosts):
+                assert np.array_equal(decode(host.view, t.size, t.dtype)[0], t)
+            call(0, None)
+            ctx.synchronize()
+            assert np.array_equal(decode(hosts[0].view, tensors[0].size, tensors[0].dtype)[0], tensors[0])
+        for host in hosts:
+            host.free()

@@ -24,20 +24,24 @@ bool stream_is_captured(hipStream_t stream) {
     return status != hipStreamCaptureStatusNone;
 }
 
-// Cleared on a stream of the context and waited for: the context's streams do not wait for the default one, and clearing returns
-// before it is done.
-void* zeroed_device_memory(vdnn_ctx* ctx, size_t bytes) {
+// Cleared on a stream of its own and waited for: the context's streams do not wait for the default one, clearing returns before it is done,
+// and any other stream may be the one a caller is capturing. Allocating is refused beside a capture unless the thread says that it
+// does not belong to it.
+void* zeroed_device_memory(size_t bytes) {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
     void* p = nullptr;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return nullptr;
-    }
-    if (hipMemsetAsync(p, 0, bytes, ctx->pack) != hipSuccess || hipStreamSynchronize(ctx->pack) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipFree(p);
-        return nullptr;
-    }
-    return p;
+    hipStream_t stream = nullptr;
+    bool ok = hipMalloc(&p, bytes) == hipSuccess && hipStreamCreateWithFlags(&stream, hipStreamNonBlocking) == hipSuccess &&
+              hipMemsetAsync(p, 0, bytes, stream) == hipSuccess && hipStreamSynchronize(stream) == hipSuccess;
+    if (!ok) (void)hipGetLastError();
+    if (stream) (void)hipStreamDestroy(stream);
+    if (!ok && p) (void)hipFree(p);
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return ok ? p : nullptr;
 }
 
 unsigned* tile_counters_of(vdnn_ctx* ctx, hipStream_t stream) {
@@ -96,7 +100,7 @@ int vdnn_ctx_create(vdnn_ctx** out, int device, int flags) {
             return VDNN_EDEVICE;
         }
         // (split reductions are added up by a second kernel where there are no counters)
-        ctx->tile_counters = (unsigned*)zeroed_device_memory(ctx, sizeof(unsigned) * kTileCounters * kTileCounterSets);
+        ctx->tile_counters = (unsigned*)zeroed_device_memory(sizeof(unsigned) * kTileCounters * kTileCounterSets);
         if (noalloc_prepare_current_device() != VDNN_OK) {
             vdnn_ctx_destroy(ctx);
             return VDNN_EDEVICE;

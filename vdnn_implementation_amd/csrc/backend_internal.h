@@ -60,8 +60,8 @@ inline hipStream_t stream_of(vdnn_ctx* ctx, vdnn_stream_t s) { return s ? (hipSt
 
 // whether launches on the stream are being recorded into a graph (which may then run on any stream)
 bool stream_is_captured(hipStream_t stream);
-// `bytes` of device memory, zero before the call returns; null (and no error left behind) where there is none
-void* zeroed_device_memory(vdnn_ctx* ctx, size_t bytes);
+// `bytes` of device memory, zero before the call returns, also while streams are captured; null (and no error left behind) where there is none
+void* zeroed_device_memory(size_t bytes);
 // the counters of a stream's launches; null while it is captured, and for streams beyond the first kTileCounterSets
 unsigned* tile_counters_of(vdnn_ctx* ctx, hipStream_t stream);
 

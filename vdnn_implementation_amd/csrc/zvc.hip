@@ -350,7 +350,7 @@ __global__ __launch_bounds__(kZvcThreads) void zvc_unpack_kernel(const unsigned 
 }
 
 static int zvc_ensure_counters(vdnn_ctx* ctx) {
-    if (!ctx->zvc_counters) ctx->zvc_counters = (unsigned long long*)zeroed_device_memory(ctx, sizeof(unsigned long long));
+    if (!ctx->zvc_counters) ctx->zvc_counters = (unsigned long long*)zeroed_device_memory(sizeof(unsigned long long));
     if (!ctx->zvc_counters) { set_error("no device memory for the offload's counter"); return VDNN_EDEVICE; }
     return VDNN_OK;
 }
@@ -364,7 +364,7 @@ static ZvcCursor* zvc_cursor(vdnn_ctx* ctx, hipStream_t stream) {
     size_t i = captured ? owners.size() : size_t(std::find(owners.begin(), owners.end(), stream) - owners.begin());
     if (i == owners.size()) {
         if (i == ctx->zvc_cursor_blocks.size() * kZvcCursors) {
-            void* block = zeroed_device_memory(ctx, sizeof(ZvcCursor) * kZvcCursors);
+            void* block = zeroed_device_memory(sizeof(ZvcCursor) * kZvcCursors);
             if (!block) return nullptr;
             ctx->zvc_cursor_blocks.push_back(block);
         }
