@@ -57,7 +57,8 @@ def test_against_oracle(geom, staged):
 
 
 # n, c, h, w, k, window, pad, stride; whether forward takes the copy
-ROUTES = [((12, 96, 27, 27, 130, 5, 2, 1), True), ((24, 608, 45, 45, 80, 5, 2, 2), False),  # (no room left for eight splits)
+ROUTES = [((12, 96, 27, 27, 130, 5, 2, 1), True), ((24, 608, 45, 45, 80, 5, 2, 2), False),  # (one of five splits left)
+          ((34, 111, 160, 45, 5, 5, 0, 2), True),    # two of seven splits left, whose rounds take as long
           ((2, 255, 120, 218, 3, 3, 0, 1), False),   # pairs of pixels, nine taps
           ((20, 96, 40, 40, 192, 5, 2, 1), True),    # pairs, twenty-five taps
           ((123, 16, 38, 38, 16, 5, 2, 1), True),    # pairs; sixteen channels are multiplied as a block of thirty-two

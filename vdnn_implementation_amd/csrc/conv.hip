@@ -567,10 +567,12 @@ static const float* rounded_filter_copy(vdnn_ctx* ctx, hipStream_t st, StagingCa
 // from a copy in nine parts; 118 x 64 x 131 x 131, 82 of 5x5 1048, 1090), and a 1x1 window reads it once anyway (6 x 64 x 105 x 105, 704 of
 // 1x1 41, 44). Where the copy's trip through memory is less than what it saves of the product, rows in whole blocks of 64 and channels in
 // whole blocks of 32, as both ways multiply them: much of a product that fetches single values, little of one that fetches pairs, and less the
-// fewer the taps. And where the room behind the copy leaves a fifth of the splits of a grid that needs them (with a half to a fifth still 1.2 to
-// 1.5 times as fast; 24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, eight splits before and one behind 59 MB: 150 us, 244).
-// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3704 take the copy: 1.2 times as fast in the mean, 63 of them more than 5 %
-// slower. By the operations alone, half of every product saved, 3668 did, 188 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
+// fewer the taps. And where the splits that the room behind the copy leaves take at most twice the rounds' time of those there would be
+// without it (24 x 608 x 45 x 45, 80 of 5x5 at stride 2 forward, a hundred tiles, five splits before and one behind 59 MB: 137 us, 242). Of 260 drawn calls
+// with less than half of their splits left, timed both ways, 222 take the copy: 1.1 % behind the faster way in the mean, 18 calls by more than 5 %,
+// at most 1.3 times its time (by a fifth of the splits 1.4 %, 20, 1.8 times; by a third 5.5 %, 50, 1.9 times).
+// Of 9494 drawn calls of 2x2 to 7x7 whose copy fits, timed both ways, 3704 took the copy by a fifth of the splits: 1.2 times as fast in the mean, 63 of
+// them more than 5 % slower. By the operations alone, half of every product saved, 3668 did, 188 of them slower, by up to 1.8 times (2 x 255 x 120 x 218, 3 of
 // 3x3 forward 44, 52; 27 x 347 x 78 x 78, 80 of 2x2 gated 115, 156); with a part block of channels counted as it is stored, calls that gain were left
 // (93 x 16 x 38 x 38, 16 of 5x5 backward data 36, 50 without).
 template <int MODE>
@@ -586,7 +588,9 @@ static int launch_staged(vdnn_ctx* ctx, hipStream_t st, const PassNames& names, 
     if (RS == 1 || lead + copy_bytes > scratch_bytes || saved * us <= copy_us) return VDNN_OK;
     const int TM = rows <= 64 ? 64 : 128, TN = rows <= 64 ? 256 : 128;
     const size_t room = scratch_bytes - lead - copy_bytes;
-    if (5 * pixel_product_splits(rows, (int)N, K, TM, TN, KH, room, ctx->num_cu) < pixel_product_splits(rows, (int)N, K, TM, TN, KH, scratch_bytes, ctx->num_cu)) return VDNN_OK;
+    const long tiles = (long)((rows + TM - 1) / TM) * ((N + TN - 1) / TN);
+    const int whole = pixel_product_splits(rows, (int)N, K, TM, TN, KH, scratch_bytes, ctx->num_cu), behind = pixel_product_splits(rows, (int)N, K, TM, TN, KH, room, ctx->num_cu);
+    if (split_rounds_us(tiles, K, behind, ctx->num_cu, 1.0) > 2.0 * split_rounds_us(tiles, K, whole, ctx->num_cu, 1.0)) return VDNN_OK;
     *taken = true;
     unsigned short* copy = (unsigned short*)(scratch + lead);
     ep.partial = (float*)(scratch + lead + copy_bytes);

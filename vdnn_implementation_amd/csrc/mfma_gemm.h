@@ -174,6 +174,16 @@ struct GemmDims {
 // worth; one more workgroup than that starts a nearly empty round. The estimate below counts, per
 // compute unit, rounds x (slices per split + a fixed prologue/epilogue) with the measured efficiency
 // of a round count, plus the traffic of writing and re-reading one partial result per split.
+// (the rounds of s splits, without the partial results' traffic)
+static inline double split_rounds_us(long tiles, long K, long s, int num_cu, double us_per_slice, long* splits = nullptr) {
+    long kchunk = (K + s - 1) / s;
+    kchunk = (kchunk + KB - 1) / KB * KB;
+    const long made = (K + kchunk - 1) / kchunk;
+    const long rounds = (tiles * made + num_cu - 1) / num_cu;
+    const double eff = rounds == 1 ? 0.72 : rounds == 2 ? 0.92 : rounds == 4 ? 0.93 : rounds % 3 == 0 ? 1.0 : 0.97;
+    if (splits) *splits = made;
+    return (double)rounds * (double)(kchunk / KB + 6) * us_per_slice / eff;
+}
 static inline int choose_splits(long tiles, long K, long max_splits, int num_cu, size_t out_bytes, double tile_flops_per_slice) {
     if (max_splits < 1) max_splits = 1;
     const long useful = 12l * num_cu / tiles + 1; // beyond twelve rounds the estimate only grows
@@ -183,12 +193,9 @@ static inline int choose_splits(long tiles, long K, long max_splits, int num_cu,
     double best = 0.0;
     int best_s = 1;
     for (long s = 1; s <= max_splits; s++) {
-        long kchunk = (K + s - 1) / s;
-        kchunk = (kchunk + KB - 1) / KB * KB;
-        const long splits = (K + kchunk - 1) / kchunk;
-        const long rounds = (tiles * splits + num_cu - 1) / num_cu;
-        const double eff = rounds == 1 ? 0.72 : rounds == 2 ? 0.92 : rounds == 4 ? 0.93 : rounds % 3 == 0 ? 1.0 : 0.97;
-        const double cost = (double)rounds * (double)(kchunk / KB + 6) * us_per_slice / eff + (splits > 1 ? (double)splits * us_per_split : 0.0);
+        long splits;
+        const double rounds_us = split_rounds_us(tiles, K, s, num_cu, us_per_slice, &splits);
+        const double cost = rounds_us + (splits > 1 ? (double)splits * us_per_split : 0.0);
         if (s == 1 || cost < best) { best = cost; best_s = (int)s; }
     }
     return best_s;
