@@ -168,13 +168,7 @@ struct GemmDims {
     unsigned* counters = nullptr; // the 64x64 tile: splits are added up by the workgroup that ends last (sum_splits), one counter a split tile
 };
 
-// Number of reduction splits for a grid of `tiles` output tiles over a reduction of K, at most
-// max_splits. Measured on the part: workgroups are resident three to a compute unit, so a grid runs
-// fastest when it is a little under a multiple of the unit count, best a multiple of three units'
-// worth; one more workgroup than that starts a nearly empty round. The estimate below counts, per
-// compute unit, rounds x (slices per split + a fixed prologue/epilogue) with the measured efficiency
-// of a round count, plus the traffic of writing and re-reading one partial result per split.
-// (the rounds of s splits, without the partial results' traffic)
+// The rounds' part of the estimate of choose_splits: s splits of a reduction of K for `tiles` output tiles; *splits: how many that makes.
 static inline double split_rounds_us(long tiles, long K, long s, int num_cu, double us_per_slice, long* splits = nullptr) {
     long kchunk = (K + s - 1) / s;
     kchunk = (kchunk + KB - 1) / KB * KB;
@@ -184,6 +178,13 @@ static inline double split_rounds_us(long tiles, long K, long s, int num_cu, dou
     if (splits) *splits = made;
     return (double)rounds * (double)(kchunk / KB + 6) * us_per_slice / eff;
 }
+
+// Number of reduction splits for a grid of `tiles` output tiles over a reduction of K, at most
+// max_splits. Measured on the part: workgroups are resident three to a compute unit, so a grid runs
+// fastest when it is a little under a multiple of the unit count, best a multiple of three units'
+// worth; one more workgroup than that starts a nearly empty round. The estimate below counts, per
+// compute unit, rounds x (slices per split + a fixed prologue/epilogue) with the measured efficiency
+// of a round count, plus the traffic of writing and re-reading one partial result per split.
 static inline int choose_splits(long tiles, long K, long max_splits, int num_cu, size_t out_bytes, double tile_flops_per_slice) {
     if (max_splits < 1) max_splits = 1;
     const long useful = 12l * num_cu / tiles + 1; // beyond twelve rounds the estimate only grows
@@ -515,7 +516,7 @@ __device__ __forceinline__ bool sum_splits(floatx16& acc, float* staging, const 
 // - AHEAD slices are on their way from memory (four, or one where there are few), so that a slice's values are there when they are
 //   written to LDS: operands that another kernel has just written 0.37 -> 0.33 us a slice. (0.21 are the matrix instructions; with
 //   one wavefront per SIMD the rest is the issue of some hundred instructions and the barrier.)
-// - What the result is combined with (bias, gate, old values) is read before the loop, and the epilogue branches on what is
+// - What the result is combined with (bias, gate, old values) is read before the loop (behind it in the instances that fill the chip), and the epilogue branches on what is
 //   uniform only, once per tile: 2.7 -> 0.9 us.
 // One call: forward 1 x 64 x 56 x 56, 128 of 3x3 17.7 -> 16.4 us; 49 x 38 x 8 x 8, 224 of 3x3 17.3 -> 14.1; fully connected 79 rows, 1473 -> 108, all
 // four passes 30.0 -> 23.6; backward 21 x 70 x 53 x 37, 130 of 3x3 at stride 2 108.9 -> 104.6.
